@@ -1,5 +1,4 @@
-// MFMA GEMM main loop shared by the TriMul kernels and the generic batched
-// GEMM (gfx950, 256 threads = 4 waves per workgroup).
+// MFMA GEMM main loop of the batched GEMM (gfx950, 256 threads = 4 waves per workgroup).
 //
 //   acc(m, n) = sum_{k in [kbeg, kend)} A(m, k) * B(n, k)
 //
@@ -20,9 +19,6 @@
 //      of k-row r stored at slot c ^ ((r & 3) << 1); fragments come from
 //      transposing LDS reads (ds_read_b64_tr_b16), so no transposed copy of
 //      the operand ever exists in memory.
-// A KC operand may gather its rows: row m of batch item m / nn is read from
-// physical row (m / nn) * nn + (p % n) * n + p / n, p = m % nn (the
-// transposed pair order of the incoming TriMul direction).
 #pragma once
 
 #include "common.hpp"
@@ -51,8 +47,6 @@ struct GemmOperand {
   const __bf16* p;  // element (0, 0) of this batch item
   int64_t ld;       // leading dimension in elements
   int rows;         // extent of the m (or n) dimension
-  int gather_n;     // KC row gather (0 = none); nn = gather_n^2
-  FastDiv div_n, div_nn;  // division by gather_n and gather_n^2 (gather only)
   int kmax = 0x7fffffff;  // MN: k rows that exist (rows past it read zeros)
 };
 
@@ -93,16 +87,7 @@ struct TileLoader {
       for (int t = 0; t < NI; ++t) {
         const int row = r0 + rpi * (NI * w + t) + rin;
         uint32_t off = kBufOOB;
-        if (row < op.rows) {
-          int64_t prow = row;
-          if (op.gather_n > 0) {
-            const uint32_t n = op.gather_n, nn = op.div_nn.d;
-            const uint32_t b = fdiv((uint32_t)row, op.div_nn), p = (uint32_t)row - b * nn;
-            const uint32_t i = fdiv(p, op.div_n), k = p - i * n;
-            prow = (int64_t)b * nn + (int64_t)k * n + i;
-          }
-          off = (uint32_t)(prow * op.ld * 2);
-        }
+        if (row < op.rows) off = (uint32_t)((int64_t)row * op.ld * 2);
         row_off[t] = off;
       }
     } else {

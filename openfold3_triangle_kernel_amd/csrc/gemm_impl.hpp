@@ -41,8 +41,8 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmArgs& g, int64_t T, cha
   const int m0 = mt * TM, n0 = nt * TM;
   const int kbeg = split * g.k_chunk;
   const int kend = min(g.K, kbeg + g.k_chunk);
-  GemmOperand A{g.A + (int64_t)z * g.a_bs, g.a_ld, g.M, g.a_gather_n, g.a_div_n, g.a_div_nn};
-  GemmOperand B{g.B + (int64_t)z * g.b_bs, g.b_ld, g.N, 0, {}, {}, g.b_kmax > 0 ? g.b_kmax : 0x7fffffff};
+  GemmOperand A{g.A + (int64_t)z * g.a_bs, g.a_ld, g.M};
+  GemmOperand B{g.B + (int64_t)z * g.b_bs, g.b_ld, g.b_rows > 0 ? g.b_rows : g.N, g.b_kmax > 0 ? g.b_kmax : 0x7fffffff};
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rl = lane & 31, hl = lane >> 5, wm = w >> 1, wn = w & 1;
   char* Cb = (char*)g.C + ((int64_t)z * g.c_bs + (int64_t)split * g.c_split) * (OUT_F32 ? 4 : 2);
@@ -150,12 +150,6 @@ static inline int gemm_prepare(GemmArgs& g, int a_kc, int b_kc, int out_f32, int
       (g.b_bs % 8))
     return set_error(TPF_ERR_SHAPE, "%s: GEMM operand pitch/padding/alignment requirement violated",
                      fn);
-  if (g.a_gather_n > 0 && !a_kc)
-    return set_error(TPF_ERR_ARG, "%s: row gather needs a K-contiguous A", fn);
-  if (g.a_gather_n > 0) {
-    g.a_div_n = make_fastdiv((uint32_t)g.a_gather_n);
-    g.a_div_nn = make_fastdiv((uint32_t)g.a_gather_n * (uint32_t)g.a_gather_n);
-  }
   // Buffer offsets of one batch item must stay below 2^31 bytes.
   const int64_t a_span = a_kc ? (int64_t)g.M * g.a_ld : (int64_t)g.K * g.a_ld;
   const int64_t b_span = b_kc ? (int64_t)g.N * g.b_ld : (int64_t)g.K * g.b_ld;

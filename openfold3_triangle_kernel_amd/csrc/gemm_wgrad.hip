@@ -1,5 +1,5 @@
 // Split-K weight-gradient products (MN-contiguous operands, f32 partials
-// folded in fixed order): the TriMul dW5 / dW_z pair and the pair-stack
+// folded in fixed order): the TriMul dW5 and the pair-stack
 // projection weight gradients.  Own translation unit for its stage shape:
 // 64-deep k-steps, two stages (measured best for these long-K, few-tile
 // products; the contraction shape in gemm.hip is 32 deep, three stages).
@@ -16,19 +16,6 @@ int gemm_launch_wgrad(const GemmArgs& g0, hipStream_t stream, const char* fn) {
   if (rc) return rc;
   dim3 grid((unsigned)((gemm_tiles(g) + 7) / 8 * 8));
   hipLaunchKernelGGL((gemm_bf16_kernel<false, false, true>), grid, dim3(256), 0, stream, g);
-  return check_launch(fn);
-}
-
-int gemm_launch_pair_wgrad(const GemmArgs& p0, const GemmArgs& p1, hipStream_t stream,
-                           const char* fn) {
-  GemmArgs g0 = p0, g1 = p1;
-  int rc = gemm_prepare(g0, 0, 0, 1, p0.batch > 0 ? p0.batch : 1, fn);
-  if (rc) return rc;
-  if ((rc = gemm_prepare(g1, 0, 0, 1, p1.batch > 0 ? p1.batch : 1, fn))) return rc;
-  const int64_t blocks = (gemm_tiles(g0) + 7) / 8 * 8 + (gemm_tiles(g1) + 7) / 8 * 8;
-  if (blocks > INT32_MAX) return set_error(TPF_ERR_SHAPE, "%s: GEMM grid too large", fn);
-  hipLaunchKernelGGL((gemm_bf16_pair_kernel<false, false, false, false, true>), dim3((unsigned)blocks),
-                     dim3(256), 0, stream, g0, g1);
   return check_launch(fn);
 }
 

@@ -15,10 +15,9 @@ struct GemmArgs {
   int M, N, K;
   int ksplit, k_chunk;                   // K range of split s: [s*k_chunk, (s+1)*k_chunk)
   float alpha;
-  int a_gather_n;                        // KC row gather of A (0 = none), see gemm_core.hpp
-  FastDiv a_div_n, a_div_nn;             // set by gemm_launch when a_gather_n > 0
   int batch;                             // set by gemm_launch
   int b_kmax;                            // MN B: k rows that exist (0 = all K)
+  int b_rows;                            // KC B: rows that exist (0 = all N; the rest read zeros)
 };
 
 // FP32 variant (gemm_core_f32.hpp); bias (nullable) is added per column n.
@@ -43,11 +42,9 @@ int gemm_launch(const GemmArgs& g, int a_kc, int b_kc, int out_f32, int batch,
 // operand layout; instantiated for the layout pairs TriMul uses.
 int gemm_launch_pair(const GemmArgs& g0, int a_kc0, int b_kc0, const GemmArgs& g1, int a_kc1,
                      int b_kc1, int out_f32, hipStream_t stream, const char* fn, int tm = 128);
-// Split-K weight-gradient products (both operands MN-contiguous, f32 output):
-// one problem, or two in one launch (gemm_wgrad.hip).
+// Split-K weight-gradient product (both operands MN-contiguous, f32 output;
+// gemm_wgrad.hip).
 int gemm_launch_wgrad(const GemmArgs& g, hipStream_t stream, const char* fn);
-int gemm_launch_pair_wgrad(const GemmArgs& g0, const GemmArgs& g1, hipStream_t stream,
-                           const char* fn);
 int gemm_f32_launch(const GemmArgsF32& g, int a_kc, int b_kc, int batch, hipStream_t stream,
                     const char* fn);
 int fold_launch(const float* part, float* out, int64_t n, int64_t stride, int splits,

@@ -1,6 +1,6 @@
-// Triangle multiplicative update (TriMul) on gfx950, built on the MFMA GEMM
-// main loop of gemm_core.hpp with the gating / LayerNorm work fused into
-// GEMM prologues and epilogues.
+// Triangle multiplicative update (TriMul) on gfx950: weight-stationary row
+// kernels that fuse the projections with the gating and LayerNorm work, and
+// the channel contractions on the batched MFMA GEMM.
 //
 // Stock math (openfold3/core/model/layers/triangular_multiplicative_update.py
 // :1263-1284 and :734-760; LayerNorm openfold3/core/model/primitives/
@@ -10,7 +10,7 @@
 //   out = (LN_out(x) Wz^T) * sigmoid(gl),  gl = zln Wg^T
 //
 // Storage (C == H channels, natural rows rho = (b*N + r)*N + s of z [B,N,N,C]):
-//   z, zln, gl, out, dz, dy: [R][C] bf16 row-major; xln [R][H];
+//   z, zln, gl, out, dz: [R][C] bf16 row-major; xln [R][H];
 //   dproj5 [R][5H] with column blocks [d a_p | d a_g | d b_p | d b_g | d gl]
 //   (the row order of W5 = [W_ap; W_ag; W_bp; W_bg; W_g]);
 //   a, b (and da, db): channel-major "stored" matrices A_c[i][k], B_c[j][k]
@@ -18,23 +18,19 @@
 //   zero): outgoing A_c[i][k] = a[i,k,c]; incoming A_c[i][k] = a[k,i,c], so
 //   both directions contract as the NT GEMM x_c = A_c B_c^T;
 //   x, dx: channel-major [B*H][N][Np] in natural (i, j) order.
-// The projection kernels walk rows in stored-matrix order m (position
-// p = m % NN of batch item m / NN): the natural row is m itself (outgoing) or
-// the transposed position (incoming), read through the GEMM's row gather.
+// The projection kernels walk plane positions in stored-matrix order: the
+// natural row of a position is the one it names (outgoing) or the transposed
+// one (incoming).
 //
 // Kernels of one direction:
 //   forward:  tm_ln_rows (LN_in) -> tm_in_proj_fwd (a, b, gl) -> GEMM x ->
 //             tm_ln_planes (LN_out) -> tm_out_proj<fwd> (out)
-//   backward: tm_out_proj<bwd> (dy, d gl) -> tm_ln_bwd<planes> (dx, LN_out
-//             partials) -> GEMMs da, db -> tm_in_proj_bwd (d a_p .. d b_g)
-//             -> tm_ln_bwd<rows> (dz, LN_in partials) -> split-K weight
-//             GEMMs -> fixed-order folds.
-// 32-deep k stages: every TriMul GEMM has K = C or 5H (small).
-#define TPF_GEMM_GK 32
+//   backward: tm_out_bwd (d gl, dx, LN_out and dWz partials) -> GEMMs da, db
+//             -> tm_in_proj_bwd (d a_p .. d b_g) -> tm_ln_in_bwd (dz, LN_in
+//             partials) -> split-K dW5 GEMM -> fixed-order folds.
 #include <type_traits>
 
 #include "common.hpp"
-#include "gemm_core.hpp"
 #include "tpf_gemm.hpp"
 #include "tpf_status.hpp"
 
@@ -45,14 +41,11 @@ struct TmGeom {
   int64_t NN;  // N*N positions per batch item
   int64_t PS;  // N*Np elements per channel-major plane
   int64_t R;   // B*N*N rows (< 2^30)
+  int64_t Rp;  // B*N*Np plane positions (R when N is a multiple of 8)
   int outgoing;
-  int ntg;     // gated 128-column weight tiles per branch (64 channels each)
-  FastDiv div_n, div_nn;
+  FastDiv div_np, div_ps;
 };
 
-constexpr int kSP = 136;  // bf16 pitch of 128-wide LDS staging tiles
-// LDS of a kernel = max(main loop ring, epilogue staging).
-// LDS of a kernel whose epilogue staging reuses its NS-stage GEMM ring.
 // Block walk of the persistent row kernels: a workgroup runs the virtual
 // blocks [bbeg, bend) and pb(blk) is the 32-row block a virtual block reads:
 // one contiguous range per workgroup, or (strided) blocks g, g + G, ... for
@@ -83,51 +76,47 @@ constexpr int kSP = 136;  // bf16 pitch of 128-wide LDS staging tiles
 // no bit of the results.
 inline int tm_contract_tile(int64_t N) { return N % 192 == 0 ? 192 : 128; }
 
-constexpr int lds_bytes(int epilogue, int ns = kGNS) {
-  return epilogue > gemm_ring_bytes(ns) ? epilogue : gemm_ring_bytes(ns);
+// The row kernels that touch channel-major planes walk plane positions
+// m = (b*N + r)*Np + s in blocks of 32 instead of rows: with Np a multiple of
+// 8, the eight positions of a 16-byte chunk always lie in one plane row, so
+// odd N streams the same 64-byte plane segments as an aligned N (at N = 1021
+// the forward projection took 748 us with two-byte plane stores in row order).
+// Positions s >= N have no row (PAD instances): their row operands read
+// zeros, their row stores are dropped and their plane stores write the
+// planes' zero pad columns.  PAD is false when Np == N, where a position is
+// its row.
+constexpr uint32_t kNoRow = 0xFFFFFFFFu;
+// Natural row of plane position m of planes in natural (i, j) order.
+template <bool PAD>
+__device__ __forceinline__ uint32_t tm_nat_row(const TmGeom& g, uint32_t m) {
+  if constexpr (!PAD) return m;
+  const uint32_t bi = fdiv(m, g.div_np), j = m - bi * (uint32_t)g.Np;
+  return j < (uint32_t)g.N ? bi * (uint32_t)g.N + j : kNoRow;
 }
-// Ring depths per kernel (measured): the short-K projections keep two
-// stages (occupancy), the long-K / large-epilogue kernels take more.
-constexpr int kInProjBwdNS = 3, kOutProjNS = 4;
-constexpr int kLnOutBwdNS = 2;
-constexpr int kInProjLds = lds_bytes((64 + 128) * kSP * 2, kInProjBwdNS);  // d tile + [dp | dg] tile
-constexpr int kOutProjLds = lds_bytes(2 * 128 * kSP * 2, kOutProjNS);  // gate + dout tiles
-constexpr int kLnOutBwdLds = lds_bytes(128 * kSP * 2, kLnOutBwdNS);  // x tile
-
-// Element offset of position p = i*N + j inside a channel-major plane.
-__device__ __forceinline__ int64_t tm_plane_off(const TmGeom& g, int64_t p) {
-  if (g.Np == g.N) return p;
-  const uint32_t i = fdiv((uint32_t)p, g.div_n);
-  return (int64_t)i * g.Np + ((uint32_t)p - i * (uint32_t)g.N);
+// Natural row of plane position m of the stored matrices (incoming: the
+// transposed position).
+template <bool PAD>
+__device__ __forceinline__ uint32_t tm_stored_row(const TmGeom& g, uint32_t m) {
+  if (g.outgoing) return tm_nat_row<PAD>(g, m);
+  const uint32_t b = fdiv(m, g.div_ps), p = m - b * (uint32_t)g.PS;
+  const uint32_t i = fdiv(p, g.div_np), k = p - i * (uint32_t)g.Np;
+  if (PAD && k >= (uint32_t)g.N) return kNoRow;
+  return b * (uint32_t)g.NN + k * (uint32_t)g.N + i;
 }
-// Batch item and position of row m.
-__device__ __forceinline__ void tm_bp(const TmGeom& g, int64_t m, int64_t& b, int64_t& p) {
-  const uint32_t bb = fdiv((uint32_t)m, g.div_nn);
-  b = bb;
-  p = (uint32_t)m - bb * (uint32_t)g.NN;
-}
-// Natural row of stored-order row m.
-__device__ __forceinline__ int64_t tm_phys_row(const TmGeom& g, int64_t m) {
-  if (g.outgoing) return m;
-  int64_t b, p;
-  tm_bp(g, m, b, p);
-  const uint32_t i = fdiv((uint32_t)p, g.div_n), k = (uint32_t)p - i * (uint32_t)g.N;
-  return b * g.NN + (int64_t)k * g.N + i;
+// Element offset of plane position m in channel plane c (plane tensors hold
+// fewer than 2^30 elements, checked by tm_geom).
+__device__ __forceinline__ uint32_t tm_plane_elem32(const TmGeom& g, uint32_t m, int c) {
+  const uint32_t b = fdiv(m, g.div_ps), p = m - b * (uint32_t)g.PS;
+  return (b * (uint32_t)g.H + (uint32_t)c) * (uint32_t)g.PS + p;
 }
 
 // ---------------------------------------------------------------------------
 // Weight packing (per call, tiny): the f32 module weights to bf16 GEMM
 // operands.
-//   Wp tile t < 2*ntg (branch t / ntg, channel block q = t % ntg): rows
-//   [p c0..c0+31 | g c0..c0+31 | p c0+32..c0+63 | g c0+32..c0+63], c0 = 64q,
-//   so the wave holding output columns 64wn.. sees p and g of the same 32
-//   channels in its two accumulator columns (the projection backward's B
-//   operand).
 //   W5 = [W_ap; W_ag; W_bp; W_bg; W_g] [5H][C] (the reference's d_w5 order;
-//   also the forward projections' stationary operand);
+//   the stationary operand of the input projections, both ways);
 //   Wz = W_z [C][H]; W5t = W5^T [C][5H] and Wzt = W_z^T [H][C] (stationary
-//   operands of the LN_in / LN_out backward kernels).  Missing channels are
-//   zero rows.
+//   operands of the LN_in / LN_out backward kernels).
 // ---------------------------------------------------------------------------
 struct TmWeights {
   const float* ap;
@@ -138,15 +127,13 @@ struct TmWeights {
   const float* z;
 };
 
-__global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w, __bf16* __restrict__ wp,
+__global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w,
                                                               __bf16* __restrict__ w5,
                                                               __bf16* __restrict__ wz,
                                                               __bf16* __restrict__ w5t,
-                                                              __bf16* __restrict__ wzt, int C,
-                                                              int ntg) {
+                                                              __bf16* __restrict__ wzt, int C) {
   const int cpr = C / 8;
-  const int wp_rows = 2 * ntg * 128;
-  const int64_t total = (int64_t)(wp_rows + 6 * C) * cpr;
+  const int64_t total = (int64_t)6 * C * cpr;
   const float* const mats[5] = {w.ap, w.ag, w.bp, w.bg, w.g};
   // W5^T [C][5C] (C x 5C / 8 chunks) and Wz^T [H][C] (H x C / 8 chunks)
   // after the row-copied part.
@@ -177,29 +164,19 @@ __global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w, __bf1
       continue;
     }
     const int row = (int)(idx / cpr), ch = (int)(idx % cpr);
-    const float* src = nullptr;
+    const float* src;
     __bf16* dst;
-    if (row < wp_rows) {
-      dst = wp + (int64_t)row * C + ch * 8;
-      const int t = row / 128, rr = row % 128;
-      const int br = t / ntg, q = t % ntg;
-      const int c = 64 * q + 32 * (rr / 64) + (rr & 31);
-      const bool isg = (rr >> 5) & 1;
-      if (c < C) src = (br ? (isg ? w.bg : w.bp) : (isg ? w.ag : w.ap)) + (int64_t)c * C;
-    } else if (row < wp_rows + 5 * C) {
-      const int j = row - wp_rows, blk = j / C, c = j % C;
-      dst = w5 + (int64_t)j * C + ch * 8;
-      src = mats[blk] + (int64_t)c * C;
+    if (row < 5 * C) {
+      dst = w5 + (int64_t)row * C + ch * 8;
+      src = mats[row / C] + (int64_t)(row % C) * C;
     } else {
-      const int c = row - wp_rows - 5 * C;
+      const int c = row - 5 * C;
       dst = wz + (int64_t)c * C + ch * 8;
       src = w.z + (int64_t)c * C;
     }
-    bf16x8 o = zero8();
-    if (src) {
+    bf16x8 o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = f2bf(src[ch * 8 + e]);
-    }
+    for (int e = 0; e < 8; ++e) o[e] = f2bf(src[ch * 8 + e]);
     st8(dst, o);
   }
 }
@@ -292,7 +269,8 @@ __global__ __launch_bounds__(256) void tm_ln_rows_kernel(const __bf16* __restric
 
 // ---------------------------------------------------------------------------
 // LN_out over the channels of the channel-major product x, written as
-// row-major xln.  Workgroup = 128 positions (natural order) x up to 128
+// row-major xln.  Workgroup = 128 plane positions (natural order; the pad
+// positions of N % 8 != 0 write nothing) x up to 128
 // channels; wave = (64-position half wv / 2) x (64-channel half wv % 2);
 // lane = (8-position group pg = lane % 8, 8-channel group lane / 8): it
 // reads its 8 channels' 16-byte position runs (128-byte runs per plane
@@ -309,8 +287,8 @@ __global__ __launch_bounds__(256) void tm_ln_rows_kernel(const __bf16* __restric
 // its next tile while it normalises the current one.  Tiles are independent,
 // so the results do not depend on the grid.
 constexpr int kLnPlanesWgsPerCu = 2;
-static inline int64_t tm_ln_planes_grid(int64_t NN, int64_t B) {
-  const int64_t nt = (NN + 127) / 128;
+static inline int64_t tm_ln_planes_grid(int64_t PS, int64_t B) {
+  const int64_t nt = (PS + 127) / 128;
   const int64_t cap = ((int64_t)device_cus() * kLnPlanesWgsPerCu + B - 1) / B;
   return nt < cap ? nt : cap;
 }
@@ -328,8 +306,7 @@ __global__ __launch_bounds__(256) void tm_ln_planes_kernel(const __bf16* __restr
   const int pg = lane & 7, cg = (lane >> 3) + 8 * (wv & 1);
   const int p0 = 64 * (wv >> 1) + pg * 8;  // first position in the tile
   const bool chan = cg * 8 < H;
-  const int64_t nt = (g.NN + T - 1) / T;
-  const bool vec = g.Np == g.N;
+  const int64_t nt = (g.PS + T - 1) / T;
   const int cgl = chan ? cg : 0;
   float wc[8], bc[8];
   {
@@ -343,22 +320,13 @@ __global__ __launch_bounds__(256) void tm_ln_planes_kernel(const __bf16* __restr
       bc[i] = b0[i]; bc[4 + i] = b1[i];
     }
   }
-  // v[c][e]: channel cg*8 + c, position pb + e of tile t.  Full tiles of
-  // unpadded planes load unconditionally, 16 bytes per channel.
+  // v[c][e]: channel cg*8 + c, position pb + e of tile t (16 bytes per
+  // channel; threads past the plane re-read its first positions).
   auto load = [&](int64_t t, bf16x8 (&v)[8]) {
     const int64_t pb = t * T + p0;
-    if (vec && pb + 8 <= g.NN) {
 #pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] = ld8(x + ((int64_t)b * H + cgl * 8 + c) * g.PS + pb);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const __bf16* plane = x + ((int64_t)b * H + cgl * 8 + c) * g.PS;
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          v[c][e] = pb + e < g.NN ? plane[tm_plane_off(g, pb + e)] : static_cast<__bf16>(0.f);
-      }
-    }
+    for (int c = 0; c < 8; ++c)
+      v[c] = ld8(x + ((int64_t)b * H + cgl * 8 + c) * g.PS + (pb < g.PS ? pb : 0));
   };
   // Sum over all channels of q[e] (this thread's 8 channels already summed);
   // the two sums of a tile use the two halves of `red`, so one barrier each.
@@ -384,6 +352,11 @@ __global__ __launch_bounds__(256) void tm_ln_planes_kernel(const __bf16* __restr
     for (int c = 0; c < 8; ++c) v[c] = chan ? nxt[c] : zero8();
     if (t + gridDim.x < nt) load(t + gridDim.x, nxt);
     const int64_t pb = t * T + p0;  // first position of this thread
+    // Its plane row, and how many of its eight positions have a row of xln.
+    const uint32_t pr = fdiv((uint32_t)pb, g.div_np);
+    const int col = (int)((uint32_t)pb - pr * (uint32_t)g.Np);
+    const int valid = pb < g.PS ? g.N - col : 0;
+    const int64_t row0 = (int64_t)b * g.NN + (int64_t)pr * g.N + col;
     float mean[8], rstd[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -415,142 +388,21 @@ __global__ __launch_bounds__(256) void tm_ln_planes_kernel(const __bf16* __restr
     if (chan) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        if (pb + e >= g.NN) continue;
+        if (e >= valid) continue;
         bf16x8 o;
 #pragma unroll
         for (int c = 0; c < 8; ++c) o[c] = f2bf((bf2f(v[c][e]) - mean[e]) * rstd[e] * wc[c] + bc[c]);
-        st8(xln + ((int64_t)b * g.NN + pb + e) * H + cg * 8, o);
+        st8(xln + (row0 + e) * H + cg * 8, o);
       }
     }
     if (cg == 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        if (pb + e < g.NN) {
-          mean_out[(int64_t)b * g.NN + pb + e] = mean[e];
-          rstd_out[(int64_t)b * g.NN + pb + e] = rstd[e];
+        if (e < valid) {
+          mean_out[row0 + e] = mean[e];
+          rstd_out[row0 + e] = rstd[e];
         }
     }
-  }
-}
-
-// Accumulator coordinates of this lane inside the 128 x 128 tile.
-struct AccPos {
-  int rl, hl, wm, wn;
-  __device__ __forceinline__ AccPos() {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    rl = lane & 31; hl = lane >> 5; wm = w >> 1; wn = w & 1;
-  }
-  __device__ __forceinline__ int row(int i, int r) const {
-    return 64 * wm + 32 * i + 8 * (r >> 2) + 4 * hl + (r & 3);
-  }
-  __device__ __forceinline__ int col(int j) const { return 64 * wn + 32 * j + rl; }
-};
-
-// Copy a [128 rows][ncols] bf16 LDS tile (pitch kSP) to rows rho_s[row] of a
-// row-major global matrix (pitch ld, column offset c0); rows < 0 skipped.
-__device__ __forceinline__ void tm_store_rows(const __bf16* S, int ncols, const int64_t* rho_s,
-                                              __bf16* __restrict__ dst, int64_t ld, int c0) {
-  const int cpr = ncols / 8;
-  for (int idx = threadIdx.x; idx < 128 * 16; idx += 256) {
-    const int row = idx >> 4, ch = idx & 15;
-    const int64_t rho = rho_s[row];
-    if (rho >= 0 && ch < cpr)
-      st8(dst + rho * ld + c0 + ch * 8, *reinterpret_cast<const bf16x8*>(&S[row * kSP + ch * 8]));
-  }
-}
-
-// Store an LDS tile S[c * kSP + pos] of [nch channels][128 positions] to
-// channel-major planes (plane b*H + c0 + c, position of tile row m0 + pos
-// within its batch item).
-__device__ __forceinline__ void tm_store_planes(const __bf16* S, int nch, __bf16* planes,
-                                                const TmGeom& g, int64_t m0, int c0) {
-  for (int idx = threadIdx.x; idx < nch * 16; idx += 256) {
-    const int cl = idx >> 4, chn = idx & 15;
-    const int c = c0 + cl;
-    if (c >= g.H) continue;
-    const int64_t mb = m0 + 8 * chn;
-    const __bf16* s = S + cl * kSP + 8 * chn;
-    if (g.Np == g.N && mb + 7 < g.R) {
-      // NN is a multiple of 64 here, so the 8 positions share a batch item.
-      int64_t b, p;
-          tm_bp(g, mb, b, p);
-      st8(planes + ((int64_t)b * g.H + c) * g.PS + p, *reinterpret_cast<const bf16x8*>(s));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int64_t m = mb + e;
-        if (m < g.R) {
-          int64_t b, p;
-          tm_bp(g, m, b, p);
-          planes[((int64_t)b * g.H + c) * g.PS + tm_plane_off(g, p)] = s[e];
-        }
-      }
-    }
-  }
-}
-
-// Register staging of an epilogue operand tile: fetched from HBM before the
-// GEMM main loop (so its latency overlaps the main loop) and written to LDS
-// after it.  Chunk k of thread t is tile chunk idx = t + 256 k.
-struct RegTile {
-  bf16x8 v[8];
-};
-// [128 rows][ncols] of a row-major matrix, natural rows m0 + row.
-__device__ __forceinline__ void fetch_rows(RegTile& t, const __bf16* __restrict__ src, int64_t ld,
-                                           int ncols, int64_t m0, int64_t R) {
-  const int cpr = ncols / 8;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = threadIdx.x + 256 * k;
-    const int row = idx >> 4, ch = idx & 15;
-    const int64_t m = m0 + row;
-    t.v[k] = (ch < cpr && m < R) ? ld8(src + m * ld + ch * 8) : zero8();
-  }
-}
-__device__ __forceinline__ void put_rows(__bf16* S, const RegTile& t) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = threadIdx.x + 256 * k;
-    *reinterpret_cast<bf16x8*>(&S[(idx >> 4) * kSP + (idx & 15) * 8]) = t.v[k];
-  }
-}
-// [nch channels][128 positions] of channel-major planes (channels c0 + c,
-// positions of tile rows m0 ..); nch * 16 <= 2048.
-__device__ __forceinline__ void fetch_planes(RegTile& t, const __bf16* __restrict__ planes,
-                                             const TmGeom& g, int nch, int64_t m0, int c0) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = threadIdx.x + 256 * k;
-    const int cl = idx >> 4, chn = idx & 15;
-    const int c = c0 + cl;
-    const int64_t mb = m0 + 8 * chn;
-    bf16x8 v = zero8();
-    if (cl < nch && c < g.H) {
-      if (g.Np == g.N && mb + 7 < g.R) {
-        int64_t b, p;
-          tm_bp(g, mb, b, p);
-        v = ld8(planes + ((int64_t)b * g.H + c) * g.PS + p);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t m = mb + e;
-          if (m < g.R) {
-            int64_t b, p;
-          tm_bp(g, m, b, p);
-            v[e] = planes[((int64_t)b * g.H + c) * g.PS + tm_plane_off(g, p)];
-          }
-        }
-      }
-    }
-    t.v[k] = v;
-  }
-}
-__device__ __forceinline__ void put_planes(__bf16* S, const RegTile& t, int nch) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = threadIdx.x + 256 * k;
-    const int cl = idx >> 4, chn = idx & 15;
-    if (cl < nch) *reinterpret_cast<bf16x8*>(&S[cl * kSP + 8 * chn]) = t.v[k];
   }
 }
 
@@ -558,8 +410,8 @@ __device__ __forceinline__ void put_planes(__bf16* S, const RegTile& t, int nch)
 // Forward input projections, weight-stationary.  One wave per 16 channels
 // (C / 16 waves) holds the bf16 rows of W_ap, W_ag, W_bp, W_bg and W_g for
 // its channels in registers (the B operands of v_mfma_f32_16x16x32_bf16) for
-// the whole kernel; workgroups are persistent and walk 32-row blocks of zln
-// in stored row order.
+// the whole kernel; workgroups are persistent and walk blocks of 32 stored
+// positions.
 //   * loads: the first half of the waves stream each block's rows straight
 //     into a 4-deep LDS ring (buffer_load ... lds, three blocks ahead; the
 //     chunk order within a row is rotated by the row so the A-fragment
@@ -628,15 +480,14 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_fwd_kernel(
       const int ci = (2 * w + j) * 64 + lane;
       const int r = ci / CPR, slot = ci % CPR;
       const int gc = (slot - r % CPR + CPR) % CPR;
-      const int64_t m = pb(blk) * 32 + r;
-      const bool ok = blk < bend && m < g.R;
-      const uint32_t off = ok ? (uint32_t)((tm_phys_row(g, m) * C + 8 * gc) * 2) : kBufOOB;
-      buf2lds16(rs_z, off, &As[stage][(2 * w + j) * 512]);
+      const uint32_t m = (uint32_t)pb(blk) * 32 + r;
+      const uint32_t row = blk < bend && m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+      buf2lds16(rs_z, row != kNoRow ? (row * C + 8 * gc) * 2 : kBufOOB, &As[stage][(2 * w + j) * 512]);
     }
     if (w == 0) {
-      const int64_t m = pb(blk) * 32 + lane;
-      const bool ok = lane < 32 && blk < bend && m < g.R;
-      buf2lds4(rs_m, ok ? (uint32_t)(tm_phys_row(g, m) * 4) : kBufOOB, &Ms[stage][0]);
+      const uint32_t m = (uint32_t)pb(blk) * 32 + lane;
+      const uint32_t row = lane < 32 && blk < bend && m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+      buf2lds4(rs_m, row != kNoRow ? row * 4 : kBufOOB, &Ms[stage][0]);
     }
   };
   auto mma = [&](int64_t blk, f32x4 (&acc)[5][2]) {
@@ -684,7 +535,7 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_fwd_kernel(
     const int sb = (int)(blk & 1);
     const __bf16* G = Sg[sb];
     const int st = tid - 2 * C;
-    const int64_t mb0 = pb(blk) * 32;
+    const uint32_t mb0 = (uint32_t)pb(blk) * 32;
     bf16x8 v[6];
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
@@ -702,33 +553,18 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_fwd_kernel(
       const int q = st + 2 * C * it;       // < 8C: a then b, (channel, 8-position part)
       const int t = it >> 1;
       const int c = (q - 4 * C * t) >> 2, part = q & 3;
-      const int64_t mb = mb0 + 8 * part;
-      if (!PAD) {
-        // N % 8 == 0: the 8 positions are contiguous in one plane row.
-        int64_t bb, pp;
-        tm_bp(g, mb < g.R ? mb : 0, bb, pp);
-        const uint32_t off = mb < g.R ? (uint32_t)((((int64_t)bb * g.H + c) * g.PS + pp) * 2) : kBufOOB;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), t ? rs_b : rs_a, off, 0, 0);
-      } else {
-        __bf16* planes = t ? b_pl : a_pl;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t m = mb + e;
-          if (m < g.R) {
-            int64_t bb, pp;
-            tm_bp(g, m, bb, pp);
-            planes[((int64_t)bb * g.H + c) * g.PS + tm_plane_off(g, pp)] = v[it][e];
-          }
-        }
-      }
+      const uint32_t mb = mb0 + 8 * part;
+      const uint32_t off = mb < (uint32_t)g.Rp ? tm_plane_elem32(g, mb, c) * 2 : kBufOOB;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), t ? rs_b : rs_a, off, 0, 0);
     }
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int q = st + 2 * C * it;       // < 4C: (row, chunk)
       const int row = q / CPR, c8 = q % CPR;
-      const int64_t m = mb0 + row;
-      const uint32_t off = m < g.R ? (uint32_t)((tm_phys_row(g, m) * C + 8 * c8) * 2) : kBufOOB;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[4 + it]), rs_g, off, 0, 0);
+      const uint32_t m = mb0 + row;
+      const uint32_t r = m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[4 + it]), rs_g,
+                                             r != kNoRow ? (r * C + 8 * c8) * 2 : kBufOOB, 0, 0);
     }
   };
   // Pipeline: iteration blk issues the loads of blk + 3, multiplies blk + 1
@@ -774,7 +610,7 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Input projections, backward, weight-stationary (N % 8 == 0).  The same
+// Input projections, backward, weight-stationary.  The same
 // persistent walk over 32-row blocks as the forward, with W_ap, W_ag, W_bp,
 // W_bg rows of the wave's 16 channels in registers as the A operand, so the
 // accumulators come out transposed (register r of lane l: channel
@@ -787,22 +623,8 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_fwd_kernel(
 // LDS staging tile [32 rows][4C] and are stored as 8C-byte row segments of
 // dproj5 by the storing waves.  Two barriers per block (staging reuse).
 // ---------------------------------------------------------------------------
-// 32-bit forms of the row / plane index helpers (R < 2^30 rows and plane
-// tensors below 2^30 elements, both checked by tm_geom).
-__device__ __forceinline__ uint32_t tm_phys_row32(const TmGeom& g, uint32_t m) {
-  if (g.outgoing) return m;
-  const uint32_t b = fdiv(m, g.div_nn), p = m - b * (uint32_t)g.NN;
-  const uint32_t i = fdiv(p, g.div_n), k = p - i * (uint32_t)g.N;
-  return b * (uint32_t)g.NN + k * (uint32_t)g.N + i;
-}
-// Element offset of stored row m in channel plane c (N % 8 == 0: Np == N).
-__device__ __forceinline__ uint32_t tm_plane_elem32(const TmGeom& g, uint32_t m, int c) {
-  const uint32_t b = fdiv(m, g.div_nn), p = m - b * (uint32_t)g.NN;
-  return (b * (uint32_t)g.H + (uint32_t)c) * (uint32_t)g.PS + p;
-}
-
 constexpr int kInBwdDepth = 4;
-template <int C>
+template <int C, bool PAD>
 __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
     const __bf16* __restrict__ zln, const __bf16* __restrict__ w5, const float* __restrict__ mask,
     const __bf16* __restrict__ da, const __bf16* __restrict__ db, __bf16* __restrict__ dproj5,
@@ -843,9 +665,8 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
       const int r = ci / CPR, slot = ci % CPR;
       const int gc = (slot - r % CPR + CPR) % CPR;
       const uint32_t m = (uint32_t)pb(blk) * 32 + r;
-      const bool ok = blk < bend && m < (uint32_t)g.R;
-      const uint32_t off = ok ? (tm_phys_row32(g, m) * C + 8 * gc) * 2 : kBufOOB;
-      buf2lds16(rs_z, off, &As[stage][(2 * w + j) * 512]);
+      const uint32_t row = blk < bend && m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+      buf2lds16(rs_z, row != kNoRow ? (row * C + 8 * gc) * 2 : kBufOOB, &As[stage][(2 * w + j) * 512]);
     }
     // Plane chunks gi = (4 w + j) * 64 + lane over [t][channel][4 parts].
 #pragma unroll
@@ -854,7 +675,7 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
       const int t = (4 * w + j) * 64 / (4 * C), rem = gi - t * 4 * C;  // t wave-uniform
       const int c = rem >> 2, part = rem & 3;
       const uint32_t mb = (uint32_t)pb(blk) * 32 + 8 * part;
-      const bool ok = blk < bend && mb < (uint32_t)g.R;
+      const bool ok = blk < bend && mb < (uint32_t)g.Rp;
       const uint32_t off = ok ? tm_plane_elem32(g, mb, c) * 2 : kBufOOB;
       // The first 4C chunks are da, the rest db (each wave's 4 instructions
       // stay within one tensor: 4C is a multiple of 256).
@@ -862,8 +683,8 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
     }
     if (w == 0) {
       const uint32_t m = (uint32_t)pb(blk) * 32 + lane;
-      const bool ok = lane < 32 && blk < bend && m < (uint32_t)g.R;
-      buf2lds4(rs_m, ok ? tm_phys_row32(g, m) * 4 : kBufOOB, &Ms[stage][0]);
+      const uint32_t row = lane < 32 && blk < bend && m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+      buf2lds4(rs_m, row != kNoRow ? row * 4 : kBufOOB, &Ms[stage][0]);
     }
   };
   auto mma = [&](int64_t blk, f32x4 (&acc)[4][2]) {
@@ -927,8 +748,9 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
       for (int it = 0; it < 4; ++it) {
         const int q = st + 2 * C * (4 * h + it), row = q / (C / 2), k = q % (C / 2);
         const uint32_t m = (uint32_t)mb0 + row;
-        const uint32_t off = m < (uint32_t)g.R ? (tm_phys_row32(g, m) * 5 * C + 8 * k) * 2 : kBufOOB;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), rs_o, off, 0, 0);
+        const uint32_t r = m < (uint32_t)g.Rp ? tm_stored_row<PAD>(g, m) : kNoRow;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), rs_o,
+                                               r != kNoRow ? (r * 5 * C + 8 * k) * 2 : kBufOOB, 0, 0);
       }
     }
   };
@@ -963,140 +785,6 @@ __global__ __launch_bounds__(4 * C) void tm_in_proj_bwd_ws_kernel(
   // The ring loads issued past the last block still write LDS: let them land
   // before the workgroup releases its LDS.
   if (loader) wait_vmcnt<0>();
-}
-
-// ---------------------------------------------------------------------------
-// Input projections, backward (stored row order): recompute p, g for 64
-// channels of branch a or b and write d p = d * mask * s(g),
-// d g = d * mask * p * s(g) (1 - s(g)) into dproj5, d = da / db.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 2) void tm_in_proj_bwd_kernel(
-    const __bf16* __restrict__ zln, const __bf16* __restrict__ wp, const float* __restrict__ mask,
-    const __bf16* __restrict__ a_pl, const __bf16* __restrict__ b_pl,
-    __bf16* __restrict__ dproj5, TmGeom g, int C) {
-  __shared__ __attribute__((aligned(1024))) char smem[kInProjLds];
-  __shared__ float mask_s[128];
-  __shared__ int64_t rho_s[128];
-  const int H = g.H;
-  const int tn = 2 * g.ntg;
-  const int64_t tm = (g.R + 127) / 128;
-  const int64_t T = xcd_order(tm * tn);
-  if (T < 0) return;
-  const int nt = (int)(T % tn);
-  const int64_t m0 = (T / tn) * 128;
-  if (threadIdx.x < 128) {
-    const int64_t m = m0 + threadIdx.x;
-    const int64_t rho = m < g.R ? tm_phys_row(g, m) : -1;
-    rho_s[threadIdx.x] = rho;
-    mask_s[threadIdx.x] = rho >= 0 ? mask[rho] : 0.f;
-  }
-  GemmOperand A{zln, C, (int)g.R, g.outgoing ? 0 : g.N, g.div_n, g.div_nn};
-  GemmOperand W{wp, C, 2 * g.ntg * 128, 0, {}, {}};
-  RegTile dreg;
-  fetch_planes(dreg, (nt / g.ntg) ? b_pl : a_pl, g, 64, m0, 64 * (nt % g.ntg));
-  f32x16 acc[2][2];
-  gemm_tile<true, true, kInProjBwdNS>(A, W, (int)m0, nt * 128, 0, C, smem, acc);
-  const AccPos ap;
-  __bf16* S0 = reinterpret_cast<__bf16*>(smem);
-  const int br = nt / g.ntg, q = nt % g.ntg;
-  const int cl = 32 * ap.wn + ap.rl;  // channel 64q + cl
-  // Backward: d tile [64 ch][128 pos] in S0, outputs [128 rows][dp 64 | dg 64] in So.
-  __bf16* So = S0 + 64 * kSP;
-  put_planes(S0, dreg, 64);
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = ap.row(i, r);
-      const float d = bf2f(S0[cl * kSP + row]) * mask_s[row];
-      const float p = acc[i][0][r];
-      const float s = sigmoidf(acc[i][1][r]);
-      So[row * kSP + cl] = f2bf(d * s);
-      So[row * kSP + 64 + cl] = f2bf(d * p * s * (1.f - s));
-    }
-  __syncthreads();
-  const int nvalid = min(64, H - 64 * q) / 8;  // 8-channel chunks inside H
-  for (int idx = threadIdx.x; idx < 128 * 16; idx += 256) {
-    const int row = idx >> 4, k = idx & 15, isg = k >> 3, c8 = k & 7;
-    const int64_t rho = rho_s[row];
-    if (rho < 0 || c8 >= nvalid) continue;
-    const int col = (2 * br + isg) * H + 64 * q + 8 * c8;
-    st8(dproj5 + rho * 5 * H + col, *reinterpret_cast<const bf16x8*>(&So[row * kSP + isg * 64 + 8 * c8]));
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Output projection backward, tile GEMM (N % 8 != 0; otherwise the fused
-// tm_out_bwd_ws_kernel runs): y = xln Wz^T recomputed (natural rows),
-// dy = dout s(gl) (row-major) and d gl = dout y s(gl) (1 - s(gl)) into the
-// last block of dproj5.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 2) void tm_out_proj_bwd_kernel(
-    const __bf16* __restrict__ xln, const __bf16* __restrict__ p_out,
-    const __bf16* __restrict__ gl, const __bf16* __restrict__ dout,
-    __bf16* __restrict__ dy, __bf16* __restrict__ dproj5, TmGeom g, int C) {
-  constexpr int kStage = 128 * kSP * 2;
-  __shared__ __attribute__((aligned(1024))) char smem[kOutProjLds];
-  __shared__ int64_t rho_s[128];
-  const int H = g.H;
-  const int64_t T = xcd_order((g.R + 127) / 128);
-  if (T < 0) return;
-  const int64_t m0 = T * 128;
-  if (threadIdx.x < 128) rho_s[threadIdx.x] = m0 + threadIdx.x < g.R ? m0 + threadIdx.x : -1;
-  GemmOperand A{xln, H, (int)g.R, 0, {}, {}};
-  GemmOperand W{p_out, H, C, 0, {}, {}};
-  RegTile greg, dreg;
-  fetch_rows(greg, gl, C, C, m0, g.R);
-  fetch_rows(dreg, dout, C, C, m0, g.R);
-  f32x16 acc[2][2];
-  gemm_tile<true, true, kOutProjNS>(A, W, (int)m0, 0, 0, H, smem, acc);
-  const AccPos ap;
-  __bf16* Sg = reinterpret_cast<__bf16*>(smem);
-  __bf16* Sd = reinterpret_cast<__bf16*>(smem + kStage);
-  put_rows(Sg, greg);
-  put_rows(Sd, dreg);
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = ap.col(j);
-      if (col >= C) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int o = ap.row(i, r) * kSP + col;
-        const float s = sigmoidf(bf2f(Sg[o]));
-        const float y = acc[i][j][r];
-        const float go = bf2f(Sd[o]);
-        Sd[o] = f2bf(go * s);
-        Sg[o] = f2bf(go * y * s * (1.f - s));
-      }
-    }
-  __syncthreads();
-  tm_store_rows(Sd, C, rho_s, dy, C, 0);
-  tm_store_rows(Sg, C, rho_s, dproj5, 5 * H, 4 * H);
-}
-
-// ---------------------------------------------------------------------------
-// LN_out backward fused onto the GEMM that produces its input gradient
-// (natural rows): G = dy Wz (A = dy [R][C], B = Wz read MN), x from the
-// channel-major planes, dx written to planes;
-//   g = G * gamma;  dx = rstd (g - mean(g) - xhat mean(g xhat));
-//   per-tile partials d gamma = sum G xhat, d beta = sum G into
-//   lnp[tile][2][W] (W channels).
-// The epilogue works on the accumulators in registers: the x tile sits in
-// LDS as [channel][row], so 8-byte reads give each lane the 4 consecutive
-// rows of one accumulator column; row sums are reduced across the 32 columns of
-// a wave with a transposing butterfly and across the two column waves in
-// LDS, column sums across the two row halves with a lane swap and across
-// the row waves in LDS.  All reductions run in a fixed order.
-// ---------------------------------------------------------------------------
-
-// x values of acc[i][j] rows 4*rq .. 4*rq+3 (of this lane's 16 registers).
-__device__ __forceinline__ bf16x4 tm_x4(const __bf16* Xt, const AccPos& ap, int i, int j, int rq) {
-  const int row = 64 * ap.wm + 32 * i + 8 * rq + 4 * ap.hl;
-  return *reinterpret_cast<const bf16x4*>(Xt + ap.col(j) * kSP + row);
 }
 
 // One level of the transposing butterfly: lanes exchange half of their
@@ -1137,126 +825,6 @@ __device__ __forceinline__ void wave_row_sums(const float* P, int r0, int lane, 
   }
   s0 = q ? o : r;
   s1 = q ? r : o;
-}
-
-__global__ __launch_bounds__(256, 2) void tm_ln_out_bwd_kernel(
-    const __bf16* __restrict__ a_op, int64_t a_ld, const __bf16* __restrict__ w_op, int K,
-    const __bf16* __restrict__ xsrc, const float* __restrict__ mean, const float* __restrict__ rstd,
-    const float* __restrict__ gamma, __bf16* __restrict__ dst, float* __restrict__ lnp,
-    TmGeom g, int W) {
-  __shared__ __attribute__((aligned(1024))) char smem[kLnOutBwdLds];
-  __shared__ __attribute__((aligned(16))) float mean_s[128], rstd_s[128];
-  __shared__ __attribute__((aligned(16))) float rsum[2][2][128];  // [quantity][wn][row]
-  __shared__ float csum[2][2][128];                               // [quantity][wm][col]
-  const int tid = threadIdx.x;
-  const int64_t T = xcd_order((g.R + 127) / 128);
-  if (T < 0) return;
-  const int64_t m0 = T * 128;
-  if (tid < 128) {
-    const int64_t m = m0 + tid;
-    const bool ok = m < g.R;
-    mean_s[tid] = ok ? mean[m] : 0.f;
-    rstd_s[tid] = ok ? rstd[m] : 0.f;
-  }
-  GemmOperand A{a_op, a_ld, (int)g.R, 0, {}, {}};
-  GemmOperand B{w_op, W, W, 0, {}, {}};
-  RegTile xreg;
-  fetch_planes(xreg, xsrc, g, 128, m0, 0);
-  f32x16 acc[2][2];
-  gemm_tile<true, false, kLnOutBwdNS>(A, B, (int)m0, 0, 0, K, smem, acc);
-  __bf16* Xt = reinterpret_cast<__bf16*>(smem);  // [ch][row]
-  put_planes(Xt, xreg, 128);
-  __syncthreads();
-  const AccPos ap;
-  const int lane = tid & 63;
-  float gam[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) gam[j] = ap.col(j) < W ? gamma[ap.col(j)] : 0.f;
-  // Pass 1: per-row partial sums over this lane's two columns, per-column
-  // partial sums over this lane's 32 rows.
-  float rs_g[32], rs_gx[32];
-  float cs_g[2] = {0.f, 0.f}, cs_gx[2] = {0.f, 0.f};
-#pragma unroll
-  for (int t = 0; t < 32; ++t) { rs_g[t] = 0.f; rs_gx[t] = 0.f; }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int rq = 0; rq < 4; ++rq) {
-      const int row0 = 64 * ap.wm + 32 * i + 8 * rq + 4 * ap.hl;
-      const f32x4 mu = *reinterpret_cast<const f32x4*>(&mean_s[row0]);
-      const f32x4 rs = *reinterpret_cast<const f32x4*>(&rstd_s[row0]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const bf16x4 xv = tm_x4(Xt, ap, i, j, rq);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = 4 * rq + e;
-          const float G = acc[i][j][r];
-          const float xh = (bf2f(xv[e]) - mu[e]) * rs[e];
-          const float gv = G * gam[j];
-          rs_g[16 * i + r] += gv;
-          rs_gx[16 * i + r] = fmaf(gv, xh, rs_gx[16 * i + r]);
-          cs_g[j] += G;
-          cs_gx[j] = fmaf(G, xh, cs_gx[j]);
-        }
-      }
-    }
-  // Transposing butterfly over the 32 columns of the wave: lane rl ends with
-  // the full sums of value index t = rl.
-  tm_butterfly<16>(rs_g, rs_gx, lane);
-  tm_butterfly<8>(rs_g, rs_gx, lane);
-  tm_butterfly<4>(rs_g, rs_gx, lane);
-  tm_butterfly<2>(rs_g, rs_gx, lane);
-  tm_butterfly<1>(rs_g, rs_gx, lane);
-  {
-    const int t = ap.rl, i = t >> 4, r = t & 15;
-    const int row = ap.row(i, r);
-    rsum[0][ap.wn][row] = rs_g[0];
-    rsum[1][ap.wn][row] = rs_gx[0];
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const float a0 = xor32_sum(cs_g[j]), a1 = xor32_sum(cs_gx[j]);
-    if (ap.hl == 0) {
-      csum[0][ap.wm][ap.col(j)] = a0;
-      csum[1][ap.wm][ap.col(j)] = a1;
-    }
-  }
-  __syncthreads();
-  if (tid < W) {
-    float* part = lnp + T * 2 * W;
-    part[tid] = csum[1][0][tid] + csum[1][1][tid];
-    part[W + tid] = csum[0][0][tid] + csum[0][1][tid];
-  }
-  // Pass 2: dx in place of x (each element is read and written by one lane).
-  const float invW = 1.f / W;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int rq = 0; rq < 4; ++rq) {
-      const int row0 = 64 * ap.wm + 32 * i + 8 * rq + 4 * ap.hl;
-      const f32x4 mu = *reinterpret_cast<const f32x4*>(&mean_s[row0]);
-      const f32x4 rs = *reinterpret_cast<const f32x4*>(&rstd_s[row0]);
-      const f32x4 sg0 = *reinterpret_cast<const f32x4*>(&rsum[0][0][row0]);
-      const f32x4 sg1 = *reinterpret_cast<const f32x4*>(&rsum[0][1][row0]);
-      const f32x4 sx0 = *reinterpret_cast<const f32x4*>(&rsum[1][0][row0]);
-      const f32x4 sx1 = *reinterpret_cast<const f32x4*>(&rsum[1][1][row0]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const bf16x4 xv = tm_x4(Xt, ap, i, j, rq);
-        bf16x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float mg = (sg0[e] + sg1[e]) * invW, mgx = (sx0[e] + sx1[e]) * invW;
-          const float xh = (bf2f(xv[e]) - mu[e]) * rs[e];
-          const float gv = acc[i][j][4 * rq + e] * gam[j];
-          o[e] = f2bf(rs[e] * (gv - mg - xh * mgx));
-        }
-        *reinterpret_cast<bf16x4*>(Xt + ap.col(j) * kSP + row0) = o;
-      }
-    }
-  __syncthreads();
-  tm_store_planes(Xt, 128, dst, g, m0, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1504,7 +1072,7 @@ __global__ __launch_bounds__(4 * C) void tm_ln_in_bwd_ws_kernel(
 
 // ---------------------------------------------------------------------------
 // Output projection backward and LN_out backward in one persistent,
-// weight-stationary kernel (N % 8 == 0), per 32-row block of natural rows:
+// weight-stationary kernel, per block of 32 plane positions in natural order:
 //   y = xln Wz^T (recomputed), s = s(gl):  dy = dout s,  d gl = dout y s (1 - s);
 //   G = dy Wz, then the LN_out backward of x (planes) into dx (planes).
 // Wave w owns channels 16 w .. 16 w + 15 of both products: its rows of Wz
@@ -1524,7 +1092,7 @@ __global__ __launch_bounds__(4 * C) void tm_ln_in_bwd_ws_kernel(
 // all of a workgroup's blocks and go to lnp [workgroup][2][C].
 // ---------------------------------------------------------------------------
 constexpr int kOutBwdDepth = 3;
-template <int C>
+template <int C, bool PAD>
 __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
     const __bf16* __restrict__ xln, const __bf16* __restrict__ wz, const __bf16* __restrict__ wzt,
     const __bf16* __restrict__ gl, const __bf16* __restrict__ dout, const __bf16* __restrict__ x,
@@ -1578,22 +1146,23 @@ __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
         const int r = ci / CPR, slot = ci % CPR;
         const int gc = (slot - r % CPR + CPR) % CPR;
         const uint32_t m = (uint32_t)pb(blk) * 32 + r;
-        const bool ok = blk < bend && m < (uint32_t)g.R;
-        buf2lds16(rs_in[t], ok ? (m * C + 8 * gc) * 2 : kBufOOB, &Rg[stage][t][(2 * w + j) * 512]);
+        const uint32_t row = blk < bend && m < (uint32_t)g.Rp ? tm_nat_row<PAD>(g, m) : kNoRow;
+        buf2lds16(rs_in[t], row != kNoRow ? (row * C + 8 * gc) * 2 : kBufOOB,
+                  &Rg[stage][t][(2 * w + j) * 512]);
       }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int ci = (2 * w + j) * 64 + lane;  // (channel ci / 4, 8-position part ci % 4)
       const int c = ci >> 2, part = ci & 3;
       const uint32_t mb = (uint32_t)pb(blk) * 32 + 8 * part;
-      const bool ok = blk < bend && mb < (uint32_t)g.R;
+      const bool ok = blk < bend && mb < (uint32_t)g.Rp;
       buf2lds16(rs_x, ok ? tm_plane_elem32(g, mb, c) * 2 : kBufOOB, &Rg[stage][3][(2 * w + j) * 512]);
     }
     if (w == 0) {
       const uint32_t m = (uint32_t)pb(blk) * 32 + lane;
-      const bool ok = lane < 32 && blk < bend && m < (uint32_t)g.R;
-      buf2lds4(rs_mu, ok ? m * 4 : kBufOOB, &Ss[stage][0][0]);
-      buf2lds4(rs_rs, ok ? m * 4 : kBufOOB, &Ss[stage][1][0]);
+      const uint32_t row = lane < 32 && blk < bend && m < (uint32_t)g.Rp ? tm_nat_row<PAD>(g, m) : kNoRow;
+      buf2lds4(rs_mu, row != kNoRow ? row * 4 : kBufOOB, &Ss[stage][0][0]);
+      buf2lds4(rs_rs, row != kNoRow ? row * 4 : kBufOOB, &Ss[stage][1][0]);
     }
   };
 
@@ -1687,6 +1256,10 @@ __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         xh[rt][e] = (bf2f(xv[e]) - mu[e]) * rsd[e];
+        // rstd reads 0 at positions without a row, whose x is not defined:
+        // their dx (the zero pad the contraction reads) and their share of
+        // the column sums stay 0 whatever is stored there.
+        if (PAD && rsd[e] == 0.f) xh[rt][e] = 0.f;
         const float G = acc[rt][e];
         gv[rt][e] = G * gam;
         a[4 * rt + e] = gv[rt][e];
@@ -1735,13 +1308,13 @@ __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
       for (int it = 0; it < 2; ++it) {
         const int q = st + 2 * C * it, row = q / CPR, k = q % CPR;
         const uint32_t m = (uint32_t)pb(blk) * 32 + row;
-        const bool ok = m < (uint32_t)g.R;
+        const uint32_t r = m < (uint32_t)g.Rp ? tm_nat_row<PAD>(g, m) : kNoRow;
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[2 + it]), rs_dp,
-                                               ok ? (m * 5 * C + 4 * C + 8 * k) * 2 : kBufOOB, 0, 0);
+                                               r != kNoRow ? (r * 5 * C + 4 * C + 8 * k) * 2 : kBufOOB, 0, 0);
         const uint32_t mb = (uint32_t)pb(blk) * 32 + 8 * (q & 3);
         __builtin_amdgcn_raw_buffer_store_b128(
             __builtin_bit_cast(u32x4, v[4 + it]), rs_dx,
-            mb < (uint32_t)g.R ? tm_plane_elem32(g, mb, q >> 2) * 2 : kBufOOB, 0, 0);
+            mb < (uint32_t)g.Rp ? tm_plane_elem32(g, mb, q >> 2) * 2 : kBufOOB, 0, 0);
       }
     }
   }
@@ -1762,8 +1335,7 @@ __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Output projection forward, weight-stationary (N % 8 == 0 not required:
-// rows are natural, row-major): out = (xln Wz^T) s(gl), persistent
+// Output projection forward, weight-stationary (natural rows): out = (xln Wz^T) s(gl), persistent
 // workgroups of C / 16 waves over 32-row blocks.  Wave w holds the Wz rows of
 // channels 16 w .. 16 w + 15 (B operands of v_mfma_f32_16x16x32_bf16); the
 // loading waves stream xln and gl rows (chunk-rotated) into a 4-deep LDS
@@ -1867,21 +1439,6 @@ __global__ __launch_bounds__(4 * C) void tm_out_proj_fwd_ws_kernel(
   if (loader) wait_vmcnt<0>();
 }
 
-// Zero-fill (used instead of hipMemsetAsync so callers may capture graphs).
-__global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    p[i] = 0u;
-}
-
-static int zero_fill(void* p, int64_t bytes, hipStream_t s, const char* fn) {
-  const int64_t n = bytes / 4;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 8192) blocks = 8192;
-  if (blocks < 1) return TPF_OK;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (uint32_t*)p, n);
-  return check_launch(fn);
-}
-
 }  // namespace tpf
 
 // ---------------------------------------------------------------------------
@@ -1916,22 +1473,19 @@ static int tm_geom(TmGeom* g, int64_t B, int64_t N, int64_t C, int outgoing, con
                      (long long)B, (long long)N, (long long)C,
                      backward ? "pair, plane or dproj5" : "pair or plane");
   g->B = (int)B; g->N = (int)N; g->Np = (int)Np; g->H = (int)C;
-  g->NN = N * N; g->PS = N * Np; g->R = R; g->outgoing = outgoing ? 1 : 0;
-  g->ntg = (int)((C + 63) / 64);
-  g->div_n = make_fastdiv((uint32_t)N);
-  g->div_nn = make_fastdiv((uint32_t)(N * N));
+  g->NN = N * N; g->PS = N * Np; g->R = R; g->Rp = B * N * Np; g->outgoing = outgoing ? 1 : 0;
+  g->div_np = make_fastdiv((uint32_t)Np);
+  g->div_ps = make_fastdiv((uint32_t)(N * Np));
   return TPF_OK;
 }
 
 static int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
-static int64_t tm_wp_rows(int64_t C) { return 2 * ((C + 63) / 64) * 128; }
 static int64_t tm_weights_bytes(int64_t C) {
-  return align256(tm_wp_rows(C) * C * 2) + 2 * align256(5 * C * C * 2) + 2 * align256(C * C * 2);
+  return 2 * align256(5 * C * C * 2) + 2 * align256(C * C * 2);
 }
 
 // Packed bf16 weights at the start of a workspace.
 struct TmPacked {
-  __bf16* wp;
   __bf16* w5;
   __bf16* wz;
   __bf16* w5t;
@@ -1940,8 +1494,6 @@ struct TmPacked {
 static TmPacked tm_packed(void* ws, int64_t C) {
   char* p = (char*)ws;
   TmPacked k;
-  k.wp = (__bf16*)p;
-  p += align256(tm_wp_rows(C) * C * 2);
   k.w5 = (__bf16*)p;
   p += align256(5 * C * C * 2);
   k.wz = (__bf16*)p;
@@ -1952,15 +1504,12 @@ static TmPacked tm_packed(void* ws, int64_t C) {
   return k;
 }
 
-static int tm_pack(const TmWeights& w, const TmPacked& k, int C, int ntg, hipStream_t s,
-                   const char* fn) {
-  const int64_t chunks = (tm_wp_rows(C) + 12 * C) * (C / 8);
+static int tm_pack(const TmWeights& w, const TmPacked& k, int C, hipStream_t s, const char* fn) {
+  const int64_t chunks = 12 * C * (C / 8);
   hipLaunchKernelGGL(tm_pack_weights_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
-                     s, w, k.wp, k.w5, k.wz, k.w5t, k.wzt, C, ntg);
+                     s, w, k.w5, k.wz, k.w5t, k.wzt, C);
   return check_launch(fn);
 }
-
-static unsigned tm_grid(int64_t tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
 
 
 #define TM_DISPATCH_C(C, KERNEL, GRID, ...)                                                   \
@@ -2004,22 +1553,13 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   hipStream_t s = (hipStream_t)stream;
   const TmPacked k = tm_packed(workspace, C);
   const TmWeights w{w_ap, w_ag, w_bp, w_bg, w_g, w_z};
-  if ((rc = tm_pack(w, k, (int)C, g.ntg, s, fn))) return rc;
-  if (g.Np != g.N) {
-    // The contraction reads whole rows of Np; pad columns must be zero.  It
-    // stores only the N real columns of x, so x's pad is cleared too: the
-    // saved state is then a function of the inputs alone.
-    if ((rc = zero_fill(a, B * C * g.PS * 2, s, fn))) return rc;
-    if ((rc = zero_fill(b, B * C * g.PS * 2, s, fn))) return rc;
-    if ((rc = zero_fill(x, B * C * g.PS * 2, s, fn))) return rc;
-  }
+  if ((rc = tm_pack(w, k, (int)C, s, fn))) return rc;
   TM_DISPATCH_C(C, tm_ln_rows_kernel, dim3((unsigned)tm_ln_rows_grid(g.R)), (const __bf16*)z, ln_in_w,
                 ln_in_b, (__bf16*)zln, mean_in, rstd_in, g.R);
   if ((rc = check_launch("tpf_trimul_forward_bf16(ln_in)"))) return rc;
-  const int64_t tiles = (g.R + 127) / 128;
   {
     // Persistent: one workgroup of C / 16 waves per CU share at C = 128.
-    const int64_t nblk = (g.R + 31) / 32;
+    const int64_t nblk = (g.Rp + 31) / 32;
     const int64_t cap = (int64_t)device_cus() * (128 / C);
     const unsigned grid = (unsigned)(nblk < cap ? nblk : cap);
     switch (C) {
@@ -2043,11 +1583,15 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   ga.A = (const __bf16*)a; ga.a_ld = g.Np; ga.a_bs = g.PS;
   ga.B = (const __bf16*)b; ga.b_ld = g.Np; ga.b_bs = g.PS;
   ga.C = x; ga.c_ld = g.Np; ga.c_bs = g.PS;
-  ga.M = (int)N; ga.N = (int)N; ga.K = g.Np; ga.ksplit = 1; ga.k_chunk = g.Np; ga.alpha = 1.f;
+  // B's rows past N read zeros, so the product's pad columns are written as
+  // zeros (the saved state is a function of the inputs alone) and every
+  // store is a whole 16-byte chunk.
+  ga.M = (int)N; ga.N = g.Np; ga.K = g.Np; ga.ksplit = 1; ga.k_chunk = g.Np; ga.alpha = 1.f;
+  ga.b_rows = (int)N;
   if ((rc = gemm_launch(ga, 1, 1, 0, (int)(B * C), s, "tpf_trimul_forward_bf16(contract)",
                         tm_contract_tile(N))))
     return rc;
-  TM_DISPATCH_C(C, tm_ln_planes_kernel, dim3((unsigned)tm_ln_planes_grid(g.NN, B), (unsigned)B),
+  TM_DISPATCH_C(C, tm_ln_planes_kernel, dim3((unsigned)tm_ln_planes_grid(g.PS, B), (unsigned)B),
                 (const __bf16*)x, ln_out_w, ln_out_b, (__bf16*)xln, mean_out, rstd_out, g);
   if ((rc = check_launch("tpf_trimul_forward_bf16(ln_out)"))) return rc;
   {
@@ -2067,26 +1611,17 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   return check_launch("tpf_trimul_forward_bf16(out_proj)");
 }
 
-// Backward workspace (each region 256-byte aligned): packed weights, dy
-// [R][C], dproj5 [R][5H], dx / da / db channel-major planes, LN_out
-// parameter partials [tiles][2][C], LN_in parameter partials [<= R/32][2][C],
-// split-K partials of dW5 and dWz.
-static int tm_split(int64_t R, int64_t per, int cap) {
-  int64_t s = R / per;
-  if (s < 1) s = 1;
-  if (s > cap) s = cap;
-  return (int)s;
-}
-// dWz on the split-K GEMM (N % 8 != 0) takes K ranges of 2304 rows
-// (measured at N = 384: 576-row ranges cost 18 us more per out + in step, in
-// the larger fold).  dW5 takes as many K ranges as fill one round of 512
+// Backward workspace (each region 256-byte aligned): packed weights, dproj5
+// [R][5H], dx / da / db channel-major planes, LN_out and LN_in parameter
+// partials and dWz partials per workgroup, split-K partials of dW5.
+// dW5 takes as many K ranges as fill one round of 512
 // workgroups with its ceil(5C / 128) x ceil(C / 128) output tiles (at least
 // 256 rows each): shape-only, so its fold order is the same on any device.
 static int tm_w5_splits(int64_t R, int64_t C) {
   const int64_t tiles = ((5 * C + 127) / 128) * ((C + 127) / 128);
-  return tm_split(R, 256, (int)(512 / tiles));
+  const int64_t cap = 512 / tiles, s = R / 256;
+  return (int)(s < 1 ? 1 : s > cap ? cap : s);
 }
-static int tm_wz_splits(int64_t R) { return tm_split(R, 2304, 64); }
 // Workgroups of the persistent backward kernels that leave per-workgroup
 // partials (LN parameter and dWz sums): a fixed plan of 256 CUs, so the
 // partition of the rows, and every summation order, depends on the shape
@@ -2098,17 +1633,14 @@ static int64_t tm_bwd_grid(int64_t R, int64_t C) {
 }
 
 int64_t tpf_trimul_backward_workspace_bytes(int64_t B, int64_t N, int64_t C) {
-  const int64_t Np = (N + 7) / 8 * 8, R = B * N * N;
-  const int64_t tiles = (R + 127) / 128;
+  const int64_t Np = (N + 7) / 8 * 8, R = B * N * N, Rp = B * N * Np;
   int64_t t = tm_weights_bytes(C);
-  t += align256(R * C * 2);                        // dy
   t += align256(R * 5 * C * 2);                    // dproj5
   t += 3 * align256(B * C * N * Np * 2);           // dx, da, db
-  t += align256((R + 31) / 32 * 2 * C * 4);        // LN_out parameter partials (tiles or workgroups)
-  t += align256((R + 31) / 32 * 2 * C * 4);        // LN_in parameter partials (per workgroup)
+  t += align256(tm_bwd_grid(Rp, C) * 2 * C * 4);   // LN_out parameter partials
+  t += align256(tm_bwd_grid(R, C) * 2 * C * 4);    // LN_in parameter partials
   t += align256((int64_t)tm_w5_splits(R, C) * 5 * C * C * 4);
-  const int64_t wz_parts = tm_wz_splits(R) > tm_bwd_grid(R, C) ? tm_wz_splits(R) : tm_bwd_grid(R, C);
-  t += align256(wz_parts * C * C * 4);  // dWz partials (split-K GEMM or per workgroup)
+  t += align256(tm_bwd_grid(Rp, C) * C * C * 4);   // dWz partials
   return t;
 }
 
@@ -2140,59 +1672,48 @@ static int trimul_backward_impl(
                      (long long)workspace_bytes, (long long)need);
   hipStream_t s = (hipStream_t)stream;
   const int64_t R = g.R, H = C;
-  const int64_t tiles = (R + 127) / 128;
-  const int s5 = tm_w5_splits(R, C), sz = tm_wz_splits(R);
+  const int s5 = tm_w5_splits(R, C);
+  const int out_grid = (int)tm_bwd_grid(g.Rp, C), ln_grid = (int)tm_bwd_grid(R, C);
   const TmPacked k = tm_packed(workspace, C);
   const TmWeights w{w_ap, w_ag, w_bp, w_bg, w_g, w_z};
   char* wp_ = (char*)workspace + tm_weights_bytes(C);
   auto take = [&](int64_t bytes) { char* p = wp_; wp_ += align256(bytes); return p; };
-  __bf16* dy = (__bf16*)take(R * C * 2);
   __bf16* dproj5 = (__bf16*)take(R * 5 * H * 2);
   const int64_t plane_bytes = B * C * g.PS * 2;
   __bf16* dx = (__bf16*)take(plane_bytes);
   __bf16* da = (__bf16*)take(plane_bytes);
   __bf16* db = (__bf16*)take(plane_bytes);
-  float* lnp = (float*)take((R + 31) / 32 * 2 * C * 4);
-  float* lnin = (float*)take((R + 31) / 32 * 2 * C * 4);
+  float* lnp = (float*)take((int64_t)out_grid * 2 * C * 4);
+  float* lnin = (float*)take((int64_t)ln_grid * 2 * C * 4);
   float* w5p = (float*)take((int64_t)s5 * 5 * C * C * 4);
-  float* wzp = (float*)take((int64_t)(sz > tm_bwd_grid(R, C) ? sz : tm_bwd_grid(R, C)) * C * C * 4);
-  if ((rc = tm_pack(w, k, (int)C, g.ntg, s, fn))) return rc;
-  // Pad columns of dx are read by the dA GEMM (K = Np) and must be zero.
-  if (g.Np != g.N && (rc = zero_fill(dx, plane_bytes, s, fn))) return rc;
-  const unsigned grid_rows = tm_grid(tiles);
-  int lnp_splits = (int)tiles;  // LN_out parameter partials
-  if (g.Np == g.N) {
-    // Output projection backward + LN_out backward in one pass.
-    const int64_t nblk = (R + 31) / 32;
-    lnp_splits = (int)tm_bwd_grid(R, C);
-    switch (C) {
+  float* wzp = (float*)take((int64_t)out_grid * C * C * 4);
+  if ((rc = tm_pack(w, k, (int)C, s, fn))) return rc;
+  // Output projection backward + LN_out backward in one pass.
+  const int64_t nblk = (g.Rp + 31) / 32;
+  switch (C) {
+#define TM_OUT_BWD_P(CC, PAD)                                                                   \
+  hipLaunchKernelGGL((tm_out_bwd_ws_kernel<CC, PAD>), dim3(out_grid), dim3(4 * CC), 0, s,       \
+                     (const __bf16*)xln, k.wz, k.wzt, (const __bf16*)gate,                      \
+                     (const __bf16*)grad_out, (const __bf16*)x, mean_out, rstd_out, ln_out_w,   \
+                     dproj5, dx, lnp, wzp, g, nblk)
 #define TM_OUT_BWD(CC)                                                                          \
   case CC:                                                                                      \
-    hipLaunchKernelGGL(tm_out_bwd_ws_kernel<CC>, dim3(lnp_splits), dim3(4 * CC), 0, s,          \
-                       (const __bf16*)xln, k.wz, k.wzt, (const __bf16*)gate,                    \
-                       (const __bf16*)grad_out, (const __bf16*)x, mean_out, rstd_out, ln_out_w, \
-                       dproj5, dx, lnp, wzp, g, nblk);                                          \
+    if (g.Np == g.N) TM_OUT_BWD_P(CC, false);                                                   \
+    else TM_OUT_BWD_P(CC, true);                                                                \
     break;
-      TM_OUT_BWD(32) TM_OUT_BWD(64) TM_OUT_BWD(96) TM_OUT_BWD(128)
+    TM_OUT_BWD(32) TM_OUT_BWD(64) TM_OUT_BWD(96) TM_OUT_BWD(128)
 #undef TM_OUT_BWD
-    }
-    if ((rc = check_launch("tpf_trimul_backward_bf16(out_proj + ln_out_bwd)"))) return rc;
-  } else {
-    hipLaunchKernelGGL(tm_out_proj_bwd_kernel, dim3(grid_rows), dim3(256), 0, s,
-                       (const __bf16*)xln, k.wz, (const __bf16*)gate, (const __bf16*)grad_out,
-                       dy, dproj5, g, (int)C);
-    if ((rc = check_launch("tpf_trimul_backward_bf16(out_proj)"))) return rc;
-    hipLaunchKernelGGL(tm_ln_out_bwd_kernel, dim3(grid_rows), dim3(256), 0, s, (const __bf16*)dy,
-                       (int64_t)C, k.wz, (int)C, (const __bf16*)x, mean_out,
-                       rstd_out, ln_out_w, dx, lnp, g, (int)H);
-    if ((rc = check_launch("tpf_trimul_backward_bf16(ln_out_bwd)"))) return rc;
+#undef TM_OUT_BWD_P
   }
+  if ((rc = check_launch("tpf_trimul_backward_bf16(out_proj + ln_out_bwd)"))) return rc;
   // Contraction backward: dA_c = dX_c B_c, dB_c = dX_c^T A_c (stored layouts).
   GemmArgs ga{};
   ga.A = dx; ga.a_ld = g.Np; ga.a_bs = g.PS;
   ga.B = (const __bf16*)b; ga.b_ld = g.Np; ga.b_bs = g.PS;
   ga.C = da; ga.c_ld = g.Np; ga.c_bs = g.PS;
-  ga.M = (int)N; ga.N = (int)N; ga.K = g.Np; ga.ksplit = 1; ga.k_chunk = g.Np; ga.alpha = 1.f;
+  // The outputs' pad columns are written too (zeros: those of B_c and A_c
+  // are), so that every store is a whole 16-byte chunk.
+  ga.M = (int)N; ga.N = g.Np; ga.K = g.Np; ga.ksplit = 1; ga.k_chunk = g.Np; ga.alpha = 1.f;
   // K = Np runs over dX's zero pad columns; the matching rows of B_c past N
   // do not exist (past the last plane they are past the tensor): read zeros.
   ga.b_kmax = (int)N;
@@ -2200,34 +1721,33 @@ static int trimul_backward_impl(
   gb.A = dx; gb.a_ld = g.Np; gb.a_bs = g.PS;
   gb.B = (const __bf16*)a; gb.b_ld = g.Np; gb.b_bs = g.PS;
   gb.C = db; gb.c_ld = g.Np; gb.c_bs = g.PS;
-  gb.M = (int)N; gb.N = (int)N; gb.K = (int)N; gb.ksplit = 1; gb.k_chunk = (int)N; gb.alpha = 1.f;
+  gb.M = (int)N; gb.N = g.Np; gb.K = (int)N; gb.ksplit = 1; gb.k_chunk = (int)N; gb.alpha = 1.f;
   // dA and dB in one launch (2 x B*C batched tiles keep the tail short).
   ga.batch = (int)(B * C);
   gb.batch = (int)(B * C);
   if ((rc = gemm_launch_pair(ga, 1, 0, gb, 0, 0, 0, s, "tpf_trimul_backward_bf16(dA, dB)",
                              tm_contract_tile(N))))
     return rc;
-  if (g.Np == g.N) {
-    const int64_t nblk = (R + 31) / 32;
+  {
     const int64_t cap = (int64_t)device_cus() * (128 / C);
     const unsigned grid = (unsigned)(nblk < cap ? nblk : cap);
     switch (C) {
+#define TM_IN_BWD_P(CC, PAD)                                                                     \
+  hipLaunchKernelGGL((tm_in_proj_bwd_ws_kernel<CC, PAD>), dim3(grid), dim3(4 * CC), 0, s,        \
+                     (const __bf16*)zln, k.w5, mask, (const __bf16*)da, (const __bf16*)db,       \
+                     dproj5, g, nblk)
 #define TM_IN_BWD(CC)                                                                            \
   case CC:                                                                                       \
-    hipLaunchKernelGGL(tm_in_proj_bwd_ws_kernel<CC>, dim3(grid), dim3(4 * CC), 0, s,             \
-                       (const __bf16*)zln, k.w5, mask, (const __bf16*)da, (const __bf16*)db,     \
-                       dproj5, g, nblk);                                                         \
+    if (g.Np == g.N) TM_IN_BWD_P(CC, false);                                                     \
+    else TM_IN_BWD_P(CC, true);                                                                  \
     break;
       TM_IN_BWD(32) TM_IN_BWD(64) TM_IN_BWD(96) TM_IN_BWD(128)
 #undef TM_IN_BWD
+#undef TM_IN_BWD_P
     }
-  } else {
-    hipLaunchKernelGGL(tm_in_proj_bwd_kernel, dim3(tm_grid(tiles * 2 * g.ntg)), dim3(256), 0, s,
-                       (const __bf16*)zln, k.wp, mask, da, db, dproj5, g, (int)C);
   }
   if ((rc = check_launch("tpf_trimul_backward_bf16(in_proj)"))) return rc;
   const int64_t ln_blk = (R + 31) / 32;
-  const int ln_grid = (int)tm_bwd_grid(R, C);
   switch (C) {
 #define TM_LN_IN(CC)                                                                            \
   case CC:                                                                                      \
@@ -2247,25 +1767,10 @@ static int trimul_backward_impl(
   gw.C = w5p; gw.c_ld = C; gw.c_bs = 0; gw.c_split = 5 * C * C;
   gw.M = (int)(5 * H); gw.N = (int)C; gw.K = (int)R; gw.ksplit = s5;
   gw.k_chunk = (int)((R + s5 - 1) / s5); gw.alpha = 1.f;
-  GemmArgs gz{};
-  gz.A = dy; gz.a_ld = C; gz.a_bs = 0;
-  gz.B = (const __bf16*)xln; gz.b_ld = H; gz.b_bs = 0;
-  gz.C = wzp; gz.c_ld = H; gz.c_bs = 0; gz.c_split = C * H;
-  gz.M = (int)C; gz.N = (int)H; gz.K = (int)R; gz.ksplit = sz;
-  gz.k_chunk = (int)((R + sz - 1) / sz); gz.alpha = 1.f;
   gw.batch = 1;
-  gz.batch = 1;
-  const bool wz_fused = g.Np == g.N;  // tm_out_bwd_ws_kernel left per-workgroup dWz partials
-  if (wz_fused) {
-    if ((rc = gemm_launch_wgrad(gw, s, "tpf_trimul_backward_bf16(dW5)"))) return rc;
-  } else {
-    // dW5 and dWz are independent split-K GEMMs of ~300 tiles each: one
-    // launch keeps both in flight together.
-    if ((rc = gemm_launch_pair_wgrad(gw, gz, s, "tpf_trimul_backward_bf16(dW5, dWz)")))
-      return rc;
-  }
+  if ((rc = gemm_launch_wgrad(gw, s, "tpf_trimul_backward_bf16(dW5)"))) return rc;
   // The four weight-gradient folds in one launch per pass; the LayerNorm
-  // partials ([tiles][ln_out_w | ln_out_b] and [workgroups][ln_in_w |
+  // partials ([workgroups][ln_out_w | ln_out_b] and [workgroups][ln_in_w |
   // ln_in_b]) land directly in the four parameter gradients.
   // The W5 partials fold as two segments: rows ap | ag | bp | bg (four
   // H x C pieces) and g; each element's fold is the same either way.
@@ -2276,9 +1781,9 @@ static int trimul_backward_impl(
   for (int j = 0; j < 4; ++j) f.dst[0][j] = w5dst[j];
   f.part[4] = w5p + 4 * H * C; f.n[4] = C * C; f.stride[4] = 5 * C * C; f.splits[4] = s5;
   f.piece[4] = C * C; f.dst[4][0] = w5dst[4];
-  f.part[1] = wzp; f.n[1] = C * H; f.stride[1] = C * H; f.splits[1] = wz_fused ? lnp_splits : sz;
+  f.part[1] = wzp; f.n[1] = C * H; f.stride[1] = C * H; f.splits[1] = out_grid;
   f.piece[1] = C * H; f.dst[1][0] = d_w_z;
-  f.part[2] = lnp; f.n[2] = 2 * C; f.stride[2] = 2 * C; f.splits[2] = lnp_splits;
+  f.part[2] = lnp; f.n[2] = 2 * C; f.stride[2] = 2 * C; f.splits[2] = out_grid;
   f.piece[2] = C;
   f.dst[2][0] = d_ln_out_w; f.dst[2][1] = d_ln_out_b;
   f.part[3] = lnin; f.n[3] = 2 * C; f.stride[3] = 2 * C; f.splits[3] = ln_grid;

@@ -274,6 +274,8 @@ def _trimul_bwd_native(grad_out, z_bf, mask_f, z_ln, gate, a, b, x, xlnT, mean_i
                          rstd_out, w_ap, w_ag, w_bp, w_bg, w_g, w_z, g_in, g_out))
     grad = grad_out.to(torch.bfloat16).contiguous()
     mask_f = mask_f.to(torch.float32).contiguous()
+    if x.data_ptr() % 16:  # the kernels read the planes in 16-byte chunks at every N
+        x = x.clone()
     *wts, gin, gout = _f32_all((w_ap, w_ag, w_bp, w_bg, w_g, w_z, g_in, g_out))
     f32 = dict(device=dev, dtype=torch.float32)
     d_z = torch.empty((B, N, N, C), device=dev, dtype=torch.bfloat16)

@@ -53,12 +53,14 @@ def run_turbo(z, mask, w, dout, outgoing, dev):
     return {k: v.detach().float().cpu().numpy() for k, v in got.items()}
 
 
-# N % 8 == 0 runs the persistent weight-stationary kernels (B = 2 crosses a
-# batch item inside the walk; N = 200 gives workgroups several 32-row blocks
-# and an uneven last share), other N the tile kernels.  N % 192 == 0 runs
+# The row kernels walk 32-position blocks of the planes (B = 2 crosses a batch
+# item inside the walk; N = 200 gives workgroups several blocks and an uneven
+# last share); N % 8 != 0 has pad positions without rows (7 of 8 in the last
+# chunk of N = 17, 33 and 113, 1 of 8 at N = 239).  N % 192 == 0 runs
 # the channel contractions on 192 x 192 tiles (128 x 128 otherwise).
 CASES = [(1, 64, 128), (1, 128, 128), (2, 33, 64), (1, 101, 32), (1, 113, 96), (1, 17, 128),
-         (2, 48, 64), (1, 72, 96), (1, 40, 32), (1, 200, 128), (1, 192, 64), (2, 192, 32)]
+         (2, 48, 64), (1, 72, 96), (1, 40, 32), (1, 200, 128), (1, 192, 64), (2, 192, 32),
+         (2, 9, 128), (1, 239, 128), (1, 1, 32)]
 
 
 @pytest.mark.gpu
