@@ -45,8 +45,9 @@ int tpf_abi_version(void);
  *   ((bb * H + h) * N + k) * N + q: the ending node's transposed pair bias,
  *   read in place).
  * out: bf16 [B, O, N, H, D].  lse, delta: f32 [B, O, H, N].
- * Requirements: N % 64 == 0 (pad on the host with -inf mask entries),
- * D % 8 == 0 and 8 <= D <= 64, B*O <= 65535.  scale = 1/sqrt(D_true): when
+ * Requirements: N % 64 == 0 (pad on the host with -inf mask entries) unless
+ * TPF_ANY_N is given (forward, forward_shadow and the single-reconstruction
+ * backward entries), D % 8 == 0 and 8 <= D <= 64, B*O <= 65535.  scale = 1/sqrt(D_true): when
  * the host zero-pads D it passes the unpadded D's scale.
  * ---------------------------------------------------------------------- */
 
@@ -55,6 +56,8 @@ enum {
   TPF_BIAS_TRANSPOSED = 2, /* bias given as the transpose of a contiguous tensor */
   TPF_DBIAS_BF16 = 4,      /* backward: dbias is bf16 (the f32 fold rounded once), stored
                               in the bias's own order (transposed with TPF_BIAS_TRANSPOSED) */
+  TPF_ANY_N = 8,           /* N need not be a multiple of 64: no tensor is padded, the result is
+                              that of the padded problem restricted to the N positions */
 };
 
 /* Bytes of device workspace tpf_attn_forward_bf16 needs (the bias in f32,
@@ -183,7 +186,7 @@ int tpf_attn_backward_fused_bf16(const void* q, const void* k, const void* v, co
 
 /* Split backward route for direct callers (not on the facade path), from
  * caller-supplied lse and delta, in the layouts and flags of
- * tpf_attn_backward_bf16 (TPF_DBIAS_BF16 excluded).
+ * tpf_attn_backward_bf16 (TPF_DBIAS_BF16 and TPF_ANY_N excluded).
  *
  * dK / dV only: dk, dv bf16 in Q/K/V storage order.  With delta_true
  * (nullable, f32 [B, O, H, N]) the call also forms delta_true = sum_k P dP

@@ -27,11 +27,12 @@ import torch
 
 from . import _native
 
-_PAD_QUANTUM = 64  # kernels tile the sequence in 64-key blocks
-# Layout bits of the C ABI (include/tpf_amd.h TPF_QKV_SEQ_MAJOR, TPF_BIAS_TRANSPOSED).
+# Layout bits of the C ABI (include/tpf_amd.h TPF_QKV_SEQ_MAJOR, TPF_BIAS_TRANSPOSED,
+# TPF_DBIAS_BF16, TPF_ANY_N).
 _QKV_SEQ_MAJOR = 1
 _BIAS_TRANSPOSED = 2
 _DBIAS_BF16 = 4  # backward: bf16 dbias in the bias's own storage order
+_ANY_N = 8  # the kernels' 64-key tiles end inside the sequence (no padded copies)
 _MAX_HEAD_DIM = 64
 _MAX_GRID_YZ = 65_535
 _SUPPORT_CACHE: dict = {}
@@ -217,7 +218,7 @@ def set_sr_workspace_budget(budget_bytes: int | None) -> None:
 def sr_workspace_plan(B: int, O: int, H: int, N: int, D: int,
                       budget_bytes: int | None = None) -> tuple[int, int]:
     """(workspace bytes, slabs) of the backward plan for a kernel-shaped problem
-    (N a multiple of 64, D a multiple of 8).  Below the one-run minimum the
+    (D a multiple of 8).  Below the one-run minimum the
     minimum is returned, as the reference's planner does for its irreducible tile."""
     budget = _SR_WORKSPACE_BUDGET if budget_bytes is None else int(budget_bytes)
     ws = int(_native.query("tpf_attn_backward_workspace_bytes_budget", B, O, H, N, D, budget))
@@ -228,9 +229,9 @@ def sr_workspace_plan(B: int, O: int, H: int, N: int, D: int,
 class _TriangleAttentionFn(torch.autograd.Function):
     """Owns the kernels' saved state (reference ``:223-320``).
 
-    Inputs are the flattened, padded kernel operands; ``bias_k`` is the
+    Inputs are the flattened kernel operands (D padded to a multiple of 8); ``bias_k`` is the
     detached kernel bias with ``Bb`` in {1, B} batches, ``source_bias`` keeps
-    the autograd edge to the caller's (dtype-converted, padded) bias.
+    the autograd edge to the caller's (dtype-converted) bias.
     """
 
     @staticmethod
@@ -318,7 +319,7 @@ class _TriangleAttentionFn(torch.autograd.Function):
 
 
 def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
-    """Validate, pad and run triangle attention, then remove padding.
+    """Validate and run triangle attention (head channels padded to a multiple of 8).
 
     Same signature and behaviour as the reference facade
     ``turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias)``
@@ -352,19 +353,6 @@ def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
         q = torch.nn.functional.pad(q, (0, head_pad))
         k = torch.nn.functional.pad(k, (0, head_pad))
         v = torch.nn.functional.pad(v, (0, head_pad))
-    # Sequence: pad to the 64-key tile; padded keys get a -inf mask.
-    seq_pad = (-sequence) % _PAD_QUANTUM
-    if seq_pad:
-        pad_qkv = (0, 0, 0, seq_pad)
-        q = torch.nn.functional.pad(q, pad_qkv)
-        k = torch.nn.functional.pad(k, pad_qkv)
-        v = torch.nn.functional.pad(v, pad_qkv)
-        pair_bias = torch.nn.functional.pad(pair_bias, (0, seq_pad, 0, seq_pad))
-        padded = res_mask.new_full(tuple(res_mask.shape[:-1]) + (sequence + seq_pad,), float("-inf"))
-        padded[..., :sequence] = res_mask
-        res_mask = padded
-    n_k = sequence + seq_pad
-
     tail = tuple(q.shape[-4:])
     qf, kf, vf = (t.reshape((batch,) + tail) for t in (q, k, v))
     orders = {_storage_order(t) for t in (qf, kf, vf)}
@@ -376,7 +364,7 @@ def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
 
     mask_f = (
         res_mask.expand(prefix + tuple(res_mask.shape[-4:]))
-        .reshape(batch, outer, n_k)
+        .reshape(batch, outer, sequence)
         .to(torch.float32)
         .contiguous()
     )
@@ -390,16 +378,16 @@ def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
         if not pair_bias.is_contiguous() and bias_t.is_contiguous():
             # The ending node's bias.transpose(-1, -2) of a contiguous tensor:
             # the kernels read it in place (TPF_BIAS_TRANSPOSED).
-            bias_k = bias_t.reshape(nbb, heads, n_k, n_k).detach()
+            bias_k = bias_t.reshape(nbb, heads, sequence, sequence).detach()
             bias_transposed = True
         else:
-            bias_k = pair_bias.reshape(nbb, heads, n_k, n_k).detach().contiguous()
+            bias_k = pair_bias.reshape(nbb, heads, sequence, sequence).detach().contiguous()
     else:
         # Partial broadcast: per-batch gradients, then a sum over the
         # broadcast prefix dimensions (reference ``dq_dbias.py:326-376``).
         bias_k = (
             pair_bias.expand(prefix + tuple(pair_bias.shape[-4:]))
-            .reshape(batch, heads, n_k, n_k)
+            .reshape(batch, heads, sequence, sequence)
             .detach()
             .contiguous()
         )
@@ -420,11 +408,14 @@ def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
             qf, kf, vf = (t.contiguous() for t in (qf, kf, vf))
             seq_major = False
     layout = (_QKV_SEQ_MAJOR if seq_major else 0) | (_BIAS_TRANSPOSED if bias_transposed else 0)
+    if sequence % 64:
+        layout |= _ANY_N
+    # The residual serves the backward only.
+    shadow = shadow and torch.is_grad_enabled() and any(
+        t.requires_grad for t in (qf, kf, vf, pair_bias))
     out = _TriangleAttentionFn.apply(
         qf, kf, vf, mask_f, bias_k, pair_bias, layout, scale, bias_reduce, shadow
     )
-    if seq_pad:
-        out = out[:, :, :sequence]
     if head_pad:
         out = out[..., :head_dim]
     if not out.is_contiguous():

@@ -23,7 +23,14 @@
 //          points).
 //   mask   [B, O, N] f32 additive.    bias [Bb, H, N, N] bf16, Bb in {1, B}.
 //   out    [B, O, N, H, D] bf16.      lse / delta [B, O, H, N] f32.
-// N must be a multiple of 64 (the host pads) and D a multiple of 8, D <= 64.
+// D is a multiple of 8, D <= 64.  The tensors of the caller hold N positions;
+// the kernels work on tiles of 64 keys and 32 queries, i.e. on NP = N rounded
+// up to 64 positions, and everything in the workspace (prescaled bias, row
+// statistics, dQ and dBias partials) has the pitch NP.  Rows past N of Q, K,
+// V and dO read zeros through the range of their buffer resource, keys past N
+// carry a -inf mask, and outputs past N are not stored, so a ragged N costs
+// no padded copies (at N = 437 the host-side padding of q, k, v, mask and
+// bias took 146 of 256 us of a forward).
 #include <algorithm>
 #include <mutex>
 
@@ -35,6 +42,7 @@ namespace tpf {
 
 struct AttnGeom {
   int B, O, H, N, D;
+  int NP;                  // N rounded up to 64
   int64_t s_row, s_head;   // Q/K/V element strides
   int64_t s_plane;         // elements between (b, o) planes of Q/K/V
   int64_t o_row, o_head;   // dQ/dK/dV element strides (the Q/K/V ones unless the
@@ -44,6 +52,13 @@ struct AttnGeom {
   int og_t;                // pair-row core: og rows in transposed pair order (O == N)
   int64_t gate_pitch;      // pair-row core: row pitch of the gate rows [B*O*N][gate_pitch]
 };
+
+// Bytes from the start of a (plane, head)'s row 0 to the end of its row N - 1:
+// the range of a buffer resource that reads zeros past N.
+__device__ __forceinline__ int row_range(int N, int64_t s_row, int D) {
+  const int64_t b = (((int64_t)N - 1) * s_row + D) * 2;
+  return (int)(b < 0x7FFFFFFF ? b : 0x7FFFFFFF);
+}
 
 // Element strides of a pair bias bias[bb, h, q, k]: the standalone op's
 // contiguous [Bb, H, N, N] (s_k = 1), or the pair-bias columns of the
@@ -104,28 +119,30 @@ __device__ __forceinline__ bool xcd_tile(int64_t total, int qtiles, int planes, 
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void attn_bias_prescale_kernel(const __bf16* __restrict__ bias,
                                                                  float* __restrict__ out,
-                                                                 int64_t items, int N,
+                                                                 int64_t items, int N, int NP,
                                                                  float inv_scale, BiasView bv) {
   const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (it >= items) return;
-  const int64_t i = bias_item_order(it, (int64_t)(N / 32) * (N / 32) * 256, bv);  // (block, j, lane)
+  const int nkb = NP / 32;
+  const int64_t i = bias_item_order(it, (int64_t)nkb * nkb * 256, bv);  // (block, j, lane)
   const int lane = (int)(i & 63), j = (int)((i >> 6) & 3);
   const int64_t blk = i >> 8;
-  const int nkb = N / 32;
   const int kb = (int)(blk % nkb);
-  const int64_t hq = blk / nkb;            // (bb * H + h) * (N / 32) + qb
-  const int qb = (int)(hq % (N / 32));
-  const int64_t bh = hq / (N / 32);
+  const int64_t hq = blk / nkb;            // (bb * H + h) * nkb + qb
+  const int qb = (int)(hq % nkb);
+  const int64_t bh = hq / nkb;
   const int ql = lane & 31, hl = lane >> 5;
-  const __bf16* src = bias_at(bias, bv, bh, qb * 32 + ql, kb * 32 + 8 * j + 4 * hl);
+  const int qi = qb * 32 + ql, k0 = kb * 32 + 8 * j + 4 * hl;
+  const __bf16* src = bias_at(bias, bv, bh, qi, k0);
   f32x4 o;
-  if (bv.s_k == 1) {
+  if (bv.s_k == 1 && N == NP) {
     const bf16x4 v = ld4(src);
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = bf2f(v[e]) * inv_scale;
   } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = bf2f(src[e * bv.s_k]) * inv_scale;
+    for (int e = 0; e < 4; ++e)
+      o[e] = qi < N && k0 + e < N ? bf2f(src[e * bv.s_k]) * inv_scale : 0.f;
   }
   *reinterpret_cast<f32x4*>(out + i * 4) = o;
 }
@@ -206,7 +223,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ql = lane & 31, hl = lane >> 5;
-  const int N = g.N, D = g.D;
+  const int N = g.N, NP = g.NP, D = g.D;
   // Groups of PL consecutive outer rows of one batch (the last group of a
   // batch may hold fewer: its missing planes recompute the first one and
   // store nothing).
@@ -220,6 +237,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
   const int q0 = tile.qt * QT + w * 32;
   const bool active = q0 < N;
   const int qi = q0 + ql;
+  const bool qok = qi < N;
   int plane[PL];
   bool pvalid[PL];
 #pragma unroll
@@ -231,10 +249,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
   const float c2 = g.scale * kLog2e;
   const float inv_scale = 1.f / g.scale;
   const float thr = 8.f / c2;  // lazy-rescale threshold in raw units
-  const int ntiles = N / 64, nblk = N / 32;
+  const int ntiles = NP / 64, nblk = NP / 32;
 
+  // Bytes from a (plane, head)'s first row to the end of its last: the range
+  // of the K / V resources, so that rows past N read zeros.
+  const int kv_bytes = row_range(N, g.s_row, D);
   // Q rows of this wave for every plane (B operand of S^T = K Q^T), zeros
-  // past D.
+  // past D and past N.
   bf16x8 qreg[PL][DP / 16];
 #pragma unroll
   for (int p = 0; p < PL; ++p) {
@@ -242,7 +263,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 #pragma unroll
     for (int s2 = 0; s2 < DP / 16; ++s2) {
       const int d0 = 16 * s2 + 8 * hl;
-      qreg[p][s2] = buf_ld8(rq, (active && d0 < D) ? (uint32_t)(((int64_t)qi * g.s_row + d0) * 2) : kBufOOB);
+      qreg[p][s2] = buf_ld8(rq, (qok && d0 < D) ? (uint32_t)(((int64_t)qi * g.s_row + d0) * 2) : kBufOOB);
     }
   }
 
@@ -254,8 +275,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 #pragma unroll
   for (int p = 0; p < PL; ++p) {
     const int64_t off = (int64_t)plane[p] * g.s_plane + (int64_t)h * g.s_head;
-    rkv[2 * p] = raw_rsrc(k + off);
-    rkv[2 * p + 1] = raw_rsrc(v + off);
+    rkv[2 * p] = raw_rsrc(k + off, kv_bytes);
+    rkv[2 * p + 1] = raw_rsrc(v + off, kv_bytes);
   }
   uint32_t vkv[CPT];
 #pragma unroll
@@ -285,7 +306,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
   // the PL planes.
   const __amdgpu_buffer_rsrc_t rs_b = raw_rsrc(
       bias_s + (int64_t)b * g.bias_bstride +
-      ((int64_t)h * (N / 32) + (active ? q0 / 32 : 0)) * (int64_t)(N / 32) * 1024);
+      ((int64_t)h * nblk + (active ? q0 / 32 : 0)) * (int64_t)nblk * 1024);
   const uint32_t vb_lane = (uint32_t)lane * 16;
   auto load_bias = [&](int blk) {
     // Blocks past the last one reload the last one (never consumed).
@@ -309,7 +330,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
   // Tiles whose 64 mask entries are all zero in every plane skip the mask
   // add (uniform flags); computed up front so no wait on the mask sits
   // inside the pipelined loop.  Each wave ballots the 64-key tiles it
-  // stages (its 64 lanes take one tile per pass; N % 64 == 0), so the flags
+  // stages (its 64 lanes take one tile per pass; NP % 64 == 0), so the flags
   // cost no round trips to memory beyond the staging loads (one ballot
   // load per tile and plane measured 3 us slower at N = 384); the waves'
   // words meet after the first barrier of the tile loop.
@@ -318,9 +339,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 #pragma unroll
   for (int p = 0; p < PL; ++p) {
     const float* mrow = mask + (int64_t)plane[p] * N;
-    for (int i = tid; i < N; i += 64 * NW) {
-      const float mv = mrow[i];
-      Ms[p * N + i] = mv * inv_scale;
+    for (int i = tid; i < NP; i += 64 * NW) {
+      const float mv = i < N ? mrow[i] : -INFINITY;
+      Ms[p * NP + i] = mv * inv_scale;
       if (__any(mv != 0.f)) wbits |= 1ull << ((i >> 6) & 63);
     }
   }
@@ -369,7 +390,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
       for (int p = 0; p < PL; ++p)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const f32x4 mv = *reinterpret_cast<const f32x4*>(&Ms[p * N + kt + sb * 32 + 8 * j + 4 * hl]);
+          const f32x4 mv = *reinterpret_cast<const f32x4*>(&Ms[p * NP + kt + sb * 32 + 8 * j + 4 * hl]);
 #pragma unroll
           for (int i = 0; i < 4; ++i) s[p][4 * j + i] += mv[i];
         }
@@ -432,9 +453,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 
   // Tile t: in LDS buffer t % 2 (written before the barrier); tile t+1 is
   // loaded into registers during the tile's first block and written to the
-  // other buffer at its end.  Waves past N (the last query tile when
-  // N % (32 NW) != 0) compute on zero Q rows and store nothing: no branch
-  // splits the loads' register state.
+  // other buffer at its end.  Waves and lanes past N (the last query tile)
+  // compute on zero Q rows and store nothing: no branch splits the loads'
+  // register state.
 #pragma unroll 1
   for (int t = 0; t < ntiles; ++t) {
     __syncthreads();
@@ -496,7 +517,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
           pr[2 * pp + 1][e] = rr[1];
         }
         const int d0 = db * 32 + 16 * pp + 8 * hl;
-        if (d0 < D) {
+        if (qok && d0 < D) {
           const u32x4 ov = {po[2 * pp][0], po[2 * pp][1], po[2 * pp + 1][0], po[2 * pp + 1][1]};
           *reinterpret_cast<u32x4*>(orow + d0) = ov;
           if (res) {
@@ -517,7 +538,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
         }
       }
     }
-    if (hl == 0) {
+    if (qok && hl == 0) {
       lse[((int64_t)plane[p] * g.H + h) * N + qi] =
           l_tot > 0.f ? (m[p] * c2 + log2f(l_tot)) * kLn2 : -INFINITY;
     }
@@ -533,14 +554,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
 // (workgroup w takes items [w * per, (w + 1) * per), per a multiple of D/8)
 // and are added in chunk order.
 // ---------------------------------------------------------------------------
-// Row sums of one workgroup's items: returns the delta index [plane][h][q]
-// of the row the calling thread finalises, with its sum in *sum (-1 for
-// every other thread).
+// Row sums of one workgroup's items: returns the (plane, head) index of the
+// row the calling thread finalises, its query in *qrow and its sum in *sum
+// (-1 for every other thread).
 template <bool SHADOW>
 __device__ __forceinline__ int64_t delta_row(const __bf16* __restrict__ dout,
                                              const __bf16* __restrict__ out,
                                              const __bf16* __restrict__ res, int64_t items,
-                                             int per, int H, int N, int D, float* sum) {
+                                             int per, int H, int N, int D, float* sum,
+                                             int* qrow) {
   __shared__ float part[256];
   const int tid = threadIdx.x;
   const int64_t t = (int64_t)blockIdx.x * per + tid;
@@ -569,9 +591,9 @@ __device__ __forceinline__ int64_t delta_row(const __bf16* __restrict__ dout,
   const int64_t r = t / d8;
   const int hh = (int)(r % H);
   const int64_t pq = r / H;
-  const int qq = (int)(pq % N);
+  *qrow = (int)(pq % N);
   const int64_t plane = pq / N;
-  return (plane * H + hh) * N + qq;
+  return plane * H + hh;
 }
 
 template <bool SHADOW>
@@ -580,15 +602,17 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(
     const __bf16* __restrict__ res, float* __restrict__ delta, int64_t items, int per, int H,
     int N, int D) {
   float sum;
-  const int64_t idx = delta_row<SHADOW>(dout, out, res, items, per, H, N, D, &sum);
-  if (idx >= 0) delta[idx] = sum;
+  int qq;
+  const int64_t ph = delta_row<SHADOW>(dout, out, res, items, per, H, N, D, &sum, &qq);
+  if (ph >= 0) delta[ph * N + qq] = sum;
 }
 
 // ---------------------------------------------------------------------------
 // Backward preparation.
 //   rowprep: nl2 = -lse * log2(e) (-inf for fully masked rows, whose P is 0)
 //            and nd = -delta, so that in the reconstruction kernel
-//              P = exp2(S_raw * c2 + nl2),  dP - delta = MFMA(dO, V^T; C = nd).
+//              P = exp2(S_raw * c2 + nl2),  dP - delta = MFMA(dO, V^T; C = nd);
+//            rows [planes * heads][NP], -inf and 0 (P = dS = 0) past N.
 //   bias_bwd: bias / scale in the fragment-major layout of the S = Q K^T
 //            accumulator: for every 32-key x 32-query block (kb, qb) of head
 //            h, [j][lane][i] holds (query 32*qb + 8*j + 4*hl + i,
@@ -599,21 +623,23 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(
 // One bias item: 4 values of the fragment-major prescaled bias (item i =
 // (fragment block, j, lane)).
 __device__ __forceinline__ void bwd_bias_item(const __bf16* __restrict__ bias,
-                                              float* __restrict__ out, int64_t it, int N,
+                                              float* __restrict__ out, int64_t it, int N, int NP,
                                               float inv_scale, const BiasView& bv) {
-  const int64_t i = bias_item_order(it, (int64_t)(N / 32) * (N / 32) * 256, bv);
+  const int nb = NP / 32;
+  const int64_t i = bias_item_order(it, (int64_t)nb * nb * 256, bv);
   const int lane = (int)(i & 63), j = (int)((i >> 6) & 3);
   const int64_t blk = i >> 8;
-  const int nb = N / 32;
   const int qb = (int)(blk % nb);
   const int64_t bk = blk / nb;             // (bh) * nb + kb
   const int kb = (int)(bk % nb);
   const int64_t bh = bk / nb;
   const int kl = lane & 31, hl = lane >> 5;
-  const __bf16* src = bias_at(bias, bv, bh, qb * 32 + 8 * j + 4 * hl, kb * 32 + kl);
+  const int q0 = qb * 32 + 8 * j + 4 * hl, key = kb * 32 + kl;
+  const __bf16* src = bias_at(bias, bv, bh, q0, key);
   f32x4 o;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = bf2f(src[(int64_t)e * bv.s_q]) * inv_scale;
+  for (int e = 0; e < 4; ++e)
+    o[e] = q0 + e < N && key < N ? bf2f(src[(int64_t)e * bv.s_q]) * inv_scale : 0.f;
   *reinterpret_cast<f32x4*>(out + i * 4) = o;
 }
 
@@ -630,39 +656,58 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const float* __restr
                                                             int64_t row_blocks,
                                                             const __bf16* __restrict__ bias,
                                                             float* __restrict__ out, int64_t items,
-                                                            int N, float inv_scale, BiasView bv) {
+                                                            int N, int NP, float inv_scale,
+                                                            BiasView bv) {
   if ((int64_t)blockIdx.x < row_blocks) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (plane, head, position)
     if (i >= rows) return;
-    nl2[i] = neg_lse_log2(lse[i]);
-    nd[i] = -delta[i];
+    if (N == NP) {
+      nl2[i] = neg_lse_log2(lse[i]);
+      nd[i] = -delta[i];
+    } else {
+      const int64_t ph = i / NP;
+      const int qq = (int)(i - ph * NP);
+      nl2[i] = qq < N ? neg_lse_log2(lse[ph * N + qq]) : -INFINITY;
+      nd[i] = qq < N ? -delta[ph * N + qq] : 0.f;
+    }
     return;
   }
   const int64_t i = ((int64_t)blockIdx.x - row_blocks) * 256 + threadIdx.x;
-  if (i < items) bwd_bias_item(bias, out, i, N, inv_scale, bv);
+  if (i < items) bwd_bias_item(bias, out, i, N, NP, inv_scale, bv);
 }
 
 // Delta and the backward preparation in one launch (the fused backward
 // entry point): workgroups [0, delta_blocks) compute delta rows as
 // attn_delta_kernel does and write nd = -delta and nl2 = -lse * log2(e) for
-// them; the rest take bias items.
+// them; the next pad_blocks write the statistics of positions past N; the
+// rest take bias items.
 template <bool SHADOW>
 __global__ __launch_bounds__(256) void attn_bwd_rows_kernel(
     const __bf16* __restrict__ dout, const __bf16* __restrict__ out,
     const __bf16* __restrict__ res, const float* __restrict__ lse, float* __restrict__ nl2,
-    float* __restrict__ nd, int64_t items, int per, int H, int N, int D, int64_t delta_blocks,
-    const __bf16* __restrict__ bias, float* __restrict__ bias_out, int64_t bias_items,
-    float inv_scale, BiasView bv) {
+    float* __restrict__ nd, int64_t items, int per, int H, int N, int NP, int D,
+    int64_t delta_blocks, int64_t pad_blocks, int64_t pad_items, const __bf16* __restrict__ bias,
+    float* __restrict__ bias_out, int64_t bias_items, float inv_scale, BiasView bv) {
+  if ((int64_t)blockIdx.x >= delta_blocks + pad_blocks) {
+    const int64_t i = ((int64_t)blockIdx.x - delta_blocks - pad_blocks) * 256 + threadIdx.x;
+    if (i < bias_items) bwd_bias_item(bias, bias_out, i, N, NP, inv_scale, bv);
+    return;
+  }
   if ((int64_t)blockIdx.x >= delta_blocks) {
     const int64_t i = ((int64_t)blockIdx.x - delta_blocks) * 256 + threadIdx.x;
-    if (i < bias_items) bwd_bias_item(bias, bias_out, i, N, inv_scale, bv);
+    if (i < pad_items) {
+      const int64_t ph = i / (NP - N), at = ph * NP + N + (i - ph * (NP - N));
+      nd[at] = 0.f;
+      nl2[at] = -INFINITY;
+    }
     return;
   }
   float sum;
-  const int64_t idx = delta_row<SHADOW>(dout, out, res, items, per, H, N, D, &sum);
-  if (idx >= 0) {
-    nd[idx] = -sum;
-    nl2[idx] = neg_lse_log2(lse[idx]);
+  int qq;
+  const int64_t ph = delta_row<SHADOW>(dout, out, res, items, per, H, N, D, &sum, &qq);
+  if (ph >= 0) {
+    nd[ph * NP + qq] = -sum;
+    nl2[ph * NP + qq] = neg_lse_log2(lse[ph * N + qq]);
   }
 }
 
@@ -808,7 +853,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int pw = w & 3, kh = w >> 2;            // outer row in the group, key half
   const int kl = lane & 31, hl = lane >> 5;
-  const int N = g.N, D = g.D, H = g.H;
+  const int N = g.N, NP = g.NP, D = g.D, H = g.H;
   const int nkb = (N + 64 * KH - 1) / (64 * KH);
   const int groups = (g.O + kBwdGroup - 1) / kBwdGroup;
   const int runs = (groups + run - 1) / run;
@@ -830,13 +875,13 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   const int b = brun / runs;
   const int og_lo = (brun % runs) * run, og_hi = min(groups, og_lo + run);
   const int key_base = kblk * 64 * KH + 64 * kh;
-  // A key half past N (N % 128 == 64) runs with every key masked: P = dS = 0.
+  // A key half past N runs with every key masked: P = dS = 0.
   const bool keys_ok = key_base < N;
   const float c2 = g.scale * kLog2e;
   const float inv_scale = 1.f / g.scale;
   __bf16* const Ss = dSbase + w * SSE;  // this wave's dS^T tile, and its K tile at setup
   __bf16* const Kt = Ss;
-  float* const dbp = dbias_part + ((int64_t)brun * H + h) * N * N;
+  float* const dbp = dbias_part + ((int64_t)brun * H + h) * NP * NP;
 
 #pragma unroll 1
   for (int og = og_lo; og < og_hi; ++og) {
@@ -856,25 +901,25 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   }
 
   const int64_t bb = (g.bias_bstride == 0) ? 0 : b;
-  const int nb32 = N / 32;
+  const int nb32 = NP / 32;
   // Fragment blocks (kb32, qb) of this head: [(bb*H + h)*nb32 + kb32][qb][1024].
   const float* bfrag = bias_f + ((bb * H + h) * nb32 + kblk * 2 * KH) * (int64_t)nb32 * 1024;
   const int64_t do_plane = (int64_t)plane * N * H * D + (int64_t)h * D;  // dO is [B,O,N,H,D]
-  const int64_t st_plane = ((int64_t)plane * H + h) * N;                // row statistics
+  const int64_t st_plane = ((int64_t)plane * H + h) * NP;               // row statistics
   // dQ partials of the slab's planes [key block][plane - plane0][h][q][D].
-  __bf16* dqp = dq_part + ((int64_t)kblk * sl.planes + (plane_ok ? plane - sl.plane0 : 0)) * H * N * D +
-                (int64_t)h * N * D;
+  __bf16* dqp = dq_part + ((int64_t)kblk * sl.planes + (plane_ok ? plane - sl.plane0 : 0)) * H * NP * D +
+                (int64_t)h * NP * D;
   const int key_blk0 = kblk * 64 * KH;  // first key of the workgroup
   // Partial stores through buffer resources: per-lane offsets fixed for the
   // walk, the step's offset in a scalar.  dQ: this wave's outer row and
-  // head; dBias: the (run, head) N x N block, which the first group of the
+  // head; dBias: the (run, head) NP x NP block, which the first group of the
   // run writes and the later ones read back (range 0: reads give zeros) and
   // rewrite with their rows added.
   const __amdgpu_buffer_rsrc_t rs_dq = __builtin_amdgcn_make_buffer_rsrc(dqp, 0, 0x7FFFFFFF, 0x00020000);
   const uint32_t vdq = (uint32_t)(kl * D * 2);  // query row kl of the step
   const __amdgpu_buffer_rsrc_t rs_db = __builtin_amdgcn_make_buffer_rsrc(dbp, 0, 0x7FFFFFFF, 0x00020000);
   const int dbkey = tid % (64 * KH), dbqb = tid / (64 * KH);
-  const uint32_t vdb = key_blk0 + dbkey < N ? (uint32_t)((8 * dbqb * N + key_blk0 + dbkey) * 4) : kBufOOB;
+  const uint32_t vdb = key_blk0 + dbkey < NP ? (uint32_t)((8 * dbqb * NP + key_blk0 + dbkey) * 4) : kBufOOB;
   // The run's partial so far: read back by the thread that writes it
   // (range 0 for the run's first group: zeros), at device scope (sc1), so
   // the load misses the CU's L1, which may hold an older copy of the line.
@@ -893,10 +938,14 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   asm volatile("v_mov_b32 %0, 0x3f80" : "=v"(sel_lo_bits));
   // Buffer loads with per-lane byte offsets fixed for the whole walk; each
   // step advances only a scalar offset.  Lanes past D and the lanes of an
-  // idle wave read zeros (kBufOOB).
+  // idle wave read zeros (kBufOOB), and so do Q / dO rows past N (the range
+  // of their resources).
   const i32x4 rs_bias = buffer_rsrc(bfrag);
-  const i32x4 rs_q = buffer_rsrc(q + plane_off);
-  const i32x4 rs_do = buffer_rsrc(dout + do_plane);
+  const int q_bytes = row_range(N, g.s_row, D);
+  i32x4 rs_q = buffer_rsrc(q + plane_off);
+  rs_q[2] = q_bytes;
+  i32x4 rs_do = buffer_rsrc(dout + do_plane);
+  rs_do[2] = row_range(N, (int64_t)H * D, D);
   // Bias: wave w loads kilobytes 2w and 2w+1 of the step's 8*KH KB (32-key
   // blocks past N read zeros).  Q / dO: key half kh loads its share of its
   // outer row's tiles.
@@ -905,7 +954,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
     const int kbx = 2 * w + x, cb = kbx >> 2, j = kbx & 3;
-    vb[x] = key_blk0 + 32 * cb < N ? (uint32_t)((cb * nb32 * 1024 + j * 256 + lane * 4) * 4)
+    vb[x] = key_blk0 + 32 * cb < NP ? (uint32_t)((cb * nb32 * 1024 + j * 256 + lane * 4) * 4)
                                    : kBufOOB;
   }
 #pragma unroll
@@ -947,7 +996,8 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   float mk2[2];
   {
     // All loads first (branch-free, zeros outside the tensor), one wait.
-    const __amdgpu_buffer_rsrc_t rk = raw_rsrc(k + plane_off), rv = raw_rsrc(v + plane_off);
+    const __amdgpu_buffer_rsrc_t rk = raw_rsrc(k + plane_off, q_bytes),
+                                 rv = raw_rsrc(v + plane_off, q_bytes);
     const __amdgpu_buffer_rsrc_t rm = raw_rsrc(mask + (int64_t)plane * N);
     float mraw[2];
 #pragma unroll
@@ -960,14 +1010,14 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
         kB[cb][s] = buf_ld8(rk, off);
         vB[cb][s] = buf_ld8(rv, off);
       }
-      mraw[cb] = buf_ldf(rm, active ? (uint32_t)(key * 4) : kBufOOB);
+      mraw[cb] = buf_ldf(rm, active && key < N ? (uint32_t)(key * 4) : kBufOOB);
     }
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
 #pragma unroll
       for (int s = 0; s < DP / 16; ++s)
         *reinterpret_cast<bf16x8*>(&Kt[(cb * 32 + kl) * KT + 16 * s + 8 * hl]) = kB[cb][s];
-      mk2[cb] = active ? mraw[cb] * inv_scale : (keys_ok ? 0.f : -INFINITY);
+      mk2[cb] = key_base + cb * 32 + kl >= N ? -INFINITY : active ? mraw[cb] * inv_scale : 0.f;
     }
   }
   const bool wmask = __any(mk2[0] != 0.f || mk2[1] != 0.f);
@@ -995,7 +1045,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         dbprev[e] = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(rs_dbr, vdb, (q0 + e) * N * 4, 16));
+            float, __builtin_amdgcn_raw_buffer_load_b32(rs_dbr, vdb, (q0 + e) * NP * 4, 16));
     };
     // This step's loads were issued one step ago; wait for them, read the
     // shared bias fragments and the row statistics, then start the next
@@ -1213,7 +1263,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dbprev[e] + acc[e]), rs_db, vdb,
-                                              (q0 + e) * N * 4, 0);
+                                              (q0 + e) * NP * 4, 0);
     }
     }  // dQ / dBias
   };
@@ -1233,6 +1283,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
       const int key = key_base + cb * 32 + kl;
+      const bool kok = key < N;
       const int64_t row = (int64_t)plane * g.o_plane + (int64_t)h * g.o_head + (int64_t)key * g.o_row;
       uint32_t pk[4][2], pv[4][2];  // [j][pair] packed bf16
 #pragma unroll
@@ -1259,7 +1310,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
           pv[2 * p + 1][e] = rv[1];
         }
         const int d0 = db * 32 + 16 * p + 8 * hl;
-        if (d0 < D) {
+        if (kok && d0 < D) {
           const u32x4 ok = {pk[2 * p][0], pk[2 * p][1], pk[2 * p + 1][0], pk[2 * p + 1][1]};
           const u32x4 ov = {pv[2 * p][0], pv[2 * p][1], pv[2 * p + 1][0], pv[2 * p + 1][1]};
           *reinterpret_cast<u32x4*>(dk + row + d0) = ok;
@@ -1282,11 +1333,11 @@ __device__ __forceinline__ void dq_fold_block(const __bf16* __restrict__ part,
   const int t = bx * 256 + threadIdx.x;
   if (t >= g.N * D8) return;
   const int qq = t / D8, d0 = (t - qq * D8) * 8;
-  const int64_t stride = planes * g.H * g.N * g.D;
+  const int64_t stride = planes * g.H * g.NP * g.D;
   const int64_t lp = ph / g.H;  // plane within the slab
   const int hh = (int)(ph - lp * g.H);
   const int64_t plane = plane0 + lp;
-  const __bf16* src = part + (ph * g.N + qq) * g.D + d0;
+  const __bf16* src = part + (ph * g.NP + qq) * g.D + d0;
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -1326,26 +1377,45 @@ __global__ __launch_bounds__(256) void attn_dq_reduce_kernel(
 // rounded to bf16, either in that order or (transposed) in the order of a
 // transposed bias, dbias[bb, h, k, q]: then the workgroup covers an 8-query
 // x 64-key tile and writes it transposed through LDS, 16 bytes per key.
+// The partials have the pitch NP, and NP / 8 key chunks per query row are
+// walked; outputs past N are dropped, and with N % 8 != 0 the rest of a chunk
+// is stored element by element.
 __device__ __forceinline__ void dbias_fold_block(const float* __restrict__ part,
                                                  void* __restrict__ dbias, int B, int Bb,
-                                                 int groups, int H, int N, int64_t blk,
+                                                 int groups, int H, int N, int NP, int64_t blk,
                                                  bool out_bf16, bool transposed) {
   __shared__ float red[4][64][9];
   const int c = threadIdx.x & 63, sl = threadIdx.x >> 6;
-  const int64_t hnn = (int64_t)H * N * N;
+  const int64_t hnn = (int64_t)H * NP * NP;
   bool act;
   int bb;
-  int64_t e;  // offset of the thread's first output in the [H, N, N] block
+  int64_t e;       // offset of the thread's first partial in the [H, NP, NP] block
+  int64_t oe = 0;  // and of its first output in the [Bb, H, N, N] block
+  int nk = 8;      // outputs of the thread's 8 that exist
   int th = 0, tq0 = 0, tk0 = 0;  // transposed tile: head, first query, first key
   if (!transposed) {
     const int64_t idx = blk * 64 + c;
-    act = idx < (int64_t)Bb * (hnn / 8);
-    bb = act ? (int)(idx / (hnn / 8)) : 0;
-    e = act ? (idx % (hnn / 8)) * 8 : 0;
+    if (N == NP) {
+      act = idx < (int64_t)Bb * (hnn / 8);
+      bb = act ? (int)(idx / (hnn / 8)) : 0;
+      e = act ? (idx % (hnn / 8)) * 8 : 0;
+      oe = (int64_t)bb * hnn + e;
+    } else {
+      const int kc = NP / 8;
+      const int64_t row = idx / kc;  // (bb, h, q) of the N query rows
+      const int k0 = (int)(idx - row * kc) * 8;
+      act = row < (int64_t)Bb * H * N && k0 < N;
+      const int64_t bh = act ? row / N : 0;
+      const int qq = act ? (int)(row - bh * N) : 0;
+      bb = (int)(bh / H);
+      e = act ? ((bh - (int64_t)bb * H) * NP + qq) * NP + k0 : 0;
+      oe = act ? row * N + k0 : 0;
+      nk = min(8, N - k0);
+    }
   } else {
-    // Tiles of 8 queries x 64 keys (N % 64 == 0): thread c -> query c / 8,
-    // keys 8 (c % 8) .. +7.
-    const int kt_n = N / 64, tiles = (N / 8) * kt_n;
+    // Tiles of 8 queries x 64 keys: thread c -> query c / 8, keys
+    // 8 (c % 8) .. +7.
+    const int kt_n = NP / 64, tiles = ((N + 7) / 8) * kt_n;
     const int64_t bh = blk / tiles;
     const int r = (int)(blk % tiles), qt = r / kt_n, kt = r % kt_n;
     act = bh < (int64_t)Bb * H;
@@ -1353,7 +1423,7 @@ __device__ __forceinline__ void dbias_fold_block(const float* __restrict__ part,
     th = (int)(bh % H);
     tq0 = qt * 8;
     tk0 = kt * 64;
-    e = act ? (int64_t)th * N * N + (int64_t)(tq0 + c / 8) * N + tk0 + (c % 8) * 8 : 0;
+    e = act ? (int64_t)th * NP * NP + (int64_t)(tq0 + c / 8) * NP + tk0 + (c % 8) * 8 : 0;
   }
   const int b_lo = (Bb == 1) ? 0 : bb, b_hi = (Bb == 1) ? B : bb + 1;
   const int n = (b_hi - b_lo) * groups;
@@ -1400,9 +1470,17 @@ __device__ __forceinline__ void dbias_fold_block(const float* __restrict__ part,
       bf16x8 o;
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[i] = f2bf(v[i]);
-      st8((__bf16*)dbias + (int64_t)bb * hnn + e, o);
+      __bf16* d = (__bf16*)dbias + oe;
+      if (N % 8 == 0) {
+        st8(d, o);
+      } else {
+        for (int i = 0; i < nk; ++i) d[i] = f2bf(v[i]);
+      }
+    } else if (N % 8 != 0) {
+      float* d = (float*)dbias + oe;
+      for (int i = 0; i < nk; ++i) d[i] = v[i];
     } else {
-      float* d = (float*)dbias + (int64_t)bb * hnn + e;
+      float* d = (float*)dbias + oe;
       *reinterpret_cast<f32x4*>(d) = f32x4{v[0], v[1], v[2], v[3]};
       *reinterpret_cast<f32x4*>(d + 4) = f32x4{v[4], v[5], v[6], v[7]};
     }
@@ -1417,11 +1495,16 @@ __device__ __forceinline__ void dbias_fold_block(const float* __restrict__ part,
     for (int i = 0; i < 8; ++i) T[c / 8][(c % 8) * 8 + i] = f2bf(v[i]);
   }
   __syncthreads();
-  if (sl != 0 || !act) return;
+  if (sl != 0 || !act || tk0 + c >= N) return;
   bf16x8 o;
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = T[i][c];
-  st8((__bf16*)dbias + (int64_t)bb * hnn + (int64_t)th * N * N + (int64_t)(tk0 + c) * N + tq0, o);
+  __bf16* d = (__bf16*)dbias + (((int64_t)bb * H + th) * N + tk0 + c) * N + tq0;
+  if (N % 8 == 0) {
+    st8(d, o);
+  } else {
+    for (int i = 0; i < min(8, N - tq0); ++i) d[i] = T[i][c];
+  }
 }
 
 __global__ __launch_bounds__(256) void attn_fold_kernel(
@@ -1430,7 +1513,7 @@ __global__ __launch_bounds__(256) void attn_fold_kernel(
     int64_t n_db, int db_mode, int64_t plane0, int64_t planes) {
   const int64_t b = blockIdx.x;
   if (b < n_db) {
-    dbias_fold_block(db_part, dbias, g.B, Bb, groups, g.H, g.N, b, db_mode != 0, db_mode == 2);
+    dbias_fold_block(db_part, dbias, g.B, Bb, groups, g.H, g.N, g.NP, b, db_mode != 0, db_mode == 2);
   } else {
     const int64_t r = b - n_db;
     dq_fold_block(dq_part, dq, g, nkb, (int)(r % dq_bx), r / dq_bx, plane0, planes);
@@ -1580,11 +1663,15 @@ __global__ __launch_bounds__(256) void attn_dbias_pair_kernel(
 // ---------------------------------------------------------------------------
 using namespace tpf;
 
-static int check_geom(const AttnGeom& g, const char* fn) {
+static int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
+
+static int check_geom(const AttnGeom& g, bool any_n, const char* fn) {
   if (g.B < 1 || g.O < 1 || g.H < 1 || g.N < 1)
     return set_error(TPF_ERR_SHAPE, "%s: B, O, H and N must be positive", fn);
-  if (g.N % 64 != 0)
-    return set_error(TPF_ERR_SHAPE, "%s: N=%d must be a multiple of 64 (pad on the host)", fn, g.N);
+  if (g.N % 64 != 0 && !any_n)
+    return set_error(TPF_ERR_SHAPE,
+                     "%s: N=%d must be a multiple of 64 (pad on the host, or pass TPF_ANY_N)", fn,
+                     g.N);
   if (g.D < 8 || g.D > 64 || g.D % 8 != 0)
     return set_error(TPF_ERR_SHAPE, "%s: D=%d must be a multiple of 8 in [8, 64]", fn, g.D);
   if (g.H > 65535) return set_error(TPF_ERR_SHAPE, "%s: H=%d exceeds the grid-y limit", fn, g.H);
@@ -1595,24 +1682,25 @@ static int make_geom(AttnGeom* g, int64_t B, int64_t O, int64_t H, int64_t N, in
                      int layout, int64_t bias_batches, double scale, const char* fn) {
   if (B > INT32_MAX || O > INT32_MAX || N > INT32_MAX)
     return set_error(TPF_ERR_SHAPE, "%s: dimension exceeds int32", fn);
-  if (layout & ~(TPF_QKV_SEQ_MAJOR | TPF_BIAS_TRANSPOSED | TPF_DBIAS_BF16))
+  if (layout & ~(TPF_QKV_SEQ_MAJOR | TPF_BIAS_TRANSPOSED | TPF_DBIAS_BF16 | TPF_ANY_N))
     return set_error(TPF_ERR_ARG, "%s: unknown layout flags 0x%x", fn, layout);
   const bool seq_major = layout & TPF_QKV_SEQ_MAJOR;
   g->B = (int)B; g->O = (int)O; g->H = (int)H; g->N = (int)N; g->D = (int)D;
+  g->NP = (int)std::min<int64_t>(pad64(N), INT32_MAX);
   g->s_row = seq_major ? H * D : D;
   g->s_head = seq_major ? D : N * D;
   g->s_plane = H * N * D;
   if (bias_batches != 1 && bias_batches != B)
     return set_error(TPF_ERR_SHAPE, "%s: bias batch count %lld must be 1 or B=%lld", fn,
                      (long long)bias_batches, (long long)B);
-  g->bias_bstride = (bias_batches == 1) ? 0 : H * N * N;
+  g->bias_bstride = (bias_batches == 1) ? 0 : H * pad64(N) * pad64(N);
   g->o_row = g->s_row;
   g->o_head = g->s_head;
   g->o_plane = g->s_plane;
   g->scale = (float)scale;
   g->og_t = 0;
   g->gate_pitch = 0;
-  return check_geom(*g, fn);
+  return check_geom(*g, (layout & TPF_ANY_N) != 0, fn);
 }
 
 // Contiguous [Bb, H, N, N] bias, or (TPF_BIAS_TRANSPOSED in layout) the
@@ -1632,9 +1720,9 @@ static BiasView dense_bias(int64_t H, int64_t N, int64_t bias_batches, int layou
 static int attn_prescale_bias(const AttnGeom& g, const void* bias, const BiasView& bv,
                               float* bias_s, int64_t bias_batches, hipStream_t s,
                               const char* fn) {
-  const int64_t items = bias_batches * g.H * (int64_t)g.N * g.N / 4;
+  const int64_t items = bias_batches * g.H * (int64_t)g.NP * g.NP / 4;
   hipLaunchKernelGGL(attn_bias_prescale_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256),
-                     0, s, (const __bf16*)bias, bias_s, items, g.N, 1.f / g.scale, bv);
+                     0, s, (const __bf16*)bias, bias_s, items, g.N, g.NP, 1.f / g.scale, bv);
   return check_launch(fn);
 }
 
@@ -1651,15 +1739,15 @@ static int attn_forward_impl(AttnGeom g, const void* q, const void* k, const voi
                         ((g.O + pl - 1) / pl);
   if ((total + 7) / 8 * 8 > INT32_MAX)
     return set_error(TPF_ERR_SHAPE, "%s: too many query tiles", fn);
-  if (g.N > kFwdMaskLdsMaxN)
+  if (g.NP > kFwdMaskLdsMaxN)
     return set_error(TPF_ERR_SHAPE, "%s: N=%d exceeds the forward's mask staging limit %d", fn, g.N,
                      kFwdMaskLdsMaxN);
   float* bias_s = (float*)workspace;
   int rc = attn_prescale_bias(g, bias, bv, bias_s, bias_batches, s, fn);
   if (rc) return rc;
-  g.bias_bstride = (bias_batches == 1) ? 0 : (int64_t)g.H * g.N * g.N;
+  g.bias_bstride = (bias_batches == 1) ? 0 : (int64_t)g.H * g.NP * g.NP;
   dim3 grid((unsigned)((total + 7) / 8 * 8));
-  const unsigned mask_lds = (unsigned)(pl * g.N) * 4u;
+  const unsigned mask_lds = (unsigned)(pl * g.NP) * 4u;
   if (g.D <= 32)
     hipLaunchKernelGGL((attn_fwd_kernel<32, kFwdWaves, kFwdPlanes32>), grid, dim3(64 * kFwdWaves),
                        mask_lds, s, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, mask,
@@ -1696,9 +1784,9 @@ static int64_t bwd_runs(int64_t O, int run) {
   return ((O + kBwdGroup - 1) / kBwdGroup + run - 1) / run;
 }
 
-// Backward workspace: bf16 dQ partials [key blocks][slab planes][H,N,D] |
-// f32 dBias partials [B * runs][H,N,N] (one per run of outer groups) | f32
-// fragment-major bias [<=B][H,N,N] | f32 row statistics nl2, nd [B,O,H,N];
+// Backward workspace: bf16 dQ partials [key blocks][slab planes][H,NP,D] |
+// f32 dBias partials [B * runs][H,NP,NP] (one per run of outer groups) | f32
+// fragment-major bias [<=B][H,NP,NP] | f32 row statistics nl2, nd [B,O,H,NP];
 // each region 256-byte aligned.  Only the dQ partials depend on the slab.
 struct BwdParts {
   __bf16* dq;
@@ -1713,12 +1801,12 @@ static int64_t a256(int64_t v) { return (v + 255) / 256 * 256; }
 static int64_t bwd_layout(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D,
                           int64_t slab_planes, char* base, BwdParts* parts) {
   const int64_t runs = bwd_runs(O, bwd_run_len(B, O, H, N, D));
-  const int64_t rows = B * O * H * N;
+  const int64_t NP = pad64(N), rows = B * O * H * NP;
   int64_t off = 0;
   auto take = [&](int64_t bytes) { char* p = base ? base + off : nullptr; off += a256(bytes); return p; };
-  char* dq = take(bwd_key_blocks(N, D) * slab_planes * H * N * D * 2);
-  char* db = take(B * runs * H * N * N * 4);
-  char* bf = take(B * H * N * N * 4);
+  char* dq = take(bwd_key_blocks(N, D) * slab_planes * H * NP * D * 2);
+  char* db = take(B * runs * H * NP * NP * 4);
+  char* bf = take(B * H * NP * NP * 4);
   char* nl = take(rows * 4);
   char* nd = take(rows * 4);
   if (parts) {
@@ -1806,19 +1894,20 @@ static int attn_backward_rows_impl(const AttnGeom& g, const void* dout, const vo
   const int64_t items = B * O * N * H * (D / 8);
   const int per = 256 - 256 % (int)(D / 8);
   const int64_t delta_blocks = (items + per - 1) / per;
-  const int64_t bias_items = bias_batches * H * N * N / 4;
-  const int64_t blocks = delta_blocks + (bias_items + 255) / 256;
+  const int64_t NP = g.NP, bias_items = bias_batches * H * NP * NP / 4;
+  const int64_t pad_items = B * O * H * (NP - N), pad_blocks = (pad_items + 255) / 256;
+  const int64_t blocks = delta_blocks + pad_blocks + (bias_items + 255) / 256;
   if (blocks > INT32_MAX) return set_error(TPF_ERR_SHAPE, "%s: row grid too large", fn);
   if (res)
     hipLaunchKernelGGL(attn_bwd_rows_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s,
                        (const __bf16*)dout, (const __bf16*)out, (const __bf16*)res, lse, pt.nl2,
-                       pt.nd, items, per, (int)H, (int)N, (int)D, delta_blocks,
-                       (const __bf16*)bias, pt.bias_f, bias_items, 1.f / g.scale, bv);
+                       pt.nd, items, per, (int)H, (int)N, (int)NP, (int)D, delta_blocks,
+                       pad_blocks, pad_items, (const __bf16*)bias, pt.bias_f, bias_items, 1.f / g.scale, bv);
   else
     hipLaunchKernelGGL(attn_bwd_rows_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, s,
                        (const __bf16*)dout, (const __bf16*)out, (const __bf16*)nullptr, lse,
-                       pt.nl2, pt.nd, items, per, (int)H, (int)N, (int)D, delta_blocks,
-                       (const __bf16*)bias, pt.bias_f, bias_items, 1.f / g.scale, bv);
+                       pt.nl2, pt.nd, items, per, (int)H, (int)N, (int)NP, (int)D, delta_blocks,
+                       pad_blocks, pad_items, (const __bf16*)bias, pt.bias_f, bias_items, 1.f / g.scale, bv);
   return check_launch(fn);
 }
 
@@ -1827,14 +1916,14 @@ static int attn_backward_rows_impl(const AttnGeom& g, const void* dout, const vo
 static int attn_backward_prep_impl(const AttnGeom& g, const float* lse, const float* delta,
                                    const void* bias, const BiasView& bv, int64_t bias_batches,
                                    const BwdParts& pt, hipStream_t s, const char* fn) {
-  const int64_t rows = (int64_t)g.B * g.O * g.H * g.N;
-  const int64_t items = bias_batches * g.H * (int64_t)g.N * g.N / 4;
+  const int64_t rows = (int64_t)g.B * g.O * g.H * g.NP;
+  const int64_t items = bias_batches * g.H * (int64_t)g.NP * g.NP / 4;
   const int64_t row_blocks = (rows + 255) / 256;
   if (row_blocks + (items + 255) / 256 > INT32_MAX)
     return set_error(TPF_ERR_SHAPE, "%s: backward preparation grid too large", fn);
   hipLaunchKernelGGL(attn_bwd_prep_kernel, dim3((unsigned)(row_blocks + (items + 255) / 256)),
                      dim3(256), 0, s, lse, delta, pt.nl2, pt.nd, rows, row_blocks,
-                     (const __bf16*)bias, pt.bias_f, items, (int)g.N, 1.f / g.scale, bv);
+                     (const __bf16*)bias, pt.bias_f, items, g.N, g.NP, 1.f / g.scale, bv);
   return check_launch(fn);
 }
 
@@ -1885,7 +1974,12 @@ static int attn_backward_fold_impl(const AttnGeom& g, void* dq, void* dbias,
   const int64_t H = g.H, N = g.N, D = g.D;
   const int64_t nph = sl.planes * H;
   const int64_t dq_bx = (N * (D / 8) + 255) / 256;
-  const int64_t n_db = with_dbias ? (bias_batches * H * N * N / 8 + 63) / 64 : 0;
+  // dBias workgroups: 64 chunks of 8 keys, or (transposed order) a tile of
+  // 8 queries x 64 keys each.
+  const int64_t NP = g.NP;
+  const int64_t n_db = !with_dbias     ? 0
+                       : db_mode == 2 ? bias_batches * H * ((N + 7) / 8) * (NP / 64)
+                                      : (bias_batches * H * N * (NP / 8) + 63) / 64;
   if (n_db + dq_bx * nph > 0x7fffffff)
     return set_error(TPF_ERR_ARG, "%s: fold grid too large", fn);
   if (n_db + dq_bx * nph == 0) return TPF_OK;
@@ -1915,7 +2009,7 @@ extern "C" {
 int64_t tpf_attn_forward_workspace_bytes(int64_t B, int64_t H, int64_t N,
                                          int64_t bias_batches) {
   (void)B;
-  return bias_batches * H * N * N * 4;
+  return bias_batches * H * pad64(N) * pad64(N) * 4;
 }
 
 int tpf_attn_forward_bf16(const void* q, const void* k, const void* v, const float* mask,
@@ -2249,7 +2343,8 @@ int tpf_attn_dkdv_bf16(const void* q, const void* k, const void* v, const void* 
   AttnGeom g;
   int rc = make_geom(&g, B, O, H, N, D, layout, bias_batches, scale, fn);
   if (rc) return rc;
-  if (layout & TPF_DBIAS_BF16) return set_error(TPF_ERR_ARG, "%s: TPF_DBIAS_BF16 has no meaning here", fn);
+  if (layout & (TPF_DBIAS_BF16 | TPF_ANY_N))
+    return set_error(TPF_ERR_ARG, "%s: TPF_DBIAS_BF16 and TPF_ANY_N have no meaning here", fn);
   if (!q || !k || !v || !dout || !lse || !delta || !mask || !bias || !dk || !dv || !workspace)
     return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   if ((delta_true_partials == nullptr) != (delta_true == nullptr))
@@ -2297,7 +2392,8 @@ int tpf_attn_dq_dbias_bf16(const void* q, const void* k, const void* v, const vo
   int rc = attn_bwd_prepare(&g, &plan, fn, q, k, v, dout, lse, delta, mask, bias, workspace,
                             workspace_bytes, B, O, H, N, D, layout, bias_batches, scale, false);
   if (rc) return rc;
-  if (layout & TPF_DBIAS_BF16) return set_error(TPF_ERR_ARG, "%s: dbias is f32 here", fn);
+  if (layout & (TPF_DBIAS_BF16 | TPF_ANY_N))
+    return set_error(TPF_ERR_ARG, "%s: dbias is f32 and N a multiple of 64 here", fn);
   if (!dq || !dbias) return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   hipStream_t s = (hipStream_t)stream;
   BwdParts pt;

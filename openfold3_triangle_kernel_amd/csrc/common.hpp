@@ -259,10 +259,12 @@ __device__ __forceinline__ void buf2lds16_so(i32x4 rsrc, uint32_t voff, uint32_t
                :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
 
-// Raw buffer resource over [base, base + 2^31 - 1) for the load/store
-// builtins; a byte offset of kBufOOB reads zeros and drops stores.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7FFFFFFF, 0x00020000);
+// Raw buffer resource over [base, base + bytes) for the load/store builtins;
+// a byte offset (lane plus scalar offset) past it, kBufOOB always, reads zeros
+// and drops stores.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* base,
+                                                           int bytes = 0x7FFFFFFF) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
 // Branch-free 16-byte / 4-byte loads through a buffer resource (zeros at
 // kBufOOB): a run of them issues back to back and is waited on once.

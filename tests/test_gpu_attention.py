@@ -222,3 +222,55 @@ def test_transposed_bias_in_place_matches_copy(gpu):
         assert torch.equal(a, b)
     ref_out, _, _ = attention_forward(q.numpy(), k.numpy(), v.numpy(), mask.numpy(), bias.numpy())
     assert max_rel(res[0][0].numpy(), ref_out) <= TOL
+
+
+def _poisoned(t):
+    """t's values at the start of a buffer whose remainder is NaN."""
+    flat = torch.full((t.numel() + 64 * 64 * 8,), float("nan"), device=t.device, dtype=t.dtype)
+    flat[: t.numel()] = t.reshape(-1)
+    return flat[: t.numel()].view(t.shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seq_major,transposed,dtype", [
+    (False, False, torch.bfloat16), (True, True, torch.bfloat16), (True, False, torch.float32)])
+@pytest.mark.parametrize("B,O,H,N,D", [
+    (1, 3, 2, 1, 8), (1, 2, 1, 31, 32), (2, 5, 2, 33, 16), (1, 4, 2, 63, 64), (1, 6, 4, 65, 32),
+    (2, 3, 1, 100, 24), (1, 9, 2, 127, 32), (1, 4, 2, 130, 64), (1, 5, 2, 191, 40)])
+def test_any_sequence_length_equals_the_padded_problem(gpu, B, O, H, N, D, seq_major, transposed,
+                                                       dtype):
+    """N that is not a multiple of 64 (tiles of 64 keys, 32 queries and 128
+    keys of the backward ending inside the sequence) is bitwise the problem
+    padded by the caller with zero rows and -inf keys, and reads nothing
+    past its tensors (NaN there)."""
+    from openfold3_triangle_kernel_amd import turbopairformer_triangle_attention
+
+    print(f"[attn any N] {B, O, H, N, D} seq={seq_major} tr={transposed} {dtype}", flush=True)
+    q, k, v, mask, bias, dout = (t.to(gpu) for t in attention_case(B, O, H, N, D, mask_frac=0.2,
+                                                                   seed=N + D))
+    q, k, v, dout = (t.to(torch.bfloat16) for t in (q, k, v, dout))
+    bias = bias.to(dtype)
+
+    def run(q, k, v, mask, bias, dout):
+        if seq_major:
+            q, k, v = (_poisoned(t.transpose(-2, -3).contiguous()).transpose(-2, -3)
+                       for t in (q, k, v))
+        else:
+            q, k, v = (_poisoned(t) for t in (q, k, v))
+        b = _poisoned(bias.transpose(-1, -2).contiguous()).transpose(-1, -2) if transposed \
+            else _poisoned(bias)
+        xs = [t.requires_grad_(True) for t in (q, k, v, b)]
+        out = turbopairformer_triangle_attention(*xs[:3], _poisoned(mask), xs[3])
+        with torch.no_grad():
+            assert torch.equal(out, turbopairformer_triangle_attention(*xs[:3], mask, xs[3]))
+        return [out, *torch.autograd.grad(out, xs, _poisoned(dout))]
+
+    got = run(q, k, v, mask, bias, dout)
+    p = (-N) % 64
+    pad = torch.nn.functional.pad
+    ref = run(*(pad(t, (0, 0, 0, p)) for t in (q, k, v)), pad(mask, (0, p), value=float("-inf")),
+              pad(bias, (0, p, 0, p)), pad(dout, (0, 0, 0, 0, 0, p)))
+    ref = [ref[0][:, :, :N]] + [t[..., :N, :] for t in ref[1:4]] + [ref[4][..., :N, :N]]
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dbias"), got, ref):
+        assert a.shape == b.shape and torch.isfinite(a.float()).all(), name
+        assert torch.equal(a, b), name
