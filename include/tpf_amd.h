@@ -482,6 +482,25 @@ int tpf_pair_projection_bf16(const void* x, const void* w, int64_t B, int64_t N,
                              int64_t P, int64_t H, int64_t D, void* qkv, void* rest,
                              void* stream);
 
+/* Inference on any number of outer rows (a chunk of them, or all O = N) and
+ * any sequence length: the projection of planes * N pair rows x [planes*N, C]
+ * into qkv [3][planes][H][N][D] and rest [planes*N][P - 3*H*D], and the gated
+ * attention forward over them, qkv [3][B][O][H][N][D], gate logits in columns
+ * [0, H*D) of rest [B*O*N][rest_pitch], mask f32 [B, O, N] and the pair bias of
+ * every pair in columns [0, H) of rows bias [B*N*N][bias_pitch] (flags as above;
+ * TPF_PAIR_OG_TRANSPOSED needs O == N).  Only og and lse are written.  Results equal the calls above where
+ * those apply. */
+int tpf_pair_rows_projection_supported(int64_t P, int64_t C, int64_t H, int64_t D);
+int tpf_pair_rows_projection_bf16(const void* x, const void* w, int64_t planes, int64_t N,
+                                  int64_t C, int64_t P, int64_t H, int64_t D, void* qkv,
+                                  void* rest, void* stream);
+int64_t tpf_attn_pair_rows_forward_workspace_bytes(int64_t B, int64_t N, int64_t H);
+int tpf_attn_pair_rows_forward_bf16(const void* qkv, const void* rest, int64_t rest_pitch,
+                                    const void* bias, int64_t bias_pitch, const float* mask,
+                                    int flags, float* lse, void* og, void* workspace,
+                                    int64_t workspace_bytes, int64_t B, int64_t O, int64_t N,
+                                    int64_t H, int64_t D, double scale, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -94,6 +94,12 @@ SIGNATURES: dict[str, tuple] = {
                _I64, _I64, _F64, _P]),
     "tpf_pair_projection_supported": (_I32, [_I64] * 5),
     "tpf_pair_projection_bf16": (_I32, [_P, _P] + [_I64] * 6 + [_P, _P, _P]),
+    "tpf_pair_rows_projection_supported": (_I32, [_I64] * 4),
+    "tpf_pair_rows_projection_bf16": (_I32, [_P, _P] + [_I64] * 6 + [_P, _P, _P]),
+    "tpf_attn_pair_rows_forward_workspace_bytes": (_I64, [_I64, _I64, _I64]),
+    "tpf_attn_pair_rows_forward_bf16": (
+        _I32, [_P, _P, _I64, _P, _I64, _P, _I32, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
+               _F64, _P]),
     "tpf_layer_norm_forward_bf16": (_I32, [_P] + [_I64] * 7 + [_P, _P, _F64, _P, _P, _P, _P]),
     "tpf_layer_norm_backward_workspace_bytes": (_I64, [_I64, _I64]),
     "tpf_layer_norm_backward_bf16": (_I32, [_P, _P] + [_I64] * 10 + [_P] * 7 + [_I64, _P]),

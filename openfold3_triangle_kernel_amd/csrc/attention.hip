@@ -519,7 +519,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 8)))
         const int d0 = db * 32 + 16 * pp + 8 * hl;
         if (qok && d0 < D) {
           const u32x4 ov = {po[2 * pp][0], po[2 * pp][1], po[2 * pp + 1][0], po[2 * pp + 1][1]};
-          *reinterpret_cast<u32x4*>(orow + d0) = ov;
+          if (out) *reinterpret_cast<u32x4*>(orow + d0) = ov;
           if (res) {
             const u32x4 rv = {pr[2 * pp][0], pr[2 * pp][1], pr[2 * pp + 1][0], pr[2 * pp + 1][1]};
             *reinterpret_cast<u32x4*>(res + orow_off + d0) = rv;
@@ -2474,6 +2474,50 @@ int tpf_attn_pair_forward_bf16(const void* qkv, const void* rest, int64_t rest_p
   // The forward's epilogue applies the output gate (og = o * sigmoid(g)).
   return attn_forward_impl(g, q, q + part, q + 2 * part, mask, r + hc, bv, B, o, lse, residual,
                            workspace, s, fn, r, og);
+}
+
+int64_t tpf_attn_pair_rows_forward_workspace_bytes(int64_t B, int64_t N, int64_t H) {
+  return tpf_attn_forward_workspace_bytes(B, H, N, B);
+}
+
+int tpf_attn_pair_rows_forward_bf16(const void* qkv, const void* rest, int64_t rest_pitch,
+                                    const void* bias, int64_t bias_pitch, const float* mask,
+                                    int flags, float* lse, void* og, void* workspace,
+                                    int64_t workspace_bytes, int64_t B, int64_t O, int64_t N,
+                                    int64_t H, int64_t D, double scale, void* stream) {
+  const char* fn = "tpf_attn_pair_rows_forward_bf16";
+  if (flags & ~(TPF_PAIR_BIAS_TRANSPOSED | TPF_PAIR_OG_TRANSPOSED))
+    return set_error(TPF_ERR_ARG, "%s: unknown flags 0x%x", fn, flags);
+  AttnGeom g;
+  int rc = make_geom(&g, B, O, H, N, D, TPF_ANY_N, B, scale, fn);
+  if (rc) return rc;
+  if (rest_pitch < H * D || rest_pitch % 8 != 0)
+    return set_error(TPF_ERR_SHAPE, "%s: rest pitch %lld must be a multiple of 8 >= H*D", fn,
+                     (long long)rest_pitch);
+  if (bias_pitch < H)
+    return set_error(TPF_ERR_SHAPE, "%s: bias pitch %lld must be at least H", fn,
+                     (long long)bias_pitch);
+  if ((flags & TPF_PAIR_OG_TRANSPOSED) && O != N)
+    return set_error(TPF_ERR_SHAPE, "%s: transposed og needs O == N", fn);
+  if (!qkv || !rest || !bias || !mask || !lse || !og || !workspace)
+    return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
+  if (((uintptr_t)qkv | (uintptr_t)rest | (uintptr_t)og) % 16)
+    return set_error(TPF_ERR_ARG, "%s: qkv, rest and og must be 16-byte aligned", fn);
+  if (workspace_bytes < tpf_attn_pair_rows_forward_workspace_bytes(B, N, H))
+    return set_error(TPF_ERR_ARG, "%s: workspace too small", fn);
+  g.og_t = (flags & TPF_PAIR_OG_TRANSPOSED) != 0;
+  g.gate_pitch = rest_pitch;
+  const bool bt = (flags & TPF_PAIR_BIAS_TRANSPOSED) != 0;
+  BiasView bv;
+  bv.s_bb = N * N * bias_pitch;
+  bv.s_h = 1;
+  bv.s_q = bt ? bias_pitch : N * bias_pitch;
+  bv.s_k = bt ? N * bias_pitch : bias_pitch;
+  bv.H = (int)H;
+  const int64_t part = B * O * H * N * D;
+  const __bf16* q = (const __bf16*)qkv;
+  return attn_forward_impl(g, q, q + part, q + 2 * part, mask, bias, bv, B, nullptr, lse,
+                           nullptr, workspace, (hipStream_t)stream, fn, rest, og);
 }
 
 // Workspace: the attention backward's, then d_o [B, N, N, H*D] bf16 and

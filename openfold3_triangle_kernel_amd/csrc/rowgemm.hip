@@ -39,12 +39,14 @@ constexpr int row_depth() { return KS <= 4 ? 4 : 3; }
 // output columns [0, 3 H D) are q | k | v and go to head-major planes
 // qkv[part][b][i][h][j][d] (the layout the attention kernels stream as
 // contiguous 2 KB tiles), the rest (gate | bias | pad) to rows of pitch
-// ldy in y.  Row r = (b, i, j) of the pair grid; a 32-row block lies in one
-// (b, i) because the sequence length is a multiple of 32.
+// ldy in y.  Row r = (plane, j), plane = (b, i), of the pair grid; the blocks
+// are cut per plane (the last one of a plane holds its N % 32 rows), so a
+// block's q | k | v segments stay contiguous for every sequence length.
 struct RowSplit {
   __bf16* qkv;
-  int64_t part_elems;  // B * N * H * N * D
+  int64_t part_elems;  // planes * H * N * D
   int Nseq, H, D;
+  FastDiv fbp;         // 32-row blocks per plane
 };
 
 // Gate-backward epilogue of the triangle-attention module (MODE = kRowGate /
@@ -153,6 +155,12 @@ __global__ __launch_bounds__(64 * kRowNW) void rowgemm_ws_kernel(
     // x rows of the block: consecutive, or (og_t) the pair rows
     // (b, i, j0 + r) at dout rows (b, j0 + r, i), N rows apart.
     int64_t xrow0 = bb * 32, xstride = ldx;
+    int64_t rows = R - xrow0;  // rows the block may read
+    if constexpr (SPLIT) {
+      const uint32_t pl = fdiv((uint32_t)bb, sp.fbp), j0 = ((uint32_t)bb - pl * sp.fbp.d) * 32;
+      xrow0 = (int64_t)pl * sp.Nseq + j0;
+      rows = sp.Nseq - (int)j0;
+    }
     if constexpr (GATE) {
       if (gt.og_t) {
         const uint32_t bi = fdiv((uint32_t)bb, gt.fbp), j0 = ((uint32_t)bb - bi * gt.fbp.d) * 32;
@@ -167,7 +175,7 @@ __global__ __launch_bounds__(64 * kRowNW) void rowgemm_ws_kernel(
       const int ci = 256 * j + tid;
       const int r = ci / CPR, slot = ci % CPR;
       const int gc = (slot - r % CPR + CPR) % CPR;
-      const bool ok = vb && bb * 32 + r < R;
+      const bool ok = vb && r < rows;
       buf2lds16(rs_x, ok ? (uint32_t)((r * xstride + 8 * gc) * 2) : kBufOOB,
                 &Xs[stage][(256 * j + 64 * wv) * 8]);
     }
@@ -335,18 +343,18 @@ __global__ __launch_bounds__(64 * kRowNW) void rowgemm_ws_kernel(
         for (int i = 0; i < SIT; ++i)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[i]), rs_y, off[i], 0, 0);
       } else {
-        // Block rows r0 .. r0 + 31 = (b, i, j0 .. j0 + 31).
-        const int64_t r0 = blk * 32;
-        const int64_t bi = r0 / sp.Nseq;               // b * N + i
-        const int j0 = (int)(r0 - bi * sp.Nseq);
-        // Per-thread chunk map (the same for every block): see split_map.
-        __bf16* const qbase = sp.qkv + (bi * sp.H * sp.Nseq + j0) * sp.D;
+        // Block rows (plane, j0 ..), up to 32 of them.
+        const uint32_t pl = fdiv((uint32_t)blk, sp.fbp);
+        const int j0 = (int)((uint32_t)blk - pl * sp.fbp.d) * 32, rows = sp.Nseq - j0;
+        const int64_t r0 = (int64_t)pl * sp.Nseq + j0;
+        // Per-thread chunk map (the same for every block): see smap.
+        __bf16* const qbase = sp.qkv + ((int64_t)pl * sp.H * sp.Nseq + j0) * sp.D;
         __bf16* const rbase = y + r0 * ldy;
         bf16x8 v[SIT];
         __bf16* dst[SIT];
 #pragma unroll
         for (int i = 0; i < SIT; ++i) {
-          const bool ok = smap[i].lds >= 0 && r0 + smap[i].row < R;
+          const bool ok = smap[i].lds >= 0 && smap[i].row < rows;
           v[i] = *reinterpret_cast<const bf16x8*>(&Yb[ok ? smap[i].lds : 0]);
           dst[i] = ok ? (smap[i].rest ? rbase : qbase) + smap[i].off : nullptr;
         }
@@ -431,10 +439,33 @@ int rowgemm_gate_bwd(const __bf16* dout, const __bf16* w_o, int64_t C, const __b
 
 using namespace tpf;
 
+extern "C" int tpf_pair_rows_projection_supported(int64_t P, int64_t K, int64_t H, int64_t D) {
+  return K == 128 && P % 16 == 0 && P <= 640 && D % 8 == 0 && H >= 1 && P >= 3 * H * D + 8 &&
+         (P - 3 * H * D) % 8 == 0;
+}
+
 extern "C" int tpf_pair_projection_supported(int64_t P, int64_t K, int64_t N, int64_t H,
                                              int64_t D) {
-  return K == 128 && P % 16 == 0 && P <= 640 && N % 32 == 0 && D % 8 == 0 && H >= 1 &&
-         P >= 3 * H * D + 8 && (P - 3 * H * D) % 8 == 0;
+  return N % 32 == 0 && tpf_pair_rows_projection_supported(P, K, H, D);
+}
+
+// planes x N rows of the pair grid, any N.
+static int pair_projection(const void* x, const void* w, int64_t planes, int64_t N, int64_t C,
+                           int64_t P, int64_t H, int64_t D, void* qkv, void* rest, void* stream,
+                           const char* fn) {
+  if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)qkv | (uintptr_t)rest) % 16)
+    return set_error(TPF_ERR_ARG, "%s: pointers must be 16-byte aligned", fn);
+  const int64_t R = planes * N, rest_pitch = P - 3 * H * D;
+  const int64_t per_plane = (N + 31) / 32, nblocks = planes * per_plane;
+  if (nblocks >= (int64_t)1 << 31)
+    return set_error(TPF_ERR_SHAPE, "%s: %lld row blocks exceed 2^31", fn, (long long)nblocks);
+  const unsigned grid = (unsigned)(nblocks < device_cus() ? nblocks : device_cus());
+  const RowSplit sp{(__bf16*)qkv, R * H * D, (int)N, (int)H, (int)D,
+                    make_fastdiv((uint32_t)per_plane)};
+  hipLaunchKernelGGL((rowgemm_ws_kernel<4, 5, kRowSplit>), dim3(grid), dim3(64 * kRowNW), 0,
+                     (hipStream_t)stream, (const __bf16*)x, C, (const __bf16*)w, 1, C,
+                     (__bf16*)rest, rest_pitch, R, (int)P, nblocks, sp, RowGate{});
+  return check_launch(fn);
 }
 
 extern "C" int tpf_pair_projection_bf16(const void* x, const void* w, int64_t B, int64_t N,
@@ -445,14 +476,16 @@ extern "C" int tpf_pair_projection_bf16(const void* x, const void* w, int64_t B,
   if (B < 1 || N < 1 || !tpf_pair_projection_supported(P, C, N, H, D))
     return set_error(TPF_ERR_SHAPE, "%s: unsupported shape (C=%lld P=%lld N=%lld H=%lld D=%lld)",
                      fn, (long long)C, (long long)P, (long long)N, (long long)H, (long long)D);
-  if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)qkv | (uintptr_t)rest) % 16)
-    return set_error(TPF_ERR_ARG, "%s: pointers must be 16-byte aligned", fn);
-  const int64_t R = B * N * N, rest_pitch = P - 3 * H * D;
-  const int64_t nblocks = (R + 31) / 32;
-  const unsigned grid = (unsigned)(nblocks < device_cus() ? nblocks : device_cus());
-  const RowSplit sp{(__bf16*)qkv, B * N * H * N * D, (int)N, (int)H, (int)D};
-  hipLaunchKernelGGL((rowgemm_ws_kernel<4, 5, kRowSplit>), dim3(grid), dim3(64 * kRowNW), 0,
-                     (hipStream_t)stream, (const __bf16*)x, C, (const __bf16*)w, 1, C,
-                     (__bf16*)rest, rest_pitch, R, (int)P, nblocks, sp, RowGate{});
-  return check_launch(fn);
+  return pair_projection(x, w, B * N, N, C, P, H, D, qkv, rest, stream, fn);
+}
+
+extern "C" int tpf_pair_rows_projection_bf16(const void* x, const void* w, int64_t planes,
+                                             int64_t N, int64_t C, int64_t P, int64_t H, int64_t D,
+                                             void* qkv, void* rest, void* stream) {
+  const char* fn = "tpf_pair_rows_projection_bf16";
+  if (!x || !w || !qkv || !rest) return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
+  if (planes < 1 || N < 1 || N > INT32_MAX || !tpf_pair_rows_projection_supported(P, C, H, D))
+    return set_error(TPF_ERR_SHAPE, "%s: unsupported shape (C=%lld P=%lld N=%lld H=%lld D=%lld)",
+                     fn, (long long)C, (long long)P, (long long)N, (long long)H, (long long)D);
+  return pair_projection(x, w, planes, N, C, P, H, D, qkv, rest, stream, fn);
 }

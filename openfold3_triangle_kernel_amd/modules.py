@@ -44,9 +44,11 @@ from torch import nn
 from . import _native, routing
 from .attention import (
     _device_ctx,
+    _device_supported,
     is_turbopairformer_supported,
     shadow_enabled,
     turbopairformer_triangle_attention,
+    validate_attention_policy,
 )
 from .attention_fp32 import turbopairformer_attention_fp32
 from .layernorm import layer_norm_bf16
@@ -147,6 +149,26 @@ def _pair_projection(x2: torch.Tensor, wa: torch.Tensor, B: int, N: int, H: int,
     return qkv, proj[:, 3 * hc:].contiguous()
 
 
+def _pair_rows_projection(x2: torch.Tensor, wa: torch.Tensor, B: int, O: int, N: int, H: int,
+                          D: int):
+    """``_pair_projection`` for inference over B * O planes of any N positions:
+    qkv [3, B, O, H, N, D] and gate | bias | pad rows [B*O*N, P - 3 H D]."""
+    R, C = x2.shape
+    P, hc = wa.shape[0], H * D
+    dev = x2.device
+    qkv = torch.empty((3, B, O, H, N, D), device=dev, dtype=torch.bfloat16)
+    if _native.query("tpf_pair_rows_projection_supported", P, C, H, D):
+        rest = torch.empty((R, P - 3 * hc), device=dev, dtype=torch.bfloat16)
+        x2 = x2.contiguous()
+        with _device_ctx(dev):
+            _native.call("tpf_pair_rows_projection_bf16", x2.data_ptr(), wa.data_ptr(), B * O, N,
+                         C, P, H, D, qkv.data_ptr(), rest.data_ptr(), _native.stream_of(x2))
+        return qkv, rest
+    proj = _mm(x2, wa, True)
+    qkv.copy_(proj[:, :3 * hc].view(B, O, N, 3, H, D).permute(3, 0, 1, 4, 2, 5))
+    return qkv, proj[:, 3 * hc:].contiguous()
+
+
 def _pair_flags(transpose_bias: bool, og_t: bool) -> int:
     """Flags of the pair-row entry points (TPF_PAIR_BIAS_TRANSPOSED = 1,
     TPF_PAIR_OG_TRANSPOSED = 2)."""
@@ -232,6 +254,39 @@ class _PairAttentionCore(torch.autograd.Function):
         dx = _mm(dproj, wa, False).view(B, N, N, C) if ctx.needs_input_grad[0] else None
         dw_all = _wgrad(dproj, x2, ctx.w_dtypes[0]) if ctx.needs_input_grad[1] else None
         return dx, dw_all, dw_o, None, None, None, None, None
+
+
+class _PairAttentionInference(torch.autograd.Function):
+    """``_PairAttentionCore`` without a backward, for any N and any number of
+    outer rows: x [B, O, N, C] holds O outer rows of the pair grid (all of
+    them, or a chunk) and ``bias_rows`` ([B*N*N, pitch], the H pair-bias values
+    first) the bias of every pair; None takes it from x's own projection
+    (O == N).  The same kernels and rounding as the training core."""
+
+    @staticmethod
+    def forward(ctx, x, w_all, w_o, mask_add, bias_rows, H, D, transpose_bias, og_t):
+        B, O, N, C = x.shape
+        R, hc = B * O * N, H * D
+        dev = x.device
+        wa = w_all.to(torch.bfloat16)
+        wo = w_o.to(torch.bfloat16).contiguous()
+        qkv, rest = _pair_rows_projection(x.reshape(R, C), wa, B, O, N, H, D)
+        bias = rest[:, hc:] if bias_rows is None else bias_rows
+        og = torch.empty((R, hc), device=dev, dtype=torch.bfloat16)
+        lse = torch.empty((B, O, H, N), device=dev, dtype=torch.float32)
+        ws_bytes = int(_native.query("tpf_attn_pair_rows_forward_workspace_bytes", B, N, H))
+        ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+        with _device_ctx(dev):
+            _native.call("tpf_attn_pair_rows_forward_bf16", qkv.data_ptr(), rest.data_ptr(),
+                         rest.shape[1], bias.data_ptr(), bias.stride(0), mask_add.data_ptr(),
+                         _pair_flags(transpose_bias, og_t), lse.data_ptr(), og.data_ptr(),
+                         ws.data_ptr(), ws_bytes, B, O, N, H, D, 1.0 / math.sqrt(D),
+                         _native.stream_of(og))
+        return _mm(og, wo, True).view(B, O, N, C)
+
+    @staticmethod
+    def backward(ctx, dout):  # pragma: no cover - only called without gradients
+        raise RuntimeError("the inference core has no backward")
 
 
 class _ProjLinear(torch.autograd.Function):
@@ -413,6 +468,8 @@ class TriangleAttention(nn.Module):
         mask_bias = (self.inf * (mask.float() - 1))[..., :, None, None, :]
         m = self.mha
         H, c = m.no_heads, m.c_hidden
+        if self._pair_inference(x, chunk_size):
+            return self._pair_inference_forward(x, mask_bias, transpose_bias, chunk_size)
         if chunk_size is not None and chunk_size < x.shape[-3]:
             return self._chunked_forward(x, mask_bias, transpose_bias, chunk_size)
         # One projection GEMM for q, k, v, the gate and the pair bias.  Rows are
@@ -458,6 +515,59 @@ class TriangleAttention(nn.Module):
             return self._stock_forward_from_ln(x, mask_bias, tri_bias, q, k, v, gp)
         g = torch.sigmoid(gp).reshape(o.shape)
         return _linear((o * g).flatten(-2), m.linear_o.weight)
+
+    def _pair_inference(self, x, chunk_size) -> bool:
+        """Whether inference runs the pair-row core: BF16 square pairs on the
+        kernels' device without gradients, within the limits of the
+        per-projection route's support verdict.  Every N: at N = 613, C = 128
+        the per-projection route, with its gate and layout passes in torch,
+        takes 821 us and the core 534."""
+        H, c, N = self.mha.no_heads, self.mha.c_hidden, x.shape[-2]
+        if not (x.dtype == torch.bfloat16 and x.is_cuda and x.shape[-3] == N and x.numel() > 0
+                and c % 8 == 0 and 8 <= c <= 64 and H <= 16 and self.c_in % 8 == 0
+                and math.prod(x.shape[:-2]) <= 65_535 and N <= 8192):
+            return False
+        if x.dim() < 4 and (N % 64 or chunk_size is not None):
+            return False
+        if torch.is_grad_enabled() and (x.requires_grad or any(
+                p.requires_grad for p in self.parameters())):
+            return False
+        return _device_supported(x)[0]
+
+    def _pair_inference_forward(self, x, mask_bias, transpose_bias, chunk_size):
+        """The pair-row core over all outer rows, or over chunks of them with
+        the bias of every pair projected once (the reference's
+        ``_chunk_stable``, ``triangular_attention.py:114-158``).  A projection
+        row and an attention plane do not depend on the chunk they are in."""
+        m = self.mha
+        H, c, N, C = m.no_heads, m.c_hidden, x.shape[-2], self.c_in
+        shadow_enabled()  # the policy variables are checked as in training
+        if N % 64:
+            validate_attention_policy()
+        B = math.prod(x.shape[:-3])
+        pad = (-(4 * H * c + H)) % 64  # 128-byte aligned rows, as in training
+        zeros = self.linear_z.weight.new_zeros
+        w_all = torch.cat([m.linear_q.weight, m.linear_k.weight, m.linear_v.weight,
+                           m.linear_g.weight, self.linear_z.weight]
+                          + ([zeros(pad, C)] if pad else []))
+        x4, mask_add = x.reshape(B, N, N, C), mask_bias.reshape(B, N, N)
+        og_t = not self.starting
+        if chunk_size is None or chunk_size >= N:
+            out = _PairAttentionInference.apply(x4, w_all, m.linear_o.weight, mask_add.contiguous(),
+                                                None, H, c, bool(transpose_bias), og_t)
+            out = out.reshape(x.shape)
+            return out.transpose(-2, -3) if og_t else out
+        # 16 output channels: the row kernel's tile, so a bias value has the
+        # bits it has among the other projections.
+        w_z = torch.cat([self.linear_z.weight, zeros((-H) % 16, C)]).to(torch.bfloat16)
+        bias_rows = _mm(x4.reshape(-1, C), w_z, True)
+        out = torch.empty_like(x4)
+        for start in range(0, N, chunk_size):
+            rows = slice(start, min(start + chunk_size, N))
+            out[:, rows] = _PairAttentionInference.apply(
+                x4[:, rows].contiguous(), w_all, m.linear_o.weight, mask_add[:, rows].contiguous(),
+                bias_rows, H, c, bool(transpose_bias), False)
+        return out.reshape(x.shape)
 
     def _attend(self, q, k, v, mask_bias, tri_bias, x_dtype, fp32_inference):
         """Attention core on sequence-major q / k / v views (or None when the

@@ -192,3 +192,29 @@ def test_pair_projection_split(gpu, B, N, H, D):
     assert torch.equal(rest.view(torch.int16), y[:, 3 * hc:].contiguous().view(torch.int16))
     ref = x.double().cpu() @ w.double().cpu().t()
     assert max_rel(y.float().cpu().numpy(), ref.numpy()) <= 8e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("planes,N,H,D", [(3, 1, 4, 32), (5, 31, 2, 16), (4, 33, 4, 32), (2, 95, 1, 64)])
+def test_pair_rows_projection_any_n(gpu, planes, N, H, D):
+    """tpf_pair_rows_projection_bf16 (blocks cut per plane, the last one of a
+    plane short) is bitwise the row GEMM's plain output rearranged."""
+    from openfold3_triangle_kernel_amd import _native
+
+    C, hc, R = 128, H * D, planes * N
+    P = (4 * hc + H + 15) // 16 * 16
+    g = torch.Generator(device="cpu").manual_seed(N)
+    x = torch.randn(R, C, generator=g).to(torch.bfloat16).to(gpu)
+    w = torch.randn(P, C, generator=g).to(torch.bfloat16).to(gpu)
+    qkv = torch.full((3, planes, H, N, D), float("nan"), device=gpu, dtype=torch.bfloat16)
+    rest = torch.full((R, P - 3 * hc), float("nan"), device=gpu, dtype=torch.bfloat16)
+    y = torch.empty((R, P), device=gpu, dtype=torch.bfloat16)
+    stream = torch.cuda.current_stream().cuda_stream
+    print(f"pair rows projection planes={planes} N={N} H={H} D={D} P={P}", flush=True)
+    _native.call("tpf_pair_rows_projection_bf16", x.data_ptr(), w.data_ptr(), planes, N, C, P, H, D,
+                 qkv.data_ptr(), rest.data_ptr(), stream)
+    _native.call("tpf_gemm_bf16", x.data_ptr(), 1, C, 0, w.data_ptr(), 1, C, 0, y.data_ptr(), 0, P,
+                 0, R, P, C, 1, 1.0, stream)
+    want = y[:, :3 * hc].reshape(planes, N, 3, H, D).permute(2, 0, 3, 1, 4)
+    assert torch.equal(qkv, want)
+    assert torch.equal(rest, y[:, 3 * hc:])

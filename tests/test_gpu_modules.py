@@ -221,3 +221,36 @@ def test_trimul_module_backward(gpu, outgoing, N):
         err = max_rel(a.detach().float().cpu().numpy(), b.detach().float().cpu().numpy())
         print(f"trimul module out={outgoing} N={N} {name} max-rel {err:.3e}", flush=True)
         assert err <= 2e-2, f"{name}: {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,C,D", [(1, 2, 128, 32), (1, 33, 64, 16), (2, 50, 128, 32),
+                                     (1, 65, 128, 24), (1, 131, 128, 32), (1, 128, 64, 32)])
+@pytest.mark.parametrize("starting,transpose_bias", [(True, False), (False, False), (False, True)])
+def test_triangle_attention_module_inference_any_n(gpu, starting, transpose_bias, B, N, C, D):
+    """Inference runs the pair-row core at every N (32-row projection blocks
+    and 64-key tiles ending inside a row): max-rel <= 2e-2 against the FP32
+    stock math, and chunks of outer rows are bitwise the whole (even chunk
+    sizes: the forward pairs outer rows)."""
+    from openfold3_triangle_kernel_amd import TriangleAttention, stock_invocation_count
+
+    torch.manual_seed(N)
+    m = TriangleAttention(C, D, 4, starting=starting).to(gpu)
+    for p in m.parameters():
+        p.data = p.data.normal_(std=0.1 if p.dim() == 2 else 1.0).bfloat16().float()
+    x = torch.randn(B, N, N, C, device=gpu).bfloat16().float()
+    mask = (torch.rand(B, N, N, device=gpu) > 0.1).float()
+    mask.diagonal(dim1=1, dim2=2).fill_(1)
+    print(f"module inference B={B} N={N} C={C} D={D} starting={starting} tb={transpose_bias}",
+          flush=True)
+    with torch.no_grad():
+        ref = _stock_triangle_attention(m, x, mask, starting, transpose_bias)
+        mb, xb, kb = m.to(torch.bfloat16), x.bfloat16(), mask.bfloat16()
+        before = stock_invocation_count()
+        out = mb(xb, kb, transpose_bias=transpose_bias)
+        chunks = [mb(xb, kb, transpose_bias=transpose_bias, chunk_size=c) for c in (2, 16, N + 1)]
+    assert stock_invocation_count() == before
+    assert all(torch.equal(out, c) for c in chunks)
+    assert max_rel(out.float().cpu().numpy(), ref.cpu().numpy()) <= 2e-2
+    if N % 64 == 0:  # the training core's forward
+        assert torch.equal(out, mb(xb.requires_grad_(True), kb, transpose_bias=transpose_bias))
