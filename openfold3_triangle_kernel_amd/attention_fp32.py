@@ -6,9 +6,10 @@ Mirrors the reference's FP32 path
 (unscaled) q, all inputs FP32, q/k/v ``[*B, O, H, N, D]``, the mask
 broadcasting exactly to ``[*B, O, 1, 1, N]`` and the bias to
 ``[*B, 1, H, N, N]``; returns contiguous FP32 ``[*B, O, N, H, D]``.  No
-autograd: calling it with gradients enabled raises.  Products and sums run
-in FP32 on the matrix cores (``csrc/attention_f32.hip``); a row whose logits
-are all ``-inf`` gives zeros.
+autograd: calling it with gradients enabled raises.  Products are FP32 (each
+operand as the exact sum of three bf16 values on the matrix cores), sums and
+softmax FP32 (``csrc/attention_f32.hip``); a row whose logits are all ``-inf``
+gives zeros.
 """
 
 from __future__ import annotations
@@ -20,7 +21,7 @@ import torch
 from . import _native
 from .attention import _device_ctx, _device_supported, _storage_order
 
-_PAD_QUANTUM = 64
+_ANY_N = 8  # include/tpf_amd.h TPF_ANY_N
 _DEFAULT_WORKSPACE_BYTES = 64 * 1024 * 1024
 _INVOCATIONS = 0
 
@@ -92,17 +93,11 @@ def turbopairformer_attention_fp32(q, k, v, res_mask, pair_bias, *,
     batch = math.prod(prefix)
     scale = 1.0 / math.sqrt(head_dim)
     head_pad = (-head_dim) % 4
-    seq_pad = (-sequence) % _PAD_QUANTUM
-    n_k = sequence + seq_pad
     d_k = head_dim + head_pad
     mask = res_mask.expand(prefix + (outer, 1, 1, sequence)).reshape(batch, outer, sequence)
     bias = pair_bias
     if head_pad:
         q, k, v = (torch.nn.functional.pad(t, (0, head_pad)) for t in (q, k, v))
-    if seq_pad:
-        q, k, v = (torch.nn.functional.pad(t, (0, 0, 0, seq_pad)) for t in (q, k, v))
-        bias = torch.nn.functional.pad(bias, (0, seq_pad, 0, seq_pad))
-        mask = torch.nn.functional.pad(mask, (0, seq_pad), value=float("-inf"))
     mask = mask.contiguous()
     tail = tuple(q.shape[-4:])
     qf, kf, vf = (t.reshape((batch,) + tail) for t in (q, k, v))
@@ -116,27 +111,29 @@ def turbopairformer_attention_fp32(q, k, v, res_mask, pair_bias, *,
     aligned = (1,) * (len(prefix) - len(bias_prefix)) + bias_prefix
     if all(x == 1 for x in aligned):
         bias_batches = 1
-        bias_k = bias.reshape(1, heads, n_k, n_k).contiguous()
+        bias_k = bias.reshape(1, heads, sequence, sequence).contiguous()
     else:
         bias_batches = batch
-        bias_k = bias.expand(prefix + tuple(bias.shape[-4:])).reshape(batch, heads, n_k, n_k).contiguous()
+        bias_k = bias.expand(prefix + tuple(bias.shape[-4:])).reshape(
+            batch, heads, sequence, sequence).contiguous()
     if any(t.data_ptr() % 16 for t in (qf, kf, vf, mask, bias_k)):
         qf, kf, vf, mask, bias_k = (t.contiguous().clone() for t in (qf, kf, vf, mask, bias_k))
         seq_major = False
     dev = q.device
-    out = torch.empty((batch, outer, n_k, heads, d_k), device=dev, dtype=torch.float32)
-    ws_bytes = int(_native.query("tpf_attn_forward_f32_workspace_bytes", batch, heads, n_k,
+    out = torch.empty((batch, outer, sequence, heads, d_k), device=dev, dtype=torch.float32)
+    ws_bytes = int(_native.query("tpf_attn_forward_f32_workspace_bytes", batch, heads, sequence,
                                  bias_batches))
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
     with _device_ctx(dev):
         _native.call(
             "tpf_attn_forward_f32", qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), mask.data_ptr(),
             bias_k.data_ptr(), out.data_ptr(), None, ws.data_ptr(), ws_bytes, batch, outer, heads,
-            n_k, d_k, int(seq_major), bias_batches, scale, _native.stream_of(qf),
+            sequence, d_k, int(seq_major) | (_ANY_N if sequence % 64 else 0), bias_batches, scale,
+            _native.stream_of(qf),
         )
     _INVOCATIONS += 1
-    if seq_pad or head_pad:
-        out = out[:, :, :sequence, :, :head_dim].contiguous()
+    if head_pad:
+        out = out[..., :head_dim].contiguous()
     return out.reshape(prefix + (outer, sequence, heads, head_dim))
 
 

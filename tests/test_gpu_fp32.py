@@ -158,6 +158,8 @@ TRIMUL_CASES = [
     (1, 96, 128, 96, False, True, False, True, "bool"),
     (1, 36, 64, 150, True, False, False, True, "float"),   # 16 channels per thread, H4 pad
     (1, 32, 48, 30, False, True, False, True, "float"),    # 8 channels per thread, H4 pad
+    (2, 35, 128, 200, False, False, False, True, "float"),  # 1 pad position, 16 channels per thread
+    (1, 129, 32, 32, True, False, False, True, "float"),    # 3 pad positions, tiles end past N
 ]
 
 
@@ -188,3 +190,67 @@ def test_trimul_fp32(gpu, case):
     ref, _ = trimul_forward(z.double().numpy(), mask_np, _oracle_weights(m, C, H), outgoing)
     err = max_rel(out.cpu().numpy(), ref)
     assert err <= TOL, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seq_major", [False, True])
+@pytest.mark.parametrize("B,O,H,N,D", [(1, 2, 1, 1, 4), (1, 3, 2, 31, 32), (2, 2, 2, 33, 20),
+                                       (1, 2, 2, 63, 64), (1, 4, 2, 95, 44), (1, 3, 1, 130, 32)])
+def test_attention_fp32_any_sequence_length(gpu, B, O, H, N, D, seq_major):
+    """N that is not a multiple of 64 is bitwise the caller-padded problem and
+    reads nothing past its tensors (NaN there); <= 1e-4 against the oracle."""
+    from openfold3_triangle_kernel_amd import turbopairformer_attention_fp32
+
+    print(f"[fp32 attn any N] {B, O, H, N, D} seq={seq_major}", flush=True)
+    q, k, v, mask, bias = _f32_case(B, O, H, N, D, mask_tail=max(0, min(7, N - 1)), seed=N)
+
+    def poisoned(t):
+        flat = torch.full((t.numel() + 64 * 64 * 8,), float("nan"), device=gpu)
+        flat[: t.numel()] = t.reshape(-1)
+        return flat[: t.numel()].view(t.shape)
+
+    def run(q, k, v, mask, bias):
+        if seq_major:
+            q, k, v = (poisoned(t.transpose(-2, -3).contiguous()).transpose(-2, -3)
+                       for t in (q, k, v))
+        else:
+            q, k, v = (poisoned(t) for t in (q, k, v))
+        with torch.no_grad():
+            return turbopairformer_attention_fp32(q, k, v, poisoned(mask), poisoned(bias))
+
+    out = run(*(t.to(gpu) for t in (q, k, v, mask, bias)))
+    p, pad = (-N) % 64, torch.nn.functional.pad
+    ref = run(*(pad(t, (0, 0, 0, p)).to(gpu) for t in (q, k, v)),
+              pad(mask, (0, p), value=float("-inf")).to(gpu), pad(bias, (0, p, 0, p)).to(gpu))
+    assert torch.equal(out, ref[:, :, :N])
+    want, _, _ = attention_forward(q.numpy(), k.numpy(), v.numpy(), mask.numpy(), bias.numpy())
+    assert max_rel(out.cpu().numpy(), want) <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -60, 2.0 ** 50])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (130, 65, 36), (257, 128, 100)])
+def test_gemm_f32_products_are_fp32(gpu, M, N, K, scale):
+    """tpf_gemm_f32 forms its products from three-way bf16 splits: rel-L2
+    against FP64 within 2 K^0.5 eps (K additions of random sign; a dropped
+    split term of 2^-16 would exceed it), whatever the operands' magnitude,
+    and exact on values of one split part."""
+    from openfold3_triangle_kernel_amd import _native
+
+    g = torch.Generator().manual_seed(M + K)
+    Np = (N + 3) // 4 * 4
+    a, b = torch.randn(M, K, generator=g) * scale, torch.randn(Np, K, generator=g) * scale
+
+    def run(a, b):
+        a, b = a.to(gpu), b.to(gpu)
+        c = torch.empty(M, Np, device=gpu)
+        _native.call("tpf_gemm_f32", a.data_ptr(), 1, K, 0, b.data_ptr(), 1, K, 0, c.data_ptr(), Np,
+                     0, M, Np, K, 1, 1.0, None, torch.cuda.current_stream().cuda_stream)
+        return c.cpu().double()
+
+    ref = a.double() @ b.double().t()
+    err = ((run(a, b) - ref).norm() / ref.norm()).item()
+    print(f"gemm f32 M={M} N={N} K={K} scale={scale:.1e} rel {err:.2e}", flush=True)
+    assert err <= 2 * K ** 0.5 * 2.0 ** -24
+    ai, bi = torch.randint(-9, 10, (M, K), generator=g).float(), torch.randint(-9, 10, (Np, K), generator=g).float()
+    assert torch.equal(run(ai, bi), ai.double() @ bi.double().t())
