@@ -1,5 +1,6 @@
-// FP32 MFMA GEMM main loop (gfx950 v_mfma_f32_32x32x2_f32, 256 threads =
-// 4 waves per workgroup), for the inference-only FP32 paths.
+// FP32 GEMM main loop on the bf16 matrix cores (split_f32.hpp: every operand
+// element as three bf16 values, six products; 256 threads = 4 waves per
+// workgroup), for the inference-only FP32 paths.
 //
 //   acc(m, n) = sum_{k in [kbeg, kend)} A(m, k) * B(n, k)     (all f32)
 //
@@ -7,10 +8,10 @@
 // (wm, wn) = (w >> 1, w & 1) as 2 x 2 accumulators in the 32x32 MFMA layout
 //   acc[i][j] register r <-> m = 64 wm + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4,
 //                            n = 64 wn + 32 j + lane % 32.
-// One 32x32x2 MFMA consumes one k value per lane half; the k index is a pure
-// summation index, so within every group of 8 k the lanes of the lower half
-// supply k = 0..3 and those of the upper half k = 4..7 across four MFMAs,
-// each lane feeding all four from one 16-byte LDS read.
+// The tiles stay f32 in LDS and a wave splits its fragments after reading
+// them: 5.5 VALU instructions per element, about as many cycles as the 24
+// MFMAs of a 16-deep step of the 2 x 2 blocks, and the two waves of a SIMD
+// overlap them.
 //
 // Operands are read from HBM straight into LDS (buffer_load ... lds, zeros
 // outside the tensor), two k-stages in flight.  Either operand may be
@@ -18,11 +19,13 @@
 //      16-byte chunk c of row r stored at slot c ^ (r & 7);
 //   MN (MN-contiguous): X[k * ld + row] -- LDS tile [32 k][128 rows],
 //      fragments are 4-byte reads of consecutive rows.
-// A KC operand may gather its rows (the transposed pair order of the
-// incoming TriMul direction, as in gemm_core.hpp).
+// A KC operand may take its rows through a map (RowMap): the TriMul input
+// projection walks the positions of padded planes, in the transposed pair
+// order for the incoming direction.
 #pragma once
 
 #include "common.hpp"
+#include "split_f32.hpp"
 
 namespace tpf {
 
@@ -31,16 +34,26 @@ constexpr int kFTileBytes = kFM * kFK * 4;       // 16 KiB
 constexpr int kFStageBytes = 2 * kFTileBytes;
 constexpr int kFMainLdsBytes = 2 * kFStageBytes;  // 64 KiB
 
-__device__ __forceinline__ f32x16 mfma32f(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
+// Natural pair row of position m = (b*n + i)*np + k of planes of n rows of
+// np >= n positions: (b, i, k), or (b, k, i) when transposed; -1 for the pad
+// positions k >= n.
+struct RowMap {
+  int n = 0, np = 0, transposed = 0;  // n = 0: identity
+  FastDiv div_np{}, div_ps{};         // division by np and n * np
+  __device__ __forceinline__ int64_t row(uint32_t m) const {
+    if (n == 0) return m;
+    const uint32_t b = fdiv(m, div_ps), p = m - b * div_ps.d;
+    const uint32_t i = fdiv(p, div_np), k = p - i * (uint32_t)np;
+    if (k >= (uint32_t)n) return -1;
+    return (int64_t)b * n * n + (transposed ? (int64_t)k * n + i : (int64_t)i * n + k);
+  }
+};
 
 struct GemmOperandF32 {
   const float* p;  // element (0, 0) of this batch item
   int64_t ld;      // leading dimension in elements
   int rows;        // extent of the m (or n) dimension
-  int gather_n;    // KC row gather (0 = none)
-  FastDiv div_n, div_nn;
+  RowMap map = {};  // KC only
 };
 
 template <bool KC>
@@ -63,16 +76,8 @@ struct TileLoaderF32 {
       for (int t = 0; t < 4; ++t) {
         const int row = r0 + 8 * (4 * w + t) + rin;
         uint32_t off = kBufOOB;
-        if (row < op.rows) {
-          int64_t prow = row;
-          if (op.gather_n > 0) {
-            const uint32_t n = op.gather_n, nn = op.div_nn.d;
-            const uint32_t b = fdiv((uint32_t)row, op.div_nn), p = (uint32_t)row - b * nn;
-            const uint32_t i = fdiv(p, op.div_n), k = p - i * n;
-            prow = (int64_t)b * nn + (int64_t)k * n + i;
-          }
-          off = (uint32_t)(prow * op.ld * 4);
-        }
+        const int64_t prow = row < op.rows ? op.map.row((uint32_t)row) : -1;
+        if (prow >= 0) off = (uint32_t)(prow * op.ld * 4);
         row_off[t] = off;
       }
     } else {
@@ -101,21 +106,25 @@ struct TileLoaderF32 {
   }
 };
 
-// The four k values (group g of 8) this lane feeds for rows rbase + lane % 32.
+// The eight k values 16 s + 8 (lane / 32) .. + 7 of row rbase + lane % 32, split.
 template <bool KC>
-__device__ __forceinline__ f32x4 tile_frag_f32(const float* T, int rbase, int g) {
+__device__ __forceinline__ Split8 tile_frag_f32(const float* T, int rbase, int s) {
   const int lane = threadIdx.x & 63, hl = lane >> 5;
-  if (KC) {
-    const int r = rbase + (lane & 31);
-    const int slot = (2 * g + hl) ^ (r & 7);
-    return *reinterpret_cast<const f32x4*>(T + r * kFK + slot * 4);
-  } else {
-    const int col = rbase + (lane & 31);
-    f32x4 v;
+  const int r = rbase + (lane & 31);
+  float v[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = T[(8 * g + 4 * hl + e) * kFM + col];
-    return v;
+  for (int u = 0; u < 2; ++u) {
+    if (KC) {
+      const int slot = (4 * s + 2 * hl + u) ^ (r & 7);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(T + r * kFK + slot * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * u + e] = x[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * u + e] = T[(16 * s + 8 * hl + 4 * u + e) * kFM + r];
+    }
   }
+  return split8(v);
 }
 
 template <bool A_KC, bool B_KC>
@@ -148,19 +157,17 @@ __device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const Gem
     const float* As = reinterpret_cast<const float*>(cur);
     const float* Bs = reinterpret_cast<const float*>(cur + kFTileBytes);
 #pragma unroll
-    for (int g = 0; g < kFK / 8; ++g) {
-      f32x4 af[2], bfr[2];
+    for (int s = 0; s < kFK / 16; ++s) {
+      Split8 af[2], bfr[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        af[t] = tile_frag_f32<A_KC>(As, 64 * wm + 32 * t, g);
-        bfr[t] = tile_frag_f32<B_KC>(Bs, 64 * wn + 32 * t, g);
+        af[t] = tile_frag_f32<A_KC>(As, 64 * wm + 32 * t, s);
+        bfr[t] = tile_frag_f32<B_KC>(Bs, 64 * wn + 32 * t, s);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma32f(af[i][e], bfr[j][e], acc[i][j]);
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32_split(af[i], bfr[j], acc[i][j]);
     }
   }
   lds_barrier();

@@ -25,8 +25,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgsF32 g) {
   const int mt = (int)(r % tm);
   const int z = (int)(r / tm);
   const int m0 = mt * kFM, n0 = nt * kFN;
-  GemmOperandF32 A{g.A + (int64_t)z * g.a_bs, g.a_ld, g.M, g.a_gather_n, g.a_div_n, g.a_div_nn};
-  GemmOperandF32 B{g.B + (int64_t)z * g.b_bs, g.b_ld, g.N, 0, {}, {}};
+  GemmOperandF32 A{g.A + (int64_t)z * g.a_bs, g.a_ld, g.M};
+  GemmOperandF32 B{g.B + (int64_t)z * g.b_bs, g.b_ld, g.N};
   f32x16 acc[2][2];
   gemm_tile_f32<A_KC, B_KC>(A, B, m0, n0, 0, g.K, smem, acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -61,12 +61,6 @@ int gemm_f32_launch(const GemmArgsF32& g0, int a_kc, int b_kc, int batch, hipStr
       ((uintptr_t)g.A % 16) || ((uintptr_t)g.B % 16) || (g.a_bs % 4) || (g.b_bs % 4))
     return set_error(TPF_ERR_SHAPE, "%s: GEMM operand pitch/padding/alignment requirement violated",
                      fn);
-  if (g.a_gather_n > 0 && !a_kc)
-    return set_error(TPF_ERR_ARG, "%s: row gather needs a K-contiguous A", fn);
-  if (g.a_gather_n > 0) {
-    g.a_div_n = make_fastdiv((uint32_t)g.a_gather_n);
-    g.a_div_nn = make_fastdiv((uint32_t)g.a_gather_n * (uint32_t)g.a_gather_n);
-  }
   const int64_t a_span = a_kc ? (int64_t)g.M * g.a_ld : (int64_t)g.K * g.a_ld;
   const int64_t b_span = b_kc ? (int64_t)g.N * g.b_ld : (int64_t)g.K * g.b_ld;
   if (a_span * 4 >= (int64_t)kBufOOB || b_span * 4 >= (int64_t)kBufOOB)

@@ -28,8 +28,6 @@ struct GemmArgsF32 {
   int M, N, K;
   float alpha;
   const float* bias;
-  int a_gather_n;
-  FastDiv a_div_n, a_div_nn;
   int batch;
 };
 

@@ -1,4 +1,4 @@
-// FP32 triangle multiplicative update, inference only (gfx950 FP32 MFMA).
+// FP32 triangle multiplicative update, inference only (gfx950).
 //
 // The contract of the reference's pure-FP32 TriMul
 // (openfold3/core/kernels/turbopairformer/turbopairformer_trimul_fp32.py:155-400):
@@ -6,7 +6,8 @@
 //   a = mask sigmoid(a_g) a_p, b = mask sigmoid(b_g) b_p;
 //   x_c = A_c B_c^T (outgoing: A_c[i][k] = a[i,k,c]; incoming: a[k,i,c]);
 //   out = (LN_out(x) W_z^T (+ b_z)) * sigmoid(zln W_g^T (+ b_g)).
-// All storage and arithmetic in FP32 (v_mfma_f32_32x32x2_f32).
+// All storage, sums and pointwise arithmetic in FP32; products to within one
+// f32 rounding on the bf16 matrix cores (split_f32.hpp).
 //
 // Layouts (R = B*N*N rows, C4 / H4 = C / H rounded up to 4, zero padded):
 //   zln, gate [R][C4]; xln [R][H4]; a, b, x channel-major [B*H][N][Np]
@@ -25,10 +26,11 @@ namespace tpf {
 struct Tm32Geom {
   int B, N, Np, C, C4, H, H4;
   int64_t NN, PS, R;
+  int64_t Rp;  // B*N*Np plane positions
   int outgoing;
   int ntg;    // gated 128-column weight tiles per branch (64 channels each)
   int ntgo;   // output-gate 128-column tiles
-  FastDiv div_n, div_nn;
+  FastDiv div_np, div_ps;
 };
 
 struct Tm32Weights {
@@ -120,65 +122,9 @@ __global__ __launch_bounds__(256) void tm32_ln_rows_kernel(const float* __restri
   }
 }
 
-// LN_out over the H channels of the channel-major product: 32 positions
-// (natural order) per workgroup, 8 threads per position for the statistics,
-// rows of xln written channel-fastest.
-__global__ __launch_bounds__(256) void tm32_ln_planes_kernel(const float* __restrict__ x,
-                                                             const float* __restrict__ gamma,
-                                                             const float* __restrict__ beta,
-                                                             float eps, float* __restrict__ xln,
-                                                             Tm32Geom g) {
-  constexpr int T = 32, XP = T + 1;
-  __shared__ float Xs[256 * XP];  // [channel][position], H <= 256
-  __shared__ float mu_s[T], rs_s[T];
-  const int tid = threadIdx.x, b = blockIdx.y;
-  const int64_t p0 = (int64_t)blockIdx.x * T;
-  for (int idx = tid; idx < g.H * T; idx += 256) {
-    const int c = idx / T, pp = idx % T;
-    const int64_t p = p0 + pp;
-    float v = 0.f;
-    if (p < g.NN) {
-      const uint32_t i = fdiv((uint32_t)p, g.div_n);
-      v = x[((int64_t)b * g.H + c) * g.PS + (int64_t)i * g.Np + ((uint32_t)p - i * (uint32_t)g.N)];
-    }
-    Xs[c * XP + pp] = v;
-  }
-  __syncthreads();
-  {
-    const int pp = tid >> 3, part = tid & 7;
-    float s = 0.f;
-    for (int c = part; c < g.H; c += 8) s += Xs[c * XP + pp];
-    s = lanes_sum<8>(s);
-    const float mean = s / g.H;
-    float v2 = 0.f;
-    for (int c = part; c < g.H; c += 8) {
-      const float d = Xs[c * XP + pp] - mean;
-      v2 = fmaf(d, d, v2);
-    }
-    v2 = lanes_sum<8>(v2);
-    if (part == 0) {
-      mu_s[pp] = mean;
-      rs_s[pp] = 1.f / sqrtf(v2 / g.H + eps);
-    }
-  }
-  __syncthreads();
-  for (int idx = tid; idx < T * g.H4; idx += 256) {
-    const int pp = idx / g.H4, c = idx % g.H4;
-    const int64_t p = p0 + pp;
-    if (p >= g.NN) continue;
-    float o = 0.f;
-    if (c < g.H) {
-      o = (Xs[c * XP + pp] - mu_s[pp]) * rs_s[pp];
-      if (gamma) o *= gamma[c];
-      if (beta) o += beta[c];
-    }
-    xln[((int64_t)b * g.NN + p) * g.H4 + c] = o;
-  }
-}
-
-// Vector forms of the two LayerNorms (used when the shapes allow 16-byte
-// accesses).  Rows: 16 lanes per row, 16 rows per workgroup; lane l holds
-// the float4 chunks l, l + 16, ... of its row in registers (C <= 64 * NV).
+// LN_in with 16-byte accesses (used when the shapes allow them): 16 lanes per
+// row, 16 rows per workgroup; lane l holds the float4 chunks l, l + 16, ... of
+// its row in registers (C <= 64 * NV).
 template <int NV>
 __global__ __launch_bounds__(256) void tm32_ln_rows_vec_kernel(const float* __restrict__ x,
                                                                int64_t ld_in, int C,
@@ -228,80 +174,17 @@ __global__ __launch_bounds__(256) void tm32_ln_rows_vec_kernel(const float* __re
   }
 }
 
-// Planes: 64 positions per workgroup (N % 4 == 0, so 4 consecutive positions
-// share one row of the plane); float4 loads along positions, LDS
-// [channel][position] with pitch 65, 4 threads per position for the
-// statistics, float4 stores of 4 channels.
-__global__ __launch_bounds__(256) void tm32_ln_planes_vec_kernel(const float* __restrict__ x,
-                                                                 const float* __restrict__ gamma,
-                                                                 const float* __restrict__ beta,
-                                                                 float eps, float* __restrict__ xln,
-                                                                 Tm32Geom g) {
-  constexpr int T = 64, XP = T + 1;
-  __shared__ float Xs[256 * XP];  // [channel][position], H <= 256
-  __shared__ float mu_s[T], rs_s[T];
-  const int tid = threadIdx.x, b = blockIdx.y;
-  const int64_t p0 = (int64_t)blockIdx.x * T;
-  for (int idx = tid; idx < g.H * (T / 4); idx += 256) {
-    const int c = idx / (T / 4), q4 = idx % (T / 4);
-    const int64_t p = p0 + 4 * q4;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (p < g.NN) {
-      const uint32_t i = fdiv((uint32_t)p, g.div_n);
-      v = *reinterpret_cast<const f32x4*>(
-          x + ((int64_t)b * g.H + c) * g.PS + (int64_t)i * g.Np + ((uint32_t)p - i * (uint32_t)g.N));
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Xs[c * XP + 4 * q4 + e] = v[e];
-  }
-  __syncthreads();
-  {
-    const int pp = tid >> 2, part = tid & 3;
-    float s = 0.f;
-    for (int c = part; c < g.H; c += 4) s += Xs[c * XP + pp];
-    s = lanes_sum<4>(s);
-    const float mean = s / g.H;
-    float v2 = 0.f;
-    for (int c = part; c < g.H; c += 4) {
-      const float d = Xs[c * XP + pp] - mean;
-      v2 = fmaf(d, d, v2);
-    }
-    v2 = lanes_sum<4>(v2);
-    if (part == 0) {
-      mu_s[pp] = mean;
-      rs_s[pp] = 1.f / sqrtf(v2 / g.H + eps);
-    }
-  }
-  __syncthreads();
-  const int h4n = g.H4 / 4;
-  for (int idx = tid; idx < T * h4n; idx += 256) {
-    const int pp = idx / h4n, c0 = 4 * (idx % h4n);
-    const int64_t p = p0 + pp;
-    if (p >= g.NN) continue;
-    f32x4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int c = c0 + e;
-      float t = 0.f;
-      if (c < g.H) {
-        t = (Xs[c * XP + pp] - mu_s[pp]) * rs_s[pp];
-        if (gamma) t *= gamma[c];
-        if (beta) t += beta[c];
-      }
-      o[e] = t;
-    }
-    *reinterpret_cast<f32x4*>(xln + ((int64_t)b * g.NN + p) * g.H4 + c0) = o;
-  }
-}
-
-// Planes, register-resident: workgroup = 64 positions x all channels;
-// thread = (4-position group pg = tid % 16, channel group cg = tid / 16 of
+// LN_out over the H channels of the channel-major product, register-resident:
+// workgroup = 64 plane positions x all channels; thread = (4-position group pg = tid % 16, channel group cg = tid / 16 of
 // CPT channels).  Each thread issues all of its CPT float4 loads at once and
 // keeps the CPT x 4 block in registers; per-position channel sums go through
 // the 4 channel groups of a wave by shuffles and the 4 waves through LDS in
 // fixed order (mean first, then the centred sum of squares).  Rows of xln
 // are written as float4 runs of the thread's channels (pad channels up to
-// H4 as zeros).  Needs N % 4 == 0 and H <= 16 * CPT.
+// H4 as zeros).  Needs H <= 16 * CPT.  The walk is over plane positions (Np a
+// multiple of 4, so a thread's four share a plane row); the pad positions of
+// N % 4 != 0 write nothing (two bytes at a time over rows, N = 333 took 62 us
+// against 33).
 template <int CPT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void tm32_ln_planes_reg_kernel(
     const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
@@ -311,19 +194,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
   const int tid = threadIdx.x, wv = tid >> 6, b = blockIdx.y;
   const int pg = tid & 15, cg = tid >> 4;
   const int64_t pb = (int64_t)blockIdx.x * T + 4 * pg;  // first position of this thread
-  const bool pos_ok = pb < g.NN;                       // NN % 4 == 0: all 4 or none
+  const bool pos_ok = pb < g.PS;                       // PS % 4 == 0: all 4 or none
   const int c0 = cg * CPT;
-  int64_t off = 0;
-  if (pos_ok) {
-    const uint32_t i = fdiv((uint32_t)pb, g.div_n);
-    off = (int64_t)i * g.Np + ((uint32_t)pb - i * (uint32_t)g.N);
-  }
+  const uint32_t pi = fdiv((uint32_t)pb, g.div_np);
+  const int col = (int)((uint32_t)pb - pi * (uint32_t)g.Np);
+  const int64_t row0 = (int64_t)b * g.NN + (int64_t)pi * g.N + col;  // row of the first position
   float v[CPT][4];
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     f32x4 t = {0.f, 0.f, 0.f, 0.f};
     if (pos_ok && c0 + c < g.H)
-      t = *reinterpret_cast<const f32x4*>(x + ((int64_t)b * g.H + c0 + c) * g.PS + off);
+      t = *reinterpret_cast<const f32x4*>(x + ((int64_t)b * g.H + c0 + c) * g.PS + pb);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[c][e] = t[e];
   }
@@ -373,10 +254,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
+      if (col + e >= g.N) continue;
       f32x4 o;
 #pragma unroll
       for (int k = 0; k < 4; ++k) o[k] = (v[4 * c4 + k][e] - mean[e]) * rstd[e] * gm[k] + bt[k];
-      *reinterpret_cast<f32x4*>(xln + ((int64_t)b * g.NN + pb + e) * g.H4 + c0 + 4 * c4) = o;
+      *reinterpret_cast<f32x4*>(xln + (row0 + e) * g.H4 + c0 + 4 * c4) = o;
     }
   }
 }
@@ -385,9 +267,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 // mode's 1e-4 bound); the IEEE division made the gating epilogue VALU-bound.
 __device__ __forceinline__ float sigmoid_f32(float x) { return sigmoidf(x); }
 
-// Input projections in stored row order m (natural row = gather of m for
-// the incoming direction).  Gated tiles write a / b planes; output-gate
-// tiles write sigmoid(g) row-major.
+// Input projections over the plane positions m of the stored matrices
+// (natural rows through RowMap; positions without a row read zeros and a zero
+// mask, so their plane stores write the zero pad columns).  Gated tiles write
+// a / b planes, four positions per store; output-gate tiles write sigmoid(g)
+// row-major.
 __global__ __launch_bounds__(256, 2) void tm32_in_proj_kernel(
     const float* __restrict__ zln, const float* __restrict__ wp, const float* __restrict__ bp,
     const float* __restrict__ mask, float* __restrict__ a_pl, float* __restrict__ b_pl,
@@ -397,27 +281,20 @@ __global__ __launch_bounds__(256, 2) void tm32_in_proj_kernel(
   __shared__ float mask_s[128];
   __shared__ int64_t rho_s[128];
   const int tn = 2 * g.ntg + g.ntgo;
-  const int64_t tm = (g.R + 127) / 128;
+  const int64_t tm = (g.Rp + 127) / 128;
   const int64_t T = xcd_order(tm * tn);
   if (T < 0) return;
   const int nt = (int)(T % tn);
   const int64_t m0 = (T / tn) * 128;
+  const RowMap map{g.N, g.Np, !g.outgoing, g.div_np, g.div_ps};
   if (threadIdx.x < 128) {
     const int64_t m = m0 + threadIdx.x;
-    int64_t rho = -1;
-    if (m < g.R) {
-      rho = m;
-      if (!g.outgoing) {
-        const uint32_t bb = fdiv((uint32_t)m, g.div_nn), p = (uint32_t)m - bb * (uint32_t)g.NN;
-        const uint32_t i = fdiv(p, g.div_n), k = p - i * (uint32_t)g.N;
-        rho = (int64_t)bb * g.NN + (int64_t)k * g.N + i;
-      }
-    }
+    const int64_t rho = m < g.Rp ? map.row((uint32_t)m) : -1;
     rho_s[threadIdx.x] = rho;
     mask_s[threadIdx.x] = rho >= 0 ? mask[rho] : 0.f;
   }
-  GemmOperandF32 A{zln, g.C4, (int)g.R, g.outgoing ? 0 : g.N, g.div_n, g.div_nn};
-  GemmOperandF32 W{wp, g.C4, tn * 128, 0, {}, {}};
+  GemmOperandF32 A{zln, g.C4, (int)g.Rp, map};
+  GemmOperandF32 W{wp, g.C4, tn * 128};
   f32x16 acc[2][2];
   gemm_tile_f32<true, true>(A, W, (int)m0, nt * 128, 0, g.C4, smem, acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -459,14 +336,10 @@ __global__ __launch_bounds__(256, 2) void tm32_in_proj_kernel(
     if (c >= g.H) continue;
     const int64_t mb = m0 + 4 * chn;
     const float* s = S + c_l * SP + 4 * chn;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t m = mb + e;
-      if (m >= g.R) break;
-      const uint32_t bb = fdiv((uint32_t)m, g.div_nn), p = (uint32_t)m - bb * (uint32_t)g.NN;
-      const uint32_t i = fdiv(p, g.div_n);
-      planes[((int64_t)bb * g.H + c) * g.PS + (int64_t)i * g.Np + (p - i * (uint32_t)g.N)] = s[e];
-    }
+    if (mb >= g.Rp) continue;
+    const uint32_t bb = fdiv((uint32_t)mb, g.div_ps), p = (uint32_t)mb - bb * (uint32_t)g.PS;
+    *reinterpret_cast<f32x4*>(planes + ((int64_t)bb * g.H + c) * g.PS + p) =
+        *reinterpret_cast<const f32x4*>(s);
   }
 }
 
@@ -480,8 +353,8 @@ __global__ __launch_bounds__(256, 2) void tm32_out_proj_kernel(
   if (T < 0) return;
   const int nt = (int)(T % tn);
   const int64_t m0 = (T / tn) * 128;
-  GemmOperandF32 A{xln, g.H4, (int)g.R, 0, {}, {}};
-  GemmOperandF32 W{wz, g.H4, g.C, 0, {}, {}};
+  GemmOperandF32 A{xln, g.H4, (int)g.R};
+  GemmOperandF32 W{wz, g.H4, g.C};
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rl = lane & 31, hl = lane >> 5, wm = w >> 1, wn = w & 1;
   // The gate values of this lane's accumulator elements are loaded before
@@ -515,11 +388,6 @@ __global__ __launch_bounds__(256, 2) void tm32_out_proj_kernel(
   }
 }
 
-__global__ __launch_bounds__(256) void tm32_zero_kernel(float* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    p[i] = 0.f;
-}
-
 }  // namespace tpf
 
 using namespace tpf;
@@ -539,12 +407,12 @@ static int tm32_geom(Tm32Geom* g, int64_t B, int64_t N, int64_t C, int64_t H, in
       R > INT32_MAX / 2)
     return set_error(TPF_ERR_SHAPE, "%s: B=%lld N=%lld too large", fn, (long long)B, (long long)N);
   g->B = (int)B; g->N = (int)N; g->Np = (int)Np; g->C = (int)C; g->C4 = (int)C4;
-  g->H = (int)H; g->H4 = (int)H4; g->NN = N * N; g->PS = N * Np; g->R = R;
+  g->H = (int)H; g->H4 = (int)H4; g->NN = N * N; g->PS = N * Np; g->R = R; g->Rp = B * N * Np;
   g->outgoing = outgoing ? 1 : 0;
   g->ntg = (int)((H + 63) / 64);
   g->ntgo = (int)((C + 127) / 128);
-  g->div_n = make_fastdiv((uint32_t)N);
-  g->div_nn = make_fastdiv((uint32_t)(N * N));
+  g->div_np = make_fastdiv((uint32_t)Np);
+  g->div_ps = make_fastdiv((uint32_t)(N * Np));
   return TPF_OK;
 }
 
@@ -618,11 +486,6 @@ int tpf_trimul_forward_f32_chunked(const float* z, const float* mask, const floa
   Tm32Weights w{{w_ap, w_ag, w_bp, w_bg, w_g, w_z}, {b_ap, b_ag, b_bp, b_bg, b_g, b_z}};
   hipLaunchKernelGGL(tm32_pack_kernel, dim3(1024), dim3(256), 0, s, w, wk.wp, wk.bp, wk.wz, wk.bz, g);
   if ((rc = check_launch(fn))) return rc;
-  if (g.Np != g.N) {  // contraction reads whole rows of Np: pad columns must be zero
-    // a and b are adjacent regions ending where x begins.
-    hipLaunchKernelGGL(tm32_zero_kernel, dim3(8192), dim3(256), 0, s, wk.a, (int64_t)(wk.x - wk.a));
-    if ((rc = check_launch(fn))) return rc;
-  }
   const bool rows_vec = C % 4 == 0 && ((uintptr_t)z | (uintptr_t)ln_in_w | (uintptr_t)ln_in_b) % 16 == 0;
   const int nv = (int)((C / 4 + 15) / 16);  // float4 chunks per lane (C <= 512: <= 8)
   if (rows_vec) {
@@ -641,7 +504,7 @@ int tpf_trimul_forward_f32_chunked(const float* z, const float* mask, const floa
                        (int64_t)g.C4, g.R);
   }
   if ((rc = check_launch(fn))) return rc;
-  const int64_t tiles = (g.R + 127) / 128;
+  const int64_t tiles = (g.Rp + 127) / 128;
   const int64_t ptiles = tiles * (2 * g.ntg + g.ntgo);
   hipLaunchKernelGGL(tm32_in_proj_kernel, dim3((unsigned)((ptiles + 7) / 8 * 8)), dim3(256), 0, s,
                      wk.zln, wk.wp, wk.bp, mask, wk.a, wk.b, wk.gate, g);
@@ -660,20 +523,15 @@ int tpf_trimul_forward_f32_chunked(const float* z, const float* mask, const floa
       if ((rc = gemm_f32_launch(ga, 1, 1, (int)H, s, "tpf_trimul_forward_f32(contract)"))) return rc;
       // The chunk as a one-batch problem of rows * N positions.
       Tm32Geom gc = g;
-      gc.B = 1; gc.NN = rows * N; gc.PS = rows * g.Np; gc.R = rows * N;
+      gc.B = 1; gc.NN = rows * N; gc.PS = rows * g.Np; gc.R = rows * N; gc.Rp = gc.PS;
       const int64_t r0 = bb * g.NN + i0 * N;  // first pair row of the chunk
-      if (N % 4 == 0 && g.Np % 4 == 0 && H <= 128)
-        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<8>, dim3((unsigned)((gc.NN + 63) / 64), 1u),
-                           dim3(256), 0, s, wk.x, ln_out_w, ln_out_b, (float)ln_out_eps, wk.xln, gc);
-      else if (N % 4 == 0 && g.Np % 4 == 0 && H <= 256)
-        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<16>, dim3((unsigned)((gc.NN + 63) / 64), 1u),
-                           dim3(256), 0, s, wk.x, ln_out_w, ln_out_b, (float)ln_out_eps, wk.xln, gc);
-      else if (N % 4 == 0 && g.Np % 4 == 0)
-        hipLaunchKernelGGL(tm32_ln_planes_vec_kernel, dim3((unsigned)((gc.NN + 63) / 64), 1u),
-                           dim3(256), 0, s, wk.x, ln_out_w, ln_out_b, (float)ln_out_eps, wk.xln, gc);
+      const dim3 ln_grid((unsigned)((gc.PS + 63) / 64), 1u);
+      if (H <= 128)
+        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<8>, ln_grid, dim3(256), 0, s, wk.x, ln_out_w,
+                           ln_out_b, (float)ln_out_eps, wk.xln, gc);
       else
-        hipLaunchKernelGGL(tm32_ln_planes_kernel, dim3((unsigned)((gc.NN + 31) / 32), 1u),
-                           dim3(256), 0, s, wk.x, ln_out_w, ln_out_b, (float)ln_out_eps, wk.xln, gc);
+        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<16>, ln_grid, dim3(256), 0, s, wk.x, ln_out_w,
+                           ln_out_b, (float)ln_out_eps, wk.xln, gc);
       if ((rc = check_launch(fn))) return rc;
       const int64_t otiles = (gc.R + 127) / 128 * ((C + 127) / 128);
       hipLaunchKernelGGL(tm32_out_proj_kernel, dim3((unsigned)((otiles + 7) / 8 * 8)), dim3(256), 0,
