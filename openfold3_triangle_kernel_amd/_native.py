@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib
 import threading
 from pathlib import Path
 
@@ -167,6 +168,33 @@ def library() -> ctypes.CDLL:
                 fn.argtypes = argtypes
             _LIB = lib
     return _LIB
+
+
+HOST_PATH = LIB_PATH.with_name("_tpf_host.so")
+_PLAIN_TYPES = frozenset((torch.Tensor, torch.nn.Parameter))
+_HOST = None
+
+
+def host():
+    """The extension that runs the operators' host path for plain eager tensors
+    (``csrc/host/torch_host.cpp``), loaded once; None when only the C-ABI
+    library is built (the Python path then serves every call)."""
+    global _HOST
+    if _HOST is None:
+        with _LOCK:
+            if _HOST is None:
+                _HOST = (importlib.import_module("._tpf_host", __package__)
+                         if HOST_PATH.exists() and LIB_PATH.exists() else False)
+    return _HOST or None
+
+
+def host_eligible(*tensors) -> bool:
+    """Plain tensors (or parameters, or None) in eager code: no subclass, no
+    compilation, no tracing.  The extension checks the rest."""
+    for t in tensors:
+        if t is not None and type(t) not in _PLAIN_TYPES:
+            return False
+    return not torch.compiler.is_compiling() and not torch._C._is_tracing()
 
 
 def call(name: str, *args) -> int:

@@ -207,12 +207,14 @@ def set_sr_workspace_budget(budget_bytes: int | None) -> None:
     """Set the backward workspace budget in bytes (None restores the default)."""
     global _SR_WORKSPACE_BUDGET
     if budget_bytes is None:
-        _SR_WORKSPACE_BUDGET = DEFAULT_SR_WORKSPACE_BUDGET_BYTES
-        return
+        budget_bytes = DEFAULT_SR_WORKSPACE_BUDGET_BYTES
     budget_bytes = int(budget_bytes)
     if budget_bytes <= 0:
         raise ValueError("workspace_budget_bytes must be positive")
     _SR_WORKSPACE_BUDGET = budget_bytes
+    host = _native.host()
+    if host is not None:
+        host.set_workspace_budget(budget_bytes)
 
 
 def sr_workspace_plan(B: int, O: int, H: int, N: int, D: int,
@@ -326,11 +328,19 @@ def turbopairformer_triangle_attention(q, k, v, res_mask, pair_bias):
     (``turbopairformer_triangle_attention.py:341-472``).  Unsupported cases raise
     ``ValueError("unsupported TurboPairFormer case: ...")`` before any launch.
     """
+    global _INVOCATIONS
+    if _native.host_eligible(q, k, v, res_mask, pair_bias) and q.is_cuda and _is_gfx950(q.device):
+        # The common form entirely in C++; None (nothing launched) for any
+        # other, which the rest of this function handles or reports.
+        host = _native.host()
+        out = None if host is None else host.attention(q, k, v, res_mask, pair_bias)
+        if out is not None:
+            _INVOCATIONS += 1
+            return out
     validate_attention_policy()
     ok, reason = is_turbopairformer_supported(q, k, v, res_mask, pair_bias)
     if not ok:
         raise ValueError(f"unsupported TurboPairFormer case: {reason}")
-    global _INVOCATIONS
     _INVOCATIONS += 1
     if q.dtype == torch.float32:
         # FP32 inference keeps FP32 storage end to end (reference ``:362-370``).

@@ -3,7 +3,9 @@
 Every HIP source under ``csrc/`` is compiled with hipcc for gfx950 only and
 linked into one C-ABI shared library that sits next to this file.  The
 library exports plain ``extern "C"`` entry points (declared in
-``include/tpf_amd.h``); Python reaches them through ``ctypes``.
+``include/tpf_amd.h``); Python reaches them through ``ctypes``.  A second
+library, the Python extension ``_tpf_host.so`` (``csrc/host/``), runs the two
+operators' host path for plain tensors on top of the first.
 """
 
 from __future__ import annotations
@@ -12,12 +14,16 @@ import concurrent.futures
 import os
 import shutil
 import subprocess
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_NAME = "libtpf_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+HOST_SRC = CSRC / "host" / "torch_host.cpp"
+HOST_NAME = "_tpf_host"
+HOST_PATH = PKG_DIR / f"{HOST_NAME}.so"
 BUILD_DIR = PKG_DIR / "_build"
 ARCH = "gfx950"
 
@@ -54,7 +60,10 @@ def sources() -> list[Path]:
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
-    """Compile every source for gfx950 and link ``libtpf_amd.so`` (always rebuilds)."""
+    """Compile every source and link ``libtpf_amd.so`` and ``_tpf_host.so`` (always
+    rebuilds)."""
+    import torch  # the host extension compiles against torch's headers
+
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     common = [
@@ -74,6 +83,16 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
         extra = (DEVICE_FLAGS + FILE_FLAGS.get(src.name, [])) if src.suffix == ".hip" else []
         lang = ["-x", "hip"] if src.suffix == ".hip" else []
         cmds.append([hipcc, *common, *extra, *lang, "-c", str(src), "-o", str(obj)])
+    torch_dir = Path(torch.__file__).resolve().parent
+    inc = torch_dir / "include"
+    host_obj = BUILD_DIR / "torch_host.o"
+    cmds.insert(0, [
+        hipcc, "-O2", "-std=c++17", "-fPIC", f"-DTORCH_EXTENSION_NAME={HOST_NAME}",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM",
+        "-D__HIP_PLATFORM_AMD__=1", f"-I{PKG_DIR.parent / 'include'}", f"-isystem{inc}",
+        f"-isystem{inc / 'torch' / 'csrc' / 'api' / 'include'}",
+        f"-isystem{sysconfig.get_paths()['include']}", "-Wno-unused-command-line-argument",
+        "-c", str(HOST_SRC), "-o", str(host_obj)])  # first: the longest one
 
     def run(cmd):
         if verbose:
@@ -89,6 +108,11 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     tmp = LIB_PATH.with_suffix(".so.tmp")
     run([hipcc, "-shared", f"--offload-arch={ARCH}", "-fPIC", "-o", str(tmp), *map(str, objs)])
     os.replace(tmp, LIB_PATH)
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    run([hipcc, "-shared", "-fPIC", "-o", str(tmp), str(host_obj), f"-L{torch_dir / 'lib'}", "-lc10",
+         "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", f"-L{PKG_DIR}", f"-l:{LIB_NAME}",
+         "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, HOST_PATH)
     return LIB_PATH
 
 
