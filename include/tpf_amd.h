@@ -267,6 +267,8 @@ int64_t tpf_trimul_forward_workspace_bytes(int64_t C);
 /* Forward: LN_in + projections + gates (trimul_in_fwd), the channel
  * contraction (the reference's torch.bmm), LN_out + projection + gate
  * (trimul_out_fwd).  outgoing = 1: x_ij = sum_k a_ik b_jk; 0: sum_k a_ki b_kj.
+ * xln, mean_out and rstd_out may be null together (no backward follows):
+ * they are then not written.
  * Replaces trimul_in_fwd / torch.bmm / trimul_out_fwd of
  * _trimul_forward_impl (openfold3/core/kernels/turbopairformer/turbopairformer_trimul.py:184-292;
  * kernels turbopairformer_trimul_cuda.cu:615-1166, 1191-1530). */

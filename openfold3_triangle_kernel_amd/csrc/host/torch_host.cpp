@@ -223,18 +223,18 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
 
 int64_t a256(int64_t v) { return (v + 255) / 256 * 256; }
 
-// The forward's state in one allocation: z_ln, gate, a, b, x, xln (bf16), then
-// the LayerNorm statistics (f32).
+// The forward's state in one allocation: z_ln, gate, a, b, x (bf16), LN_in's
+// statistics (f32) and, for a backward, xln (bf16) and LN_out's (f32).
 struct TrimulState {
-  char* p[10];
+  char* p[10] = {};
   int64_t bytes;
-  TrimulState(int64_t B, int64_t N, int64_t C, char* base) {
+  TrimulState(int64_t B, int64_t N, int64_t C, bool save, char* base) {
     const int64_t rows = a256(B * N * N * C * 2);
     const int64_t planes = a256(B * C * N * tpf_trimul_plane_pitch(N) * 2);
     const int64_t stat = a256(B * N * N * 4);
-    const int64_t sizes[10] = {rows, rows, planes, planes, planes, rows, stat, stat, stat, stat};
+    const int64_t sizes[10] = {rows, rows, planes, planes, planes, stat, stat, rows, stat, stat};
     bytes = 0;
-    for (int i = 0; i < 10; ++i) {
+    for (int i = 0; i < (save ? 10 : 7); ++i) {
       p[i] = base + bytes;
       bytes += sizes[i];
     }
@@ -253,8 +253,8 @@ Tensor trimul_forward(const Tensor& z, const Tensor& mask, const variable_list& 
   check(tpf_trimul_forward_bf16(
             z.const_data_ptr(), (const float*)mask.const_data_ptr(), f(0), f(1), f(0) + cc,
             f(1) + cc, f(2), f(3), f(4), f(5), f(6), f(7), outgoing ? 1 : 0, B, N, C,
-            out.data_ptr(), st.p[0], st.p[1], st.p[2], st.p[3], st.p[4], st.p[5], (float*)st.p[6],
-            (float*)st.p[7], (float*)st.p[8], (float*)st.p[9], ws.data_ptr(), ws_bytes, stream()),
+            out.data_ptr(), st.p[0], st.p[1], st.p[2], st.p[3], st.p[4], st.p[7], (float*)st.p[5],
+            (float*)st.p[6], (float*)st.p[8], (float*)st.p[9], ws.data_ptr(), ws_bytes, stream()),
         "tpf_trimul_forward_bf16");
   return out;
 }
@@ -265,9 +265,9 @@ struct TrimulFn : torch::autograd::Function<TrimulFn> {
                         const Tensor& p_out, const Tensor& n_in_w, const Tensor& n_in_b,
                         const Tensor& n_out_w, const Tensor& n_out_b, bool outgoing) {
     const int64_t B = z.size(0), N = z.size(1), C = z.size(3);
-    Tensor state = at::empty({TrimulState(B, N, C, nullptr).bytes}, like(z, at::kByte));
+    Tensor state = at::empty({TrimulState(B, N, C, true, nullptr).bytes}, like(z, at::kByte));
     Tensor out = trimul_forward(z, mask, {p_in, g_in, g_out, p_out, n_in_w, n_in_b, n_out_w, n_out_b},
-                                outgoing, TrimulState(B, N, C, (char*)state.data_ptr()));
+                                outgoing, TrimulState(B, N, C, true, (char*)state.data_ptr()));
     ctx->save_for_backward({z, mask, state, p_in, g_in, g_out, p_out, n_in_w, n_out_w});
     ctx->saved_data["outgoing"] = outgoing;
     return out;
@@ -277,7 +277,7 @@ struct TrimulFn : torch::autograd::Function<TrimulFn> {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &z = s[0], &mask = s[1], &state = s[2];
     const int64_t B = z.size(0), N = z.size(1), C = z.size(3), cc = C * C;
-    const TrimulState st(B, N, C, (char*)state.data_ptr());
+    const TrimulState st(B, N, C, true, (char*)state.data_ptr());
     const Tensor g = grads[0].to(at::kBFloat16).contiguous();
     const auto f32 = like(z, at::kFloat);
     Tensor dz = at::empty({B, N, N, C}, like(z, at::kBFloat16));
@@ -292,7 +292,7 @@ struct TrimulFn : torch::autograd::Function<TrimulFn> {
     check(tpf_trimul_backward_named_bf16(
               g.const_data_ptr(), z.const_data_ptr(), (const float*)mask.const_data_ptr(), f(3),
               f(4), f(3) + cc, f(4) + cc, f(5), f(6), f(7), f(8), st.p[0], st.p[1], st.p[2],
-              st.p[3], st.p[4], st.p[5], (const float*)st.p[6], (const float*)st.p[7],
+              st.p[3], st.p[4], st.p[7], (const float*)st.p[5], (const float*)st.p[6],
               (const float*)st.p[8], (const float*)st.p[9],
               ctx->saved_data["outgoing"].toBool() ? 1 : 0, B, N, C, dz.data_ptr(), o(dp), o(dg),
               o(dgo), o(dpo), o(dn[0]), o(dn[1]), o(dn[2]), o(dn[3]), ws.data_ptr(), ws_bytes,
@@ -340,8 +340,8 @@ std::optional<Tensor> trimul(const Tensor& z, const std::optional<Tensor>& mask_
   if (grad) {
     out = TrimulFn::apply(z4, mask, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], outgoing);
   } else {
-    Tensor scratch = at::empty({TrimulState(B, N, C, nullptr).bytes}, like(z, at::kByte));
-    out = trimul_forward(z4, mask, w, outgoing, TrimulState(B, N, C, (char*)scratch.data_ptr()));
+    Tensor scratch = at::empty({TrimulState(B, N, C, false, nullptr).bytes}, like(z, at::kByte));
+    out = trimul_forward(z4, mask, w, outgoing, TrimulState(B, N, C, false, (char*)scratch.data_ptr()));
   }
   return z.dim() == 4 ? out : out.view(z.sizes());
 }

@@ -24,7 +24,7 @@
 //
 // Kernels of one direction:
 //   forward:  tm_ln_rows (LN_in) -> tm_in_proj_fwd (a, b, gl) -> GEMM x ->
-//             tm_ln_planes (LN_out) -> tm_out_proj<fwd> (out)
+//             tm_out_fwd (LN_out, out)
 //   backward: tm_out_bwd (d gl, dx, LN_out and dWz partials) -> GEMMs da, db
 //             -> tm_in_proj_bwd (d a_p .. d b_g) -> tm_ln_in_bwd (dz, LN_in
 //             partials) -> split-K dW5 GEMM -> fixed-order folds.
@@ -48,23 +48,29 @@ struct TmGeom {
 
 // Block walk of the persistent row kernels: a workgroup runs the virtual
 // blocks [bbeg, bend) and pb(blk) is the 32-row block a virtual block reads:
-// one contiguous range per workgroup, or (strided) blocks g, g + G, ... for
-// workgroup g of G, which keeps the grid on a compact window of rows.  Each
-// kernel takes the walk measured faster for it at N = 384 (strided: LN_in
-// backward 59.2 -> 55.8 us, output projection 23.8 -> 21.4 us; contiguous:
-// the projection backward, whose 64-byte plane stores of consecutive blocks
-// merge, 71.6 against 79.7 us, the projection forward and the output
-// backward).  Either walk depends on the shape and grid only.
+// one contiguous range per workgroup, or (window) blocks l, l + G, ... for
+// logical workgroup l of G, which keeps the grid on a compact window of rows;
+// l numbers the workgroups XCD by XCD (workgroup i runs on XCD i % 8), so that
+// the two 64-byte plane segments of a 128-byte line, in consecutive blocks,
+// meet in one L2 (l = i instead: output pass 33.9 -> 32 us at N = 384, 26.9 ->
+// 25 us at N = 301, 170 -> 168 us at N = 1021).  Each kernel takes the walk
+// measured faster for it (window: LN_in backward 61 -> 58.5 us at N = 384 and
+// the output pass, 34.3 -> 32 us, at N = 1021 186 -> 168 us; contiguous: the
+// projection backward, whose 64-byte plane stores of consecutive blocks merge,
+// 71.4 against 75.7 us, the output backward, 62 against 67.8 us, and the
+// projection forward, at N = 1021 317 against 367 us).  Either walk depends on
+// the shape and grid only.
 #define TM_BLOCKS_CONTIGUOUS(nblocks)                                            \
   const int64_t per = ((nblocks) + gridDim.x - 1) / gridDim.x;                   \
   const int64_t bbeg = blockIdx.x * per;                                         \
   const int64_t bend = bbeg + per < (nblocks) ? bbeg + per : (nblocks);          \
   auto pb = [&](int64_t v) { return v; }
-#define TM_BLOCKS_STRIDED(nblocks)                                               \
+#define TM_BLOCKS_WINDOW(nblocks)                                                \
+  const uint32_t wg_l =                                                          \
+      (gridDim.x & 7) ? blockIdx.x : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); \
   const int64_t bbeg = 0;                                                        \
-  const int64_t bend =                                                           \
-      blockIdx.x < (nblocks) ? ((nblocks) - blockIdx.x + gridDim.x - 1) / gridDim.x : 0; \
-  auto pb = [&](int64_t v) { return v * (int64_t)gridDim.x + blockIdx.x; }
+  const int64_t bend = wg_l < (nblocks) ? ((nblocks) - wg_l + gridDim.x - 1) / gridDim.x : 0; \
+  auto pb = [&](int64_t v) { return v * (int64_t)gridDim.x + wg_l; }
 
 // Tile size of the channel contractions (forward x = A B^T, backward dA and
 // dB): 192 x 192 when N is a multiple of 192 (N = 384: 4 tiles per channel
@@ -263,145 +269,6 @@ __global__ __launch_bounds__(256) void tm_ln_rows_kernel(const __bf16* __restric
           rstd_out[row] = rstd;
         }
       }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// LN_out over the channels of the channel-major product x, written as
-// row-major xln.  Workgroup = 128 plane positions (natural order; the pad
-// positions of N % 8 != 0 write nothing) x up to 128
-// channels; wave = (64-position half wv / 2) x (64-channel half wv % 2);
-// lane = (8-position group pg = lane % 8, 8-channel group lane / 8): it
-// reads its 8 channels' 16-byte position runs (128-byte runs per plane
-// along pg) and keeps the 8 x 8 block in registers, so no LDS transpose is
-// needed.  Per-position sums over channels: the 8 channel groups of a wave
-// by lane exchanges, the two channel halves through LDS; mean first, then
-// the centred sum of squares.  Each thread then writes its 8 channels of
-// its 8 rows as 16-byte stores, so a store instruction covers 8 rows x 128
-// contiguous bytes (16 rows x 64 bytes with 16 position groups per wave:
-// 17.3 -> 16.4 us at N=384, C=128).
-// ---------------------------------------------------------------------------
-// Workgroups of the LN_out launch per batch: a grid-stride walk over the
-// 128-position tiles at 2 workgroups per CU (over all batches), each loading
-// its next tile while it normalises the current one.  Tiles are independent,
-// so the results do not depend on the grid.
-constexpr int kLnPlanesWgsPerCu = 2;
-static inline int64_t tm_ln_planes_grid(int64_t PS, int64_t B) {
-  const int64_t nt = (PS + 127) / 128;
-  const int64_t cap = ((int64_t)device_cus() * kLnPlanesWgsPerCu + B - 1) / B;
-  return nt < cap ? nt : cap;
-}
-template <int H>
-__global__ __launch_bounds__(256) void tm_ln_planes_kernel(const __bf16* __restrict__ x,
-                                                           const float* __restrict__ w,
-                                                           const float* __restrict__ bias,
-                                                           __bf16* __restrict__ xln,
-                                                           float* __restrict__ mean_out,
-                                                           float* __restrict__ rstd_out,
-                                                           TmGeom g) {
-  constexpr int T = 128;  // positions per tile
-  __shared__ float red[2][4][8][8];
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, b = blockIdx.y;
-  const int pg = lane & 7, cg = (lane >> 3) + 8 * (wv & 1);
-  const int p0 = 64 * (wv >> 1) + pg * 8;  // first position in the tile
-  const bool chan = cg * 8 < H;
-  const int64_t nt = (g.PS + T - 1) / T;
-  const int cgl = chan ? cg : 0;
-  float wc[8], bc[8];
-  {
-    const f32x4 w0 = *reinterpret_cast<const f32x4*>(w + cgl * 8);
-    const f32x4 w1 = *reinterpret_cast<const f32x4*>(w + cgl * 8 + 4);
-    const f32x4 b0 = *reinterpret_cast<const f32x4*>(bias + cgl * 8);
-    const f32x4 b1 = *reinterpret_cast<const f32x4*>(bias + cgl * 8 + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      wc[i] = w0[i]; wc[4 + i] = w1[i];
-      bc[i] = b0[i]; bc[4 + i] = b1[i];
-    }
-  }
-  // v[c][e]: channel cg*8 + c, position pb + e of tile t (16 bytes per
-  // channel; threads past the plane re-read its first positions).
-  auto load = [&](int64_t t, bf16x8 (&v)[8]) {
-    const int64_t pb = t * T + p0;
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      v[c] = ld8(x + ((int64_t)b * H + cgl * 8 + c) * g.PS + (pb < g.PS ? pb : 0));
-  };
-  // Sum over all channels of q[e] (this thread's 8 channels already summed);
-  // the two sums of a tile use the two halves of `red`, so one barrier each.
-  auto channel_sum = [&](float (&q)[8], int half) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) q[e] = xor32_sum(xor16_sum(q[e] + dpp_f<kDppXor8>(q[e])));
-    if ((lane & 56) == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) red[half][wv][pg][e] = q[e];
-    }
-    __syncthreads();
-    const int w0 = wv & 2;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) q[e] = red[half][w0][pg][e] + red[half][w0 + 1][pg][e];
-  };
-  bf16x8 nxt[8];
-  int64_t t = blockIdx.x;
-  if (t < nt) load(t, nxt);
-#pragma unroll 1
-  for (; t < nt; t += gridDim.x) {
-    bf16x8 v[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = chan ? nxt[c] : zero8();
-    if (t + gridDim.x < nt) load(t + gridDim.x, nxt);
-    const int64_t pb = t * T + p0;  // first position of this thread
-    // Its plane row, and how many of its eight positions have a row of xln.
-    const uint32_t pr = fdiv((uint32_t)pb, g.div_np);
-    const int col = (int)((uint32_t)pb - pr * (uint32_t)g.Np);
-    const int valid = pb < g.PS ? g.N - col : 0;
-    const int64_t row0 = (int64_t)b * g.NN + (int64_t)pr * g.N + col;
-    float mean[8], rstd[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float s = 0.f;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) s += bf2f(v[c][e]);
-      mean[e] = s;
-    }
-    // red[0] was last read before the previous tile's second barrier, red[1]
-    // before this tile's first: no barrier is needed between tiles.
-    channel_sum(mean, 0);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) mean[e] *= 1.f / H;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float s = 0.f;
-      if (chan) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const float d = bf2f(v[c][e]) - mean[e];
-          s = fmaf(d, d, s);
-        }
-      }
-      rstd[e] = s;
-    }
-    channel_sum(rstd, 1);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) rstd[e] = rsqrtf(rstd[e] * (1.f / H) + 1e-5f);
-    if (chan) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (e >= valid) continue;
-        bf16x8 o;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) o[c] = f2bf((bf2f(v[c][e]) - mean[e]) * rstd[e] * wc[c] + bc[c]);
-        st8(xln + (row0 + e) * H + cg * 8, o);
-      }
-    }
-    if (cg == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (e < valid) {
-          mean_out[row0 + e] = mean[e];
-          rstd_out[row0 + e] = rstd[e];
-        }
     }
   }
 }
@@ -895,7 +762,7 @@ __global__ __launch_bounds__(4 * C) void tm_ln_in_bwd_ws_kernel(
   const i32x4 rs_mu = buffer_rsrc(mean);
   const i32x4 rs_rs = buffer_rsrc(rstd);
   const __amdgpu_buffer_rsrc_t rs_o = __builtin_amdgcn_make_buffer_rsrc(dz, 0, 0x7FFFFFFF, 0x00020000);
-  TM_BLOCKS_STRIDED(nblocks);
+  TM_BLOCKS_WINDOW(nblocks);
   // Loads per block and loading wave: 2 z instructions and, by wave 0, the
   // two statistics rows (load j < 2, block blk, into the 2-deep ring), then PI
   // dproj5 instructions (load j >= 2, into the 3-deep ring).
@@ -1335,64 +1202,173 @@ __global__ __launch_bounds__(4 * C) void tm_out_bwd_ws_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Output projection forward, weight-stationary (natural rows): out = (xln Wz^T) s(gl), persistent
-// workgroups of C / 16 waves over 32-row blocks.  Wave w holds the Wz rows of
-// channels 16 w .. 16 w + 15 (B operands of v_mfma_f32_16x16x32_bf16); the
-// loading waves stream xln and gl rows (chunk-rotated) into a 4-deep LDS
-// ring; gl is read back transposed to match the accumulators; out is staged
-// as [row][channel] and stored as full rows by the storing waves.
+// LN_out and the output projection in one persistent, weight-stationary pass,
+// per block of 32 plane positions in natural order:
+//   xln = LN over the channels of x (planes);  out = (xln Wz^T) s(gl).
+// One barrier per block: in interval i the waves multiply block i (its
+// normalised rows Xn were written in interval i - 1) and write its gated
+// outputs to LDS, normalise block i + 1 from the ring into the other Xn
+// buffer, and the storing waves write block i - 1's output rows and, with
+// SAVE, block i's xln rows (the backward's state).
+//   * loads: the first half of the waves stream x plane segments ([channel][32
+//     positions], 64 bytes each) and gl rows (chunk-rotated) into a 4-deep
+//     LDS ring.  The channels of a 32-channel group are stored transposed
+//     (8 x 4) and the four 8-position chunks rotated by the group, so that the
+//     sixteen channel groups of a wave read distinct banks;
+//   * LayerNorm: lane (channel group cg = lane % CGP of 8 channels, position
+//     lane / CGP), so a wave holds whole rows and the channel sums stay
+//     within it: mean first, then the centred sum of squares, groups paired
+//     cg ^ 1, ^ 2, ^ 4, ^ 8;
+//   * product: wave w holds the Wz rows of channels 16 w .. 16 w + 15 (B
+//     operands of v_mfma_f32_16x16x32_bf16).
+// Bound by memory: 3 tensors of [R][C] in inference (x, gl, out), 4 with SAVE.
+// As two kernels (LN_out to row-major xln, then the projection): 17 + 24 us
+// with SAVE at N = 384 against 32 (4.7 TB/s), 100 + 157 us in inference at
+// N = 1021 against 168 (4.8 TB/s).
 // ---------------------------------------------------------------------------
 constexpr int kOutFwdDepth = 4;
-template <int C>
-__global__ __launch_bounds__(4 * C) void tm_out_proj_fwd_ws_kernel(
-    const __bf16* __restrict__ xln, const __bf16* __restrict__ wz, const __bf16* __restrict__ gl,
-    __bf16* __restrict__ out, TmGeom g, int64_t nblocks) {
+template <int C, bool PAD, bool SAVE>
+__global__ __launch_bounds__(4 * C) void tm_out_fwd_kernel(
+    const __bf16* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
+    const __bf16* __restrict__ wz, const __bf16* __restrict__ gl, __bf16* __restrict__ out,
+    __bf16* __restrict__ xln, float* __restrict__ mean_out, float* __restrict__ rstd_out, TmGeom g,
+    int64_t nblocks) {
   constexpr int NW = C / 16;         // waves
-  constexpr int CPR = C / 8;         // 16-byte chunks per row
+  constexpr int CPR = C / 8;         // 16-byte chunks per row = channel groups
   constexpr int KS = C / 32;         // 32-deep k steps
-  constexpr int RP = C + 8;          // staging pitch (bf16)
-  __shared__ __attribute__((aligned(1024))) __bf16 Rg[kOutFwdDepth][2][32 * C];  // xln | gl
+  constexpr int RP = C + 8;          // output staging pitch (bf16)
+  constexpr int CGP = CPR <= 4 ? 4 : CPR <= 8 ? 8 : 16;  // channel-group lanes
+  constexpr int PPW = 64 / CGP;      // positions per wave pass
+  __shared__ __attribute__((aligned(1024))) __bf16 Rg[kOutFwdDepth][2][32 * C];  // x | gl
+  __shared__ __attribute__((aligned(16))) __bf16 Xn[2][32 * C];                  // normalised rows
   __shared__ __attribute__((aligned(16))) __bf16 Or[2][32 * RP];
+  __shared__ float St[2][2][32];  // mean, rstd
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, lg = lane >> 4;
   const int ch = 16 * w + l16;
   const bool loader = w < NW / 2;
+  const int cg = lane % CGP, pl = lane / CGP;
+  const bool chan = cg < CPR;
 
   bf16x8 wf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) wf[ks] = ld8(wz + (int64_t)ch * C + 8 * (4 * ks + lg));
-  const i32x4 rs_in[2] = {buffer_rsrc(xln), buffer_rsrc(gl)};
-  const __amdgpu_buffer_rsrc_t rs_o = __builtin_amdgcn_make_buffer_rsrc(out, 0, 0x7FFFFFFF, 0x00020000);
-  TM_BLOCKS_STRIDED(nblocks);
-  // Loads per block and loading wave: 2 instructions each for xln and gl.
+  float wc[8], bc[8];  // LayerNorm weights of the lane's channel group
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    wc[e] = gamma[8 * (chan ? cg : 0) + e];
+    bc[e] = beta[8 * (chan ? cg : 0) + e];
+  }
+  const i32x4 rs_x = buffer_rsrc(x), rs_g = buffer_rsrc(gl);
+  const __amdgpu_buffer_rsrc_t rs_o = raw_rsrc(out), rs_n = raw_rsrc(xln);
+  TM_BLOCKS_WINDOW(nblocks);
+  auto row_of = [&](uint32_t m) { return m < (uint32_t)g.Rp ? tm_nat_row<PAD>(g, m) : kNoRow; };
+  // Loads per block and loading wave: 2 instructions each for x and gl.
   auto issue = [&](int64_t blk) {
     const int stage = (int)(blk % kOutFwdDepth);
+    const bool vb = blk < bend;
+    const uint32_t m0 = (uint32_t)pb(vb ? blk : 0) * 32;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int j = 0; j < 2; ++j) {
+      const int ci = (2 * w + j) * 64 + lane;
+      const int r = ci >> 2;  // LDS row r: the channel of its slot
+      const int c = (r & ~31) + (r & 3) * 8 + ((r >> 2) & 7);
+      const int part = (ci - (r >> 5)) & 3;
+      const uint32_t mb = m0 + 8 * part;
+      buf2lds16(rs_x, vb && mb < (uint32_t)g.Rp ? tm_plane_elem32(g, mb, c) * 2 : kBufOOB,
+                &Rg[stage][0][(2 * w + j) * 512]);
+    }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int ci = (2 * w + j) * 64 + lane;
-        const int r = ci / CPR, slot = ci % CPR;
-        const int gc = (slot - r % CPR + CPR) % CPR;
-        const uint32_t m = (uint32_t)pb(blk) * 32 + r;
-        const bool ok = blk < bend && m < (uint32_t)g.R;
-        buf2lds16(rs_in[t], ok ? (m * C + 8 * gc) * 2 : kBufOOB, &Rg[stage][t][(2 * w + j) * 512]);
+    for (int j = 0; j < 2; ++j) {
+      const int ci = (2 * w + j) * 64 + lane;
+      const int r = ci / CPR, slot = ci % CPR;
+      const int gc = (slot - r % CPR + CPR) % CPR;
+      const uint32_t row = vb ? row_of(m0 + r) : kNoRow;
+      buf2lds16(rs_g, row != kNoRow ? (row * C + 8 * gc) * 2 : kBufOOB, &Rg[stage][1][(2 * w + j) * 512]);
+    }
+  };
+  // LayerNorm of block blk into Xn[blk % 2] (rows chunk-rotated).
+  auto normalise = [&](int64_t blk) {
+    const __bf16* X = Rg[blk % kOutFwdDepth][0];
+    __bf16* Y = Xn[blk & 1];
+#pragma unroll
+    for (int q = 0; q < (32 / PPW + NW - 1) / NW; ++q) {
+      const int grp = w + NW * q;
+      if (grp * PPW >= 32) break;  // wave-uniform (C = 96: eight groups for six waves)
+      const int p = grp * PPW + pl;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int c = 8 * (chan ? cg : 0) + e;
+        const int r = (c & ~31) + (c & 7) * 4 + ((c >> 3) & 3);
+        v[e] = bf2f(X[r * 32 + 8 * (((p >> 3) + (c >> 5)) & 3) + (p & 7)]);
       }
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += chan ? v[e] : 0.f;
+      const float mean = lanes_sum<CGP>(s) * (1.f / C);
+      s = 0.f;
+      if (chan) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = v[e] - mean;
+          s = fmaf(d, d, s);
+        }
+      }
+      const float rstd = rsqrtf(lanes_sum<CGP>(s) * (1.f / C) + 1e-5f);
+      if (chan) {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = f2bf((v[e] - mean) * rstd * wc[e] + bc[e]);
+        *reinterpret_cast<bf16x8*>(&Y[p * C + 8 * ((cg + p) % CPR)]) = o;
+      }
+      if (SAVE && cg == 0) {
+        St[blk & 1][0][p] = mean;
+        St[blk & 1][1][p] = rstd;
+      }
+    }
+  };
+  // 4 C chunks (32 rows x C / 8) of block blk over the 2 C storing threads:
+  // out rows from the staging tile, or (xn) the normalised rows.
+  auto store_rows = [&](int64_t blk, bool xn) {
+    const int st = tid - 2 * C;
+    bf16x8 v[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int q = st + 2 * C * it, row = q / CPR, k = q % CPR;
+      v[it] = *reinterpret_cast<const bf16x8*>(xn ? &Xn[blk & 1][row * C + 8 * ((k + row) % CPR)]
+                                                  : &Or[blk & 1][row * RP + 8 * k]);
+    }
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int q = st + 2 * C * it, row = q / CPR, k = q % CPR;
+      const uint32_t r = row_of((uint32_t)pb(blk) * 32 + row);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), xn ? rs_n : rs_o,
+                                             r != kNoRow ? (r * C + 8 * k) * 2 : kBufOOB, 0, 0);
+    }
+    if (xn && st < 32) {
+      const uint32_t r = row_of((uint32_t)pb(blk) * 32 + st);
+      if (r != kNoRow) {
+        mean_out[r] = St[blk & 1][0][st];
+        rstd_out[r] = St[blk & 1][1][st];
+      }
+    }
   };
   if (loader) {
 #pragma unroll
     for (int d = 0; d < kOutFwdDepth - 1; ++d) issue(bbeg + d);
-    wait_vmcnt<4 * (kOutFwdDepth - 2)>();  // block bbeg landed
+    wait_vmcnt<4 * (kOutFwdDepth - 3)>();  // blocks bbeg, bbeg + 1 landed
   }
   __syncthreads();
+  normalise(bbeg);
+  lds_barrier();
 #pragma unroll 1
   for (int64_t blk = bbeg; blk < bend; ++blk) {
     const int stage = (int)(blk % kOutFwdDepth);
-    const int sb = (int)(blk & 1);
     if (loader) issue(blk + kOutFwdDepth - 1);
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    const __bf16* Xl = Rg[stage][0];
+    const __bf16* Xl = Xn[blk & 1];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -1402,6 +1378,7 @@ __global__ __launch_bounds__(4 * C) void tm_out_proj_fwd_ws_kernel(
             *reinterpret_cast<const bf16x8*>(&Xl[row * C + 8 * ((4 * ks + lg + row) % CPR)]);
         acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, wf[ks], acc[rt], 0, 0, 0);
       }
+    if (blk + 1 < bend) normalise(blk + 1);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       // gl for rows 16 rt + 4 lg + e, channel ch: lane L of a 16-lane group
@@ -1412,28 +1389,16 @@ __global__ __launch_bounds__(4 * C) void tm_out_proj_fwd_ws_kernel(
           (lds_bf16x4*)&Rg[stage][1][rr * C + 8 * (((cc >> 3) + rr) % CPR) + (cc & 7)]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        Or[sb][(16 * rt + 4 * lg + e) * RP + ch] = f2bf(acc[rt][e] * sigmoidf(bf2f(gv4[e])));
+        Or[blk & 1][(16 * rt + 4 * lg + e) * RP + ch] = f2bf(acc[rt][e] * sigmoidf(bf2f(gv4[e])));
     }
-    if (loader) wait_vmcnt<4 * (kOutFwdDepth - 2)>();  // block blk + 1 landed
-    __syncthreads();
     if (!loader) {
-      // 4 C chunks (32 rows x C / 8) over the 2 C storing threads.
-      const int st = tid - 2 * C;
-      bf16x8 v[2];
-#pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const int q = st + 2 * C * it, row = q / CPR, k = q % CPR;
-        v[it] = *reinterpret_cast<const bf16x8*>(&Or[sb][row * RP + 8 * k]);
-      }
-#pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const int q = st + 2 * C * it, row = q / CPR, k = q % CPR;
-        const uint32_t m = (uint32_t)pb(blk) * 32 + row;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[it]), rs_o,
-                                               m < (uint32_t)g.R ? (m * C + 8 * k) * 2 : kBufOOB, 0, 0);
-      }
+      if (blk > bbeg) store_rows(blk - 1, false);
+      if (SAVE) store_rows(blk, true);
     }
+    if (loader) wait_vmcnt<4 * (kOutFwdDepth - 3)>();  // block blk + 2 landed
+    lds_barrier();
   }
+  if (!loader && bbeg < bend) store_rows(bend - 1, false);
   // The ring loads issued past the last block still write LDS: let them land
   // before the workgroup releases its LDS.
   if (loader) wait_vmcnt<0>();
@@ -1544,8 +1509,8 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   int rc = tm_geom(&g, B, N, C, outgoing, fn, false);
   if (rc) return rc;
   if (!z || !mask || !w_ap || !w_ag || !w_bp || !w_bg || !w_g || !w_z || !ln_in_w || !ln_in_b ||
-      !ln_out_w || !ln_out_b || !out || !zln || !gate || !a || !b || !x || !xln || !mean_in ||
-      !rstd_in || !mean_out || !rstd_out || !workspace)
+      !ln_out_w || !ln_out_b || !out || !zln || !gate || !a || !b || !x || !mean_in ||
+      !rstd_in || !workspace || !xln != !mean_out || !xln != !rstd_out)
     return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   if (workspace_bytes < tm_weights_bytes(C))
     return set_error(TPF_ERR_ARG, "%s: workspace %lld < required %lld", fn,
@@ -1591,24 +1556,27 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   if ((rc = gemm_launch(ga, 1, 1, 0, (int)(B * C), s, "tpf_trimul_forward_bf16(contract)",
                         tm_contract_tile(N))))
     return rc;
-  TM_DISPATCH_C(C, tm_ln_planes_kernel, dim3((unsigned)tm_ln_planes_grid(g.PS, B), (unsigned)B),
-                (const __bf16*)x, ln_out_w, ln_out_b, (__bf16*)xln, mean_out, rstd_out, g);
-  if ((rc = check_launch("tpf_trimul_forward_bf16(ln_out)"))) return rc;
   {
-    const int64_t nblk = (g.R + 31) / 32;
+    const int64_t nblk = (g.Rp + 31) / 32;
     const int64_t cap = (int64_t)device_cus() * (128 / C);
     const unsigned grid = (unsigned)(nblk < cap ? nblk : cap);
+    const bool pad = g.Np != g.N;
     switch (C) {
-#define TM_OUT_FWD(CC)                                                                          \
-  case CC:                                                                                      \
-    hipLaunchKernelGGL(tm_out_proj_fwd_ws_kernel<CC>, dim3(grid), dim3(4 * CC), 0, s,           \
-                       (const __bf16*)xln, k.wz, (const __bf16*)gate, (__bf16*)out, g, nblk);   \
+#define TM_OUT_FWD_P(CC, PAD, SAVE)                                                              \
+  hipLaunchKernelGGL((tm_out_fwd_kernel<CC, PAD, SAVE>), dim3(grid), dim3(4 * CC), 0, s,         \
+                     (const __bf16*)x, ln_out_w, ln_out_b, k.wz, (const __bf16*)gate,            \
+                     (__bf16*)out, (__bf16*)xln, mean_out, rstd_out, g, nblk)
+#define TM_OUT_FWD(CC)                                                                           \
+  case CC:                                                                                       \
+    if (xln) { if (pad) TM_OUT_FWD_P(CC, true, true); else TM_OUT_FWD_P(CC, false, true); }      \
+    else { if (pad) TM_OUT_FWD_P(CC, true, false); else TM_OUT_FWD_P(CC, false, false); }        \
     break;
       TM_OUT_FWD(32) TM_OUT_FWD(64) TM_OUT_FWD(96) TM_OUT_FWD(128)
 #undef TM_OUT_FWD
+#undef TM_OUT_FWD_P
     }
   }
-  return check_launch("tpf_trimul_forward_bf16(out_proj)");
+  return check_launch("tpf_trimul_forward_bf16(ln_out + out_proj)");
 }
 
 // Backward workspace (each region 256-byte aligned): packed weights, dproj5

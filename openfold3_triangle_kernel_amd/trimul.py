@@ -164,12 +164,15 @@ def _trimul_fwd_impl(
     a = torch.empty((B * H, N * Np), device=dev, dtype=torch.bfloat16)
     b = torch.empty((B * H, N * Np), device=dev, dtype=torch.bfloat16)
     x = torch.empty((B * H, N, Np), device=dev, dtype=torch.bfloat16)
-    xln = torch.empty((rows, H), device=dev, dtype=torch.bfloat16)
     f32 = dict(device=dev, dtype=torch.float32)
     mean_in, rstd_in = torch.empty(rows, **f32), torch.empty(rows, **f32)
-    mean_out, rstd_out = torch.empty(rows, **f32), torch.empty(rows, **f32)
+    if save_state:
+        xln = torch.empty((rows, H), device=dev, dtype=torch.bfloat16)
+        mean_out, rstd_out = torch.empty(rows, **f32), torch.empty(rows, **f32)
+        ln_out = (xln.data_ptr(), mean_out.data_ptr(), rstd_out.data_ptr())
+    else:  # the output pass keeps the normalised product on the chip
+        ln_out = (None, None, None)
     lnw = [g_in32, b_in32, g_out32, b_out32]
-    state = (z_ln, xln, mean_out, rstd_out)
     with _device_ctx(dev):
         _native.call(
             "tpf_trimul_forward_bf16",
@@ -177,14 +180,12 @@ def _trimul_fwd_impl(
             lnw[0].data_ptr(), lnw[1].data_ptr(), lnw[2].data_ptr(), lnw[3].data_ptr(),
             int(bool(outgoing)), B, N, C,
             out.data_ptr(), z_ln.data_ptr(), gate.data_ptr(), a.data_ptr(), b.data_ptr(),
-            x.data_ptr(), xln.data_ptr(), mean_in.data_ptr(), rstd_in.data_ptr(),
-            mean_out.data_ptr(), rstd_out.data_ptr(), ws.data_ptr(), ws_bytes,
-            _native.stream_of(z_bf),
+            x.data_ptr(), ln_out[0], mean_in.data_ptr(), rstd_in.data_ptr(), ln_out[1], ln_out[2],
+            ws.data_ptr(), ws_bytes, _native.stream_of(z_bf),
         )
     if not save_state:
-        # The scratch state dies here (its memory returns to the caching
+        # The scratch z_ln dies here (its memory returns to the caching
         # allocator in stream order); only zero-row tensors leave the op.
-        del state
         z_ln, xln = z_bf.new_empty((0, C)), z_bf.new_empty((0, H))
         mean_out, rstd_out = torch.empty(0, **f32), torch.empty(0, **f32)
     return (out, z_ln, gate, a, b, x, xln, mean_in, rstd_in, mean_out, rstd_out)

@@ -161,3 +161,23 @@ def test_trimul_backward_ignores_memory_past_the_planes(gpu, outgoing):
     for c, d in zip(clean, dirty):
         assert torch.isfinite(d.float()).all()
         assert torch.equal(c, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outgoing", [True, False], ids=["outgoing", "incoming"])
+@pytest.mark.parametrize("B,N,C", [(1, 200, 128), (2, 33, 64), (1, 113, 96), (2, 41, 32), (1, 1, 128)])
+def test_trimul_inference_equals_training_forward(gpu, B, N, C, outgoing):
+    """Without a backward the row passes write no saved state; the output is
+    the same arithmetic: bitwise equal."""
+    from openfold3_triangle_kernel_amd import turbo_trimul
+
+    print(f"[trimul inference] B={B} N={N} C={C} outgoing={outgoing}", flush=True)
+    z, mask, w, _ = trimul_case(B, N, C, seed=N)
+    w = {k: v.to(gpu) for k, v in w.items()}
+    args = ("outgoing" if outgoing else "incoming", mask.to(gpu), w["g_in"], w["b_in"],
+            torch.cat([w["w_ap"], w["w_bp"]]), torch.cat([w["w_ag"], w["w_bg"]]), w["g_out"],
+            w["b_out"], w["w_z"], w["w_g"])
+    z = z.to(gpu, torch.bfloat16)
+    train = turbo_trimul(z.clone().requires_grad_(True), *args)
+    with torch.no_grad():
+        assert torch.equal(turbo_trimul(z, *args), train)
