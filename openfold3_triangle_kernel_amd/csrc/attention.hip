@@ -689,9 +689,8 @@ __global__ __launch_bounds__(256) void attn_bwd_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Backward.  One workgroup = (key block of 64*KH keys, head, group of 4 outer
-// rows), KH = 2 for D <= 32 (8 waves) and 1 for D = 64 (4 waves, LDS-bound);
-// wave w owns outer row o = 4*group + (w % 4) and key half w / 4 and keeps its
+// Backward for D <= 32, in one kernel.  One workgroup = (128 keys, head, group
+// of 4 outer rows), 8 waves; wave w owns outer row o = 4*group + (w % 4) and key half w / 4 and keeps its
 // dK / dV accumulators for those 64 keys in registers while streaming all
 // queries in 32-row steps.  Scores are
 // formed as S = Q K^T (lane = key column) so the C-layout P and dS tiles are
@@ -723,11 +722,11 @@ struct BwdSlab {
   int brun0, nbrun;
   int64_t plane0, planes;
 };
-// Key halves per backward workgroup (keys per workgroup = 64 * KH).
-__host__ __device__ constexpr int bwd_kh(int dp) { return dp == 32 ? 2 : 1; }
-// Backward key blocks (= dQ partials) for head dimension D.
+// Backward blocks per head and run: 128 keys for D <= 32 (one dQ partial
+// each), 64 keys or queries for D > 32 (whose workspace plan keeps room for a
+// partial per block: callers budget by it; the staged route uses one).
 static inline int64_t bwd_key_blocks(int64_t N, int64_t D) {
-  const int64_t kw = 64 * bwd_kh(D <= 32 ? 32 : 64);
+  const int64_t kw = D <= 32 ? 128 : 64;
   return (N + kw - 1) / kw;
 }
 
@@ -736,7 +735,7 @@ static inline int64_t bwd_key_blocks(int64_t N, int64_t D) {
 // row reads of 8 consecutive rows avoid bank conflicts.
 template <int DP>
 __device__ __forceinline__ int qd_swz(int r) {
-  return (DP == 32) ? (((r >> 1) & 1) << 1) : ((r & 3) << 1);
+  return (DP == 32) ? (((r >> 1) & 1) << 1) : ((r & 3) << 1) | ((r >> 2) & 1);
 }
 template <int DP>
 __device__ __forceinline__ int qd_off(int r, int col) {  // element offset of (row, col)
@@ -797,8 +796,8 @@ __device__ __forceinline__ void lds_read_rows4(u32x4* out, unsigned a0, unsigned
   for (int i = 0; i < 4; ++i) out[i] = u32x4{rs[i][0], rs[i][1], rs[i][2], rs[i][3]};
 }
 
-template <int DP, int MODE>
-__global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
+template <int MODE>
+__global__ __launch_bounds__(512, 1) void attn_bwd_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ k,
     const __bf16* __restrict__ v, const __bf16* __restrict__ dout,
     const float* __restrict__ nl2_g, const float* __restrict__ nd_g,
@@ -806,10 +805,11 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
     __bf16* __restrict__ dk, __bf16* __restrict__ dv,
     __bf16* __restrict__ dq_part, float* __restrict__ dbias_part, AttnGeom g, int run,
     BwdSlab sl, float* __restrict__ dtrue_part) {
+  constexpr int DP = 32;
   constexpr int KT = DP + 16;  // K tile pitch at setup (bf16)
   constexpr int SP = 32 + 4;   // dS^T tile [64 keys][32 queries] pitch (bf16): the
                                // 8-byte row writes of 32 lanes cover all banks once
-  constexpr int KH = bwd_kh(DP);               // key halves of 64 keys
+  constexpr int KH = 2;                         // key halves of 64 keys
   constexpr int NW = 4 * KH;                    // waves
   constexpr int NT = 64 * NW;                   // threads
   constexpr int QDE = 32 * DP;                 // elements of one Q (or dO) tile
@@ -825,7 +825,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
   __shared__ __attribute__((aligned(16))) __bf16 dSs[NW * SSE];
   __bf16* const dSbase = dSs;
   // Key half 1's dQ^T tiles for key half 0 [outer row][d block][16 regs][lane].
-  __shared__ __attribute__((aligned(16))) float Xq[KH == 2 ? 4 : 1][DP / 32][16][64];
+  __shared__ __attribute__((aligned(16))) float Xq[4][DP / 32][16][64];
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int pw = w & 3, kh = w >> 2;            // outer row in the group, key half
@@ -1029,12 +1029,11 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
     // step's loads so they overlap this step's compute.
     // Younger than those loads: this wave's previous-step partial loads
     // (8 read-backs) and stores (8 dBias, plus dQ on key half 0), all issued
-    // by every wave; with two key halves they may stay in flight (different
-    // rows from this step's; measured faster), with one (D = 64) waiting for
-    // them measured faster.  The first step of a group waits for
+    // by every wave; they may stay in flight (different rows from this
+    // step's; measured faster).  The first step of a group waits for
     // everything: its setup loads are younger, and the last group's partial
     // stores must land before this group reads the same addresses back.
-    if (q0 == 0 || KH == 1 || MODE == kBwdDKDV)
+    if (q0 == 0 || MODE == kBwdDKDV)
       wait_vmcnt<0>();
     else
       wait_vmcnt<16>();
@@ -1168,7 +1167,7 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
         acc = mfma32(kA[db][t], sb, acc);
       }
       dqacc[db] = acc;
-      if (KH == 2 && kh == 1) {
+      if (kh == 1) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) Xq[pw][db][r][lane] = acc[r];
       }
@@ -1179,13 +1178,11 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
 #pragma unroll
       for (int db = 0; db < DP / 32; ++db) {
         f32x16 acc = dqacc[db];
-        if (KH == 2) {
-          // All 16 values in one batch of LDS reads and one wait (at full
-          // register pressure the compiler issues them one pair at a time).
-          const u32x16 x = lds_read_col16(lds_offset(&Xq[pw][db][0][lane]));
+        // All 16 values in one batch of LDS reads and one wait (at full
+        // register pressure the compiler issues them one pair at a time).
+        const u32x16 x = lds_read_col16(lds_offset(&Xq[pw][db][0][lane]));
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[r] += __uint_as_float(x[r]);
-        }
+        for (int r = 0; r < 16; ++r) acc[r] += __uint_as_float(x[r]);
         // Lane-pair exchange as for dK / dV below: 16-byte stores of
         // channels 16p + 8hl .. +7 (chunks past D dropped by the range check).
         uint32_t pq[4][2];
@@ -1297,6 +1294,498 @@ __global__ __launch_bounds__(256 * bwd_kh(DP), 1) void attn_bwd_kernel(
     }
   }
   }  // outer groups of the run
+}
+
+// Tile of a workgroup of the D > 32 backward kernels, ordered XCD-aware by
+// (head, run of outer groups, block of 64 keys or queries), so the workgroups
+// that stream one group's rows run side by side on one XCD (L2 reuse).
+struct Bwd64Tile {
+  int blk, h, b, brun, og_lo, og_hi;
+};
+__device__ __forceinline__ bool bwd64_tile(const AttnGeom& g, int run, const BwdSlab& sl,
+                                           Bwd64Tile* t) {
+  const int nblk = g.NP / 64, groups = (g.O + kBwdGroup - 1) / kBwdGroup;
+  const int runs = (groups + run - 1) / run;
+  const int64_t total = (int64_t)g.H * nblk * sl.nbrun, L = blockIdx.x, per = (total + 7) / 8;
+  const int64_t T = (L % 8) * per + L / 8;
+  if (T >= total) return false;
+  t->blk = (int)(T % nblk);
+  const int64_t hb = T / nblk;
+  t->brun = sl.brun0 + (int)(hb % sl.nbrun);
+  t->h = (int)(hb / sl.nbrun);
+  t->b = t->brun / runs;
+  t->og_lo = (t->brun % runs) * run;
+  t->og_hi = min(groups, t->og_lo + run);
+  return true;
+}
+
+// Store of a transposed accumulator (register 4j + i of lane (kl, hl) and
+// block db: channel 32 db + 8 j + 4 hl + i of row kl) as the bf16 row at dst,
+// scaled.  One exchange with lane l ^ 32 per register pair gives a lane 8
+// consecutive channels, so each store instruction writes 32 contiguous bytes
+// per row.
+__device__ __forceinline__ void bwd64_store_row(const f32x16 (&acc)[2], float scale, int D, bool ok,
+                                                __bf16* dst) {
+  const int hl = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int db = 0; db < 2; ++db) {
+    uint32_t pk[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        pk[j][e] = __builtin_bit_cast(uint32_t, bf16x2{f2bf(acc[db][4 * j + 2 * e] * scale),
+                                                       f2bf(acc[db][4 * j + 2 * e + 1] * scale)});
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        auto r = __builtin_amdgcn_permlane32_swap(pk[2 * p][e], pk[2 * p + 1][e], false, false);
+        pk[2 * p][e] = r[0];
+        pk[2 * p + 1][e] = r[1];
+      }
+      const int d0 = db * 32 + 16 * p + 8 * hl;
+      if (ok && d0 < D)
+        *reinterpret_cast<u32x4*>(dst + d0) =
+            u32x4{pk[2 * p][0], pk[2 * p][1], pk[2 * p + 1][0], pk[2 * p + 1][1]};
+    }
+  }
+}
+// ---------------------------------------------------------------------------
+// Backward for 32 < D <= 64, in two kernels of the same tile geometry: keys
+// outside (dK / dV) and queries outside (dQ / dBias).  One workgroup = (head,
+// run of groups of 4 outer rows, 64 keys or queries); its 8 waves are 4 outer
+// rows x 2 halves of 32 keys (queries), two waves to a SIMD.
+//
+// Why two: the one-kernel form needs 224 registers of resident operands and
+// accumulators per wave at D = 64, so one wave per SIMD, whose matrix
+// instructions, exponentials and waits follow one another, and it leaves a
+// bf16 dQ partial per 64 keys (12 x 604 MB written and read back at N = 768,
+// H = 8).  Split, a wave holds 32 keys: dQ is summed in registers over all
+// keys and no partial is written, for S, dP and P formed twice (56 instead of
+// 40 matrix instructions per 32 x 64 scores).  At N = 768, H = 8, D = 64:
+// 5840 us + 1490 us of folds in one kernel, 2850 + 3400 us (dK / dV, dQ /
+// dBias) + 38 us of folds here; 660 -> 623 us forward and backward at N = 384,
+// H = 4.  Bound by latency within a step: the matrix unit is busy 30 %, the
+// vector unit 30 % and the LDS 34 % of the time, in turns, and taking any one
+// of the loads, the exponentials or half the products out of the dK / dV
+// kernel saves at most 12 %.  Measured no faster there: three buffers, LDS
+// reads in batches (2950 us), the two waves of a SIMD half a step apart (3100).
+//
+// Scores are formed as S = Q K^T (lane = key, registers = queries), seeded
+// with the prescaled bias; dP is seeded with -delta:
+//   P = exp2(S * c2 + nl2),  dS = P * dP.
+// ---------------------------------------------------------------------------
+template <bool DTRUE>
+__global__ __launch_bounds__(512, 1) void attn_dkdv64_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
+    const __bf16* __restrict__ dout, const float* __restrict__ nl2_g,
+    const float* __restrict__ nd_g, const float* __restrict__ mask,
+    const float* __restrict__ bias_f, __bf16* __restrict__ dk, __bf16* __restrict__ dv, AttnGeom g,
+    int run, BwdSlab sl, float* __restrict__ dtrue_part) {
+  constexpr int DP = 64, QDE = 32 * DP;
+  __shared__ __attribute__((aligned(1024))) __bf16 QD[2][4][2 * QDE];  // [buf][outer row] Q | dO
+  __shared__ __attribute__((aligned(1024))) float Bf[2][2][1024];      // [buf][key half] bias
+  __shared__ __attribute__((aligned(16))) float RS[2][4][64];          // [buf][outer row] nl2 | nd
+  __shared__ float Td[DTRUE ? 4 : 1][32];  // key half 1's delta_true sums
+
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int pw = w & 3, half = w >> 2, kl = lane & 31, hl = lane >> 5;
+  const int N = g.N, NP = g.NP, D = g.D, H = g.H;
+  Bwd64Tile t;
+  if (!bwd64_tile(g, run, sl, &t)) return;
+  const int key = t.blk * 64 + 32 * half + kl;
+  const float c2 = g.scale * kLog2e, inv_scale = 1.f / g.scale;
+  const int nb32 = NP / 32;
+  const float* bfrag = bias_f + (((int64_t)(g.bias_bstride == 0 ? 0 : t.b) * H + t.h) * nb32 +
+                                 t.blk * 2) * (int64_t)nb32 * 1024;
+  const i32x4 rs_bias = buffer_rsrc(bfrag);
+  // Wave w loads kilobyte w % 4 of key half w / 4's fragments.
+  const uint32_t vb = (uint32_t)((half * nb32 * 1024 + pw * 256 + lane * 4) * 4);
+  const int q_bytes = row_range(N, g.s_row, D);
+
+#pragma unroll 1
+  for (int og = t.og_lo; og < t.og_hi; ++og) {
+    if (og != t.og_lo) __syncthreads();  // the previous group's LDS reads are done
+    const int o = og * kBwdGroup + pw;
+    const bool plane_ok = o < g.O, active = plane_ok && t.blk * 64 + 32 * half < N;
+    const int plane = t.b * g.O + (plane_ok ? o : 0);
+    const int64_t plane_off = (int64_t)plane * g.s_plane + (int64_t)t.h * g.s_head;
+    const int64_t do_plane = ((int64_t)plane * N * H + t.h) * D;  // dO is [B,O,N,H,D]
+    const int64_t st_plane = ((int64_t)plane * H + t.h) * NP;     // row statistics
+    if (!plane_ok && half == 0) {  // an idle outer row: P = 0 everywhere
+#pragma unroll
+      for (int x = 0; x < 2; ++x) RS[x][pw][lane] = lane < 32 ? -INFINITY : 0.f;
+    }
+    i32x4 rs_q = buffer_rsrc(q + plane_off), rs_do = buffer_rsrc(dout + do_plane);
+    rs_q[2] = q_bytes;
+    rs_do[2] = row_range(N, (int64_t)H * D, D);
+    uint32_t vq[2], vdo[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int gc = (half * 2 + n) * 64 + lane, r = gc >> 3, c = (gc & 7) ^ qd_swz<DP>(r);
+      const bool ld = plane_ok && c * 8 < D;
+      vq[n] = ld ? (uint32_t)((r * g.s_row + c * 8) * 2) : kBufOOB;
+      vdo[n] = ld ? (uint32_t)((r * H * D + c * 8) * 2) : kBufOOB;
+    }
+    // Loads of step q0 (rows past N read zeros) into buffer `buf`.
+    auto issue = [&](int q0, int buf) {
+      buf2lds16_so(rs_bias, vb, (uint32_t)q0 * 128u, &Bf[buf][half][pw * 256]);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const int nn = half * 2 + n;
+        buf2lds16_so(rs_q, vq[n], (uint32_t)(q0 * g.s_row * 2), &QD[buf][pw][nn * 512]);
+        buf2lds16_so(rs_do, vdo[n], (uint32_t)(q0 * H * D * 2), &QD[buf][pw][QDE + nn * 512]);
+      }
+      if (plane_ok && half == 0 && lane < 16) {
+        const float* src = (lane < 8 ? nl2_g : nd_g) + st_plane + q0 + (lane & 7) * 4;
+        g2lds16(src, &RS[buf][pw][0]);
+      }
+    };
+    issue(0, 0);
+    bf16x8 kB[4], vB[4];  // B operands of S and dP (lane = key)
+    const __amdgpu_buffer_rsrc_t rk = raw_rsrc(k + plane_off, q_bytes),
+                                 rv = raw_rsrc(v + plane_off, q_bytes);
+    const __amdgpu_buffer_rsrc_t rm = raw_rsrc(mask + (int64_t)plane * N);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int d0 = 16 * s + 8 * hl;
+      const uint32_t off =
+          active && d0 < D ? (uint32_t)(((int64_t)key * g.s_row + d0) * 2) : kBufOOB;
+      kB[s] = buf_ld8(rk, off);
+      vB[s] = buf_ld8(rv, off);
+    }
+    const float mraw = buf_ldf(rm, active && key < N ? (uint32_t)(key * 4) : kBufOOB);
+    const float mk = key >= N ? -INFINITY : active ? mraw * inv_scale : 0.f;
+    const bool wmask = __any(mk != 0.f);
+    f32x16 dKacc[2], dVacc[2];
+#pragma unroll
+    for (int db = 0; db < 2; ++db) { dKacc[db] = zero16(); dVacc[db] = zero16(); }
+
+    // The operands have landed before the loop (each passes through an asm): with
+    // one pending, the compiler would wait for all loads in every step.
+#pragma unroll
+    for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(kB[s]), "+v"(vB[s]));
+    wait_vmcnt<0>();
+#pragma unroll 1
+    for (int q0 = 0; q0 < N; q0 += 32) {
+      const int buf = (q0 >> 5) & 1;
+      wait_vmcnt<0>();
+      lds_barrier();
+      // The other buffer was last read before the barrier.
+      if (q0 + 32 < N) issue(q0 + 32, buf ^ 1);
+      const __bf16* Qs = QD[buf][pw];
+      const __bf16* dOs = Qs + QDE;
+      f32x16 sacc, dp, nl2v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&Bf[buf][half][j * 256 + lane * 4]);
+        const f32x4 a4 = *reinterpret_cast<const f32x4*>(&RS[buf][pw][8 * j + 4 * hl]);
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(&RS[buf][pw][32 + 8 * j + 4 * hl]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sacc[4 * j + i] = x[i];
+          nl2v[4 * j + i] = a4[i];
+          dp[4 * j + i] = d4[i];
+        }
+      }
+      [[maybe_unused]] const f32x16 ndv = dp;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int c = 16 * s + 8 * hl;
+        sacc = mfma32(*reinterpret_cast<const bf16x8*>(&Qs[qd_off<DP>(kl, c)]), kB[s], sacc);
+        dp = mfma32(*reinterpret_cast<const bf16x8*>(&dOs[qd_off<DP>(kl, c)]), vB[s], dp);
+      }
+      if (wmask) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sacc[r] += mk;
+      }
+      f32x16 P, dS;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        P[r] = fast_exp2(fmaf(sacc[r], c2, nl2v[r]));
+        dS[r] = P[r] * dp[r];
+      }
+      if constexpr (DTRUE) {
+        // delta_true partial of the workgroup's 64 keys (dP is the accumulator
+        // minus its -delta seed): the 32 key lanes of a half summed on DPP /
+        // permlane, then half 0 + half 1 (fixed order).
+        float ts[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ts[r] = lanes_sum<32>(P[r] * (dp[r] - ndv[r]));
+        if (half == 1 && kl == 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) Td[pw][8 * (r >> 2) + 4 * hl + (r & 3)] = ts[r];
+        }
+        lds_barrier();
+        if (half == 0 && active && kl == 0) {
+          float* dst = dtrue_part +
+                       (((int64_t)plane * H + t.h) * ((N + 63) / 64) + t.blk) * N + q0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            f32x4 x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = ts[4 * j + i] + Td[pw][8 * j + 4 * hl + i];
+            *reinterpret_cast<f32x4*>(dst + 8 * j + 4 * hl) = x;
+          }
+        }
+      }
+      // dV^T += dO^T P, dK^T += Q^T dS over two 16-query steps (C-layout order).
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const bf16x8 pP = pack8(P, 8 * tt), pS = pack8(dS, 8 * tt);
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+          const bf16x8 da = cat8(qd_tr_col4<DP>(dOs, 16 * tt, 16 * tt + 4, 32 * db),
+                                 qd_tr_col4<DP>(dOs, 16 * tt + 8, 16 * tt + 12, 32 * db));
+          const bf16x8 qa = cat8(qd_tr_col4<DP>(Qs, 16 * tt, 16 * tt + 4, 32 * db),
+                                 qd_tr_col4<DP>(Qs, 16 * tt + 8, 16 * tt + 12, 32 * db));
+          dVacc[db] = mfma32(da, pP, dVacc[db]);
+          dKacc[db] = mfma32(qa, pS, dKacc[db]);
+        }
+      }
+    }
+    // dK (scaled) and dV in Q/K/V storage order.
+    if (active) {
+      const int64_t row = (int64_t)plane * g.o_plane + (int64_t)t.h * g.o_head + (int64_t)key * g.o_row;
+      bwd64_store_row(dKacc, g.scale, D, key < N, dk + row);
+      bwd64_store_row(dVacc, 1.f, D, key < N, dv + row);
+    }
+  }
+}
+
+// dQ and the dBias partials: queries outside.  Q, dO and the row statistics of
+// a wave's 32 queries stay in registers while the keys stream in steps of 32
+// (K / V tiles through LDS).  dS goes to LDS as bf16 [key][query]: the dQ
+// operand (transposing reads, dQ^T += K^T dS^T) and the sum over the 4 outer
+// rows that is added to the run's f32 dBias partial.
+// dq: final (scaled) dQ in Q's storage order; else dq_part: the unscaled bf16
+// sum as the slab's one partial [plane - plane0][h][q < NP][D].
+__global__ __launch_bounds__(512, 1) void attn_dqdb64_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
+    const __bf16* __restrict__ dout, const float* __restrict__ nl2_g,
+    const float* __restrict__ nd_g, const float* __restrict__ mask,
+    const float* __restrict__ bias_f, __bf16* __restrict__ dq, __bf16* __restrict__ dq_part,
+    float* __restrict__ dbias_part, AttnGeom g, int run, BwdSlab sl) {
+  constexpr int DP = 64, KVE = 32 * DP;
+  constexpr int SP = 32 + 4;  // dS^T tile pitch: 32 lanes' 8-byte accesses cover all banks once
+  constexpr int SSE = 32 * SP;
+  __shared__ __attribute__((aligned(1024))) __bf16 KV[2][4][2 * KVE];  // [buf][outer row] K | V
+  __shared__ __attribute__((aligned(1024))) float Bf[2][2][1024];      // [buf][query half] bias
+  __shared__ __attribute__((aligned(16))) __bf16 dSs[8 * SSE];         // [wave][32 keys][SP]
+
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int pw = w & 3, half = w >> 2, kl = lane & 31, hl = lane >> 5;
+  const int N = g.N, NP = g.NP, D = g.D, H = g.H;
+  Bwd64Tile t;
+  if (!bwd64_tile(g, run, sl, &t)) return;
+  const int qb0 = t.blk * 64 + 32 * half, qrow = qb0 + kl;  // first query of the wave, lane's query
+  const float c2 = g.scale * kLog2e, inv_scale = 1.f / g.scale;
+  const int nb32 = NP / 32;
+  const float* bfrag = bias_f + ((int64_t)(g.bias_bstride == 0 ? 0 : t.b) * H + t.h) * nb32 *
+                                    (int64_t)nb32 * 1024;
+  const i32x4 rs_bias = buffer_rsrc(bfrag);
+  // Wave w loads kilobyte w % 4 of query half w / 4's fragments; a step of 32
+  // keys is nb32 fragment blocks.
+  const uint32_t vb = (uint32_t)(((t.blk * 2 + half) * 1024 + pw * 256 + lane * 4) * 4);
+  const int q_bytes = row_range(N, g.s_row, D);
+  __bf16* const Ss = dSs + w * SSE;
+  float* const dbp = dbias_part + ((int64_t)t.brun * H + t.h) * NP * NP;
+  const __amdgpu_buffer_rsrc_t rs_db = raw_rsrc(dbp);
+  // dBias phase: thread = (key, 4 queries).
+  const int dbkey = tid & 31, dbq = tid >> 5;
+  const uint32_t vdb = (uint32_t)(((t.blk * 64 + 4 * dbq) * NP + dbkey) * 4);
+  const __bf16* const dbsrc = dSs + 4 * (dbq >> 3) * SSE + dbkey * SP + 4 * (dbq & 7);
+  // bf16 pairs (1, 0) and (0, 1) for the dBias sum; the first is kept out of
+  // the compiler's sight, which would encode it as the inline constant 1.0
+  // (read by v_dot2 as the f32 pattern, the pair (0, 1)).
+  uint32_t sel_lo_bits;
+  asm volatile("v_mov_b32 %0, 0x3f80" : "=v"(sel_lo_bits));
+
+#pragma unroll 1
+  for (int og = t.og_lo; og < t.og_hi; ++og) {
+    const bool first = og == t.og_lo;
+    if (!first) __syncthreads();  // the previous group's LDS reads are done
+    const int o = og * kBwdGroup + pw;
+    const bool plane_ok = o < g.O;
+    const int plane = t.b * g.O + (plane_ok ? o : 0);
+    const int64_t plane_off = (int64_t)plane * g.s_plane + (int64_t)t.h * g.s_head;
+    const int64_t do_plane = ((int64_t)plane * N * H + t.h) * D;
+    const int64_t st_plane = ((int64_t)plane * H + t.h) * NP;
+    // The run's partial so far: read back by the thread that wrote it (range
+    // 0 for the run's first group: zeros), at device scope (sc1), so the load
+    // misses the CU's L1, which may hold an older copy of the line.
+    const __amdgpu_buffer_rsrc_t rs_dbr = raw_rsrc(dbp, first ? 0 : 0x7FFFFFFF);
+    i32x4 rs_k = buffer_rsrc(k + plane_off), rs_v = buffer_rsrc(v + plane_off);
+    rs_k[2] = q_bytes;
+    rs_v[2] = q_bytes;
+    uint32_t vkv[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int gc = (half * 2 + n) * 64 + lane, r = gc >> 3, c = (gc & 7) ^ qd_swz<DP>(r);
+      vkv[n] = plane_ok && c * 8 < D ? (uint32_t)((r * g.s_row + c * 8) * 2) : kBufOOB;
+    }
+    const __amdgpu_buffer_rsrc_t rm = raw_rsrc(mask + (int64_t)plane * N);
+    auto issue = [&](int k0, int buf) {
+      // The mask first: older than the tiles, whose wait then covers it.
+      const float m = buf_ldf(rm, plane_ok && k0 + kl < N ? (uint32_t)((k0 + kl) * 4) : kBufOOB);
+      buf2lds16_so(rs_bias, vb, (uint32_t)k0 * (uint32_t)nb32 * 128u, &Bf[buf][half][pw * 256]);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const int nn = half * 2 + n;
+        buf2lds16_so(rs_k, vkv[n], (uint32_t)(k0 * g.s_row * 2), &KV[buf][pw][nn * 512]);
+        buf2lds16_so(rs_v, vkv[n], (uint32_t)(k0 * g.s_row * 2), &KV[buf][pw][KVE + nn * 512]);
+      }
+      return m;
+    };
+    // The run's partial so far of the thread's dBias outputs of step k0.
+    auto load_db = [&](int k0, float (&x)[4]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[e] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(rs_dbr, vdb, (k0 + e * NP) * 4, 16));
+    };
+    // Mask and partials of even and odd steps: fixed registers, so no copy
+    // waits for a load in flight.
+    wait_vmcnt<0>();  // the last group's partials have landed
+    float m0 = issue(0, 0), m1, db0[4], db1[4];
+    load_db(0, db0);
+    bf16x8 qA[4], doA[4];  // A operands of S and dP (lane = query)
+    const __amdgpu_buffer_rsrc_t rq = raw_rsrc(q + plane_off, q_bytes),
+                                 rdo = raw_rsrc(dout + do_plane, row_range(N, (int64_t)H * D, D));
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int d0 = 16 * s + 8 * hl;
+      const bool ld = plane_ok && qrow < N && d0 < D;
+      qA[s] = buf_ld8(rq, ld ? (uint32_t)(((int64_t)qrow * g.s_row + d0) * 2) : kBufOOB);
+      doA[s] = buf_ld8(rdo, ld ? (uint32_t)(((int64_t)qrow * H * D + d0) * 2) : kBufOOB);
+    }
+    f32x16 nl2v, ndv;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 a4 = *reinterpret_cast<const f32x4*>(nl2_g + st_plane + qb0 + 8 * j + 4 * hl);
+      const f32x4 d4 = *reinterpret_cast<const f32x4*>(nd_g + st_plane + qb0 + 8 * j + 4 * hl);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // an idle outer row: P = dS = 0
+        nl2v[4 * j + i] = plane_ok ? a4[i] : -INFINITY;
+        ndv[4 * j + i] = plane_ok ? d4[i] : 0.f;
+      }
+    }
+    f32x16 dQacc[2] = {zero16(), zero16()};
+
+    auto step = [&](int k0, int buf, float& mcur, float (&dbprev)[4], float& mnext,
+                    float (&dbnext)[4]) {
+      // Younger than this step's loads: the last step's 4 partial loads and 4
+      // stores.
+      wait_vmcnt<8>();
+      lds_barrier();
+      asm volatile("" : "+v"(mcur));
+      const float mk = k0 + kl >= N ? -INFINITY : mcur * inv_scale;
+      // (After the last step: its own loads again, read by nobody, so that a
+      // step's loads are a constant.)
+      const int kn = min(k0 + 32, NP - 32);
+      mnext = issue(kn, buf ^ 1);
+      load_db(kn, dbnext);
+      const __bf16* Ks = KV[buf][pw];
+      const __bf16* Vs = Ks + KVE;
+      f32x16 sacc, dp = ndv;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&Bf[buf][half][j * 256 + lane * 4]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sacc[4 * j + i] = x[i];
+      }
+      // LDS reads in batches ahead of their use (left alone, the compiler reads
+      // one operand at a time and waits out its latency).
+      bf16x8 kf[4], vf[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int c = 16 * s + 8 * hl;
+        kf[s] = *reinterpret_cast<const bf16x8*>(&Ks[qd_off<DP>(kl, c)]);
+        vf[s] = *reinterpret_cast<const bf16x8*>(&Vs[qd_off<DP>(kl, c)]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        sacc = mfma32(qA[s], kf[s], sacc);
+        dp = mfma32(doA[s], vf[s], dp);
+      }
+      bf16x8 ka[2][2];  // [16-key step][32-channel block]
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+          ka[tt][db] = cat8(qd_tr_col4<DP>(Ks, 16 * tt, 16 * tt + 8, 32 * db),
+                            qd_tr_col4<DP>(Ks, 16 * tt + 4, 16 * tt + 12, 32 * db));
+      __builtin_amdgcn_sched_barrier(0);
+      if (__any(mk != 0.f)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sacc[r] += mk;
+      }
+      f32x16 dS;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dS[r] = fast_exp2(fmaf(sacc[r], c2, nl2v[r])) * dp[r];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const bf16x8 h8 = pack8(dS, 8 * tt);
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+          bf16x4 s4;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s4[i] = h8[4 * jj + i];
+          *reinterpret_cast<bf16x4*>(&Ss[kl * SP + 8 * (2 * tt + jj) + 4 * hl]) = s4;
+        }
+      }
+      // dQ^T (d x 32 queries) += K^T dS^T over two 16-key steps.
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const bf16x8 sb = cat8(tr_col4(Ss, SP, 16 * tt, 16 * tt + 8, 0),
+                               tr_col4(Ss, SP, 16 * tt + 4, 16 * tt + 12, 0));
+#pragma unroll
+        for (int db = 0; db < 2; ++db) dQacc[db] = mfma32(ka[tt][db], sb, dQacc[db]);
+      }
+      lds_barrier();
+      // dBias: the 4 outer rows' bf16 dS^T tiles summed in the fixed order
+      // ((o0 + o1) + o2) + o3 (one v_dot2 with a one-hot pair per add), then
+      // added to the run's partial; a store instruction writes 32 consecutive
+      // keys of two query rows.
+      const bf16x2 sel[2] = {__builtin_bit_cast(bf16x2, sel_lo_bits),
+                             {static_cast<__bf16>(0.f), static_cast<__bf16>(1.f)}};
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) {
+        const u32x2 rows = *reinterpret_cast<const u32x2*>(dbsrc + ww * SSE);
+        const uint32_t lo = rows[0], hi = rows[1];
+        acc[0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, lo), sel[0], acc[0], false);
+        acc[1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, lo), sel[1], acc[1], false);
+        acc[2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, hi), sel[0], acc[2], false);
+        acc[3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, hi), sel[1], acc[3], false);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dbprev[e] + acc[e]), rs_db, vdb,
+                                              (k0 + e * NP) * 4, 0);
+    };
+    // The operands have landed before the loop (each passes through an asm): with
+    // one pending, the compiler would wait for all loads in every step.
+#pragma unroll
+    for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(qA[s]), "+v"(doA[s]));
+    asm volatile("" : "+v"(nl2v), "+v"(ndv), "+v"(m0), "+v"(db0[0]), "+v"(db0[1]), "+v"(db0[2]),
+                 "+v"(db0[3]));
+    wait_vmcnt<0>();
+#pragma unroll 1
+    for (int k0 = 0; k0 < NP; k0 += 64) {
+      step(k0, 0, m0, db0, m1, db1);
+      step(k0 + 32, 1, m1, db1, m0, db0);
+    }
+    wait_vmcnt<0>();  // the loads issued past the last step land in LDS
+    if (dq)
+      bwd64_store_row(dQacc, g.scale, D, plane_ok && qrow < N,
+                      dq + (int64_t)plane * g.o_plane + (int64_t)t.h * g.o_head + (int64_t)qrow * g.o_row);
+    else
+      bwd64_store_row(dQacc, 1.f, D, plane_ok,
+                      dq_part + (((int64_t)plane - sl.plane0) * H + t.h) * NP * D + (int64_t)qrow * D);
+  }
 }
 
 // dQ = bf16(scale * sum_kb partial[kb]) in ascending key-block order; bf16
@@ -1904,14 +2393,15 @@ static int attn_backward_prep_impl(const AttnGeom& g, const float* lse, const fl
   return check_launch(fn);
 }
 
-// The reconstruction kernel over one slab (dK, dV of its planes and their
-// dQ / dBias partials).
-template <int DP, int MODE>
+// The reconstruction over one slab (dK, dV of its planes and their dQ / dBias
+// partials).  D > 32: dQ itself goes to `dq` when given, else to the slab's
+// one partial.
+template <int MODE>
 static void bwd_kernel_launch(dim3 grid, const AttnGeom& g, const void* q, const void* k,
                               const void* v, const void* dout, const float* mask, void* dk,
                               void* dv, const BwdParts& pt, const BwdPlan& plan,
                               const BwdSlab& sl, float* dtrue, hipStream_t s) {
-  hipLaunchKernelGGL((attn_bwd_kernel<DP, MODE>), grid, dim3(256 * bwd_kh(DP)), 0, s,
+  hipLaunchKernelGGL((attn_bwd_kernel<MODE>), grid, dim3(512), 0, s,
                      (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, (const __bf16*)dout,
                      pt.nl2, pt.nd, mask, pt.bias_f, (__bf16*)dk, (__bf16*)dv, pt.dq, pt.db, g,
                      plan.run, sl, dtrue);
@@ -1919,37 +2409,50 @@ static void bwd_kernel_launch(dim3 grid, const AttnGeom& g, const void* q, const
 static int attn_backward_slab_impl(const AttnGeom& g, const void* q, const void* k,
                                    const void* v, const void* dout, const float* mask,
                                    void* dk, void* dv, const BwdParts& pt, const BwdPlan& plan,
-                                   const BwdSlab& sl, hipStream_t s, const char* fn,
+                                   const BwdSlab& sl, void* dq, hipStream_t s, const char* fn,
                                    int mode = kBwdSR, float* dtrue = nullptr) {
   const int64_t H = g.H, N = g.N, D = g.D;
   const int64_t total = H * bwd_key_blocks(N, D) * sl.nbrun;
   if ((total + 7) / 8 * 8 > INT32_MAX)
     return set_error(TPF_ERR_SHAPE, "%s: too many backward tiles", fn);
   dim3 grid((unsigned)((total + 7) / 8 * 8));
-#define TPF_BWD_LAUNCH(DP, MODE) \
-  bwd_kernel_launch<DP, MODE>(grid, g, q, k, v, dout, mask, dk, dv, pt, plan, sl, dtrue, s)
+#define TPF_BWD_LAUNCH(MODE) \
+  bwd_kernel_launch<MODE>(grid, g, q, k, v, dout, mask, dk, dv, pt, plan, sl, dtrue, s)
   if (D <= 32) {
-    if (mode == kBwdDKDV) TPF_BWD_LAUNCH(32, kBwdDKDV);
-    else if (mode == kBwdDQDB) TPF_BWD_LAUNCH(32, kBwdDQDB);
-    else TPF_BWD_LAUNCH(32, kBwdSR);
+    if (mode == kBwdDKDV) TPF_BWD_LAUNCH(kBwdDKDV);
+    else if (mode == kBwdDQDB) TPF_BWD_LAUNCH(kBwdDQDB);
+    else TPF_BWD_LAUNCH(kBwdSR);
   } else {
-    if (mode == kBwdDKDV) TPF_BWD_LAUNCH(64, kBwdDKDV);
-    else if (mode == kBwdDQDB) TPF_BWD_LAUNCH(64, kBwdDQDB);
-    else TPF_BWD_LAUNCH(64, kBwdSR);
+#define TPF_DKDV64(DTRUE)                                                                        \
+  hipLaunchKernelGGL((attn_dkdv64_kernel<DTRUE>), grid, dim3(512), 0, s, (const __bf16*)q,       \
+                     (const __bf16*)k, (const __bf16*)v, (const __bf16*)dout, pt.nl2, pt.nd,     \
+                     mask, pt.bias_f, (__bf16*)dk, (__bf16*)dv, g, plan.run, sl, dtrue)
+    if (mode != kBwdDQDB) {
+      if (dtrue) TPF_DKDV64(true);
+      else TPF_DKDV64(false);
+    }
+#undef TPF_DKDV64
+    if (mode != kBwdDKDV)
+      hipLaunchKernelGGL(attn_dqdb64_kernel, grid, dim3(512), 0, s, (const __bf16*)q,
+                         (const __bf16*)k, (const __bf16*)v, (const __bf16*)dout, pt.nl2, pt.nd,
+                         mask, pt.bias_f, (__bf16*)dq, pt.dq, pt.db, g, plan.run, sl);
   }
 #undef TPF_BWD_LAUNCH
   return check_launch(fn);
 }
 
-// Folds of one slab: its planes' dQ, and (with_dbias, after the last slab)
-// every dBias partial.  db_mode: 0 = f32 dBias, 1 = bf16, 2 = bf16 in
+// Folds of one slab: its planes' dQ (with_dq; D > 32 leaves one partial), and
+// (with_dbias, after the last slab) every dBias partial.  db_mode: 0 = f32 dBias, 1 = bf16, 2 = bf16 in
 // transposed-bias order.
+static inline int bwd_dq_partials(int64_t N, int64_t D) {
+  return D > 32 ? 1 : (int)bwd_key_blocks(N, D);
+}
 static int attn_backward_fold_impl(const AttnGeom& g, void* dq, void* dbias,
                                    int64_t bias_batches, const BwdParts& pt, const BwdPlan& plan,
-                                   const BwdSlab& sl, bool with_dbias, hipStream_t s,
-                                   const char* fn, int db_mode) {
+                                   const BwdSlab& sl, bool with_dq, bool with_dbias,
+                                   hipStream_t s, const char* fn, int db_mode) {
   const int64_t H = g.H, N = g.N, D = g.D;
-  const int64_t nph = sl.planes * H;
+  const int64_t nph = with_dq ? sl.planes * H : 0;
   const int64_t dq_bx = (N * (D / 8) + 255) / 256;
   // dBias workgroups: 64 chunks of 8 keys, or (transposed order) a tile of
   // 8 queries x 64 keys each.
@@ -1961,7 +2464,7 @@ static int attn_backward_fold_impl(const AttnGeom& g, void* dq, void* dbias,
     return set_error(TPF_ERR_ARG, "%s: fold grid too large", fn);
   if (n_db + dq_bx * nph == 0) return TPF_OK;
   hipLaunchKernelGGL(attn_fold_kernel, dim3((unsigned)(n_db + dq_bx * nph)), dim3(256), 0, s,
-                     pt.dq, (__bf16*)dq, g, (int)bwd_key_blocks(N, D), (int)dq_bx, pt.db, dbias,
+                     pt.dq, (__bf16*)dq, g, bwd_dq_partials(N, D), (int)dq_bx, pt.db, dbias,
                      (int)bias_batches, plan.runs, n_db, db_mode, sl.plane0, sl.planes);
   return check_launch(fn);
 }
@@ -2183,7 +2686,7 @@ int tpf_attn_backward_main_bf16(const void* q, const void* k, const void* v, con
                                     bias_batches, pt, s, fn)))
     return rc;
   return attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan, bwd_slab(plan, B, O, 0),
-                                 s, fn);
+                                 nullptr, s, fn);
 }
 
 // Stage 2 of the backward: fixed-order folds of the dQ and dBias partials.
@@ -2200,7 +2703,7 @@ int tpf_attn_backward_finish_bf16(void* dq, void* dbias, const void* workspace, 
   BwdParts pt;
   bwd_layout(B, O, H, N, D, B * O, (char*)workspace, &pt);
   return attn_backward_fold_impl(g, dq, dbias, bias_batches, pt, plan, bwd_slab(plan, B, O, 0),
-                                 true, (hipStream_t)stream, fn, db_mode);
+                                 true, true, (hipStream_t)stream, fn, db_mode);
 }
 
 // Every slab of a plan: reconstruction, then that slab's dQ fold; the dBias
@@ -2210,12 +2713,20 @@ static int attn_backward_slabs(const AttnGeom& g, const BwdPlan& plan, const voi
                                void* dq, void* dk, void* dv, void* dbias, int64_t bias_batches,
                                const BwdParts& pt, hipStream_t s, const char* fn, int db_mode,
                                int mode = kBwdSR) {
+  if (g.D > 32) {  // dQ leaves no partials: every run at once
+    const BwdSlab all{0, g.B * plan.runs, 0, (int64_t)g.B * g.O};
+    int rc = attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan, all, dq, s, fn, mode);
+    if (rc) return rc;
+    return attn_backward_fold_impl(g, dq, dbias, bias_batches, pt, plan, all, false, true, s, fn,
+                                   db_mode);
+  }
   for (int i = 0; i < plan.slabs; ++i) {
     const BwdSlab sl = bwd_slab(plan, g.B, g.O, i);
-    int rc = attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan, sl, s, fn, mode);
+    int rc = attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan, sl, nullptr, s, fn,
+                                     mode);
     if (rc) return rc;
-    rc = attn_backward_fold_impl(g, dq, dbias, bias_batches, pt, plan, sl, i + 1 == plan.slabs, s,
-                                 fn, db_mode);
+    rc = attn_backward_fold_impl(g, dq, dbias, bias_batches, pt, plan, sl, true,
+                                 i + 1 == plan.slabs, s, fn, db_mode);
     if (rc) return rc;
   }
   return TPF_OK;
@@ -2339,7 +2850,7 @@ int tpf_attn_dkdv_bf16(const void* q, const void* k, const void* v, const void* 
   const BwdPlan plan = bwd_plan(B, O, H, N, D, INT64_MAX);
   for (int i = 0; i < plan.slabs; ++i)
     if ((rc = attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan,
-                                      bwd_slab(plan, B, O, i), s, fn, kBwdDKDV,
+                                      bwd_slab(plan, B, O, i), nullptr, s, fn, kBwdDKDV,
                                       delta_true_partials)))
       return rc;
   if (delta_true) {
@@ -2563,13 +3074,15 @@ static int pair_backward_impl(const void* qkv, const void* rest, int64_t rest_pi
   const BwdPlan plan = bwd_plan(B, N, H, N, D, INT64_MAX);
   if ((rc = attn_backward_prep_impl(g, lse, delta, r + hc, bv, B, pt, s, fn))) return rc;
   if ((rc = attn_backward_slab_impl(g, q, q + part, q + 2 * part, d_o, mask, dp + hc, dp + 2 * hc,
-                                    pt, plan, bwd_slab(plan, B, N, 0), s, fn)))
+                                    pt, plan, bwd_slab(plan, B, N, 0), dp, s, fn)))
     return rc;
-  const int64_t nph = B * N * H;
-  hipLaunchKernelGGL(attn_dq_reduce_kernel,
-                     dim3((unsigned)((N * (D / 8) + 255) / 256), (unsigned)(nph < 65535 ? nph : 65535)),
-                     dim3(256), 0, s, pt.dq, dp, g, (int)bwd_key_blocks(N, D));
-  if ((rc = check_launch(fn))) return rc;
+  if (D <= 32) {
+    const int64_t nph = B * N * H;
+    hipLaunchKernelGGL(attn_dq_reduce_kernel,
+                       dim3((unsigned)((N * (D / 8) + 255) / 256), (unsigned)(nph < 65535 ? nph : 65535)),
+                       dim3(256), 0, s, pt.dq, dp, g, (int)bwd_key_blocks(N, D));
+    if ((rc = check_launch(fn))) return rc;
+  }
   const int64_t groups = plan.runs;
   const dim3 db_grid((unsigned)(B * N * N / 512));
   hipLaunchKernelGGL(attn_dbias_pair_kernel, db_grid, dim3(256), 0, s, pt.db, (int)B, (int)B,

@@ -274,3 +274,46 @@ def test_any_sequence_length_equals_the_padded_problem(gpu, B, O, H, N, D, seq_m
     for name, a, b in zip(("out", "dq", "dk", "dv", "dbias"), got, ref):
         assert a.shape == b.shape and torch.isfinite(a.float()).all(), name
         assert torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,O,H,N,D", [(1, 98, 16, 128, 40), (2, 13, 2, 192, 64)])
+def test_wide_head_backward_runs_and_stages(gpu, B, O, H, N, D):
+    """D > 32: runs of several outer groups with idle rows in the last one
+    (98 rows: 25 groups in runs of 4), against the oracle; the two-stage
+    entries leave dQ as one bf16 sum that the second stage scales, so it is
+    the fused dQ up to one bf16 rounding (2^-9 relative) on either side."""
+    from openfold3_triangle_kernel_amd import _native
+
+    print(f"[attn wide heads] {B, O, H, N, D}", flush=True)
+    case = attention_case(B, O, H, N, D, mask_frac=0.2, seed=D)
+    ref = attention_backward(*(t.numpy() for t in case))
+    got = _run(case, gpu)[1:]
+    for n, a, r in zip(("dq", "dk", "dv", "dbias"), got, ref):
+        assert max_rel(a, r) <= TOL, n
+
+    q, k, v, mask, bias, dout = (t.to(gpu).bfloat16() if i not in (3,) else t.to(gpu)
+                                 for i, t in enumerate(case))
+    f32 = dict(device=gpu, dtype=torch.float32)
+    out, lse = torch.empty(B, O, N, H, D, device=gpu, dtype=torch.bfloat16), torch.empty(B, O, H, N, **f32)
+    delta, st, scale = torch.empty_like(lse), _native.stream_of(q), D ** -0.5
+    ws = torch.empty(int(_native.query("tpf_attn_backward_workspace_bytes", B, O, H, N, D)),
+                     device=gpu, dtype=torch.uint8)
+    ptr = [t.data_ptr() for t in (q, k, v, mask.contiguous(), bias.contiguous())]
+    tail = (B, O, H, N, D, 0, 1, scale, st)
+    _native.call("tpf_attn_forward_bf16", *ptr, out.data_ptr(), lse.data_ptr(), ws.data_ptr(),
+                 ws.numel(), *tail)
+    _native.call("tpf_attn_delta_bf16", dout.data_ptr(), out.data_ptr(), delta.data_ptr(), B, O, H,
+                 N, D, st)
+    args = (*ptr[:3], dout.data_ptr(), lse.data_ptr(), delta.data_ptr(), *ptr[3:])
+    grads = [[torch.empty_like(q) for _ in range(3)] + [torch.empty(1, H, N, N, **f32)]
+             for _ in range(2)]
+    dq, dk, dv, db = (t.data_ptr() for t in grads[0])
+    _native.call("tpf_attn_backward_bf16", *args, dq, dk, dv, db, ws.data_ptr(), ws.numel(), *tail)
+    dq, dk, dv, db = (t.data_ptr() for t in grads[1])
+    _native.call("tpf_attn_backward_main_bf16", *args, dk, dv, ws.data_ptr(), ws.numel(), *tail)
+    _native.call("tpf_attn_backward_finish_bf16", dq, db, ws.data_ptr(), *tail)
+    one, two = grads
+    assert all(torch.equal(a, b) for a, b in zip(one[1:], two[1:]))
+    a, b = one[0].float(), two[0].float()
+    assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 1e-30).all()
