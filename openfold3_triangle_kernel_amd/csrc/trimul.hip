@@ -133,19 +133,24 @@ struct TmWeights {
   const float* z;
 };
 
-__global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w,
-                                                              __bf16* __restrict__ w5,
-                                                              __bf16* __restrict__ wz,
-                                                              __bf16* __restrict__ w5t,
-                                                              __bf16* __restrict__ wzt, int C) {
+// The pack by workgroups [0, wgs), this one being wg; the forward stops before
+// the transposed parts (w5t null).
+struct TmPacked {
+  __bf16* w5;
+  __bf16* wz;
+  __bf16* w5t;
+  __bf16* wzt;
+};
+__device__ __forceinline__ void tm_pack_weights(const TmWeights& w, const TmPacked& k, int C,
+                                                int64_t wg, int64_t wgs) {
   const int cpr = C / 8;
   const int64_t total = (int64_t)6 * C * cpr;
   const float* const mats[5] = {w.ap, w.ag, w.bp, w.bg, w.g};
   // W5^T [C][5C] (C x 5C / 8 chunks) and Wz^T [H][C] (H x C / 8 chunks)
   // after the row-copied part.
   const int64_t t5 = total + (int64_t)C * 5 * cpr;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < t5 + (int64_t)C * cpr;
-       idx += (int64_t)gridDim.x * 256) {
+  const int64_t end = k.w5t ? t5 + (int64_t)C * cpr : total;
+  for (int64_t idx = wg * 256 + threadIdx.x; idx < end; idx += wgs * 256) {
     // The transposed parts take consecutive source columns on consecutive
     // lanes (coalesced loads; the 16-byte stores are the scattered side).
     if (idx >= t5) {
@@ -154,7 +159,7 @@ __global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w,
       bf16x8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = f2bf(w.z[(int64_t)(c0 + e) * C + h]);
-      st8(wzt + (int64_t)h * C + c0, o);
+      st8(k.wzt + (int64_t)h * C + c0, o);
       continue;
     }
     if (idx >= total) {
@@ -163,21 +168,21 @@ __global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w,
       bf16x8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int k = k0 + e;
-        o[e] = f2bf(mats[k / C][(int64_t)(k % C) * C + c]);
+        const int r = k0 + e;
+        o[e] = f2bf(mats[r / C][(int64_t)(r % C) * C + c]);
       }
-      st8(w5t + (int64_t)c * 5 * C + k0, o);
+      st8(k.w5t + (int64_t)c * 5 * C + k0, o);
       continue;
     }
     const int row = (int)(idx / cpr), ch = (int)(idx % cpr);
     const float* src;
     __bf16* dst;
     if (row < 5 * C) {
-      dst = w5 + (int64_t)row * C + ch * 8;
+      dst = k.w5 + (int64_t)row * C + ch * 8;
       src = mats[row / C] + (int64_t)(row % C) * C;
     } else {
       const int c = row - 5 * C;
-      dst = wz + (int64_t)c * C + ch * 8;
+      dst = k.wz + (int64_t)c * C + ch * 8;
       src = w.z + (int64_t)c * C;
     }
     bf16x8 o;
@@ -186,10 +191,15 @@ __global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w,
     st8(dst, o);
   }
 }
+__global__ __launch_bounds__(256) void tm_pack_weights_kernel(TmWeights w, TmPacked k, int C) {
+  tm_pack_weights(w, k, C, blockIdx.x, gridDim.x);
+}
 
 // ---------------------------------------------------------------------------
-// LN_in over rows of z (16 lanes per row, 8 channels per lane).  A thread
-// handles kLnRowsRPT rows 16 apart, their loads issued together.
+// LN_in over rows of z (16 lanes per row, 8 channels per lane) by the first
+// nwg workgroups; the rest pack the weights for the launches that follow (a
+// launch of its own took 4.1 us of 23 at N = 64).  A thread handles kLnRowsRPT
+// rows 16 apart, their loads issued together.
 // ---------------------------------------------------------------------------
 constexpr int kLnRowsRPT = 2;
 // Workgroups of the LN_in launch: one per 16 * kLnRowsRPT rows (the kernel
@@ -205,7 +215,12 @@ __global__ __launch_bounds__(256) void tm_ln_rows_kernel(const __bf16* __restric
                                                          const float* __restrict__ bias,
                                                          __bf16* __restrict__ out,
                                                          float* __restrict__ mean_out,
-                                                         float* __restrict__ rstd_out, int64_t R) {
+                                                         float* __restrict__ rstd_out, int64_t R,
+                                                         int64_t nwg, TmWeights pw, TmPacked pk) {
+  if ((int64_t)blockIdx.x >= nwg) {
+    tm_pack_weights(pw, pk, C, blockIdx.x - nwg, gridDim.x - nwg);
+    return;
+  }
   const int l16 = threadIdx.x & 15;
   const bool chan = l16 < C / 8;
   const int64_t nb = (R + 16 * kLnRowsRPT - 1) / (16 * kLnRowsRPT);
@@ -233,13 +248,13 @@ __global__ __launch_bounds__(256) void tm_ln_rows_kernel(const __bf16* __restric
   int64_t blk = blockIdx.x;
   load(blk, nxt);
 #pragma unroll 1
-  for (; blk < nb; blk += gridDim.x) {
+  for (; blk < nb; blk += nwg) {
     float x[kLnRowsRPT][8];
 #pragma unroll
     for (int k = 0; k < kLnRowsRPT; ++k)
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[k][e] = chan ? bf2f(nxt[k][e]) : 0.f;
-    if (blk + gridDim.x < nb) load(blk + gridDim.x, nxt);
+    if (blk + nwg < nb) load(blk + nwg, nxt);
     const int64_t row0 = blk * 16 * kLnRowsRPT + (threadIdx.x >> 4);
 #pragma unroll
     for (int k = 0; k < kLnRowsRPT; ++k) {
@@ -1450,12 +1465,6 @@ static int64_t tm_weights_bytes(int64_t C) {
 }
 
 // Packed bf16 weights at the start of a workspace.
-struct TmPacked {
-  __bf16* w5;
-  __bf16* wz;
-  __bf16* w5t;
-  __bf16* wzt;
-};
 static TmPacked tm_packed(void* ws, int64_t C) {
   char* p = (char*)ws;
   TmPacked k;
@@ -1472,7 +1481,7 @@ static TmPacked tm_packed(void* ws, int64_t C) {
 static int tm_pack(const TmWeights& w, const TmPacked& k, int C, hipStream_t s, const char* fn) {
   const int64_t chunks = 12 * C * (C / 8);
   hipLaunchKernelGGL(tm_pack_weights_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
-                     s, w, k.w5, k.wz, k.w5t, k.wzt, C);
+                     s, w, k, C);
   return check_launch(fn);
 }
 
@@ -1518,9 +1527,10 @@ int tpf_trimul_forward_bf16(const void* z, const float* mask, const float* w_ap,
   hipStream_t s = (hipStream_t)stream;
   const TmPacked k = tm_packed(workspace, C);
   const TmWeights w{w_ap, w_ag, w_bp, w_bg, w_g, w_z};
-  if ((rc = tm_pack(w, k, (int)C, s, fn))) return rc;
-  TM_DISPATCH_C(C, tm_ln_rows_kernel, dim3((unsigned)tm_ln_rows_grid(g.R)), (const __bf16*)z, ln_in_w,
-                ln_in_b, (__bf16*)zln, mean_in, rstd_in, g.R);
+  const int64_t ln_wgs = tm_ln_rows_grid(g.R), pack_wgs = (6 * C * (C / 8) + 255) / 256;
+  const TmPacked pk{k.w5, k.wz, nullptr, nullptr};
+  TM_DISPATCH_C(C, tm_ln_rows_kernel, dim3((unsigned)(ln_wgs + pack_wgs)), (const __bf16*)z, ln_in_w,
+                ln_in_b, (__bf16*)zln, mean_in, rstd_in, g.R, ln_wgs, w, pk);
   if ((rc = check_launch("tpf_trimul_forward_bf16(ln_in)"))) return rc;
   {
     // Persistent: one workgroup of C / 16 waves per CU share at C = 128.
