@@ -298,7 +298,7 @@ def main():
     bwd_flops = 10.0 * B * O * H * N * N * D
     achieved = bwd_flops / (bwd_kernel_ms * 1e-3) / 1e12
     roofline = {
-        "kernel": "attn_bwd_kernel<32> (timed with its attn_bwd_prep_kernel launch)",
+        "kernel": "attn_bwd_kernel (timed with its attn_bwd_prep_kernel launch)",
         "bound": "mfma",
         "achieved": round(achieved, 2),
         "peak": MFMA_BF16_PEAK_TFLOPS,

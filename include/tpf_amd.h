@@ -115,7 +115,8 @@ int tpf_attn_delta_shadow_bf16(const void* dout, const void* out, const void* re
 /* Bytes of device workspace of the one-slab backward plan (dQ partials of
  * every outer row, one f32 dBias partial per run of outer groups, the
  * prescaled bias and the row statistics).  tpf_attn_backward_main_bf16 /
- * _finish_bf16 need this much. */
+ * _finish_bf16 need this much.  D > 32: the plan keeps room for a dQ partial
+ * per 64 keys, of which the kernels use one (main / finish) or none. */
 int64_t tpf_attn_backward_workspace_bytes(int64_t B, int64_t O, int64_t H, int64_t N,
                                           int64_t D);
 

@@ -16,10 +16,11 @@ selected by default here:
 
 * attention, stable: LayerNorm (FP32 statistics; the BF16 LayerNorm kernel),
   the additive mask ``inf * (mask - 1)``, one projection GEMM for q / k / v,
-  the gate and the pair bias ``linear_z``; for N a multiple of 64 the
-  pair-row core (``tpf_attn_pair_*``: attention and gate read the projection
-  rows in place, gradients land in one projection-gradient buffer), else the
-  triangle-attention facade on sequence-major views; ``linear_o``.  The
+  the gate and the pair bias ``linear_z``; in inference, and in training for
+  N a multiple of 64, the pair-row core (``tpf_attn_pair_*``: attention and
+  gate read the projection rows in place, gradients land in one
+  projection-gradient buffer), else the triangle-attention facade on
+  sequence-major views; ``linear_o``.  The
   projection weight gradients (contractions over all B*N^2 pair rows) run on
   the split-K MFMA GEMM.  FP32 activations under ``torch.no_grad()`` take
   the FP32 inference kernel; FP32 training inputs take the stock FP32 math
