@@ -560,11 +560,17 @@ __device__ __forceinline__ int64_t delta_row(const __bf16* __restrict__ dout,
   part[tid] = s;
   __syncthreads();
   const int d8 = D / 8;
-  if (!act || (t % d8) != 0) return -1;
+  if (!act || tid % d8 != 0) return -1;  // per is a multiple of d8
   float acc = 0.f;
   for (int u = 0; u < d8; ++u) acc += part[tid + u];
   *sum = acc;
-  // r enumerates [plane][q][h]; delta is [plane][h][q].
+  // r enumerates [plane][q][h]; delta is [plane][h][q].  (32-bit divisions
+  // where they do: the 64-bit ones are about a hundred instructions each.)
+  if (items <= UINT32_MAX) {
+    const uint32_t r = (uint32_t)t / (uint32_t)d8, pq = r / (uint32_t)H, plane = pq / (uint32_t)N;
+    *qrow = (int)(pq - plane * (uint32_t)N);
+    return (int64_t)plane * H + (r - pq * (uint32_t)H);
+  }
   const int64_t r = t / d8;
   const int hh = (int)(r % H);
   const int64_t pq = r / H;
@@ -614,9 +620,14 @@ __device__ __forceinline__ void bwd_bias_item(const __bf16* __restrict__ bias,
   const int q0 = qb * 32 + 8 * j + 4 * hl, key = kb * 32 + kl;
   const __bf16* src = bias_at(bias, bv, bh, q0, key);
   f32x4 o;
+  if (N == NP) {  // unpredicated, so the four loads are in flight together
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = q0 + e < N && key < N ? bf2f(src[(int64_t)e * bv.s_q]) * inv_scale : 0.f;
+    for (int e = 0; e < 4; ++e) o[e] = bf2f(src[(int64_t)e * bv.s_q]) * inv_scale;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = q0 + e < N && key < N ? bf2f(src[(int64_t)e * bv.s_q]) * inv_scale : 0.f;
+  }
   *reinterpret_cast<f32x4*>(out + i * 4) = o;
 }
 
