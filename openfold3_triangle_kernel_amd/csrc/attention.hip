@@ -701,9 +701,9 @@ __global__ __launch_bounds__(256) void attn_bwd_rows_kernel(
 
 // ---------------------------------------------------------------------------
 // Backward for D <= 32, in one kernel.  One workgroup = (128 keys, head, group
-// of 4 outer rows), 8 waves; wave w owns outer row o = 4*group + (w % 4) and key half w / 4 and keeps its
-// dK / dV accumulators for those 64 keys in registers while streaming all
-// queries in 32-row steps.  Scores are
+// of 4 outer rows), 8 waves; wave w owns outer row o = 4*group + (w % 4) and
+// key half w / 4 and keeps its dK / dV accumulators for those 64 keys in
+// registers while streaming all queries in 32-row steps.  Scores are
 // formed as S = Q K^T (lane = key column) so the C-layout P and dS tiles are
 // the B operands of dV^T += dO^T P and dK^T += Q^T dS without data movement;
 // the transposed A operands (dO^T, Q^T) and dS^T for dQ^T = K^T dS^T come
