@@ -170,6 +170,16 @@ def _pair_rows_projection(x2: torch.Tensor, wa: torch.Tensor, B: int, O: int, N:
     return qkv, proj[:, 3 * hc:].contiguous()
 
 
+def _mask_rows(mask_bias: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """The additive mask [*, I, 1, 1, J] of pairs x [*, I, J, C] as [B, I, J],
+    a broadcast one (over the batch or a pair axis) written out."""
+    I, J = x.shape[-3:-1]
+    full = x.shape[:-2] + (1, 1, J)
+    if mask_bias.numel() != math.prod(full):
+        mask_bias = mask_bias.expand(full)
+    return mask_bias.reshape(-1, I, J)
+
+
 def _pair_flags(transpose_bias: bool, og_t: bool) -> int:
     """Flags of the pair-row entry points (TPF_PAIR_BIAS_TRANSPOSED = 1,
     TPF_PAIR_OG_TRANSPOSED = 2)."""
@@ -469,7 +479,7 @@ class TriangleAttention(nn.Module):
         mask_bias = (self.inf * (mask.float() - 1))[..., :, None, None, :]
         m = self.mha
         H, c = m.no_heads, m.c_hidden
-        if self._pair_inference(x, chunk_size):
+        if self._pair_inference(x, mask_bias, chunk_size):
             return self._pair_inference_forward(x, mask_bias, transpose_bias, chunk_size)
         if chunk_size is not None and chunk_size < x.shape[-3]:
             return self._chunked_forward(x, mask_bias, transpose_bias, chunk_size)
@@ -489,7 +499,7 @@ class TriangleAttention(nn.Module):
                           + ([self.linear_z.weight.new_zeros(pad, self.c_in)] if pad else []))
         if pair_core:
             B = math.prod(prefix)
-            mask_add = mask_bias.reshape(B, N, N).contiguous()
+            mask_add = _mask_rows(mask_bias, x).contiguous()
             # The ending node's x is the transposed view of the caller's
             # pair rows: the core returns its output in the caller's order,
             # handed back as the transposed view the caller transposes again
@@ -517,10 +527,10 @@ class TriangleAttention(nn.Module):
         g = torch.sigmoid(gp).reshape(o.shape)
         return _linear((o * g).flatten(-2), m.linear_o.weight)
 
-    def _pair_inference(self, x, chunk_size) -> bool:
+    def _pair_inference(self, x, mask_bias, chunk_size) -> bool:
         """Whether inference runs the pair-row core: BF16 square pairs on the
-        kernels' device without gradients, within the limits of the
-        per-projection route's support verdict.  Every N: at N = 613, C = 128
+        kernels' device without gradients, a mask that broadcasts to them, and
+        the limits of the per-projection route's support verdict.  Every N: at N = 613, C = 128
         the per-projection route, with its gate and layout passes in torch,
         takes 821 us and the core 534."""
         H, c, N = self.mha.no_heads, self.mha.c_hidden, x.shape[-2]
@@ -529,6 +539,10 @@ class TriangleAttention(nn.Module):
                 and math.prod(x.shape[:-2]) <= 65_535 and N <= 8192):
             return False
         if x.dim() < 4 and (N % 64 or chunk_size is not None):
+            return False
+        if mask_bias.dim() > x.dim() + 1 or any(
+                m not in (1, t) for m, t in zip(mask_bias.shape[-4::-1], x.shape[-3::-1])) \
+                or mask_bias.shape[-1] not in (1, N):
             return False
         if torch.is_grad_enabled() and (x.requires_grad or any(
                 p.requires_grad for p in self.parameters())):
@@ -551,7 +565,7 @@ class TriangleAttention(nn.Module):
         w_all = torch.cat([m.linear_q.weight, m.linear_k.weight, m.linear_v.weight,
                            m.linear_g.weight, self.linear_z.weight]
                           + ([zeros(pad, C)] if pad else []))
-        x4, mask_add = x.reshape(B, N, N, C), mask_bias.reshape(B, N, N)
+        x4, mask_add = x.reshape(B, N, N, C), _mask_rows(mask_bias, x)
         og_t = not self.starting
         if chunk_size is None or chunk_size >= N:
             out = _PairAttentionInference.apply(x4, w_all, m.linear_o.weight, mask_add.contiguous(),

@@ -254,3 +254,33 @@ def test_triangle_attention_module_inference_any_n(gpu, starting, transpose_bias
     assert max_rel(out.float().cpu().numpy(), ref.cpu().numpy()) <= 2e-2
     if N % 64 == 0:  # the training core's forward
         assert torch.equal(out, mb(xb.requires_grad_(True), kb, transpose_bias=transpose_bias))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,chunk", [(33, None), (64, None), (33, 16), (64, 16)])
+@pytest.mark.parametrize("starting", [True, False])
+@pytest.mark.parametrize("shape", [(1, -1, -1), (-1, -1), (2, 1, -1), (2, -1, 1)], ids=str)
+def test_triangle_attention_module_broadcast_mask(gpu, shape, starting, N, chunk):
+    """A mask that broadcasts over the batch or over a pair axis gives the
+    bits of the same mask given whole, in inference (whole and in chunks) and,
+    where the training core serves the mask, in training."""
+    from openfold3_triangle_kernel_amd import TriangleAttention
+
+    torch.manual_seed(N)
+    m = TriangleAttention(128, 32, 4, starting=starting).to(gpu).bfloat16()
+    for p in m.parameters():
+        p.data.normal_(std=0.1)
+    x = torch.randn(2, N, N, 128, device=gpu).bfloat16()
+    mask = (torch.rand([N if s < 0 else s for s in shape], device=gpu) > 0.2).bfloat16()
+    whole = mask.expand(2, N, N).contiguous()
+    print(f"broadcast mask {tuple(mask.shape)} N={N} chunk={chunk} starting={starting}", flush=True)
+    with torch.no_grad():
+        out = m(x, mask, chunk_size=chunk)
+        assert out.shape == x.shape and torch.equal(out, m(x, whole, chunk_size=chunk))
+    if chunk is None and (N % 64 == 0 or shape[-2:] == (-1, -1)):
+        res = []
+        for k in (mask, whole):
+            xg = x.clone().requires_grad_(True)
+            y = m(xg, k)
+            res.append([y, *torch.autograd.grad(y, [xg, *m.parameters()], x)])
+        assert all(torch.equal(a, b) for a, b in zip(*res))
