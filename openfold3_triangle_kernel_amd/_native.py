@@ -216,6 +216,12 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy where its storage does not start on the 16 bytes that
+    the kernels load at a time (a contiguous view into a larger buffer)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 

@@ -279,6 +279,7 @@ class _TriangleAttentionFn(torch.autograd.Function):
         d_out = d_out.contiguous()
         if d_out.dtype != torch.bfloat16:
             d_out = d_out.to(torch.bfloat16)
+        d_out = _native.aligned(d_out)
         with _device_ctx(q.device):
             stream = _native.stream_of(q)
             if ctx.seq_major:

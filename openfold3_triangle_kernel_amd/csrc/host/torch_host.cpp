@@ -70,6 +70,12 @@ bool plain(const Tensor& t, c10::DeviceIndex dev) {
 
 bool aligned16(const Tensor& t) { return (uintptr_t)t.const_data_ptr() % 16 == 0; }
 
+// An upstream gradient as the kernels read it: bf16, contiguous, 16-byte aligned.
+Tensor kernel_grad(const Tensor& g) {
+  const Tensor t = g.to(at::kBFloat16).contiguous();
+  return aligned16(t) ? t : t.clone();
+}
+
 at::TensorOptions like(const Tensor& t, at::ScalarType dtype) {
   return at::TensorOptions().device(t.device()).dtype(dtype);
 }
@@ -125,7 +131,7 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
     const int64_t layout = ctx->saved_data["layout"].toInt();
     const int64_t batches = ctx->saved_data["batches"].toInt();
     const int64_t B = q.size(0), O = q.size(1), H = q.size(2), N = q.size(3), D = q.size(4);
-    const Tensor dout = grads[0].contiguous().to(at::kBFloat16);
+    const Tensor dout = kernel_grad(grads[0]);
     Tensor d[3];
     for (Tensor& t : d)
       t = layout & TPF_QKV_SEQ_MAJOR
@@ -278,7 +284,7 @@ struct TrimulFn : torch::autograd::Function<TrimulFn> {
     const Tensor &z = s[0], &mask = s[1], &state = s[2];
     const int64_t B = z.size(0), N = z.size(1), C = z.size(3), cc = C * C;
     const TrimulState st(B, N, C, true, (char*)state.data_ptr());
-    const Tensor g = grads[0].to(at::kBFloat16).contiguous();
+    const Tensor g = kernel_grad(grads[0]);
     const auto f32 = like(z, at::kFloat);
     Tensor dz = at::empty({B, N, N, C}, like(z, at::kBFloat16));
     Tensor dp = at::empty({2 * C, C}, f32), dg = at::empty({2 * C, C}, f32);

@@ -77,7 +77,7 @@ def _operands(q, k, v, d_output, logsumexp, delta, mask, pair_bias, fn):
         bias, bias_batches = pair_bias[:1].contiguous(), 1
     else:
         bias, bias_batches = pair_bias.contiguous(), B
-    flat = (d_output.contiguous(), logsumexp.reshape(-1).float().contiguous(),
+    flat = (_native.aligned(d_output.contiguous()), logsumexp.reshape(-1).float().contiguous(),
             delta.reshape(-1).float().contiguous(), mask.reshape(-1).float().contiguous(), bias)
     return (B, O, H, N, D), layout, flat, bias_batches
 

@@ -150,7 +150,7 @@ def _trimul_fwd_impl(
     H = C
     dev = z_bf.device
     _check_devices(dev, (mask_f, w_ap, w_ag, w_bp, w_bg, w_g, w_z, g_in, b_in, g_out, b_out))
-    z_bf = z_bf.contiguous()
+    z_bf = _native.aligned(z_bf.contiguous())
     mask_f = mask_f.to(torch.float32).contiguous()
     Np = int(_native.query("tpf_trimul_plane_pitch", N))
     rows = B * N * N
@@ -273,10 +273,10 @@ def _trimul_bwd_native(grad_out, z_bf, mask_f, z_ln, gate, a, b, x, xlnT, mean_i
     dev = z_bf.device
     _check_devices(dev, (grad_out, mask_f, z_ln, gate, a, b, x, xlnT, mean_in, rstd_in, mean_out,
                          rstd_out, w_ap, w_ag, w_bp, w_bg, w_g, w_z, g_in, g_out))
-    grad = grad_out.to(torch.bfloat16).contiguous()
+    # The kernels read these in 16-byte chunks at every N.
+    grad = _native.aligned(grad_out.to(torch.bfloat16).contiguous())
+    z_bf, x = _native.aligned(z_bf), _native.aligned(x)
     mask_f = mask_f.to(torch.float32).contiguous()
-    if x.data_ptr() % 16:  # the kernels read the planes in 16-byte chunks at every N
-        x = x.clone()
     *wts, gin, gout = _f32_all((w_ap, w_ag, w_bp, w_bg, w_g, w_z, g_in, g_out))
     f32 = dict(device=dev, dtype=torch.float32)
     d_z = torch.empty((B, N, N, C), device=dev, dtype=torch.bfloat16)

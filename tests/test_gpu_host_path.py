@@ -169,3 +169,55 @@ def test_host_path_saved_tensor_hooks_and_checkpoint(gpu):
     got = checkpoint(lambda x, b: attn(x, x, x, mask, b).float().sum(), q, bias, use_reentrant=False)
     for a, b in zip(ref, torch.autograd.grad(got, (q, bias))):
         assert torch.equal(a, b)
+
+
+def _misaligned(t):
+    """t's values, contiguous, starting 2 bytes past a 16-byte boundary."""
+    out = torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
+    assert out.is_contiguous() and out.data_ptr() % 16 == 2
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,D", [(33, 32), (64, 32), (33, 64), (64, 64)])
+def test_attention_misaligned_upstream_gradient(gpu, python_path, N, D):
+    """The kernels load 16 bytes at a time: an upstream gradient that starts
+    off that boundary gives the bits of the aligned one on both host paths."""
+    from openfold3_triangle_kernel_amd import turbopairformer_triangle_attention as attn
+
+    print(f"[misaligned dO] N={N} D={D}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(N)
+    xs = [torch.randn(1, 5, 2, N, D, device=gpu, generator=g).bfloat16() for _ in range(3)]
+    xs = [t.requires_grad_(True) for t in
+          (*xs, torch.randn(1, 1, 2, N, N, device=gpu, generator=g).bfloat16())]
+    mask = torch.zeros(1, 5, 1, 1, N, device=gpu)
+    dout = torch.randn(1, 5, N, 2, D, device=gpu, generator=g).bfloat16()
+
+    def run(d):
+        return torch.autograd.grad(attn(*xs[:3], mask, xs[3]), xs, d)
+
+    ref = run(dout)
+    for got in (run(_misaligned(dout)), python_path(lambda: run(_misaligned(dout)))):
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,C", [(17, 64), (24, 128)])
+def test_trimul_misaligned_pair_and_gradient(gpu, python_path, N, C):
+    """As above for TriMul's upstream gradient and for its pair input."""
+    from openfold3_triangle_kernel_amd import turbo_trimul
+
+    print(f"[misaligned trimul] N={N} C={C}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(N)
+    z, dout = (torch.randn(1, N, N, C, device=gpu, generator=g).bfloat16() for _ in range(2))
+    w = [torch.randn(s, device=gpu, generator=g) / C ** 0.5
+         for s in ((C,), (C,), (2 * C, C), (2 * C, C), (C,), (C,), (C, C), (C, C))]
+
+    def run(z, d):
+        xs = [z.detach().requires_grad_(True), *(t.detach().requires_grad_(True) for t in w)]
+        return torch.autograd.grad(turbo_trimul(xs[0], "incoming", None, *xs[1:]), xs, d)
+
+    ref = run(z, dout)
+    bad = _misaligned(z), _misaligned(dout)
+    for got in (run(z, bad[1]), run(*bad), python_path(lambda: run(*bad))):
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
