@@ -224,8 +224,9 @@ int tpf_attn_dq_dbias_bf16(const void* q, const void* k, const void* v, const vo
 /* FP32 forward (inference): q, k, v, bias f32 in the layouts above (layout:
  * TPF_QKV_SEQ_MAJOR and TPF_ANY_N only; the bias is contiguous), out f32
  * [B, O, N, H, D], lse (nullable) f32 [B, O, H, N].  Requirements: N % 64 == 0
- * unless TPF_ANY_N, D % 4 == 0 and 4 <= D <= 64.  Products to within one f32
- * rounding (three-way bf16 splits on the matrix cores), f32 sums.
+ * unless TPF_ANY_N, D % 4 == 0 and 4 <= D <= 64.  Products to within half a
+ * unit in the last place of the f32 product (three-way bf16 splits on the
+ * matrix cores), f32 sums.
  * Replaces turbopairformer_attention_fp32_forward
  * (openfold3/core/kernels/turbopairformer/turbopairformer_attention_fp32.py:139-224). */
 int64_t tpf_attn_forward_f32_workspace_bytes(int64_t B, int64_t H, int64_t N,

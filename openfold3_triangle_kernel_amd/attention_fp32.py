@@ -6,9 +6,10 @@ Mirrors the reference's FP32 path
 (unscaled) q, all inputs FP32, q/k/v ``[*B, O, H, N, D]``, the mask
 broadcasting exactly to ``[*B, O, 1, 1, N]`` and the bias to
 ``[*B, 1, H, N, N]``; returns contiguous FP32 ``[*B, O, N, H, D]``.  No
-autograd: calling it with gradients enabled raises.  Products are FP32 (each
-operand as the exact sum of three bf16 values on the matrix cores), sums and
-softmax FP32 (``csrc/attention_f32.hip``); a row whose logits are all ``-inf``
+autograd: calling it with gradients enabled raises.  Each operand enters its
+products as the exact sum of three bf16 values on the matrix cores, within half
+a unit in the last place of the FP32 products (``csrc/split_f32.hpp``); sums
+and softmax are FP32 (``csrc/attention_f32.hip``); a row whose logits are all ``-inf``
 gives zeros.
 """
 

@@ -2,9 +2,9 @@
 //
 //   out[b,o,q,h,:] = sum_k softmax_k(scale <q, k> + mask[b,o,k] + bias[bb,h,q,k]) v[k,:]
 //
-// in FP32: products of three-way bf16 splits on the bf16 matrix cores, which
-// are f32 products to within one f32 rounding (split_f32.hpp), f32 sums and
-// softmax; the contract of the reference's inference-only FP32 path
+// in FP32: products of three-way bf16 splits on the bf16 matrix cores, within
+// half a unit in the last place of the f32 products (split_f32.hpp), f32 sums
+// and softmax; the contract of the reference's inference-only FP32 path
 // (openfold3/core/kernels/turbopairformer/turbopairformer_attention_fp32.py:139-224):
 // a row whose logits are all -inf produces zeros.
 //

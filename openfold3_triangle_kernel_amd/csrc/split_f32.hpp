@@ -1,13 +1,29 @@
-// FP32 products on the bf16 matrix cores.
+// FP32 products on the bf16 matrix cores, by the three-term bfloat16 splitting
+// of Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial Intelligence
+// Datatype For Higher-Precision Computations", ARITH 2019).
 //
-// A float is the exact sum of three bf16 values cut from its mantissa 8 bits
-// at a time, x = h + m + l (h = x with its low 16 bits cleared, m the same of
-// x - h, l the rest; both differences are exact).  A product keeps the six
-// terms h h, h m, m h, m m, h l, l h; what is dropped, m l + l m + l l, is
-// below 2^-23 of |x y| (2^-25 on average), the size of one f32 rounding.  Each
-// term is an exact f32 product inside the MFMA.  On gfx950 a bf16 MFMA does 16
-// times the work of the f32 one per cycle, so six of them cost 3/8 of the f32
-// instructions they replace.  Infinite and NaN inputs give NaN.
+// A float is the exact sum of three bf16 values, x = h + m + l: h is x rounded
+// to nearest, m the rounded x - h, l the rest (both differences are exact and
+// l has at most 8 significant bits).  With x in [1, 2) 2^e, |m| <= 2^-8 2^e and
+// |l| <= 2^-17 2^e, of either sign.  A product keeps the six terms h h, h m,
+// m h, m m, h l, l h; what is dropped, m l + l m + l l, is below 2^-24 |x y|
+// (1 + 2^-9), half a unit in the last place of an f32 product, and of either
+// sign, so it averages out over a sum.  Each kept term is an exact f32 product
+// inside the MFMA, whose sums round within one unit in the last place.
+//
+// Error against 64 bits in 2^-24 of sum |x y|, rms over 2^18 sums: K = 16
+// operands of one sign 0.65 (f32 MFMA: 1.05), close to 1 + 2^-7 0.73 (1.03), of
+// both signs 0.21 (0.46); K = 384: 3.3 (4.7), 3.6 (4.9), 0.40 (0.47).  A product
+// alone is worse, 0.56 (0.42) and at most 2.4 (1.0).  Parts cut instead of
+// rounded all have x's sign: the dropped terms reach 2^-21 of every product,
+// one way (3.9 close to 1 + 2^-7 at K = 16), for 2 % less time (197 against
+// 201 us for the attention forward at N = 384).  Operands below 2^-109 have
+// parts that are subnormal in bf16, which the matrix cores read as zero: an
+// error of up to 2^-126 times the other operand.
+//
+// On gfx950 a bf16 MFMA does 16 times the work of the f32 one per cycle, so
+// six of them cost 3/8 of the f32 instructions they replace; the split takes
+// 11 VALU instructions per pair of elements.  Infinite and NaN inputs give NaN.
 #pragma once
 
 #include "common.hpp"
@@ -21,22 +37,23 @@ struct Split4 {
   bf16x4 h, m, l;
 };
 
-// The upper halves of two floats as a bf16 pair (x0 in the low half).
-__device__ __forceinline__ uint32_t hi_pair(float x0, float x1) {
-  return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+// Two floats rounded to a bf16 pair (x0 in the low half), and its halves as
+// floats.  The pair passes through an asm: left alone, the compiler rounds x0
+// a second time for its half (13 instructions per pair).
+__device__ __forceinline__ uint32_t bf_pair(float x0, float x1) {
+  uint32_t p = __builtin_bit_cast(uint32_t, bf16x2{f2bf(x0), f2bf(x1)});
+  asm("" : "+v"(p));
+  return p;
 }
-// (Forming x - h by a dot product with the packed pair, 7 instructions per
-// pair instead of 11, measured slower: 208 against 195 us on the attention
-// forward at N = 384.)
-__device__ __forceinline__ float below_hi(float x) {
-  return x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u);
-}
+__device__ __forceinline__ float pair_lo(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float pair_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& h, uint32_t& m,
                                            uint32_t& l) {
-  h = hi_pair(x0, x1);
-  const float r0 = below_hi(x0), r1 = below_hi(x1);
-  m = hi_pair(r0, r1);
-  l = hi_pair(below_hi(r0), below_hi(r1));
+  h = bf_pair(x0, x1);
+  x0 -= pair_lo(h);
+  x1 -= pair_hi(h);
+  m = bf_pair(x0, x1);
+  l = bf_pair(x0 - pair_lo(m), x1 - pair_hi(m));
 }
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   u32x4 h, m, l;

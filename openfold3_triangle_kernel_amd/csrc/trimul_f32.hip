@@ -6,8 +6,9 @@
 //   a = mask sigmoid(a_g) a_p, b = mask sigmoid(b_g) b_p;
 //   x_c = A_c B_c^T (outgoing: A_c[i][k] = a[i,k,c]; incoming: a[k,i,c]);
 //   out = (LN_out(x) W_z^T (+ b_z)) * sigmoid(zln W_g^T (+ b_g)).
-// All storage, sums and pointwise arithmetic in FP32; products to within one
-// f32 rounding on the bf16 matrix cores (split_f32.hpp).
+// All storage, sums and pointwise arithmetic in FP32; products on the bf16
+// matrix cores, within half a unit in the last place of the f32 products
+// (split_f32.hpp).
 //
 // Layouts (R = B*N*N rows, C4 / H4 = C / H rounded up to 4, zero padded):
 //   zln, gate [R][C4]; xln [R][H4]; a, b, x channel-major [B*H][N][Np]

@@ -233,8 +233,8 @@ def test_attention_fp32_any_sequence_length(gpu, B, O, H, N, D, seq_major):
 def test_gemm_f32_products_are_fp32(gpu, M, N, K, scale):
     """tpf_gemm_f32 forms its products from three-way bf16 splits: rel-L2
     against FP64 within 2 K^0.5 eps (K additions of random sign; a dropped
-    split term of 2^-16 would exceed it), whatever the operands' magnitude,
-    and exact on values of one split part."""
+    split term of 2^-16 would exceed it), for operands of ordinary and of
+    extreme magnitude, and exact on values of one split part."""
     from openfold3_triangle_kernel_amd import _native
 
     g = torch.Generator().manual_seed(M + K)
@@ -254,3 +254,48 @@ def test_gemm_f32_products_are_fp32(gpu, M, N, K, scale):
     assert err <= 2 * K ** 0.5 * 2.0 ** -24
     ai, bi = torch.randint(-9, 10, (M, K), generator=g).float(), torch.randint(-9, 10, (Np, K), generator=g).float()
     assert torch.equal(run(ai, bi), ai.double() @ bi.double().t())
+
+
+def _gemm_f32(a, b, dev):
+    """a [M, K] @ b [N, K]^T on tpf_gemm_f32 (K and N multiples of 4), as FP64."""
+    from openfold3_triangle_kernel_amd import _native
+
+    (M, K), N = a.shape, b.shape[0]
+    a, b, c = a.to(dev), b.to(dev), torch.empty(M, N, device=dev)
+    _native.call("tpf_gemm_f32", a.data_ptr(), 1, K, 0, b.data_ptr(), 1, K, 0, c.data_ptr(), N, 0,
+                 M, N, K, 1, 1.0, None, torch.cuda.current_stream().cuda_stream)
+    return c.cpu().double()
+
+
+@pytest.mark.gpu
+def test_gemm_f32_single_products(gpu):
+    """One product per output, over random significands and those whose split
+    parts are largest: the dropped terms are below 2^-24 of it and the last sum
+    rounds within one unit in the last place, 2^-23 of it (the sums before are
+    below 2^-7 of it, hence the factor)."""
+    g = torch.Generator().manual_seed(0)
+    bits = torch.randint(1 << 23, (256,), generator=g)
+    bits[:8] = torch.tensor([0x00FFFF, 0x7FFFFF, 0x008080, 0x008000, 0x007FFF, 0x7F7FFF, 0x018181,
+                             0x000001])
+    x = ((bits + 0x3F800000).to(torch.int32)).view(torch.float32)
+    a = torch.zeros(256, 4)
+    a[:, 0] = x
+    ref = a.double() @ a.double().t()
+    err = ((_gemm_f32(a, a, gpu) - ref).abs() / ref).max().item()
+    print(f"single products: largest error {err * 2 ** 24:.3f} * 2^-24", flush=True)
+    assert err <= 3 * 2.0 ** -24 * (1 + 2.0 ** -7)
+
+
+@pytest.mark.gpu
+def test_gemm_f32_same_sign_sums_are_unbiased(gpu):
+    """Operands of one sign just below 1 + 2^-7 (K = 16, one MFMA step): every
+    sum within its 16 roundings and the dropped terms, and no error of one
+    sign: the mean over 2^16 sums stays below a quarter of one rounding."""
+    g = torch.Generator().manual_seed(1)
+    a, b = (1 + 2.0 ** -7 * (1 - 0.1 * torch.rand(256, 16, generator=g)) for _ in range(2))
+    ref = a.double() @ b.double().t()
+    err = (_gemm_f32(a, b, gpu) - ref) / ref
+    print(f"same-sign sums: mean {err.mean() * 2 ** 24:.3f}, largest "
+          f"{err.abs().max() * 2 ** 24:.3f} (* 2^-24)", flush=True)
+    assert err.abs().max() <= 17 * 2.0 ** -24
+    assert err.mean().abs() <= 2.0 ** -26
