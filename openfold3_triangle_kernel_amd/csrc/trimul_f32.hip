@@ -358,8 +358,11 @@ __global__ __launch_bounds__(256, 2) void tm32_out_proj_kernel(
   GemmOperandF32 W{wz, g.H4, g.C};
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rl = lane & 31, hl = lane >> 5, wm = w >> 1, wn = w & 1;
-  // The gate values of this lane's accumulator elements are loaded before
-  // the main loop, so their latency overlaps it.
+  f32x16 acc[2][2];
+  gemm_tile_f32<true, true>(A, W, (int)m0, nt * 128, 0, g.H4, smem, acc);
+  // The gate values of this lane's accumulator elements, all loads in flight
+  // together.  (Loaded before the main loop they do not fit the registers
+  // beside its fragments.)
   float gv[2][2][16];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -372,8 +375,6 @@ __global__ __launch_bounds__(256, 2) void tm32_out_proj_kernel(
         gv[j][i][r] = (c < g.C && rho < g.R) ? gate[rho * g.C4 + c] : 0.f;
       }
   }
-  f32x16 acc[2][2];
-  gemm_tile_f32<true, true>(A, W, (int)m0, nt * 128, 0, g.H4, smem, acc);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int c = nt * 128 + 64 * wn + 32 * j + rl;
