@@ -14,9 +14,11 @@
 // seeded with the prescaled, fragment-major bias, online softmax with a
 // lazily raised running max, V^T operands through transposing reads.  K and V
 // are split once per workgroup, when a tile is written to LDS (three bf16
-// tiles each), Q once per wave, and P in registers on its way into the P V
-// product.  A sequence that ends inside a tile reads zeros past N through the
+// tiles each), Q once per wave, and P (finite, or NaN where a score is +inf or
+// NaN) in registers on its way into the P V product.  A sequence that ends inside a tile reads zeros past N through the
 // range of the buffer resources and masks those keys.
+#include <type_traits>
+
 #include "attn_tile.hpp"
 #include "common.hpp"
 #include "split_f32.hpp"
@@ -117,7 +119,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[4 * u + e] = y[e];
       }
-      qs[s] = split8(x);
+      bool ok;
+      qs[s] = split8(x, &ok);
+      if (!__all(ok)) qs[s] = split8<true>(x);
     }
   }
   // K / V chunk it of this thread: row (it * 256 + tid) / CH of the tile.  The
@@ -143,12 +147,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 
       vr[it] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, vkv[it], 0, 0));
     }
   };
-  auto store_kv = [&](int buf) {
+  auto store_split = [&](int buf, auto all) {  // whether the split served every element
+    bool ok = true;
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int idx = it * 256 + tid;
       const int off = kv_off<DP>(idx / CH, 4 * (idx % CH));
-      const Split4 ks = split4(kr[it]), vs = split4(vr[it]);
+      bool okk, okv;
+      const Split4 ks = split4<decltype(all)::value>(kr[it], &okk);
+      const Split4 vs = split4<decltype(all)::value>(vr[it], &okv);
+      ok &= okk & okv;
       *reinterpret_cast<bf16x4*>(&KVs[buf][0][0][off]) = ks.h;
       *reinterpret_cast<bf16x4*>(&KVs[buf][0][1][off]) = ks.m;
       *reinterpret_cast<bf16x4*>(&KVs[buf][0][2][off]) = ks.l;
@@ -156,6 +164,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 
       *reinterpret_cast<bf16x4*>(&KVs[buf][1][1][off]) = vs.m;
       *reinterpret_cast<bf16x4*>(&KVs[buf][1][2][off]) = vs.l;
     }
+    return ok;
+  };
+  auto store_kv = [&](int buf) {
+    if (!__all(store_split(buf, std::false_type{}))) store_split(buf, std::true_type{});
   };
   const __amdgpu_buffer_rsrc_t rs_b = raw_rsrc(
       bias_s + (int64_t)b * g.bias_bstride +

@@ -107,7 +107,7 @@ struct TileLoaderF32 {
 };
 
 // The eight k values 16 s + 8 (lane / 32) .. + 7 of row rbase + lane % 32, split.
-template <bool KC>
+template <bool KC, bool ALL>
 __device__ __forceinline__ Split8 tile_frag_f32(const float* T, int rbase, int s) {
   const int lane = threadIdx.x & 63, hl = lane >> 5;
   const int r = rbase + (lane & 31);
@@ -124,13 +124,17 @@ __device__ __forceinline__ Split8 tile_frag_f32(const float* T, int rbase, int s
       for (int e = 0; e < 4; ++e) v[4 * u + e] = T[(16 * s + 8 * hl + 4 * u + e) * kFM + r];
     }
   }
-  return split8(v);
+  return split8<ALL>(v);
 }
 
-template <bool A_KC, bool B_KC>
-__device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const GemmOperandF32& B,
-                                              int m0, int n0, int kbeg, int kend, char* smem,
-                                              f32x16 (&acc)[2][2]) {
+// The tile's products with one kind of split (split_pair), the same on all
+// threads: returns whether any sum of the tile is NaN.
+template <bool A_KC, bool B_KC, bool ALL>
+__device__ __forceinline__ bool gemm_tile_f32_pass(const GemmOperandF32& A,
+                                                   const GemmOperandF32& B, int m0, int n0,
+                                                   int kbeg, int kend, char* smem,
+                                                   f32x16 (&acc)[2][2]) {
+  __shared__ int nan_s[4];
   const int w = threadIdx.x >> 6;
   const int wm = w >> 1, wn = w & 1;
 #pragma unroll
@@ -142,7 +146,7 @@ __device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const Gem
   la.init(A, m0);
   lb.init(B, n0);
   const int nk = (kend - kbeg + kFK - 1) / kFK;
-  if (nk <= 0) return;
+  if (nk <= 0) return false;
   la.issue(kbeg, kend, smem);
   lb.issue(kbeg, kend, smem + kFTileBytes);
   for (int kt = 0; kt < nk; ++kt) {
@@ -161,8 +165,8 @@ __device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const Gem
       Split8 af[2], bfr[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        af[t] = tile_frag_f32<A_KC>(As, 64 * wm + 32 * t, s);
-        bfr[t] = tile_frag_f32<B_KC>(Bs, 64 * wn + 32 * t, s);
+        af[t] = tile_frag_f32<A_KC, ALL>(As, 64 * wm + 32 * t, s);
+        bfr[t] = tile_frag_f32<B_KC, ALL>(Bs, 64 * wn + 32 * t, s);
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
@@ -170,7 +174,26 @@ __device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const Gem
         for (int j = 0; j < 2; ++j) acc[i][j] = mfma32_split(af[i], bfr[j], acc[i][j]);
     }
   }
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bad |= __builtin_isunordered(acc[i][0][r], acc[i][1][r]);
+  const int any = __any(bad);
+  if ((threadIdx.x & 63) == 0) nan_s[w] = any;
   lds_barrier();
+  return __builtin_amdgcn_readfirstlane(nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;
+}
+
+// Operands are taken to be finite floats below the largest bf16; where one is
+// not, some sum is NaN, and the tile is formed again with the split that
+// serves every float (no test of the operands in the main loop).
+template <bool A_KC, bool B_KC>
+__device__ __forceinline__ void gemm_tile_f32(const GemmOperandF32& A, const GemmOperandF32& B,
+                                              int m0, int n0, int kbeg, int kend, char* smem,
+                                              f32x16 (&acc)[2][2]) {
+  if (gemm_tile_f32_pass<A_KC, B_KC, false>(A, B, m0, n0, kbeg, kend, smem, acc))
+    gemm_tile_f32_pass<A_KC, B_KC, true>(A, B, m0, n0, kbeg, kend, smem, acc);
 }
 
 }  // namespace tpf

@@ -23,7 +23,7 @@
 //
 // On gfx950 a bf16 MFMA does 16 times the work of the f32 one per cycle, so
 // six of them cost 3/8 of the f32 instructions they replace; the split takes
-// 11 VALU instructions per pair of elements.  Infinite and NaN inputs give NaN.
+// 11 VALU instructions per pair of elements.
 #pragma once
 
 #include "common.hpp"
@@ -47,41 +47,71 @@ __device__ __forceinline__ uint32_t bf_pair(float x0, float x1) {
 }
 __device__ __forceinline__ float pair_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float pair_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
-__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& h, uint32_t& m,
+// Two floats split.  False where a part is NaN: for a NaN, an infinity, or a
+// float above the largest bf16 (h rounds to infinity).
+//
+// ALL splits those too, so that products are those of f32 arithmetic: an
+// infinity is (+-1, 0, +-inf), whose l meets only the other operand's h (of the
+// same sign, 0 if the operand is 0: NaN as it should be) and whose h and m
+// meet finite parts or the other infinity; a large float takes the largest
+// bf16 as h.
+template <bool ALL>
+__device__ __forceinline__ bool split_pair(float x0, float x1, uint32_t& h, uint32_t& m,
                                            uint32_t& l) {
-  h = bf_pair(x0, x1);
-  x0 -= pair_lo(h);
-  x1 -= pair_hi(h);
-  m = bf_pair(x0, x1);
-  l = bf_pair(x0 - pair_lo(m), x1 - pair_hi(m));
+  if constexpr (ALL) {
+    const float big = __uint_as_float(0x7F7F0000u);
+    const bool i0 = __builtin_isinf(x0), i1 = __builtin_isinf(x1);
+    auto head = [&](float x, bool inf) {
+      return inf || fabsf(x) > big ? copysignf(inf ? 1.f : big, x) : x;
+    };
+    h = bf_pair(head(x0, i0), head(x1, i1));
+    const float r0 = i0 ? 0.f : x0 - pair_lo(h), r1 = i1 ? 0.f : x1 - pair_hi(h);
+    m = bf_pair(r0, r1);
+    l = bf_pair(i0 ? x0 : r0 - pair_lo(m), i1 ? x1 : r1 - pair_hi(m));
+    return true;
+  } else {
+    h = bf_pair(x0, x1);
+    x0 -= pair_lo(h);
+    x1 -= pair_hi(h);
+    m = bf_pair(x0, x1);
+    x0 -= pair_lo(m);
+    x1 -= pair_hi(m);
+    l = bf_pair(x0, x1);
+    return !__builtin_isunordered(x0, x1);
+  }
 }
-__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+template <bool ALL = false>
+__device__ __forceinline__ Split8 split8(const float (&x)[8], bool* ok = nullptr) {
   u32x4 h, m, l;
+  bool good = true;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     uint32_t a, b, c;
-    split_pair(x[2 * e], x[2 * e + 1], a, b, c);
+    good &= split_pair<ALL>(x[2 * e], x[2 * e + 1], a, b, c);
     h[e] = a;
     m[e] = b;
     l[e] = c;
   }
+  if (ok) *ok = good;
   return Split8{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m),
                 __builtin_bit_cast(bf16x8, l)};
 }
-__device__ __forceinline__ Split4 split4(const f32x4& x) {
+template <bool ALL = false>
+__device__ __forceinline__ Split4 split4(const f32x4& x, bool* ok = nullptr) {
   u32x2 h, m, l;
+  bool good = true;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     uint32_t a, b, c;
-    split_pair(x[2 * e], x[2 * e + 1], a, b, c);
+    good &= split_pair<ALL>(x[2 * e], x[2 * e + 1], a, b, c);
     h[e] = a;
     m[e] = b;
     l[e] = c;
   }
+  if (ok) *ok = good;
   return Split4{__builtin_bit_cast(bf16x4, h), __builtin_bit_cast(bf16x4, m),
                 __builtin_bit_cast(bf16x4, l)};
 }
-
 // c + a b, the small terms first.
 __device__ __forceinline__ f32x16 mfma32_split(const Split8& a, const Split8& b, f32x16 c) {
   c = mfma32(a.l, b.h, c);

@@ -299,3 +299,52 @@ def test_gemm_f32_same_sign_sums_are_unbiased(gpu):
           f"{err.abs().max() * 2 ** 24:.3f} (* 2^-24)", flush=True)
     assert err.abs().max() <= 17 * 2.0 ** -24
     assert err.mean().abs() <= 2.0 ** -26
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("special", [float("inf"), float("-inf"), float("nan"), 3.4e38, -3.4e38])
+def test_gemm_f32_infinities_and_largest_values(gpu, special):
+    """Operands that are infinite, NaN or round to infinity in bf16 act as in
+    f32 arithmetic, beside ordinary outputs that keep their values."""
+    g = torch.Generator().manual_seed(2)
+    a, b = torch.randn(130, 36, generator=g), torch.randn(68, 36, generator=g)
+    b[:, 5] = torch.tensor([1.0, -1.0, 0.5, 2.0 ** -20]).repeat(17)  # one split part: m = l = 0
+    b[7, 5] = 0.0
+    clean = _gemm_f32(a, b, gpu)
+    a[3, 5] = special
+    a[70, 5] = -special
+    got, ref = _gemm_f32(a, b, gpu), a.double() @ b.double().t()
+    rows = torch.tensor([r not in (3, 70) for r in range(130)])
+    assert torch.equal(got[rows], clean[rows])
+    ref = ref.float().double()  # overflow where f32 overflows
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    fin = ref.isfinite()
+    assert torch.equal(got[ref.isinf()], ref[ref.isinf()])
+    assert ((got - ref).abs()[fin] <= 37 * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())[fin]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,D", [(64, 32), (70, 64)])
+def test_attention_fp32_infinities(gpu, N, D):
+    """FP32 attention with an infinite value at an unmasked key, a key whose
+    score is -inf (weight 0) and a value near the largest float, against the
+    same in FP64."""
+    from openfold3_triangle_kernel_amd import turbopairformer_attention_fp32
+
+    q, k, v, mask, bias = _f32_case(1, 3, 2, N, D, seed=N)
+    q[..., 0] = q[..., 0].abs() + 0.1
+    k[0, 0, 0, 5, 0] = float("-inf")
+    v[0, 1, 1, 9, 3] = float("inf")
+    v[0, 1, 1, 11, 4] = float("-inf")
+    v[0, 2, 0, 40, 7] = 3.4e38
+    bias[..., 40] -= 30  # (its weight well below 1: the sums are unnormalised)
+    with torch.no_grad():
+        out = turbopairformer_attention_fp32(*(t.to(gpu) for t in (q, k, v, mask, bias))).cpu()
+    s = (q.double() @ k.double().transpose(-1, -2)) / D ** 0.5 + mask.double() + bias.double()
+    ref = (torch.softmax(s, -1) @ v.double()).transpose(-2, -3)
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    assert torch.equal(out[ref.isinf()].double(), ref[ref.isinf()]) and ref.isinf().any()
+    assert not ref.isnan().any()
+    fin = ref.isfinite()
+    rel = (out.double() - ref).abs()[fin] / ref.abs()[fin].clamp(min=1e-2)
+    assert rel.max() <= TOL
