@@ -176,17 +176,18 @@ __global__ __launch_bounds__(256) void tm32_ln_rows_vec_kernel(const float* __re
 }
 
 // LN_out over the H channels of the channel-major product, register-resident:
-// workgroup = 64 plane positions x all channels; thread = (4-position group pg = tid % 16, channel group cg = tid / 16 of
-// CPT channels).  Each thread issues all of its CPT float4 loads at once and
+// workgroup = 64 plane positions x all channels; thread = (4-position group
+// pg = tid % 16, channel group cg = tid / 16 of CPT channels).  Each thread issues all of its CPT float4 loads at once and
 // keeps the CPT x 4 block in registers; per-position channel sums go through
 // the 4 channel groups of a wave by shuffles and the 4 waves through LDS in
 // fixed order (mean first, then the centred sum of squares).  Rows of xln
 // are written as float4 runs of the thread's channels (pad channels up to
 // H4 as zeros).  Needs H <= 16 * CPT.  The walk is over plane positions (Np a
 // multiple of 4, so a thread's four share a plane row); the pad positions of
-// N % 4 != 0 write nothing (two bytes at a time over rows, N = 333 took 62 us
-// against 33).
-template <int CPT>
+// N % 4 != 0 (PAD) write nothing (four bytes at a time over rows, N = 333 took
+// 62 us against 33).  Without pad a position is its row: with the map and its
+// predicated stores N = 384 took 47 us against 36.
+template <int CPT, bool PAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void tm32_ln_planes_reg_kernel(
     const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
     float eps, float* __restrict__ xln, Tm32Geom g) {
@@ -197,9 +198,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
   const int64_t pb = (int64_t)blockIdx.x * T + 4 * pg;  // first position of this thread
   const bool pos_ok = pb < g.PS;                       // PS % 4 == 0: all 4 or none
   const int c0 = cg * CPT;
-  const uint32_t pi = fdiv((uint32_t)pb, g.div_np);
+  const uint32_t pi = PAD ? fdiv((uint32_t)pb, g.div_np) : 0u;
   const int col = (int)((uint32_t)pb - pi * (uint32_t)g.Np);
-  const int64_t row0 = (int64_t)b * g.NN + (int64_t)pi * g.N + col;  // row of the first position
+  // Row of the first position.
+  const int64_t row0 = (int64_t)b * g.NN + (PAD ? (int64_t)pi * g.N + col : pb);
   float v[CPT][4];
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (col + e >= g.N) continue;
+      if (PAD && col + e >= g.N) continue;
       f32x4 o;
 #pragma unroll
       for (int k = 0; k < 4; ++k) o[k] = (v[4 * c4 + k][e] - mean[e]) * rstd[e] * gm[k] + bt[k];
@@ -528,12 +530,13 @@ int tpf_trimul_forward_f32_chunked(const float* z, const float* mask, const floa
       gc.B = 1; gc.NN = rows * N; gc.PS = rows * g.Np; gc.R = rows * N; gc.Rp = gc.PS;
       const int64_t r0 = bb * g.NN + i0 * N;  // first pair row of the chunk
       const dim3 ln_grid((unsigned)((gc.PS + 63) / 64), 1u);
-      if (H <= 128)
-        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<8>, ln_grid, dim3(256), 0, s, wk.x, ln_out_w,
-                           ln_out_b, (float)ln_out_eps, wk.xln, gc);
-      else
-        hipLaunchKernelGGL(tm32_ln_planes_reg_kernel<16>, ln_grid, dim3(256), 0, s, wk.x, ln_out_w,
-                           ln_out_b, (float)ln_out_eps, wk.xln, gc);
+#define TM32_LN_OUT(CPT, PAD)                                                                  \
+  hipLaunchKernelGGL((tm32_ln_planes_reg_kernel<CPT, PAD>), ln_grid, dim3(256), 0, s, wk.x,     \
+                     ln_out_w, ln_out_b, (float)ln_out_eps, wk.xln, gc)
+      const bool pad = g.Np != N;
+      if (H <= 128) { if (pad) TM32_LN_OUT(8, true); else TM32_LN_OUT(8, false); }
+      else { if (pad) TM32_LN_OUT(16, true); else TM32_LN_OUT(16, false); }
+#undef TM32_LN_OUT
       if ((rc = check_launch(fn))) return rc;
       const int64_t otiles = (gc.R + 127) / 128 * ((C + 127) / 128);
       hipLaunchKernelGGL(tm32_out_proj_kernel, dim3((unsigned)((otiles + 7) / 8 * 8)), dim3(256), 0,
