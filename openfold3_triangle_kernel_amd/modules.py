@@ -399,7 +399,8 @@ class TriangleAttention(nn.Module):
         ``chunk_size`` (inference only on the stable route, as the reference's
         ``triangular_attention.py:114-158, 322-327``) runs the projections,
         attention, gate and output projection over chunks of outer rows with
-        the full pair bias; the output is bitwise the unchunked one.
+        the full pair bias; the output of the pair-row core and of FP32
+        inference is bitwise the unchunked one.
         ``inplace_safe`` only saves memory in the reference and is accepted.
         """
         _reject_backends(use_deepspeed_evo_attention=use_deepspeed_evo_attention,
@@ -553,7 +554,11 @@ class TriangleAttention(nn.Module):
         """The pair-row core over all outer rows, or over chunks of them with
         the bias of every pair projected once (the reference's
         ``_chunk_stable``, ``triangular_attention.py:114-158``).  A projection
-        row and an attention plane do not depend on the chunk they are in."""
+        row does not depend on the chunk it is in, and neither does an
+        attention plane for head dimensions above 32.  Up to 32 the forward
+        runs outer rows 2 i and 2 i + 1 together and raises both running maxima
+        at once, so chunks hold whole pairs (an odd ``chunk_size`` is taken one
+        smaller, 1 as 2)."""
         m = self.mha
         H, c, N, C = m.no_heads, m.c_hidden, x.shape[-2], self.c_in
         shadow_enabled()  # the policy variables are checked as in training
@@ -577,8 +582,10 @@ class TriangleAttention(nn.Module):
         w_z = torch.cat([self.linear_z.weight, zeros((-H) % 16, C)]).to(torch.bfloat16)
         bias_rows = _mm(x4.reshape(-1, C), w_z, True)
         out = torch.empty_like(x4)
-        for start in range(0, N, chunk_size):
-            rows = slice(start, min(start + chunk_size, N))
+        pair = 2 if c <= 32 else 1
+        step = max(pair, chunk_size - chunk_size % pair)
+        for start in range(0, N, step):
+            rows = slice(start, min(start + step, N))
             out[:, rows] = _PairAttentionInference.apply(
                 x4[:, rows].contiguous(), w_all, m.linear_o.weight, mask_add[:, rows].contiguous(),
                 bias_rows, H, c, bool(transpose_bias), False)
@@ -603,7 +610,8 @@ class TriangleAttention(nn.Module):
         projected once; each chunk projects its rows' q / k / v / gate, runs
         attention over its planes with the full bias, gates and projects its
         output rows.  Per-row GEMMs and per-plane attention make the output
-        bitwise that of the unchunked call."""
+        bitwise that of the unchunked call (in BF16, whose forward runs outer
+        rows in pairs, for even chunk sizes)."""
         m = self.mha
         H, c = m.no_heads, m.c_hidden
         hc = H * c

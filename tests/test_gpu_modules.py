@@ -284,3 +284,23 @@ def test_triangle_attention_module_broadcast_mask(gpu, shape, starting, N, chunk
             y = m(xg, k)
             res.append([y, *torch.autograd.grad(y, [xg, *m.parameters()], x)])
         assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,C,D", [(1, 33, 128, 32), (2, 50, 64, 16), (1, 65, 128, 64)])
+def test_triangle_attention_module_odd_chunks(gpu, B, N, C, D):
+    """Odd chunk sizes too give the bits of the whole call: the forward runs
+    outer rows in pairs, and a chunk never parts one."""
+    from openfold3_triangle_kernel_amd import TriangleAttention
+
+    torch.manual_seed(N)
+    m = TriangleAttention(C, D, 4).to(gpu).bfloat16()
+    for p in m.parameters():
+        p.data.normal_(std=1.0)  # scores that raise the running maximum often
+    x = torch.randn(B, N, N, C, device=gpu).bfloat16()
+    mask = (torch.rand(B, N, N, device=gpu) > 0.1).bfloat16()
+    print(f"odd chunks B={B} N={N} C={C} D={D}", flush=True)
+    with torch.no_grad():
+        whole = m(x, mask)
+        for c in (1, 3, 5, N - 1, N):
+            assert torch.equal(whole, m(x, mask, chunk_size=c)), f"chunk_size {c}"
