@@ -41,7 +41,8 @@ void check(int rc, const char* fn) {
 void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
 // The policy variables as the facade reads them: the canonical name, then
-// the older one, then "1"; surrounding blanks dropped.
+// the older one, then "1"; surrounding blanks dropped.  Called with the GIL
+// held: Python's os.environ assignments change the environment under it.
 std::string env_flag(const char* canonical, const char* legacy) {
   const char* v = std::getenv(canonical);
   if (!v) v = std::getenv(legacy);
@@ -156,8 +157,10 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
   }
 };
 
+// backward, shadow: the policy variables (env_flag).
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v,
-                                const Tensor& res_mask, const Tensor& pair_bias) {
+                                const Tensor& res_mask, const Tensor& pair_bias,
+                                const std::string& backward, const std::string& sh) {
   if (transforms_active() || !q.is_cuda()) return std::nullopt;
   const c10::DeviceIndex dev = c10::hip::current_device();
   for (const Tensor* t : {&q, &k, &v, &res_mask, &pair_bias})
@@ -184,9 +187,7 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   const at::IntArrayRef bp = pair_bias.sizes().slice(0, pair_bias.dim() - 4);
   const bool shared = c10::multiply_integers(bp) == 1 && bp.size() <= prefix.size();
   if (!shared && bp != prefix) return std::nullopt;
-  if (env_flag("TURBOPAIRFORMER_SR_BACKWARD", "OPENFOLD3_SR_BACKWARD") == "0") return std::nullopt;
-  const std::string sh = env_flag("TURBOPAIRFORMER_SR_SHADOW", "OPENFOLD3_SR_SHADOW");
-  if (sh != "0" && sh != "1") return std::nullopt;
+  if (backward == "0" || (sh != "0" && sh != "1")) return std::nullopt;
 
   // One storage order for q, k and v: contiguous, or the transposed view of a
   // contiguous [*B, O, N, H, D] projection.
@@ -355,7 +356,13 @@ std::optional<Tensor> trimul(const Tensor& z, const std::optional<Tensor>& mask_
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("attention", &attention, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& res_mask,
+                        const Tensor& pair_bias) {
+    const std::string backward = env_flag("TURBOPAIRFORMER_SR_BACKWARD", "OPENFOLD3_SR_BACKWARD");
+    const std::string shadow = env_flag("TURBOPAIRFORMER_SR_SHADOW", "OPENFOLD3_SR_SHADOW");
+    pybind11::gil_scoped_release nogil;
+    return attention(q, k, v, res_mask, pair_bias, backward, shadow);
+  });
   m.def("trimul", &trimul, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("set_workspace_budget", [](int64_t bytes) { g_budget.store(bytes); });
 }

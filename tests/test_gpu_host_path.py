@@ -221,3 +221,65 @@ def test_trimul_misaligned_pair_and_gradient(gpu, python_path, N, C):
     bad = _misaligned(z), _misaligned(dout)
     for got in (run(z, bad[1]), run(*bad), python_path(lambda: run(*bad))):
         assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+@pytest.mark.gpu
+def test_host_path_threads_streams_and_environment(gpu):
+    """Two threads, each on a stream of its own, run both operators forward
+    and backward while a third assigns environment variables (the policy
+    variables are read under the GIL, as those assignments are made): the bits
+    of one thread on the default stream."""
+    import os
+    import threading
+
+    from openfold3_triangle_kernel_amd import turbo_trimul
+    from openfold3_triangle_kernel_amd import turbopairformer_triangle_attention as attn
+
+    g = torch.Generator(device=gpu).manual_seed(3)
+    q, k, v = (torch.randn(1, 9, 2, 70, 32, device=gpu, generator=g).bfloat16() for _ in range(3))
+    bias = torch.randn(1, 1, 2, 70, 70, device=gpu, generator=g).bfloat16()
+    mask, z = torch.zeros(1, 9, 1, 1, 70, device=gpu), torch.randn(
+        1, 33, 33, 64, device=gpu, generator=g).bfloat16()
+    w = [torch.randn(s, device=gpu, generator=g) / 8
+         for s in ((64,), (64,), (128, 64), (128, 64), (64,), (64,), (64, 64), (64, 64))]
+
+    def both():
+        xs = [t.detach().requires_grad_(True) for t in (q, k, v, bias, z, *w)]
+        a = attn(*xs[:3], mask, xs[3])
+        t = turbo_trimul(xs[4], "outgoing", None, *xs[5:])
+        return [a, t, *torch.autograd.grad((a, t), xs, (a.detach(), t.detach()))]
+
+    ref = [t.clone() for t in both()]
+    torch.cuda.synchronize()
+    failed, done = [], threading.Event()
+
+    def work():
+        try:
+            with torch.cuda.stream(torch.cuda.Stream(gpu)):
+                for _ in range(20):
+                    got = both()
+                torch.cuda.current_stream().synchronize()
+                if not all(torch.equal(a, b) for a, b in zip(got, ref)):
+                    failed.append("outputs differ")
+        except Exception as e:  # reported by the main thread
+            failed.append(repr(e))
+
+    def assign():
+        i = 0
+        while not done.is_set() and i < 100_000:
+            os.environ[f"TPF_TEST_{i % 300}"] = "x" * (i % 50)
+            i += 1
+
+    workers = [threading.Thread(target=work) for _ in range(2)]
+    writer = threading.Thread(target=assign)
+    try:
+        for t in (writer, *workers):
+            t.start()
+        for t in workers:
+            t.join()
+    finally:
+        done.set()
+        writer.join()
+        for i in range(300):
+            os.environ.pop(f"TPF_TEST_{i}", None)
+    assert not failed, failed
