@@ -19,6 +19,7 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.utils._device import DeviceContext
 
 LIB_PATH = Path(__file__).resolve().parent / "libtpf_amd.so"
 
@@ -190,11 +191,17 @@ def host():
 
 def host_eligible(*tensors) -> bool:
     """Plain tensors (or parameters, or None) in eager code: no subclass, no
-    compilation, no tracing.  The extension checks the rest."""
+    compilation, no tracing, no TorchFunctionMode that wants to see the torch
+    calls (torch's own default-device mode acts on factories without a device,
+    which neither path uses).  The extension checks the rest."""
     for t in tensors:
         if t is not None and type(t) not in _PLAIN_TYPES:
             return False
-    return not torch.compiler.is_compiling() and not torch._C._is_tracing()
+    if torch.compiler.is_compiling() or torch._C._is_tracing():
+        return False
+    modes = torch._C._len_torch_function_stack()
+    return not modes or all(type(torch._C._get_function_stack_at(i)) is DeviceContext
+                            for i in range(modes))
 
 
 def call(name: str, *args) -> int:

@@ -283,3 +283,38 @@ def test_host_path_threads_streams_and_environment(gpu):
         for i in range(300):
             os.environ.pop(f"TPF_TEST_{i}", None)
     assert not failed, failed
+
+
+@pytest.mark.gpu
+def test_host_path_leaves_torch_function_modes_to_python(gpu):
+    """An active TorchFunctionMode sees the torch calls of both operators; a
+    default device (a mode of torch's own, for tensor factories) keeps the
+    host path."""
+    from openfold3_triangle_kernel_amd import _native, turbo_trimul
+    from openfold3_triangle_kernel_amd import turbopairformer_triangle_attention as attn
+
+    class Seen(torch.overrides.TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    q = torch.randn(1, 2, 1, 16, 8, device=gpu).bfloat16()
+    mask, bias = torch.zeros(1, 2, 1, 1, 16, device=gpu), torch.zeros(1, 1, 1, 16, 16, device=gpu)
+    z, w = torch.randn(1, 8, 8, 32, device=gpu).bfloat16(), torch.randn(64, 32, device=gpu)
+    ln = torch.ones(32, device=gpu)
+
+    def trimul():
+        return turbo_trimul(z, "outgoing", None, ln, ln, w, w, ln, ln, w[:32], w[:32])
+
+    ref = attn(q, q, q, mask, bias), trimul()
+    for call, want in zip((lambda: attn(q, q, q, mask, bias), trimul), ref):
+        with Seen() as mode:
+            assert torch.equal(call(), want)
+        assert mode.names
+        with torch.device(gpu):
+            assert _native.host_eligible(q)
+            assert torch.equal(call(), want)
