@@ -29,7 +29,8 @@ enum {
 
 /* Message of the last failed call on this thread ("" if none). */
 const char* tpf_last_error(void);
-/* ABI revision of this header (8). */
+/* ABI revision of this header, and of the library. */
+#define TPF_ABI_VERSION 8
 int tpf_abi_version(void);
 
 /* ------------------------------------------------------------------------

@@ -16,6 +16,7 @@ import contextlib
 import ctypes
 import importlib
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -179,14 +180,28 @@ _HOST = None
 def host():
     """The extension that runs the operators' host path for plain eager tensors
     (``csrc/host/torch_host.cpp``), loaded once; None when only the C-ABI
-    library is built (the Python path then serves every call)."""
+    library is built, or when the extension does not load beside the installed
+    torch (reported once): the Python path, on the same kernels, then serves
+    every call."""
     global _HOST
     if _HOST is None:
         with _LOCK:
             if _HOST is None:
-                _HOST = (importlib.import_module("._tpf_host", __package__)
-                         if HOST_PATH.exists() and LIB_PATH.exists() else False)
+                _HOST = _load_host()
     return _HOST or None
+
+
+def _load_host():
+    if not (HOST_PATH.exists() and LIB_PATH.exists()):
+        return False
+    try:
+        return importlib.import_module("._tpf_host", __package__)
+    except ImportError as e:
+        warnings.warn(f"TurboPairFormer host extension {HOST_PATH.name} not loaded ({e}); calls "
+                      "take the slower Python host path until it is built again "
+                      "(`python -m openfold3_triangle_kernel_amd.build`)", RuntimeWarning,
+                      stacklevel=2)
+        return False
 
 
 def host_eligible(*tensors) -> bool:

@@ -10,12 +10,14 @@
 // dimensions that need padding, partially broadcast biases, misaligned
 // storage, function transforms, forward-mode AD, dispatch modes.
 #include <torch/extension.h>
+#include <torch/version.h>
 
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
+#include <cctype>
 #include <cmath>
 #include <cstdlib>
 #include <optional>
@@ -355,7 +357,21 @@ std::optional<Tensor> trimul(const Tensor& z, const std::optional<Tensor>& mask_
 
 }  // namespace
 
+// Refuses the import beside another torch or C-ABI library than it was built
+// with: both are called through their headers of that time.
+void check_versions() {
+  const auto torch = pybind11::module_::import("torch").attr("__version__").cast<std::string>();
+  const std::string built = TORCH_VERSION;
+  if (torch.compare(0, built.size(), built) != 0 ||
+      (torch.size() > built.size() && std::isdigit((unsigned char)torch[built.size()])))
+    throw pybind11::import_error("built for torch " + built + ", found " + torch);
+  if (tpf_abi_version() != TPF_ABI_VERSION)
+    throw pybind11::import_error("built for library ABI " + std::to_string(TPF_ABI_VERSION) +
+                                 ", found " + std::to_string(tpf_abi_version()));
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  check_versions();
   m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& res_mask,
                         const Tensor& pair_bias) {
     const std::string backward = env_flag("TURBOPAIRFORMER_SR_BACKWARD", "OPENFOLD3_SR_BACKWARD");

@@ -318,3 +318,30 @@ def test_host_path_leaves_torch_function_modes_to_python(gpu):
         with torch.device(gpu):
             assert _native.host_eligible(q)
             assert torch.equal(call(), want)
+
+
+@pytest.mark.parametrize("version,loads", [(None, True), ("1.13.0", False), ("{0}1", False),
+                                           ("{0}+other", True)])
+def test_host_extension_declines_another_torch(version, loads):
+    """Beside another torch than it was built for the extension is reported
+    and left out, and the Python path serves the operators; the budget call
+    that forwards to it works either way."""
+    import subprocess
+    import sys
+
+    code = f"""
+import warnings, torch
+version = {version!r}
+if version:
+    torch.__version__ = version.format(torch.__version__.split('+')[0])
+warnings.simplefilter("always")
+with warnings.catch_warnings(record=True) as seen:
+    from openfold3_triangle_kernel_amd import _native, attention
+    hosts = [_native.host(), _native.host()]
+    attention.set_sr_workspace_budget(1 << 30)
+msgs = [w for w in seen if "host extension" in str(w.message)]
+assert [h is not None for h in hosts] == [{loads}] * 2 and len(msgs) == {int(not loads)}, (hosts, msgs)
+assert _native.query("tpf_abi_version") > 0
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
