@@ -116,14 +116,15 @@ int tpf_attn_delta_shadow_bf16(const void* dout, const void* out, const void* re
 /* Bytes of device workspace of the one-slab backward plan (dQ partials of
  * every outer row, one f32 dBias partial per run of outer groups, the
  * prescaled bias and the row statistics).  tpf_attn_backward_main_bf16 /
- * _finish_bf16 need this much.  D > 32: the plan keeps room for a dQ partial
- * per 64 keys, of which the kernels use one (main / finish) or none. */
+ * _finish_bf16 need this much.  D > 32: one dQ partial, which only these two
+ * use. */
 int64_t tpf_attn_backward_workspace_bytes(int64_t B, int64_t O, int64_t H, int64_t N,
                                           int64_t D);
 
 /* Workspace bytes of the backward plan under a budget: the full plan when it
  * fits, otherwise slabs of consecutive runs of outer rows whose dQ partials
- * fit (each slab's dQ folded before the next reuses the space; dBias partials
+ * fit (each slab's dQ folded before the next reuses the space; none for D > 32,
+ * whose workspace is the same for every budget; dBias partials
  * stay resident, so every summation order, and every result bit, is that of
  * the full plan).  Below the one-run minimum the minimum is returned (it
  * exceeds the budget), as the reference's planner returns its irreducible

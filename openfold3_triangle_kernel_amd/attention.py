@@ -191,14 +191,15 @@ def _storage_order(t: torch.Tensor) -> str | None:
 
 # Workspace budget of the backward (bytes).  The reference plans its SR
 # backward under a budget too (turbopairformer_triangle_dq_dbias.py:35,
-# 150-300); here the budget bounds the dQ partials, the only part of the
-# workspace that grows with O * N^2 * H * D / 64: when the full plan exceeds
-# it, the reconstruction kernel runs over slabs of outer rows, each slab's dQ
-# partials folded before the next slab reuses the space.  Results are
-# bitwise equal for every budget.  The default (8 GiB of the MI355X's 288 GB)
-# holds config-5 sized problems (N = 768, H = 8, D = 64: a 7.46 GB plan) in
-# one slab; larger problems run in slabs (each slab adds a partly filled
-# round of workgroups: two slabs at that size cost about 13 %).
+# 150-300); here the budget bounds the dQ partials of head dimensions up to
+# 32, the only part of the workspace that grows with O * N^2 * H * D / 128:
+# when the full plan exceeds it, the reconstruction kernel runs over slabs of
+# outer rows, each slab's dQ partials folded before the next slab reuses the
+# space.  Results are bitwise equal for every budget.  The default (8 GiB of
+# the MI355X's 288 GB) holds N = 768, H = 8, D = 32 (2.2 GB) in one slab; larger
+# problems run in slabs, each of which adds a partly filled round of
+# workgroups.  Above D = 32 dQ leaves no partials and every problem is one slab
+# (0.21 GB at N = 768, H = 8, D = 64).
 DEFAULT_SR_WORKSPACE_BUDGET_BYTES = 8 << 30
 _SR_WORKSPACE_BUDGET = DEFAULT_SR_WORKSPACE_BUDGET_BYTES
 

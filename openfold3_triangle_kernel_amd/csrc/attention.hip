@@ -733,12 +733,16 @@ struct BwdSlab {
   int brun0, nbrun;
   int64_t plane0, planes;
 };
-// Backward blocks per head and run: 128 keys for D <= 32 (one dQ partial
-// each), 64 keys or queries for D > 32 (whose workspace plan keeps room for a
-// partial per block: callers budget by it; the staged route uses one).
+// Backward blocks per head and run: 128 keys for D <= 32, 64 keys or queries
+// for D > 32.
 static inline int64_t bwd_key_blocks(int64_t N, int64_t D) {
   const int64_t kw = D <= 32 ? 128 : 64;
   return (N + kw - 1) / kw;
+}
+// dQ partials of a plane: one per key block for D <= 32.  For D > 32 dQ is
+// summed in registers: none, or one where the second stage stores it.
+static inline int64_t bwd_dq_partials(int64_t N, int64_t D) {
+  return D > 32 ? 1 : bwd_key_blocks(N, D);
 }
 
 // Q / dO tile of 32 rows x DP bf16 stored unpadded, 16-byte chunks permuted
@@ -2261,10 +2265,12 @@ static int64_t bwd_runs(int64_t O, int run) {
   return ((O + kBwdGroup - 1) / kBwdGroup + run - 1) / run;
 }
 
-// Backward workspace: bf16 dQ partials [key blocks][slab planes][H,NP,D] |
+// Backward workspace: bf16 dQ partials [bwd_dq_partials][dq_planes][H,NP,D] |
 // f32 dBias partials [B * runs][H,NP,NP] (one per run of outer groups) | f32
 // fragment-major bias [<=B][H,NP,NP] | f32 row statistics nl2, nd [B,O,H,NP];
-// each region 256-byte aligned.  Only the dQ partials depend on the slab.
+// each region 256-byte aligned.  dq_planes: the largest slab's for D <= 32;
+// for D > 32 none, or all in the staged entries (at N = O = 768, H = 8, D = 64
+// 0.21 GB and 0.81 GB; a partial per 64 keys took 7.46 GB).
 struct BwdParts {
   __bf16* dq;
   float* db;
@@ -2276,12 +2282,12 @@ struct BwdParts {
 static int64_t a256(int64_t v) { return (v + 255) / 256 * 256; }
 
 static int64_t bwd_layout(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D,
-                          int64_t slab_planes, char* base, BwdParts* parts) {
+                          int64_t dq_planes, char* base, BwdParts* parts) {
   const int64_t runs = bwd_runs(O, bwd_run_len(B, O, H, N, D));
   const int64_t NP = pad64(N), rows = B * O * H * NP;
   int64_t off = 0;
   auto take = [&](int64_t bytes) { char* p = base ? base + off : nullptr; off += a256(bytes); return p; };
-  char* dq = take(bwd_key_blocks(N, D) * slab_planes * H * NP * D * 2);
+  char* dq = take(bwd_dq_partials(N, D) * dq_planes * H * NP * D * 2);
   char* db = take(B * runs * H * NP * NP * 4);
   char* bf = take(B * H * NP * NP * 4);
   char* nl = take(rows * 4);
@@ -2292,15 +2298,21 @@ static int64_t bwd_layout(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D,
   }
   return off;
 }
-static int64_t bwd_full_bytes(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D) {
+// One slab with every plane's dQ partials: what the staged entries need.
+static int64_t bwd_staged_bytes(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D) {
   return bwd_layout(B, O, H, N, D, B * O, nullptr, nullptr);
+}
+// One slab of the other entries.
+static int64_t bwd_full_bytes(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D) {
+  return bwd_layout(B, O, H, N, D, D > 32 ? 0 : B * O, nullptr, nullptr);
 }
 
 // Slab plan for a workspace of `bytes`: every slab holds `per` consecutive
 // flattened runs (the last one fewer), sized evenly so the slabs' grids
 // are alike.  One slab when the full plan fits; per = 0 when not even one
 // run's dQ partials fit.  Slabs change where the dQ partials live, not any
-// summation order: results are bitwise equal to the one-slab plan.
+// summation order: results are bitwise equal to the one-slab plan.  D > 32
+// has no partials to divide: one slab.
 struct BwdPlan {
   int run;       // outer groups per run
   int runs;      // runs per batch
@@ -2321,6 +2333,7 @@ static BwdPlan bwd_plan(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D, i
     p.slabs = 1;
     return p;
   }
+  if (D > 32) { p.per = 0; p.slabs = 0; return p; }
   int lo = 0, hi = fr;  // largest per whose layout fits
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
@@ -2343,6 +2356,10 @@ static BwdPlan bwd_plan(int64_t B, int64_t O, int64_t H, int64_t N, int64_t D, i
   }
   return p;
 }
+// dQ planes of the workspace of a plan (bwd_layout).
+static int64_t bwd_dq_planes(int64_t B, int64_t O, int64_t D, const BwdPlan& p) {
+  return D > 32 ? 0 : bwd_slab_planes(B, O, p.per, p.run);
+}
 // Slab s of a plan: its flattened runs and the contiguous planes they cover.
 static BwdSlab bwd_slab(const BwdPlan& p, int64_t B, int64_t O, int s) {
   BwdSlab sl;
@@ -2364,10 +2381,10 @@ static BwdSlab bwd_slab(const BwdPlan& p, int64_t B, int64_t O, int s) {
 static int attn_backward_rows_impl(const AttnGeom& g, const void* dout, const void* out,
                                    const void* res, const float* lse, const void* bias,
                                    const BiasView& bv, int64_t bias_batches, void* workspace,
-                                   int64_t slab_planes, hipStream_t s, const char* fn) {
+                                   int64_t dq_planes, hipStream_t s, const char* fn) {
   const int64_t B = g.B, O = g.O, H = g.H, N = g.N, D = g.D;
   BwdParts pt;
-  bwd_layout(B, O, H, N, D, slab_planes, (char*)workspace, &pt);
+  bwd_layout(B, O, H, N, D, dq_planes, (char*)workspace, &pt);
   const int64_t items = B * O * N * H * (D / 8);
   const int per = 256 - 256 % (int)(D / 8);
   const int64_t delta_blocks = (items + per - 1) / per;
@@ -2455,9 +2472,6 @@ static int attn_backward_slab_impl(const AttnGeom& g, const void* q, const void*
 // Folds of one slab: its planes' dQ (with_dq; D > 32 leaves one partial), and
 // (with_dbias, after the last slab) every dBias partial.  db_mode: 0 = f32 dBias, 1 = bf16, 2 = bf16 in
 // transposed-bias order.
-static inline int bwd_dq_partials(int64_t N, int64_t D) {
-  return D > 32 ? 1 : (int)bwd_key_blocks(N, D);
-}
 static int attn_backward_fold_impl(const AttnGeom& g, void* dq, void* dbias,
                                    int64_t bias_batches, const BwdParts& pt, const BwdPlan& plan,
                                    const BwdSlab& sl, bool with_dq, bool with_dbias,
@@ -2475,7 +2489,7 @@ static int attn_backward_fold_impl(const AttnGeom& g, void* dq, void* dbias,
     return set_error(TPF_ERR_ARG, "%s: fold grid too large", fn);
   if (n_db + dq_bx * nph == 0) return TPF_OK;
   hipLaunchKernelGGL(attn_fold_kernel, dim3((unsigned)(n_db + dq_bx * nph)), dim3(256), 0, s,
-                     pt.dq, (__bf16*)dq, g, bwd_dq_partials(N, D), (int)dq_bx, pt.db, dbias,
+                     pt.dq, (__bf16*)dq, g, (int)bwd_dq_partials(N, D), (int)dq_bx, pt.db, dbias,
                      (int)bias_batches, plan.runs, n_db, db_mode, sl.plane0, sl.planes);
   return check_launch(fn);
 }
@@ -2632,14 +2646,14 @@ int tpf_attn_delta_shadow_bf16(const void* dout, const void* out, const void* re
 
 int64_t tpf_attn_backward_workspace_bytes(int64_t B, int64_t O, int64_t H, int64_t N,
                                           int64_t D) {
-  return bwd_full_bytes(B, O, H, N, D);
+  return bwd_staged_bytes(B, O, H, N, D);
 }
 
 int64_t tpf_attn_backward_workspace_bytes_budget(int64_t B, int64_t O, int64_t H, int64_t N,
                                                  int64_t D, int64_t budget_bytes) {
   if (B < 1 || O < 1 || H < 1 || N < 1 || D < 1) return -1;
   const int64_t full = bwd_full_bytes(B, O, H, N, D);
-  if (budget_bytes >= full) return full;
+  if (budget_bytes >= full || D > 32) return full;
   BwdPlan p = bwd_plan(B, O, H, N, D, budget_bytes);
   // Below the one-run minimum the minimum is returned (it exceeds the budget).
   const int per = p.per > 0 ? p.per : 1;
@@ -2665,7 +2679,7 @@ static int attn_bwd_prepare(AttnGeom* g, BwdPlan* plan, const char* fn, const vo
   if (rc) return rc;
   if (!q || !k || !v || !dout || !lse || !delta || !mask || !bias || !workspace)
     return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
-  const int64_t need = full_only ? bwd_full_bytes(B, O, H, N, D)
+  const int64_t need = full_only ? bwd_staged_bytes(B, O, H, N, D)
                                  : tpf_attn_backward_workspace_bytes_budget(B, O, H, N, D, 0);
   if (workspace_bytes < need)
     return set_error(TPF_ERR_ARG, "%s: workspace %lld < required %lld", fn,
@@ -2724,8 +2738,8 @@ static int attn_backward_slabs(const AttnGeom& g, const BwdPlan& plan, const voi
                                void* dq, void* dk, void* dv, void* dbias, int64_t bias_batches,
                                const BwdParts& pt, hipStream_t s, const char* fn, int db_mode,
                                int mode = kBwdSR) {
-  if (g.D > 32) {  // dQ leaves no partials: every run at once
-    const BwdSlab all{0, g.B * plan.runs, 0, (int64_t)g.B * g.O};
+  if (g.D > 32) {  // dQ leaves no partials: one slab
+    const BwdSlab all = bwd_slab(plan, g.B, g.O, 0);
     int rc = attn_backward_slab_impl(g, q, k, v, dout, mask, dk, dv, pt, plan, all, dq, s, fn, mode);
     if (rc) return rc;
     return attn_backward_fold_impl(g, dq, dbias, bias_batches, pt, plan, all, false, true, s, fn,
@@ -2758,7 +2772,7 @@ int tpf_attn_backward_bf16(const void* q, const void* k, const void* v, const vo
   if (!dq || !dk || !dv || !dbias) return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   hipStream_t s = (hipStream_t)stream;
   BwdParts pt;
-  bwd_layout(B, O, H, N, D, bwd_slab_planes(B, O, plan.per, plan.run), (char*)workspace, &pt);
+  bwd_layout(B, O, H, N, D, bwd_dq_planes(B, O, D, plan), (char*)workspace, &pt);
   if ((rc = attn_backward_prep_impl(g, lse, delta, bias, dense_bias(H, N, bias_batches, layout),
                                     bias_batches, pt, s, fn)))
     return rc;
@@ -2786,12 +2800,12 @@ int tpf_attn_backward_fused_bf16(const void* q, const void* k, const void* v, co
   if (!out || !dq || !dk || !dv || !dbias) return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   const BiasView bv = dense_bias(H, N, bias_batches, layout);
   hipStream_t s = (hipStream_t)stream;
-  const int64_t slab_planes = bwd_slab_planes(B, O, plan.per, plan.run);
+  const int64_t dq_planes = bwd_dq_planes(B, O, D, plan);
   rc = attn_backward_rows_impl(g, dout, out, residual, lse, bias, bv, bias_batches, workspace,
-                               slab_planes, s, fn);
+                               dq_planes, s, fn);
   if (rc) return rc;
   BwdParts pt;
-  bwd_layout(B, O, H, N, D, slab_planes, (char*)workspace, &pt);
+  bwd_layout(B, O, H, N, D, dq_planes, (char*)workspace, &pt);
   const int db_mode = !(layout & TPF_DBIAS_BF16) ? 0 : (layout & TPF_BIAS_TRANSPOSED) ? 2 : 1;
   return attn_backward_slabs(g, plan, q, k, v, dout, mask, dq, dk, dv, dbias, bias_batches, pt, s,
                              fn, db_mode);
@@ -2896,7 +2910,7 @@ int tpf_attn_dq_dbias_bf16(const void* q, const void* k, const void* v, const vo
   if (!dq || !dbias) return set_error(TPF_ERR_ARG, "%s: null pointer", fn);
   hipStream_t s = (hipStream_t)stream;
   BwdParts pt;
-  bwd_layout(B, O, H, N, D, bwd_slab_planes(B, O, plan.per, plan.run), (char*)workspace, &pt);
+  bwd_layout(B, O, H, N, D, bwd_dq_planes(B, O, D, plan), (char*)workspace, &pt);
   if ((rc = attn_backward_prep_impl(g, lse, delta, bias, dense_bias(H, N, bias_batches, layout),
                                     bias_batches, pt, s, fn)))
     return rc;
@@ -3081,8 +3095,8 @@ static int pair_backward_impl(const void* qkv, const void* rest, int64_t rest_pi
                        dp + 3 * hc, dproj_pitch, items, per, fN, (int)H, (int)D, fhc8, g.og_t);
   if (d_og && (rc = check_launch(fn))) return rc;
   BwdParts pt;
-  bwd_layout(B, N, H, N, D, B * N, (char*)workspace, &pt);
   const BwdPlan plan = bwd_plan(B, N, H, N, D, INT64_MAX);
+  bwd_layout(B, N, H, N, D, bwd_dq_planes(B, N, D, plan), (char*)workspace, &pt);
   if ((rc = attn_backward_prep_impl(g, lse, delta, r + hc, bv, B, pt, s, fn))) return rc;
   if ((rc = attn_backward_slab_impl(g, q, q + part, q + 2 * part, d_o, mask, dp + hc, dp + 2 * hc,
                                     pt, plan, bwd_slab(plan, B, N, 0), dp, s, fn)))

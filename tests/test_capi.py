@@ -131,12 +131,12 @@ def test_workspace_sizes(lib):
 
 
 def test_backward_workspace_budget_plan(lib):
-    """The budgeted plan: the full plan when it fits, otherwise slabs whose
+    """The budgeted plan (D <= 32): the full plan when it fits, otherwise slabs whose
     workspace stays within the budget, down to a one-run minimum that is
     returned (and exceeds the budget) for budgets below it."""
     from openfold3_triangle_kernel_amd import _native
 
-    for shape in ((1, 384, 4, 384, 32), (1, 768, 8, 768, 64), (2, 130, 4, 128, 32)):
+    for shape in ((1, 384, 4, 384, 32), (1, 768, 8, 768, 32), (2, 130, 4, 128, 32)):
         full = _native.query("tpf_attn_backward_workspace_bytes", *shape)
         assert _native.query("tpf_attn_backward_workspace_bytes_budget", *shape, full) == full
         assert _native.query("tpf_attn_backward_slab_count", *shape, full) == 1
@@ -151,10 +151,30 @@ def test_backward_workspace_budget_plan(lib):
             slabs = _native.query("tpf_attn_backward_slab_count", *shape, ws)
             assert slabs >= last  # fewer bytes never means fewer slabs
             last = slabs
-    # Config 5's H=8, D=64 attention needs 7.46 GB in one slab; 4 GiB gives two.
-    ws = _native.query("tpf_attn_backward_workspace_bytes_budget", 1, 768, 8, 768, 64, 4 << 30)
-    assert ws <= 4 << 30
-    assert _native.query("tpf_attn_backward_slab_count", 1, 768, 8, 768, 64, ws) == 2
+    # N = 768, H = 8, D = 32 needs 2.17 GB in one slab; 1.5 GiB gives two.
+    shape = (1, 768, 8, 768, 32)
+    ws = _native.query("tpf_attn_backward_workspace_bytes_budget", *shape, 3 << 29)
+    assert ws <= 3 << 29
+    assert _native.query("tpf_attn_backward_slab_count", *shape, ws) == 2
+
+
+def test_backward_workspace_of_wide_heads(lib):
+    """D > 32 sums dQ in registers: one slab under every budget, in a
+    workspace without dQ partials (7.25 of 7.46 GB at N = 768, H = 8, D = 64 when
+    it held one per 64 keys); the staged entries add one partial."""
+    from openfold3_triangle_kernel_amd import _native
+
+    for B, O, H, N, D in ((1, 768, 8, 768, 64), (2, 130, 4, 100, 40), (1, 5, 1, 1, 64)):
+        shape, NP = (B, O, H, N, D), (N + 63) // 64 * 64
+        full = _native.query("tpf_attn_backward_workspace_bytes_budget", *shape, 1 << 62)
+        for budget in (1, full - 1, full, 8 << 30):
+            assert _native.query("tpf_attn_backward_workspace_bytes_budget", *shape, budget) == full
+        assert _native.query("tpf_attn_backward_slab_count", *shape, full) == 1
+        assert _native.query("tpf_attn_backward_slab_count", *shape, full - 1) == 0
+        assert _native.query("tpf_attn_dq_dbias_workspace_bytes", *shape) == full
+        partial = (B * O * H * NP * D * 2 + 255) // 256 * 256
+        assert _native.query("tpf_attn_backward_workspace_bytes", *shape) == full + partial
+    assert _native.query("tpf_attn_backward_workspace_bytes_budget", 1, 768, 8, 768, 64, 1) < 1 << 28
 
 
 def test_pair_backward_dout_instances(lib):
