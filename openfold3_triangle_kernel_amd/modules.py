@@ -45,7 +45,7 @@ from torch import nn
 from . import _native, routing
 from .attention import (
     _device_ctx,
-    _device_supported,
+    _is_gfx950,
     is_turbopairformer_supported,
     shadow_enabled,
     turbopairformer_triangle_attention,
@@ -173,11 +173,10 @@ def _pair_rows_projection(x2: torch.Tensor, wa: torch.Tensor, B: int, O: int, N:
 def _mask_rows(mask_bias: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """The additive mask [*, I, 1, 1, J] of pairs x [*, I, J, C] as [B, I, J],
     a broadcast one (over the batch or a pair axis) written out."""
-    I, J = x.shape[-3:-1]
-    full = x.shape[:-2] + (1, 1, J)
-    if mask_bias.numel() != math.prod(full):
-        mask_bias = mask_bias.expand(full)
-    return mask_bias.reshape(-1, I, J)
+    shape = x.shape
+    if mask_bias.numel() * shape[-1] != x.numel():
+        mask_bias = mask_bias.expand(shape[:-2] + (1, 1, shape[-2]))
+    return mask_bias.reshape(-1, shape[-3], shape[-2])
 
 
 def _pair_flags(transpose_bias: bool, og_t: bool) -> int:
@@ -480,7 +479,7 @@ class TriangleAttention(nn.Module):
         mask_bias = (self.inf * (mask.float() - 1))[..., :, None, None, :]
         m = self.mha
         H, c = m.no_heads, m.c_hidden
-        if self._pair_inference(x, mask_bias, chunk_size):
+        if self._pair_inference(x, mask, chunk_size):
             return self._pair_inference_forward(x, mask_bias, transpose_bias, chunk_size)
         if chunk_size is not None and chunk_size < x.shape[-3]:
             return self._chunked_forward(x, mask_bias, transpose_bias, chunk_size)
@@ -528,27 +527,28 @@ class TriangleAttention(nn.Module):
         g = torch.sigmoid(gp).reshape(o.shape)
         return _linear((o * g).flatten(-2), m.linear_o.weight)
 
-    def _pair_inference(self, x, mask_bias, chunk_size) -> bool:
+    def _pair_inference(self, x, mask, chunk_size) -> bool:
         """Whether inference runs the pair-row core: BF16 square pairs on the
         kernels' device without gradients, a mask that broadcasts to them, and
         the limits of the per-projection route's support verdict.  Every N: at N = 613, C = 128
         the per-projection route, with its gate and layout passes in torch,
         takes 821 us and the core 534."""
-        H, c, N = self.mha.no_heads, self.mha.c_hidden, x.shape[-2]
-        if not (x.dtype == torch.bfloat16 and x.is_cuda and x.shape[-3] == N and x.numel() > 0
-                and c % 8 == 0 and 8 <= c <= 64 and H <= 16 and self.c_in % 8 == 0
-                and math.prod(x.shape[:-2]) <= 65_535 and N <= 8192):
+        m, shape = self.mha, x.shape
+        c, N = m.c_hidden, shape[-2]
+        if not (x.dtype == torch.bfloat16 and x.is_cuda and shape[-3] == N and x.numel() > 0
+                and c % 8 == 0 and 8 <= c <= 64 and m.no_heads <= 16 and shape[-1] % 8 == 0
+                and x.numel() // (N * shape[-1]) <= 65_535 and N <= 8192):
             return False
-        if x.dim() < 4 and (N % 64 or chunk_size is not None):
+        if len(shape) < 4 and (N % 64 or chunk_size is not None):
             return False
-        if mask_bias.dim() > x.dim() + 1 or any(
-                m not in (1, t) for m, t in zip(mask_bias.shape[-4::-1], x.shape[-3::-1])) \
-                or mask_bias.shape[-1] not in (1, N):
+        pairs = shape[:-1]
+        if mask.shape != pairs and (mask.dim() > len(pairs) or any(
+                k not in (1, p) for k, p in zip(reversed(mask.shape), reversed(pairs)))):
             return False
         if torch.is_grad_enabled() and (x.requires_grad or any(
                 p.requires_grad for p in self.parameters())):
             return False
-        return _device_supported(x)[0]
+        return _is_gfx950(x.device)
 
     def _pair_inference_forward(self, x, mask_bias, transpose_bias, chunk_size):
         """The pair-row core over all outer rows, or over chunks of them with
@@ -559,18 +559,15 @@ class TriangleAttention(nn.Module):
         runs outer rows 2 i and 2 i + 1 together and raises both running maxima
         at once, so chunks hold whole pairs (an odd ``chunk_size`` is taken one
         smaller, 1 as 2)."""
-        m = self.mha
-        H, c, N, C = m.no_heads, m.c_hidden, x.shape[-2], self.c_in
+        m, w_z = self.mha, self.linear_z.weight
+        H, c, N, C = m.no_heads, m.c_hidden, x.shape[-2], x.shape[-1]
         shadow_enabled()  # the policy variables are checked as in training
         if N % 64:
             validate_attention_policy()
-        B = math.prod(x.shape[:-3])
         pad = (-(4 * H * c + H)) % 64  # 128-byte aligned rows, as in training
-        zeros = self.linear_z.weight.new_zeros
         w_all = torch.cat([m.linear_q.weight, m.linear_k.weight, m.linear_v.weight,
-                           m.linear_g.weight, self.linear_z.weight]
-                          + ([zeros(pad, C)] if pad else []))
-        x4, mask_add = x.reshape(B, N, N, C), _mask_rows(mask_bias, x)
+                           m.linear_g.weight, w_z] + ([w_z.new_zeros(pad, C)] if pad else []))
+        x4, mask_add = x.reshape(-1, N, N, C), _mask_rows(mask_bias, x)
         og_t = not self.starting
         if chunk_size is None or chunk_size >= N:
             out = _PairAttentionInference.apply(x4, w_all, m.linear_o.weight, mask_add.contiguous(),
@@ -579,7 +576,7 @@ class TriangleAttention(nn.Module):
             return out.transpose(-2, -3) if og_t else out
         # 16 output channels: the row kernel's tile, so a bias value has the
         # bits it has among the other projections.
-        w_z = torch.cat([self.linear_z.weight, zeros((-H) % 16, C)]).to(torch.bfloat16)
+        w_z = torch.cat([w_z, w_z.new_zeros((-H) % 16, C)]).to(torch.bfloat16)
         bias_rows = _mm(x4.reshape(-1, C), w_z, True)
         out = torch.empty_like(x4)
         pair = 2 if c <= 32 else 1
