@@ -271,7 +271,9 @@ class _PairAttentionInference(torch.autograd.Function):
     outer rows: x [B, O, N, C] holds O outer rows of the pair grid (all of
     them, or a chunk) and ``bias_rows`` ([B*N*N, pitch], the H pair-bias values
     first) the bias of every pair; None takes it from x's own projection
-    (O == N).  The same kernels and rounding as the training core."""
+    (O == N).  The same kernels and rounding as the training core.  A Function
+    all the same, so that forward-mode AD and function transforms, which the
+    native calls would hide, are refused as the training core refuses them."""
 
     @staticmethod
     def forward(ctx, x, w_all, w_o, mask_add, bias_rows, H, D, transpose_bias, og_t):
@@ -326,7 +328,8 @@ class _ProjLinear(torch.autograd.Function):
 
 def _mm_f32(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """``a [R, K] @ b.t()`` for FP32 ``b [N, K]`` on the FP32 MFMA GEMM
-    (``tpf_gemm_f32``, strict FP32: no TF32-style rounding)."""
+    (``tpf_gemm_f32``: products within half a unit in the last place of the
+    FP32 ones, no TF32-style rounding)."""
     a = a.contiguous()
     b = b.contiguous()
     R, K = a.shape
