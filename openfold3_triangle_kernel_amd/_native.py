@@ -205,12 +205,12 @@ def _load_host():
 
 
 def host_eligible(*tensors) -> bool:
-    """Plain tensors (or parameters, or None) in eager code: no subclass, no
+    """Plain tensors (or parameters) in eager code: nothing else, no subclass, no
     compilation, no tracing, no TorchFunctionMode that wants to see the torch
     calls (torch's own default-device mode acts on factories without a device,
     which neither path uses).  The extension checks the rest."""
     for t in tensors:
-        if t is not None and type(t) not in _PLAIN_TYPES:
+        if type(t) not in _PLAIN_TYPES:
             return False
     if torch.compiler.is_compiling() or torch._C._is_tracing():
         return False

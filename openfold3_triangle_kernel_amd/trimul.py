@@ -526,7 +526,7 @@ def turbo_trimul(
         raise ValueError(f"direction must be 'outgoing' or 'incoming', got {direction!r}")
     given = (p_in_weight, g_in_weight, g_out_weight, p_out_weight, norm_in_weight, norm_in_bias,
              norm_out_weight, norm_out_bias)
-    if not any(t is None for t in given) and _native.host_eligible(z, mask, *given) and z.is_cuda:
+    if _native.host_eligible(z, z if mask is None else mask, *given) and z.is_cuda:
         # The common form entirely in C++; None (nothing launched) for any other.
         host = _native.host()
         out = None if host is None else host.trimul(z, mask, given, direction == "outgoing")

@@ -213,6 +213,20 @@ def test_unsupported_cases_raise_before_launch(fake, mutate, msg):
     assert fake.calls == []
 
 
+@pytest.mark.parametrize("name", ["q", "k", "v", "res_mask", "pair_bias"])
+def test_operand_that_is_no_tensor_raises_value_error(fake, name):
+    from openfold3_triangle_kernel_amd import _native, turbopairformer_triangle_attention
+
+    q, k, v, mask, bias, _ = attention_case(1, 2, 2, 64, 8, seed=1)
+    args = dict(q=q.bfloat16(), k=k.bfloat16(), v=v.bfloat16(), res_mask=mask,
+                pair_bias=bias.bfloat16())
+    args[name] = None
+    assert not _native.host_eligible(*args.values())  # the extension takes tensors only
+    with pytest.raises(ValueError, match="must be torch.Tensor instances"):
+        turbopairformer_triangle_attention(**args)
+    assert fake.calls == []
+
+
 def test_sr_backward_flag_zero_raises(fake, monkeypatch):
     from openfold3_triangle_kernel_amd import turbopairformer_triangle_attention
 
