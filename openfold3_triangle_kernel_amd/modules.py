@@ -495,7 +495,7 @@ class TriangleAttention(nn.Module):
         N = x.shape[-2]
         pair_core = (x.dtype == torch.bfloat16 and x.is_cuda and x.shape[-3] == N
                      and N % 64 == 0 and c % 8 == 0 and 8 <= c <= 64 and H <= 16
-                     and self.c_in % 8 == 0 and x.numel() > 0)
+                     and self.c_in % 8 == 0 and x.numel() > 0 and mask.device == x.device)
         pad = (-(4 * hc + H)) % (64 if pair_core else 8)
         w_all = torch.cat([m.linear_q.weight, m.linear_k.weight, m.linear_v.weight,
                            m.linear_g.weight, self.linear_z.weight]
@@ -532,7 +532,7 @@ class TriangleAttention(nn.Module):
 
     def _pair_inference(self, x, mask, chunk_size) -> bool:
         """Whether inference runs the pair-row core: BF16 square pairs on the
-        kernels' device without gradients, a mask that broadcasts to them, and
+        kernels' device without gradients, a mask there that broadcasts to them, and
         the limits of the per-projection route's support verdict.  Every N: at N = 613, C = 128
         the per-projection route, with its gate and layout passes in torch,
         takes 821 us and the core 534."""
@@ -545,7 +545,7 @@ class TriangleAttention(nn.Module):
         if len(shape) < 4 and (N % 64 or chunk_size is not None):
             return False
         pairs = shape[:-1]
-        if mask.shape != pairs and (mask.dim() > len(pairs) or any(
+        if mask.device != x.device or mask.shape != pairs and (mask.dim() > len(pairs) or any(
                 k not in (1, p) for k, p in zip(reversed(mask.shape), reversed(pairs)))):
             return False
         if torch.is_grad_enabled() and (x.requires_grad or any(

@@ -287,6 +287,31 @@ def test_triangle_attention_module_broadcast_mask(gpu, shape, starting, N, chunk
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,chunk", [(33, None), (33, 16), (64, None), (64, 16)])
+@pytest.mark.parametrize("train", [False, True])
+def test_triangle_attention_module_mask_on_another_device(gpu, monkeypatch, train, N, chunk):
+    """A mask in host memory is refused before any kernel sees its address
+    (strict mode: without it the stock math goes on, into torch's own error)."""
+    from openfold3_triangle_kernel_amd import TriangleAttention, modules, routing
+
+    m = TriangleAttention(128, 32, 4).to(gpu).bfloat16()
+    x, mask = torch.randn(1, N, N, 128, device=gpu).bfloat16(), torch.ones(1, N, N)
+    print(f"host mask N={N} chunk={chunk} train={train}", flush=True)
+    call = modules._native.call
+
+    def guarded(name, *args):
+        assert not name.startswith("tpf_attn") and "projection" not in name, name
+        return call(name, *args)
+
+    monkeypatch.setattr(modules._native, "call", guarded)
+    monkeypatch.setattr(routing, "_STRICT", True)
+    with torch.set_grad_enabled(train), pytest.raises(
+            (RuntimeError, ValueError), match="must share one device|inference-only"):
+        m(x, mask, chunk_size=chunk)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,N,C,D", [(1, 33, 128, 32), (2, 50, 64, 16), (1, 65, 128, 64)])
 def test_triangle_attention_module_odd_chunks(gpu, B, N, C, D):
     """Odd chunk sizes too give the bits of the whole call: the forward runs
