@@ -548,7 +548,7 @@ class TriangleAttention(nn.Module):
         if mask.device != x.device or mask.shape != pairs and (mask.dim() > len(pairs) or any(
                 k not in (1, p) for k, p in zip(reversed(mask.shape), reversed(pairs)))):
             return False
-        if torch.is_grad_enabled() and (x.requires_grad or any(
+        if torch.is_grad_enabled() and (x.requires_grad or mask.requires_grad or any(
                 p.requires_grad for p in self.parameters())):
             return False
         return _is_gfx950(x.device)

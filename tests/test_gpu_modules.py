@@ -287,6 +287,25 @@ def test_triangle_attention_module_broadcast_mask(gpu, shape, starting, N, chunk
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("chunk", [None, 16])
+def test_triangle_attention_module_mask_gradient_is_not_dropped(gpu, monkeypatch, chunk):
+    """A frozen module with a mask that wants a gradient does not answer from
+    the inference core, which would give it none: the kernels refuse it (and
+    without strict mode the stock math serves it)."""
+    from openfold3_triangle_kernel_amd import TriangleAttention, routing
+
+    m = TriangleAttention(128, 32, 4).to(gpu).bfloat16().requires_grad_(False)
+    x = torch.randn(1, 33, 33, 128, device=gpu).bfloat16()
+    mask = torch.ones(1, 33, 33, device=gpu, requires_grad=True)
+    print(f"mask gradient chunk={chunk}", flush=True)
+    monkeypatch.setattr(routing, "_STRICT", True)
+    with pytest.raises(RuntimeError, match="res_mask must not require gradients"):
+        m(x, mask, chunk_size=chunk)
+    with torch.no_grad():
+        assert torch.equal(m(x, mask, chunk_size=chunk), m(x, mask.detach(), chunk_size=chunk))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,chunk", [(33, None), (33, 16), (64, None), (64, 16)])
 @pytest.mark.parametrize("train", [False, True])
 def test_triangle_attention_module_mask_on_another_device(gpu, monkeypatch, train, N, chunk):
